@@ -1,7 +1,8 @@
-"""Builds ``libbam_hip.so`` (the HIP kernels + C ABI) for gfx950 with hipcc.
+"""Builds ``libbam_hip.so`` (the HIP kernels + C ABI) for gfx950 with hipcc, and ``_bam_host.so`` (the native host layer
+on top of it, a torch extension module) with the host compiler.
 
-The library has no dependency on torch or Python: plain ``hipcc -shared``.  It is built
-in-tree, next to this file, so that the very same binary is what tests, the smoke check
+The library has no dependency on torch or Python: plain ``hipcc -shared``.  Both are built
+in-tree, next to this file, so that the very same binaries are what tests, the smoke check
 and the benchmark load.
 """
 
@@ -16,6 +17,7 @@ from concurrent.futures import ThreadPoolExecutor
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libbam_hip.so")
+HOST_PATH = os.path.join(PKG_DIR, "_bam_host.so")
 # the longest compilations first: they are spread over the workers
 SOURCES = ["bwd_long.hip", "bwd_dkdv.hip", "bwd_dkdv_save.hip", "bwd_dq_saved.hip", "bwd_dq.hip", "fwd_long.hip", "fwd.hip", "tile_flags.hip", "decode.hip", "bam_abi.hip"]
 ARCH = "gfx950"
@@ -41,9 +43,43 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found: libbam_hip.so cannot be built")
 
 
+def _rocm_include() -> str:
+    return os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), "include")
+
+
+def _compile_host(objdir: str) -> str:
+    """host.cpp -> object file (it includes torch's headers, which takes longer than most kernel files)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(objdir, "host.o")
+    includes = [f"-I{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"])]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wno-attributes", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-I{_rocm_include()}", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           "-DTORCH_EXTENSION_NAME=_bam_host", *includes, "-c", os.path.join(CSRC, "host.cpp"), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{r.stderr}")
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    from torch.utils import cpp_extension
+
+    libs = [f"-L{p}" for p in cpp_extension.library_paths()]
+    tmp = HOST_PATH + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, f"-L{PKG_DIR}", "-lbam_hip", "-Wl,-rpath,$ORIGIN", *libs, "-lc10", "-lc10_hip",
+           "-ltorch", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link of the host layer failed:\n{r.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build_library(force: bool = True, verbose: bool = False) -> str:
-    """Compile every kernel file and link the shared library.  Returns its path."""
-    if not force and os.path.exists(LIB_PATH):
+    """Compile every kernel file and the host layer and link both.  Returns the path of the HIP library."""
+    if not force and os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH):
         return LIB_PATH
     hipcc = _hipcc()
     objdir = os.path.join(PKG_DIR, "build")
@@ -59,14 +95,17 @@ def build_library(force: bool = True, verbose: bool = False) -> str:
             sys.stderr.write(r.stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
+    with ThreadPoolExecutor(max_workers=min(len(SOURCES) + 1, os.cpu_count() or 4)) as ex:
+        host = ex.submit(_compile_host, objdir)
         objs = list(ex.map(compile_one, SOURCES))
+        host_obj = host.result()
     tmp = LIB_PATH + ".tmp"
     r = subprocess.run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs],
                        capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_host(host_obj)
     return LIB_PATH
 
 

@@ -204,6 +204,7 @@ void fill_sizes(bam::AttnParams& p, const MaskSource& m, int B, int Hq, int Hkv,
     p.num_n = (m.Sk + 31) / 32;
     p.num_kt = (m.Sk + 127) / 128;
     p.Sq_rounded = p.num_m * 128;
+    p.lse_sb = (int64_t)Hq * p.Sq_rounded;
     p.scale = scale;
 }
 
@@ -312,7 +313,7 @@ extern "C" {
 
 const char* bam_last_error(void) { return g_error; }
 
-int bam_abi_version(void) { return 10; }
+int bam_abi_version(void) { return 11; }
 
 int bam_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                    int64_t flags_stride_m, int B, int S, void* stream) {
@@ -417,7 +418,8 @@ int place_plan(const char* who, void* workspace, int64_t workspace_bytes, int B,
 }
 
 // second launch of every plan builder: numbers the (slice, 128-key tile) pairs that have work
-int number_pairs(const char* who, const bam_plan* plan, const PlanLayout& l, void* workspace, void* stream) {
+int number_pairs(const char* who, const bam_plan* plan, const PlanLayout& l, void* workspace, uint64_t* count_host,
+                 uint32_t count_tag, void* stream) {
     return launched(bam::launch_ds_entries(plan->fine, plan->fine_stride_b, plan->fine_stride_s, plan->B, plan->Sq, plan->Sk,
                                            const_cast<int*>(plan->ds_entry), plan->ds_entry_stride_b,
                                            const_cast<int*>(plan->ds_tile_base),
@@ -426,7 +428,8 @@ int number_pairs(const char* who, const bam_plan* plan, const PlanLayout& l, voi
                                            const_cast<int*>(plan->ds_tile_order), plan->order, plan->order_stride_b,
                                            (int*)((char*)workspace + l.group_count_off),
                                            const_cast<int*>(plan->group_order),
-                                           const_cast<int64_t*>(plan->row_workloads), (hipStream_t)stream),
+                                           const_cast<int64_t*>(plan->row_workloads), count_host, count_tag,
+                                           (hipStream_t)stream),
                     who);
 }
 }  // namespace
@@ -434,6 +437,13 @@ int number_pairs(const char* who, const bam_plan* plan, const PlanLayout& l, voi
 int bam_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                   int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
                   void* stream) {
+    return bam_tile_plan_counted(bf, bf_stride_b, flags, flags_stride_b, flags_stride_m, workspace, workspace_bytes, B, S, plan,
+                                 nullptr, 0, stream);
+}
+
+int bam_tile_plan_counted(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
+                          int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
+                          uint64_t* count_host, uint32_t count_tag, void* stream) {
     if (bf == nullptr || flags == nullptr || workspace == nullptr || plan == nullptr)
         return fail(BAM_ERR_INVALID_ARGUMENT, "bam_tile_plan: null pointer");
     if (B <= 0 || S <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_tile_plan: B and S must be positive");
@@ -446,7 +456,7 @@ int bam_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t
                                            l.fine_sb, l.fine_ss, (int*)(w + l.order_off), l.order_sb,
                                            (int*)(w + l.count_off), B, S, (hipStream_t)stream),
                      "bam_tile_plan"));
-    return number_pairs("bam_tile_plan", plan, l, workspace, stream);
+    return number_pairs("bam_tile_plan", plan, l, workspace, count_host, count_tag, stream);
 }
 
 int bam_tile_plan_static(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
@@ -479,6 +489,11 @@ int bam_tile_plan_static(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, 
 
 int bam_plan_indexed(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
                      void* stream) {
+    return bam_plan_indexed_counted(iv, workspace, workspace_bytes, B, plan, nullptr, 0, stream);
+}
+
+int bam_plan_indexed_counted(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
+                             uint64_t* count_host, uint32_t count_tag, void* stream) {
     MaskSource m;
     BAM_TRY(indexed_source(iv, m));
     if (B <= 0 || m.Sq <= 0 || m.Sk <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_plan_indexed: B, Sq and Sk must be positive");
@@ -490,11 +505,18 @@ int bam_plan_indexed(const bam_index_view* iv, void* workspace, int64_t workspac
                                               (uint8_t*)(w + l.fine_off), l.fine_sb, l.fine_ss, (int*)(w + l.order_off),
                                               l.order_sb, (int*)(w + l.count_off), B, (hipStream_t)stream),
                      "bam_plan_indexed"));
-    return number_pairs("bam_plan_indexed", plan, l, workspace, stream);
+    return number_pairs("bam_plan_indexed", plan, l, workspace, count_host, count_tag, stream);
 }
 
 int bam_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m, void* workspace,
                        int64_t workspace_bytes, int B, int Sq, int Sk, bam_plan* plan, void* stream) {
+    return bam_mask_tile_plan_counted(mask, flags, flags_stride_b, flags_stride_m, workspace, workspace_bytes, B, Sq, Sk, plan,
+                                      nullptr, 0, stream);
+}
+
+int bam_mask_tile_plan_counted(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m,
+                               void* workspace, int64_t workspace_bytes, int B, int Sq, int Sk, bam_plan* plan,
+                               uint64_t* count_host, uint32_t count_tag, void* stream) {
     if (mask == nullptr || flags == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_mask_tile_plan: null pointer");
     if (B <= 0 || Sq <= 0 || Sk <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_mask_tile_plan: B, Sq and Sk must be positive");
     if (B > 65535 || (Sq + 127) / 128 > 65535)
@@ -508,7 +530,7 @@ int bam_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stride_
                                                 (unsigned*)(w + l.col_off), l.col_sb, l.col_ss, B, Sq, Sk,
                                                 (hipStream_t)stream),
                      "bam_mask_tile_plan"));
-    return number_pairs("bam_mask_tile_plan", plan, l, workspace, stream);
+    return number_pairs("bam_mask_tile_plan", plan, l, workspace, count_host, count_tag, stream);
 }
 
 int64_t bam_ds_workspace_bytes(int Hq, int64_t pairs) {
@@ -687,6 +709,97 @@ int bam_bwd_dq_indexed(const void* q, const void* k, const void* v, const void* 
     BAM_TRY(bwd_params(p, "bam_bwd_dq_indexed", q, k, v, dout, lse, delta, dq, dk, dv, m, flags, st, B, Hq, Hkv, D, scale,
                        dtype, accumulate, true, false, bias, plan));
     return launched(launch_dq(p, dtype, stream), "bam_bwd_dq_indexed");
+}
+
+// ---- the struct form of the attention calls
+static int attn_source(const bam_attn* a, MaskSource& m) {
+    if (a->mode == BAM_MASK_INDEXED) return indexed_source(a->index, m);
+    if (a->mode == BAM_MASK_DENSE) {
+        BAM_TRY(check_mask("bam_attn", a->mask));
+        m = dense_source(a->mask, a->Sq, a->Sk);
+        return BAM_OK;
+    }
+    if (a->mode != BAM_MASK_BITFIELD) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn: unknown mode %d", a->mode);
+    if (a->Sq != a->Sk) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn: Sq and Sk must match in bitfield mode");
+    m = plain_source(a->bf, a->bf_stride_b, a->Sq);
+    return BAM_OK;
+}
+
+int bam_attn_fwd(const bam_attn* a, void* stream) {
+    if (a == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_fwd: null pointer");
+    MaskSource m;
+    BAM_TRY(attn_source(a, m));
+    const int64_t st[12] = {a->q.stride_b, a->q.stride_s, a->q.stride_h, a->k.stride_b, a->k.stride_s, a->k.stride_h,
+                            a->v.stride_b, a->v.stride_s, a->v.stride_h, a->o.stride_b, a->o.stride_s, a->o.stride_h};
+    return fwd_impl("bam_attn_fwd", a->q.ptr, a->k.ptr, a->v.ptr, a->o.ptr, a->lse, m, a->flags, st, a->flags_stride_b,
+                    a->flags_stride_m, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->bias, a->plan, stream);
+}
+
+int bam_attn_bwd(const bam_attn* a, void* stream) {
+    if (a == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: null pointer");
+    MaskSource m;
+    BAM_TRY(attn_source(a, m));
+    BAM_TRY(check_problem(a->B, m.Sq, m.Sk, a->Hq, a->Hkv, a->D, a->dtype));
+    BAM_TRY(check_half_tensor("o", a->o.ptr, a->o.stride_b, a->o.stride_s, a->o.stride_h));
+    BAM_TRY(check_half_tensor("do", a->dout.ptr, a->dout.stride_b, a->dout.stride_s, a->dout.stride_h));
+    const int runs = a->head_runs > 1 ? a->head_runs : 1;
+    if (a->Hkv % runs) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: %d runs do not divide %d kv heads", runs, a->Hkv);
+    if (runs > 1 && a->bias != nullptr)  // a bias is indexed by absolute head
+        return fail(BAM_ERR_UNSUPPORTED, "bam_attn_bwd: heads are not taken in runs with a bias");
+    bam_plan plan;
+    if (a->plan != nullptr) {
+        plan = *a->plan;
+        plan.ds_workspace = a->ds_workspace;
+        plan.ds_capacity = a->ds_capacity;
+    }
+    const int64_t st[23] = {a->q.stride_b,    a->q.stride_s,    a->q.stride_h,    a->k.stride_b,  a->k.stride_s,  a->k.stride_h,
+                            a->v.stride_b,    a->v.stride_s,    a->v.stride_h,    a->dout.stride_b, a->dout.stride_s,
+                            a->dout.stride_h, a->dq.stride_b,   a->dq.stride_s,   a->dq.stride_h, a->dk.stride_b, a->dk.stride_s,
+                            a->dk.stride_h,   a->dv.stride_b,   a->dv.stride_s,   a->dv.stride_h, a->flags_stride_b,
+                            a->flags_stride_m};
+    const int hq = a->Hq / runs, hk = a->Hkv / runs, gsz = a->accumulate ? 4 : 2;
+    bam::AttnParams all = {};
+    BAM_TRY(bwd_params(all, "bam_attn_bwd", a->q.ptr, a->k.ptr, a->v.ptr, a->dout.ptr, a->lse, a->delta, a->dq.ptr, a->dk.ptr,
+                       a->dv.ptr, m, a->flags, st, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->accumulate, true, true,
+                       a->bias, nullptr));
+    all.o = {a->o.ptr, a->o.stride_b, a->o.stride_s, a->o.stride_h};
+    BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
+    // The heads in runs of whole kv heads, every run through the same dS workspace: the launches of a stream run in
+    // order, so a run's dQ kernel has read the workspace before the next run's dK/dV kernel writes it.
+    for (int r = 0; r < runs; ++r) {
+        bam::AttnParams p = all;
+        auto skip = [&](bam::Tensor4& t, int heads, int bytes) { t.ptr = (const char*)t.ptr + (int64_t)r * heads * t.sh * bytes; };
+        skip(p.q, hq, 2);
+        skip(p.k, hk, 2);
+        skip(p.v, hk, 2);
+        skip(p.dout, hq, 2);
+        skip(p.dq, hq, gsz);
+        skip(p.dk, hk, gsz);
+        skip(p.dv, hk, gsz);
+        p.lse += (int64_t)r * hq * p.Sq_rounded;
+        p.delta += (int64_t)r * hq * p.Sq_rounded;
+        p.Hq = hq;
+        p.Hkv = hk;
+        if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
+        BAM_TRY(launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+        BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
+    }
+    return BAM_OK;
+}
+
+// ---- pinned host words the plan builders publish their pair counts to
+int bam_host_words_alloc(uint64_t** words, int n) {
+    if (words == nullptr || n <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_host_words_alloc: null pointer or no words");
+    void* p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, (size_t)n * 8, hipHostMallocPortable | hipHostMallocCoherent);
+    if (e != hipSuccess) return fail(BAM_ERR_LAUNCH, "bam_host_words_alloc: %s", hipGetErrorString(e));
+    for (int i = 0; i < n; ++i) ((uint64_t*)p)[i] = 0;
+    *words = (uint64_t*)p;
+    return BAM_OK;
+}
+int bam_host_words_free(uint64_t* words) {
+    const hipError_t e = words != nullptr ? hipHostFree(words) : hipSuccess;
+    return e == hipSuccess ? BAM_OK : fail(BAM_ERR_LAUNCH, "bam_host_words_free: %s", hipGetErrorString(e));
 }
 
 int64_t bam_decode_workspace_bytes(int B, int Sk, int Hq, int Hkv, int D, int window) {

@@ -85,6 +85,7 @@ struct AttnParams {
     int64_t col_bits_sb, col_bits_ss;
     int B, Sq, Sk, Hq, Hkv, D;
     int Sq_rounded, num_m, num_n, num_kt;  // ceil(Sq/128)*128, ceil(Sq/128), ceil(Sk/32), ceil(Sk/128)
+    int64_t lse_sb;            // batch stride of lse and delta (a run of heads is a view of the tensors of all heads)
     float scale;
 };
 
@@ -136,10 +137,11 @@ int launch_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stri
 // be null, and no order is written beyond MAX_RANKED tiles.  The same for the groups of four slices in the plan's slice
 // order (order, order_sb): group_count (B * num_m) scratch, group_order (B * num_m) = the groups by falling number of
 // 64-key tiles they visit.  row_workloads (num_m int64, or null): per 128-row block, the number of its 128 x 32 tiles
-// with an allowed pair, summed over the batch.
+// with an allowed pair, summed over the batch.  count_host (pinned host memory, or null): receives count_tag << 32 | count.
 int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int B, int Sq, int Sk, int* entry,
                       int64_t entry_sb, int* tile_base, int* count, int* tile_count, int* tile_order, const int* order,
-                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, hipStream_t stream);
+                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, uint64_t* count_host,
+                      uint32_t count_tag, hipStream_t stream);
 int launch_fwd(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_preprocess(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dkdv(const AttnParams& p, int dtype, hipStream_t stream);

@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const AttnParams p)
     }
 #pragma unroll
     for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-    if (valid && c == 0) p.delta[((int64_t)b * p.Hq + h) * p.Sq_rounded + i] = acc;
+    if (valid && c == 0) p.delta[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + i] = acc;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -220,8 +220,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         HeadBase hb;
         hb.q = (const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)h * p.q.sh);
         hb.g = (const char*)p.dout.ptr + 2 * ((int64_t)b * p.dout.sb + (int64_t)h * p.dout.sh);
-        hb.small = small == 0   ? (const char*)(p.lse + ((int64_t)b * p.Hq + h) * p.Sq_rounded)
-                   : small == 1 ? (const char*)(p.delta + ((int64_t)b * p.Hq + h) * p.Sq_rounded)
+        hb.small = small == 0   ? (const char*)(p.lse + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded)
+                   : small == 1 ? (const char*)(p.delta + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded)
                    : DENSE      ? (const char*)(p.col_bits + (int64_t)b * p.col_bits_sb + nt * 128 + (small - 2) * 64)
                                 : (const char*)bfrow;
         return hb;
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 stQ.load_ragged((const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)h * p.q.sh + (int64_t)row0 * p.q.ss), sQ[0], rows, tid);
                 stDO.load_ragged((const char*)p.dout.ptr + 2 * ((int64_t)b * p.dout.sb + (int64_t)h * p.dout.sh + (int64_t)row0 * p.dout.ss), sDO[0], rows, tid);
                 if (tid < DKDV_QT) {
-                    const int64_t off = ((int64_t)b * p.Hq + h) * p.Sq_rounded + row0;
+                    const int64_t off = (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + row0;
                     const bool ok = tid < rows;
                     sLse[0][tid] = ok ? p.lse[off + tid] : INFINITY;  // lse = +inf gives P = 0
                     sDelta[0][tid] = ok ? p.delta[off + tid] : 0.f;
@@ -733,7 +733,7 @@ __global__ __launch_bounds__(DQ_THREADS, D == 128 ? 2 : 3) void bwd_dq_kernel(co
     const int64_t qf = (!DENSE && qvalid) ? p.bfq[(int64_t)b * p.bfq_sb + qrow] : 0;
     float lse_row = 0.f, dlt = 0.f;
     if (qvalid) {
-        const int64_t off = ((int64_t)b * p.Hq + h) * p.Sq_rounded + qrow;
+        const int64_t off = (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow;
         lse_row = p.lse[off];
         dlt = p.delta[off];
     }

@@ -470,12 +470,12 @@ __global__ __launch_bounds__(FWD_THREADS, D == 128 ? 2 : 3) void fwd_kernel(cons
     const float ltot = half_swap_sum(l_i);
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
     if (hi == 0 && slice >= 0)
-        p.lse[((int64_t)b * p.Hq + h) * p.Sq_rounded + qrow] =
+        p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] =
             ltot > 0.f ? (m_i * c2 + __builtin_amdgcn_logf(ltot)) * LN2 : -INFINITY;
     // A wave without a slice (plan: slot 4 grp + wave of the order lies past the last slice) owns the 32 padding rows
     // of that slot, so that every row of the rounded lse is written whether or not a plan is given.
     if (hi == 0 && slice < 0 && 32 * (4 * grp + wave) + 31 < p.Sq_rounded)
-        p.lse[((int64_t)b * p.Hq + h) * p.Sq_rounded + 32 * (4 * grp + wave) + l32] = -INFINITY;
+        p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + 32 * (4 * grp + wave) + l32] = -INFINITY;
     if (qvalid) {
         char* op = (char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
 #pragma unroll

@@ -770,12 +770,19 @@ __global__ __launch_bounds__(DS_NUM_THREADS) void ds_entries_kernel(const uint8_
 // 64 tiles per workgroup, four threads per tile, each comparing against a quarter of all counts (staged in LDS).
 // blockIdx.y = 1 ranks a second, independent array the same way (the groups of four slices, for the forward and dQ
 // kernels); either array may be absent (n = 0).
+// count_host (optional): the number of pairs, under the caller's tag, goes straight to pinned host memory, where the host
+// polls for it; a copy on a side stream cost an event on either stream and 60-80 us of host time per plan, and its blit
+// kernel took up to 75 us when the forward had filled the chip before it.
 __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__ tile_count, int n_tiles,
                                                          int* __restrict__ tile_order,
                                                          const int* __restrict__ group_count, int n_groups,
-                                                         int* __restrict__ group_order) {
+                                                         int* __restrict__ group_order, const int* __restrict__ count,
+                                                         unsigned long long* __restrict__ count_host,
+                                                         unsigned long long count_tag) {
     __shared__ __attribute__((aligned(16))) int s_cnt[DS_MAX_ORDERED_TILES];
     const int tid = threadIdx.x;
+    if (count_host != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0)
+        __hip_atomic_store(count_host, count_tag | (unsigned)*count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (blockIdx.y == 1) {
         tile_count = group_count;
         n_tiles = n_groups;
@@ -804,7 +811,8 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__
 
 int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int B, int Sq, int Sk, int* entry,
                       int64_t entry_sb, int* tile_base, int* count, int* tile_count, int* tile_order, const int* order,
-                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, hipStream_t stream) {
+                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, uint64_t* count_host,
+                      uint32_t count_tag, hipStream_t stream) {
     const int num_m = (Sq + BLOCK_M - 1) / BLOCK_M;
     const int slots = 4 * num_m, nkt = (Sk + 127) / 128, num_n = (Sk + BLOCK_N - 1) / BLOCK_N;
     const int n_tiles = nkt * B, n_groups = num_m * B;
@@ -815,10 +823,11 @@ int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int
                        dim3(DS_NUM_THREADS), 0, stream, fine, fine_sb, fine_ss, slots, nkt, num_n, entry, entry_sb,
                        tile_base, count, tile_order != nullptr ? tile_count : nullptr, order, order_sb, group_count,
                        group_blocks, (long long*)row_workloads);
-    if (tile_order != nullptr || group_order != nullptr) {
+    if (tile_order != nullptr || group_order != nullptr || count_host != nullptr) {
         const int nt = tile_order != nullptr ? n_tiles : 0, ng = group_order != nullptr ? n_groups : 0;
-        hipLaunchKernelGGL(tile_order_kernel, dim3((max(nt, ng) + 63) / 64, group_order != nullptr ? 2 : 1), dim3(256), 0,
-                           stream, tile_count, nt, tile_order, group_count, ng, group_order);
+        hipLaunchKernelGGL(tile_order_kernel, dim3(max(1, (max(nt, ng) + 63) / 64), group_order != nullptr ? 2 : 1), dim3(256), 0,
+                           stream, tile_count, nt, tile_order, group_count, ng, group_order, count,
+                           (unsigned long long*)count_host, (unsigned long long)count_tag << 32);
     }
     return (int)hipGetLastError();
 }

@@ -15,7 +15,7 @@ BAM_DTYPE_F16 = 0
 BAM_DTYPE_BF16 = 1
 BAM_MAX_SEQLEN = 4194304
 BAM_STATIC_PLAN_BYTES = 8 << 20
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -80,7 +80,38 @@ class Plan(ctypes.Structure):
     ]
 
 
+class TensorArg(ctypes.Structure):
+    """``bam_tensor`` of include/bam_hip.h."""
+
+    _fields_ = [("ptr", ctypes.c_void_p), ("stride_b", ctypes.c_int64), ("stride_s", ctypes.c_int64), ("stride_h", ctypes.c_int64)]
+
+
+class Attn(ctypes.Structure):
+    """``bam_attn`` of include/bam_hip.h: one attention call in struct form."""
+
+    _fields_ = [
+        *((name, TensorArg) for name in ("q", "k", "v", "o", "dout", "dq", "dk", "dv")),
+        ("lse", ctypes.c_void_p),
+        ("delta", ctypes.c_void_p),
+        ("bf", ctypes.c_void_p),
+        ("bf_stride_b", ctypes.c_int64),
+        ("index", ctypes.POINTER(IndexView)),
+        ("mask", ctypes.c_void_p),
+        ("flags", ctypes.c_void_p),
+        ("flags_stride_b", ctypes.c_int64),
+        ("flags_stride_m", ctypes.c_int64),
+        ("bias", ctypes.POINTER(Bias)),
+        ("plan", ctypes.POINTER(Plan)),
+        ("ds_workspace", ctypes.c_void_p),
+        ("ds_capacity", ctypes.c_int64),
+        *((name, ctypes.c_int32) for name in ("mode", "B", "Sq", "Sk", "Hq", "Hkv", "D", "dtype", "accumulate", "head_runs")),
+        ("scale", ctypes.c_float),
+    ]
+
+
 _view = ctypes.POINTER(IndexView)
+_attn = ctypes.POINTER(Attn)
+_u32 = ctypes.c_uint32
 _bias = ctypes.POINTER(Bias)
 _plan = ctypes.POINTER(Plan)
 
@@ -89,6 +120,9 @@ SIGNATURES = {
     "bam_tile_flags": [_ptr, _i64, _ptr, _i64, _i64, _int, _int, _ptr],
     "bam_materialize_mask": [_ptr, _i64, _ptr, _int, _int, _ptr],
     "bam_tile_plan": [_ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _plan, _ptr],
+    "bam_tile_plan_counted": [_ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _plan, _ptr, _u32, _ptr],
+    "bam_host_words_alloc": [_ptr, _int],
+    "bam_host_words_free": [_ptr],
     "bam_tile_plan_static": [_ptr, _i64, _ptr, _i64, _i64, _int, _int, _plan, _ptr],
     "bam_fwd": [_ptr] * 7 + [_i64] * 15 + [_int] * 5 + [_f32, _int, _bias, _plan, _ptr],
     "bam_bwd_preprocess": [_ptr] * 3 + [_i64] * 6 + [_int] * 5 + [_ptr],
@@ -97,15 +131,19 @@ SIGNATURES = {
     "bam_bwd_dq": [_ptr] * 9 + [_i64] * 18 + [_int] * 5 + [_f32, _int, _int, _bias, _plan, _ptr],
     "bam_mask_tile_flags": [_ptr, _ptr, _i64, _i64, _int, _int, _int, _ptr],
     "bam_mask_tile_plan": [_ptr, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _int, _plan, _ptr],
+    "bam_mask_tile_plan_counted": [_ptr, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _int, _plan, _ptr, _u32, _ptr],
     "bam_fwd_masked": [_ptr] * 7 + [_i64] * 14 + [_int] * 6 + [_f32, _int, _bias, _plan, _ptr],
     "bam_bwd_dkdv_masked": [_ptr] * 10 + [_i64] * 20 + [_int] * 6 + [_f32, _int, _int, _bias, _plan, _ptr],
     "bam_bwd_dq_masked": [_ptr] * 9 + [_i64] * 17 + [_int] * 6 + [_f32, _int, _int, _bias, _plan, _ptr],
     "bam_flag_row_workloads": [_ptr, _i64, _i64, _int, _int, _int, _ptr, _ptr],
     "bam_gather_bitfields": [_ptr, _i64, _int, _ptr, _int, _ptr, _i64, _ptr, _int, _ptr],
     "bam_plan_indexed": [_view, _ptr, _i64, _int, _plan, _ptr],
+    "bam_plan_indexed_counted": [_view, _ptr, _i64, _int, _plan, _ptr, _u32, _ptr],
     "bam_fwd_indexed": [_ptr] * 5 + [_view, _ptr] + [_i64] * 14 + [_int] * 4 + [_f32, _int, _bias, _plan, _ptr],
     "bam_bwd_dkdv_indexed": [_ptr] * 8 + [_view, _ptr] + [_i64] * 20 + [_int] * 4 + [_f32, _int, _int, _bias, _plan, _ptr],
     "bam_bwd_dq_indexed": [_ptr] * 7 + [_view, _ptr] + [_i64] * 17 + [_int] * 4 + [_f32, _int, _int, _bias, _plan, _ptr],
+    "bam_attn_fwd": [_attn, _ptr],
+    "bam_attn_bwd": [_attn, _ptr],
     "bam_decode": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr],
 }
 
@@ -156,3 +194,18 @@ def call(name: str, *args) -> None:
     rc = getattr(lib, name)(*args)
     if rc != 0:
         raise BamError(f"{name} failed ({rc}): {lib.bam_last_error().decode()}")
+
+
+def _load_host():
+    """The native host layer (csrc/host.cpp), which calls the library above."""
+    try:
+        from cornstarch_amd import _bam_host
+    except ImportError as e:
+        raise BamError(
+            f"the native host layer cannot be loaded ({e}): it has not been built "
+            "(run `python -m cornstarch_amd.build`); there is no fallback path"
+        ) from e
+    return _bam_host
+
+
+host = _load_host()

@@ -12,7 +12,6 @@ module (cornstarch/kernel/attention.py:51-52, cornstarch/shardformer/layers/util
 
 from __future__ import annotations
 
-import atexit
 import math
 from typing import Optional
 
@@ -20,12 +19,11 @@ import torch
 import torch.nn.functional as F
 
 from . import _bam_hip
+from ._bam_hip import host as _host
 from .bitfield_attention import (
-    _CACHE_LOCK,
     _bias_arg,
     _BiasView,
     _plan_arg,
-    _TilePlan,
     _backward_in_head_runs,
     _dtype_code,
     _is_kernel_ready,
@@ -60,53 +58,21 @@ class _MaskPlan:
     of the mask's size in all) of a bool mask, from one pass over it.  The forward
     and, later, the backward of one call bring the same mask tensor: the last result is kept, together with the mask
     it was computed from (so its address cannot be handed to another tensor meanwhile), and reused while that is
-    unchanged."""
-
-    _last = None
+    unchanged.  (Kept by the native layer; masks that are not contiguous are made so by the caller.)"""
 
     @classmethod
     def get(cls, mask: Optional[torch.Tensor], batch: int, seqlen_q: int, seqlen_k: int, device):
         """-> (flags int8 (B, ceil(Sq/128), ceil(Sk/32)), plan or None)"""
         if mask is None:
             return mask_tile_flags(None, batch, seqlen_q, seqlen_k, device), None
-        with _CACHE_LOCK:
-            return cls._get_locked(mask, batch, seqlen_q, seqlen_k, device)
-
-    @classmethod
-    def _get_locked(cls, mask: torch.Tensor, batch: int, seqlen_q: int, seqlen_k: int, device):
-        key = (mask.data_ptr(), tuple(mask.shape), tuple(mask.stride()), mask._version, mask.device)
-        if cls._last is not None and cls._last[0] == key:
-            return cls._last[1], cls._last[2]
-        import ctypes
-
-        num_m, num_n = -(-seqlen_q // BLOCK_M), -(-seqlen_k // BLOCK_N)
-        with torch.cuda.device(device):
-            ws_bytes = _bam_hip.load().bam_mask_plan_workspace_bytes(batch, seqlen_q, seqlen_k)
-            workspace = None
-            if ws_bytes > 0:
-                try:
-                    workspace = torch.empty((ws_bytes,), dtype=torch.uint8, device=device)
-                except torch.cuda.OutOfMemoryError:
-                    workspace = None  # no room for a quarter of the mask: flags only, the kernels read the mask bytes
-            if workspace is not None:
-                flags = torch.empty((batch, num_m, num_n), dtype=torch.int8, device=device)
-                struct = _bam_hip.Plan()
-                _bam_hip.call(
-                    "bam_mask_tile_plan", mask.data_ptr(), flags.data_ptr(), flags.stride(0), flags.stride(1),
-                    workspace.data_ptr(), ws_bytes, batch, seqlen_q, seqlen_k, ctypes.byref(struct), _stream_ptr(device),
-                )
-                plan = _TilePlan(workspace, struct, flags)
-            else:
-                flags, plan = mask_tile_flags(mask, batch, seqlen_q, seqlen_k, device), None
-        cls._last = (key, flags, plan, mask)
-        return flags, plan
+        got = _host.mask_flags(mask, batch, seqlen_q, seqlen_k)
+        if got is None:  # (a tensor without a version counter: nothing to keep a plan by)
+            return mask_tile_flags(mask, batch, seqlen_q, seqlen_k, device), None
+        return got
 
     @classmethod
     def forget(cls):
-        cls._last = None
-
-
-atexit.register(_MaskPlan.forget)  # (runs before the release of the bitfield module's state, registered earlier)
+        _host.forget_mask()
 
 
 def _checked_mask(mask, batch, seqlen_q, seqlen_k):
@@ -141,15 +107,19 @@ def _flash_attn_forward(
     assert q.dtype in [torch.float16, torch.bfloat16], "Only support fp16 and bf16"
     assert q.is_cuda and k.is_cuda and v.is_cuda
     softmax_scale = softmax_scale or 1.0 / math.sqrt(d)
+    mask = _checked_mask(mask, batch, seqlen_q, seqlen_k)
+    flags, plan = _MaskPlan.get(mask, batch, seqlen_q, seqlen_k, q.device)
+    out = _host.forward(q, k, v, None, 0, mask, True, flags, bias, softmax_scale, plan)
+    if out is not None:
+        return (*out, softmax_scale)
+
+    # the general path: head dims, layouts and biases that have to be brought into the kernels' form first
     # reference attention.py:874-895
     bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k) if bias is not None else None
-    mask = _checked_mask(mask, batch, seqlen_q, seqlen_k)
-
     dp = _padded_head_dim(d)
     if dp != d:  # zero columns change neither q.k nor the first d columns of p.v
         q, k, v = (F.pad(x, (0, dp - d)) for x in (q, k, v))
     qk, kk, vk = (_kernel_ready(x, 8) for x in (q, k, v))
-    flags, plan = _MaskPlan.get(mask, batch, seqlen_q, seqlen_k, q.device)
     lse = torch.empty((batch, nheads, flags.shape[1] * BLOCK_M), device=q.device, dtype=torch.float32)
     o = torch.empty_like(qk)
     with torch.cuda.device(q.device):
@@ -193,10 +163,14 @@ def _flash_attn_backward(
     assert q.stride(-1) == k.stride(-1) == v.stride(-1) == o.stride(-1) == 1
     assert dq.stride(-1) == dk.stride(-1) == dv.stride(-1) == 1
     softmax_scale = softmax_scale or 1.0 / math.sqrt(d)
-    # the reference asserts the unit stride here instead of copying (attention.py:1002-1019)
-    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k, may_copy=False) if bias is not None else None
     mask = _checked_mask(mask, batch, seqlen_q, seqlen_k)
     flags, plan = _MaskPlan.get(mask, batch, seqlen_q, seqlen_k, q.device)
+    if _host.backward(do, q, k, v, o, lse, dq, dk, dv, False, None, 0, mask, True, flags, bias, softmax_scale, plan) is not None:
+        return
+
+    # the general path: head dims, layouts and biases that have to be brought into the kernels' form first
+    # the reference asserts the unit stride here instead of copying (attention.py:1002-1019)
+    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k, may_copy=False) if bias is not None else None
 
     dp = _padded_head_dim(d)
     outs = (dq, dk, dv)
@@ -282,5 +256,9 @@ def flash_attn_func(
     softmax_scale: Optional[float] = None,
 ):
     """Attention with an optional materialized bool mask (reference attention.py:1126-1146)."""
+    if mask is not None:
+        out = _host.masked_attention(q, k, v, bias, mask, softmax_scale)
+        if out is not None:
+            return out
     return FlashAttnFunc.apply(q, k, v, bias, mask, softmax_scale)
 

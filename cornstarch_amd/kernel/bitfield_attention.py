@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import atexit
 import contextlib
+import ctypes
 import math
 import os
 import threading
@@ -21,6 +22,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _bam_hip
+from ._bam_hip import host as _host
 
 BLOCK_M = 128  # rows of a flag tile (reference bitfield_attention.py:53)
 BLOCK_N = 32  # columns of a flag tile (reference bitfield_attention.py:54)
@@ -89,91 +91,65 @@ _DS_LIMIT_ENV = os.environ.get("BAM_DS_WORKSPACE_LIMIT_GB")
 # BAM_DS_WORKSPACE_TARGET_GB overrides the size (a value at or above the limit means: one run whenever it fits).
 _DS_RUN_TARGET = int(float(os.environ.get("BAM_DS_WORKSPACE_TARGET_GB", "16")) * (1 << 30))
 _DS_RUN_MIN_WORKGROUPS = 1024
+_DS_RECORD_BYTES = 8192  # of one (slice, key tile) pair and q head: bam_ds_workspace_bytes
+
+
+_DEVICE_LIMITS: dict = {}
 
 
 def _ds_workspace_limit(device) -> int:
     if _DS_LIMIT_ENV is not None:
         return int(float(_DS_LIMIT_ENV) * (1 << 30))
-    return min(64 << 30, torch.cuda.get_device_properties(device).total_memory // 4)
+    limit = _DEVICE_LIMITS.get(device)
+    if limit is None:
+        limit = _DEVICE_LIMITS[device] = min(64 << 30, torch.cuda.get_device_properties(device).total_memory // 4)
+    return limit
 
 
-class _PinnedInts:
-    """A small pool of pinned host ints for asynchronous device-to-host copies of single counters."""
-
-    _buf: Optional[torch.Tensor] = None
-    _next = 0
-    _SLOTS = 256
-
-    @classmethod
-    def slot(cls) -> torch.Tensor:
-        if cls._buf is None:
-            cls._buf = torch.empty((cls._SLOTS,), dtype=torch.int32, pin_memory=True)
-        i = cls._next
-        cls._next = (i + 1) % cls._SLOTS
-        return cls._buf[i : i + 1]
-
-    _streams: dict = {}
-
-    @classmethod
-    def copy_stream(cls, device) -> "torch.cuda.Stream":
-        """One side stream per device for these copies, so that they never sit between two kernels of the caller's
-        stream."""
-        key = torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device()
-        if key not in cls._streams:
-            cls._streams[key] = torch.cuda.Stream(device=device)
-        return cls._streams[key]
-
-
-# The caches below (flags + plan of the last bitfield mask, index view, mask plan) are per process, as in the
-# reference; host threads that share them take this lock while they look an entry up or replace it.
+# The caches (flags + plan of the last bitfield mask, index view, mask plan) are per process, as in the reference.  Flags
+# and plans are kept by the native layer, which replaces an entry under the interpreter lock; the index view lives here,
+# and host threads that share it take this lock while they look it up or replace it.
 _CACHE_LOCK = threading.RLock()
 
 
 def _release_device_state() -> None:
-    """Drops what this module keeps alive between calls (cached flags and plans, the pinned counter slots, the side
-    stream) while the GPU runtime is still up: left to interpreter shutdown, pinned memory and streams would be
-    released in no particular order after it."""
+    """Drops what this module keeps alive between calls (cached flags and plans, the pinned words of the pair counts)
+    while the GPU runtime is still up: left to interpreter shutdown, pinned memory would be released in no particular
+    order after it."""
     try:
         if torch.cuda.is_available() and torch.cuda.is_initialized():
             torch.cuda.synchronize()
     except Exception:  # the runtime is already gone: nothing left to wait for
         pass
     BitfieldUtils.clear_cache()
-    _IndexView.forget()
-    _PinnedInts._buf = None
-    _PinnedInts._streams.clear()
+    _host.forget_mask()
+    _host.release_host_memory()
 
 
 atexit.register(_release_device_state)
 
 
-class _TilePlan:
+class _TilePlan(_host.PlanCore):
     """What the kernels use beyond the 128 x 32 flags to skip masked work (``bam_plan`` of include/bam_hip.h):
     the class of every 32-row x 32-key tile and an order of the 32-row slices in which neighbours need the same
-    keys.  Built together with the flags, lives in one workspace tensor, and belongs to exactly one flags tensor."""
+    keys.  Built together with the flags, lives in one workspace tensor, and belongs to exactly one flags tensor
+    (``flags`` is None for plans that are not tied to one: index-tensor attention).  Created by the native layer, which
+    fills in ``workspace``, ``flags``, ``flags_version`` and the struct.
 
-    def __init__(self, workspace: torch.Tensor, struct: "_bam_hip.Plan", flags: Optional[torch.Tensor]):
-        self.workspace = workspace  # keeps the device memory alive
-        self.struct = struct
-        self.flags = flags  # None for plans that are not tied to a flags tensor (index-tensor attention)
-        self.flags_version = flags._version if flags is not None else -1  # (the builder wrote through raw pointers)
-        # The number of (slice, 128-key tile) pairs that have work is device data; it sizes the dS workspace of the
-        # backward.  Its copy to the host is enqueued here, right behind the kernels that compute it, and awaited
-        # only when a backward asks for it -- by then it has long arrived.
-        self._lock = threading.Lock()  # held while a backward has its dS workspace named in the struct
-        self._pairs: Optional[int] = None
-        self._pairs_host = _PinnedInts.slot()
-        count = torch.as_strided(workspace.view(torch.int32), (1,), (1,), (struct.ds_count - workspace.data_ptr()) // 4)
-        main = torch.cuda.current_stream(workspace.device)
-        side = _PinnedInts.copy_stream(workspace.device)
-        built = torch.cuda.Event()
-        built.record(main)
-        side.wait_event(built)
-        with torch.cuda.stream(side):
-            self._pairs_host.copy_(count, non_blocking=True)
-        workspace.record_stream(side)
-        self._pairs_event = torch.cuda.Event()
-        self._pairs_event.record(side)
+    The number of (slice, 128-key tile) pairs that have work is device data; it sizes the dS workspace of the backward.
+    The plan builder's last launch stores it to pinned host memory, and ``ds_pairs()`` waits for it there -- by the time a
+    backward asks it has usually long arrived."""
+
+    def __init__(self):
+        super().__init__()
+        self._lock = None  # held while a backward has its dS workspace named in the struct
+        self._struct = None
+
+    @property
+    def struct(self) -> "_bam_hip.Plan":
+        if self._struct is None:
+            self._struct = _bam_hip.Plan.from_address(self.struct_address)
+        return self._struct
 
     def row_workloads(self) -> torch.Tensor:
         """int64 (ceil(Sq/128),): non-empty 128 x 32 tiles of each row block, summed over the batch; a view into the
@@ -182,42 +158,42 @@ class _TilePlan:
         ws = self.workspace
         return torch.as_strided(ws.view(torch.int64), (num_m,), (1,), (self.struct.row_workloads - ws.data_ptr()) // 8)
 
-    def ds_pairs(self) -> int:
-        """How many (32-row slice, 128-key tile) pairs have work (waits for the asynchronous copy on first use)."""
-        if self._pairs is None:
-            self._pairs_event.synchronize()
-            self._pairs = int(self._pairs_host[0])
-        return self._pairs
+    def allocate_ds_workspace(self, nheads: int, head_dim: int, seqlen_k: int) -> Optional[torch.Tensor]:
+        """The dS workspace of one backward call, or None where the hand-over does not apply."""
+        if head_dim != 128 or seqlen_k > 131072:
+            return None
+        pairs = self.ds_pairs()
+        nbytes = nheads * pairs * _DS_RECORD_BYTES
+        if nbytes <= 0 or nbytes > _ds_workspace_limit(self.workspace.device) or nheads * pairs >= 1 << 31:
+            return None
+        try:
+            return self._allocate(nbytes, self.workspace.device)
+        except torch.cuda.OutOfMemoryError:
+            return None  # no room for it right now: the dQ kernel recomputes what it needs, as without a workspace
 
     def attach_ds_workspace(self, nheads: int, head_dim: int, seqlen_k: int) -> Optional[torch.Tensor]:
         """Allocates the dS workspace of one backward call and names it in the plan struct; None (and nothing
         attached) where the hand-over does not apply.  The caller detaches it after its launches."""
         self.detach_ds_workspace()
-        if head_dim != 128 or seqlen_k > 131072:
-            return None
-        pairs = self.ds_pairs()
-        nbytes = _bam_hip.load().bam_ds_workspace_bytes(nheads, pairs)
-        if nbytes <= 0 or nbytes > _ds_workspace_limit(self.workspace.device) or nheads * pairs >= 1 << 31:
-            return None
-        try:
-            ws = self._allocate(nbytes, self.workspace.device)
-        except torch.cuda.OutOfMemoryError:
-            return None  # no room for it right now: the dQ kernel recomputes what it needs, as without a workspace
-        self.struct.ds_workspace = ws.data_ptr()
-        self.struct.ds_capacity = pairs
+        ws = self.allocate_ds_workspace(nheads, head_dim, seqlen_k)
+        if ws is not None:
+            self.struct.ds_workspace = ws.data_ptr()
+            self.struct.ds_capacity = self.ds_pairs()
         return ws
 
     def ds_head_runs(self, batch: int, nheads: int, nheads_k: int, head_dim: int, seqlen_k: int) -> int:
         """Into how many runs of whole kv heads a backward splits: the smallest divisor of ``nheads_k`` for which the
         dS workspace of one run stays within the limit, and beyond that more runs while a run's workspace is above
         ``_DS_RUN_TARGET`` and its dK/dV launch keeps ``_DS_RUN_MIN_WORKGROUPS`` workgroups.  1: all heads at once
-        (also where the hand-over does not apply or no split helps: ``attach_ds_workspace`` then decides)."""
+        (also where the hand-over does not apply or no split helps: ``allocate_ds_workspace`` then decides)."""
         if head_dim != 128 or seqlen_k > 131072 or nheads % nheads_k != 0:
             return 1
         pairs = self.ds_pairs()
         limit = _ds_workspace_limit(self.workspace.device)
-        lib = _bam_hip.load()
-        nbytes = {r: lib.bam_ds_workspace_bytes(nheads // r, pairs) for r in range(1, nheads_k + 1) if nheads_k % r == 0}
+        whole = nheads * pairs * _DS_RECORD_BYTES
+        if whole <= min(limit, _DS_RUN_TARGET) and nheads * pairs < 1 << 31:
+            return 1
+        nbytes = {r: whole // r for r in range(1, nheads_k + 1) if nheads_k % r == 0}
         fits = [r for r, n in nbytes.items() if 0 < n <= limit and (nheads // r) * pairs < 1 << 31]
         if not fits:
             return 1
@@ -228,6 +204,12 @@ class _TilePlan:
                 break
             runs = r
         return runs
+
+    def backward_workspace(self, batch: int, nheads: int, nheads_k: int, head_dim: int, seqlen_k: int, splittable: bool):
+        """-> (runs of heads, dS workspace of one run or None): what the native backward asks for.  A bias is indexed
+        by absolute head: with one, the heads stay in one run (``splittable`` False)."""
+        runs = self.ds_head_runs(batch, nheads, nheads_k, head_dim, seqlen_k) if splittable else 1
+        return runs, self.allocate_ds_workspace(nheads // runs, head_dim, seqlen_k)
 
     @staticmethod
     def _allocate(nbytes: int, device) -> torch.Tensor:
@@ -242,6 +224,9 @@ class _TilePlan:
         """The launches of one backward: the dS workspace (if any) is attached on entry and detached on exit, and
         other host threads that run a backward with the same plan wait meanwhile (the struct is shared; the
         launches only enqueue work, so the wait is short)."""
+        with _CACHE_LOCK:
+            if self._lock is None:
+                self._lock = threading.Lock()
         with self._lock:
             ws = self.attach_ds_workspace(nheads, head_dim, seqlen_k)
             try:
@@ -250,8 +235,6 @@ class _TilePlan:
                 self.detach_ds_workspace()
 
     def byref(self):
-        import ctypes
-
         return ctypes.byref(self.struct)
 
     def fine_classes(self) -> torch.Tensor:
@@ -282,10 +265,22 @@ def _plan_arg(plan: Optional["_TilePlan"]):
     return plan.byref() if plan is not None else None
 
 
-class BitfieldUtils:
+class _FlagCache(type):
+    """The cached flags live in the native layer; as a class attribute they read (and assign) like the reference's."""
+
+    @property
+    def compressed_mask_cache(cls) -> Optional[torch.Tensor]:
+        return _host.cached_bitfield_flags()
+
+    @compressed_mask_cache.setter
+    def compressed_mask_cache(cls, flags: Optional[torch.Tensor]) -> None:
+        _host.set_cached_bitfield_flags(flags)
+
+
+class BitfieldUtils(metaclass=_FlagCache):
     """Cache of the tile flags ("compressed mask") of the current bitfield mask.
 
-    compressed_mask_cache: int8 (batch, ceil(S / BLOCK_M), ceil(S / BLOCK_N));
+    compressed_mask_cache: int8 (batch, ceil(S / BLOCK_M), ceil(S / BLOCK_N)):
         0: every pair of the tile is masked, the tile is skipped
         1: some pairs are allowed, the mask is evaluated
         2: every in-range pair is allowed, the mask is not evaluated
@@ -296,19 +291,10 @@ class BitfieldUtils:
     entry lives) and compares address, shape, strides and version counter.
     """
 
-    compressed_mask_cache: Optional[torch.Tensor] = None
-    _cache_key = None
-    _cache_owner: Optional[torch.Tensor] = None  # the bitfield tensor the cached flags belong to
-    _plan: Optional[_TilePlan] = None            # built with the cached flags; None for very long sequences
-
     @classmethod
     def clear_cache(cls):
-        with _CACHE_LOCK:
-            cls.compressed_mask_cache = None
-            cls._cache_key = None
-            cls._cache_owner = None
-            cls._plan = None
-            _IndexView.forget()
+        _host.forget_bitfield()
+        _IndexView.forget()
 
     @classmethod
     def plan_for(cls, compressed_mask: torch.Tensor, bitfield_mask: torch.Tensor) -> Optional[_TilePlan]:
@@ -316,73 +302,18 @@ class BitfieldUtils:
         itself and ``bitfield_mask`` is still the (unchanged) mask they were computed from.  Callers that bring
         their own flags (re-indexed context-parallel shards, for instance) get None and the kernels work from
         the flags alone."""
-        with _CACHE_LOCK:
-            plan, cached, key = cls._plan, cls.compressed_mask_cache, cls._cache_key
-        if plan is None or plan.flags is not cached:
-            return None
-        # the cache keeps its flags tensor alive, so equal address and shape mean "that tensor" (autograd may hand
+        # (the cache keeps its flags tensor alive, so equal address and shape mean "that tensor": autograd may hand
         # saved tensors back as new Python objects)
-        if compressed_mask.data_ptr() != plan.flags.data_ptr() or compressed_mask.shape != plan.flags.shape:
-            return None
-        if key != cls._key_of(bitfield_mask):
-            return None
-        return plan
-
-    @staticmethod
-    def _key_of(bitfield_mask: torch.Tensor):
-        return (
-            bitfield_mask.data_ptr(),
-            tuple(bitfield_mask.shape),
-            tuple(bitfield_mask.stride()),
-            bitfield_mask._version,
-            bitfield_mask.device,
-        )
+        return _host.plan_for(compressed_mask, bitfield_mask)
 
     @classmethod
     def materialize_compressed_mask_from_bitfield_mask(cls, bitfield_mask: torch.Tensor) -> torch.Tensor:
-        with _CACHE_LOCK:
-            return cls._materialize_locked(bitfield_mask)
-
-    @classmethod
-    def _materialize_locked(cls, bitfield_mask: torch.Tensor) -> torch.Tensor:
-        key = cls._key_of(bitfield_mask)
-        if cls.compressed_mask_cache is not None and cls._cache_key == key:
-            # _cache_owner is alive, so this address still belongs to the tensor (or a view of the
-            # tensor) the flags were computed from, and its version says it has not been written since
-            return cls.compressed_mask_cache
-
+        flags = _host.bitfield_flags(bitfield_mask)
+        if flags is not None:
+            return flags
         assert bitfield_mask.is_cuda, "bitfield attention runs on the GPU only"
         assert bitfield_mask.dtype == torch.int64 and bitfield_mask.dim() == 2
-        bf = bitfield_mask if bitfield_mask.stride(1) == 1 else bitfield_mask.contiguous()
-        batch_size, seq_len = bf.shape
-        out = torch.empty(
-            (batch_size, -(-seq_len // BLOCK_M), -(-seq_len // BLOCK_N)),
-            dtype=torch.int8,
-            device=bf.device,
-        )
-        plan = None
-        with torch.cuda.device(bf.device):
-            ws_bytes = _bam_hip.load().bam_plan_workspace_bytes(batch_size, seq_len)
-            if ws_bytes > 0:
-                workspace = torch.empty((ws_bytes,), dtype=torch.uint8, device=bf.device)
-                struct = _bam_hip.Plan()
-                import ctypes
-
-                _bam_hip.call(
-                    "bam_tile_plan", bf.data_ptr(), bf.stride(0), out.data_ptr(), out.stride(0), out.stride(1),
-                    workspace.data_ptr(), ws_bytes, batch_size, seq_len, ctypes.byref(struct), _stream_ptr(bf.device),
-                )
-                plan = _TilePlan(workspace, struct, out)
-            else:
-                _bam_hip.call(
-                    "bam_tile_flags", bf.data_ptr(), bf.stride(0), out.data_ptr(), out.stride(0), out.stride(1),
-                    batch_size, seq_len, _stream_ptr(bf.device),
-                )
-        cls.compressed_mask_cache = out
-        cls._cache_key = key
-        cls._cache_owner = bitfield_mask
-        cls._plan = plan
-        return out
+        return _host.bitfield_flags_general(bitfield_mask)
 
     @classmethod
     def nonempty_tiles_per_row_block(cls, compressed_mask: torch.Tensor) -> torch.Tensor:
@@ -391,8 +322,7 @@ class BitfieldUtils:
         sequence split sorts by (reference shardformer/layers/utils.py:161-171), computed on the GPU so that
         only this small vector has to travel to the host."""
         assert compressed_mask.is_cuda and compressed_mask.dtype == torch.int8 and compressed_mask.dim() == 3
-        with _CACHE_LOCK:
-            plan, cached = cls._plan, cls.compressed_mask_cache
+        plan, cached = _host.cached_bitfield_plan(), _host.cached_bitfield_flags()
         # the cached flags tensor itself, unwritten since it was built: its plan already holds the sums, so nothing is
         # launched; the result is a view into the plan's workspace (read it, do not write it)
         if (plan is not None and cached is not None and plan.flags is cached and plan.struct.row_workloads
@@ -438,8 +368,6 @@ class _BiasView:
         )
 
     def byref(self):
-        import ctypes
-
         return ctypes.byref(self.struct)
 
 
@@ -459,45 +387,19 @@ class _IndexView:
             raise ValueError("offsets_q and offsets_k must be given together")
         dev = bitfield_mask.device
         bf = bitfield_mask if bitfield_mask.stride(1) == 1 else bitfield_mask.contiguous()
-        batch, length = bf.shape
-        self.seqlen_q, self.seqlen_k = int(offsets_q.numel()), int(offsets_k.numel())
+        assert bf.is_cuda and bf.dtype == torch.int64 and bf.dim() == 2
         assert offsets_q.dim() == 1 and offsets_k.dim() == 1
-        self._keep = []
-        arrays = []
-        with torch.cuda.device(dev):
-            for off in (offsets_q, offsets_k):
-                idx = off.to(device=dev, dtype=torch.int64).contiguous()
-                bits = torch.empty((batch, idx.numel()), dtype=torch.int64, device=dev)
-                pos = torch.empty((idx.numel(),), dtype=torch.int32, device=dev)
-                _bam_hip.call(
-                    "bam_gather_bitfields", bf.data_ptr(), bf.stride(0), length, idx.data_ptr(), idx.numel(),
-                    bits.data_ptr(), bits.stride(0), pos.data_ptr(), batch, _stream_ptr(dev),
-                )
-                arrays.append((bits, pos))
-                self._keep.append(idx)
-        (self.q_bits, self.q_pos), (self.k_bits, self.k_pos) = arrays
-        self.struct = _bam_hip.IndexView(
-            self.q_bits.data_ptr(), self.k_bits.data_ptr(), self.q_pos.data_ptr(), self.k_pos.data_ptr(),
-            self.q_bits.stride(0), self.k_bits.stride(0), self.seqlen_q, self.seqlen_k,
-        )
-        # the plan of the shard (classes of its 32 x 32 tiles, slice order), from the gathered arrays
-        self.plan = None
-        with torch.cuda.device(dev):
-            ws_bytes = _bam_hip.load().bam_plan_workspace_bytes_rect(batch, self.seqlen_q, self.seqlen_k)
-            if ws_bytes > 0:
-                import ctypes
+        self.seqlen_q, self.seqlen_k = int(offsets_q.numel()), int(offsets_k.numel())
+        idx = tuple(off.to(device=dev, dtype=torch.int64).contiguous() for off in (offsets_q, offsets_k))
+        self.struct = _bam_hip.IndexView()
+        # gathered bitfields and positions (named in the struct), and the plan of the shard: classes of its 32 x 32 tiles,
+        # slice order
+        arrays, self.plan = _host.index_view(bf, *idx, ctypes.addressof(self.struct))
+        self._keep = (arrays, idx)
 
-                workspace = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
-                struct = _bam_hip.Plan()
-                _bam_hip.call(
-                    "bam_plan_indexed", ctypes.byref(self.struct), workspace.data_ptr(), ws_bytes, batch,
-                    ctypes.byref(struct), _stream_ptr(dev),
-                )
-                self.plan = _TilePlan(workspace, struct, None)
+        self.address = ctypes.addressof(self.struct)
 
     def byref(self):
-        import ctypes
-
         return ctypes.byref(self.struct)
 
     # The context-parallel caller runs the forward and, later, the backward of one shard with the same three
@@ -506,15 +408,11 @@ class _IndexView:
     # while those are unchanged.
     _last = None
 
-    @staticmethod
-    def _tensor_key(t: torch.Tensor):
-        return (t.data_ptr(), tuple(t.shape), tuple(t.stride()), t._version, t.device, t.dtype)
-
     @classmethod
     def get(cls, bitfield_mask: torch.Tensor, offsets_q: torch.Tensor, offsets_k: torch.Tensor) -> "_IndexView":
         if offsets_q is None or offsets_k is None:
             raise ValueError("offsets_q and offsets_k must be given together")
-        key = tuple(cls._tensor_key(t) for t in (bitfield_mask, offsets_q, offsets_k))
+        key = tuple(_host.tensor_key(t) for t in (bitfield_mask, offsets_q, offsets_k))
         with _CACHE_LOCK:
             if cls._last is not None and cls._last[0] == key:
                 return cls._last[1]
@@ -550,7 +448,6 @@ def _bitfield_attn_forward(
     assert k.shape == v.shape and k.shape[0] == batch and k.shape[3] == d
     assert nheads % nheads_k == 0
     assert bitfield_mask.dtype == torch.int64 and bitfield_mask.dim() == 2 and bitfield_mask.shape[0] == batch
-    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k) if bias is not None else None
     view = None
     if offsets_q is not None or offsets_k is not None:
         view = _IndexView.get(bitfield_mask, offsets_q, offsets_k)
@@ -559,16 +456,22 @@ def _bitfield_attn_forward(
         assert seqlen_q == seqlen_k, "without index tensors query and key sequence lengths must match"
         assert bitfield_mask.shape[1] == seqlen_k
     softmax_scale = softmax_scale or 1.0 / math.sqrt(d)
+    num_m, num_n = -(-seqlen_q // BLOCK_M), -(-seqlen_k // BLOCK_N)
+    assert compressed_mask.dtype == torch.int8 and compressed_mask.shape == (batch, num_m, num_n)
+    plan = BitfieldUtils.plan_for(compressed_mask, bitfield_mask) if view is None else view.plan
+    out = _host.forward(q, k, v, bitfield_mask, view.address if view is not None else 0, None, False, compressed_mask,
+                        bias, softmax_scale, plan)
+    if out is not None:
+        return (*out, softmax_scale)
 
+    # the general path: head dims, layouts and biases that have to be brought into the kernels' form first
+    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k) if bias is not None else None
     dp = _padded_head_dim(d)
     if dp != d:  # zero columns change neither q.k nor the first d columns of p.v
         q, k, v = (F.pad(x, (0, dp - d)) for x in (q, k, v))
     qk, kk, vk = (_kernel_ready(x, 8) for x in (q, k, v))
     bf = bitfield_mask if bitfield_mask.stride(1) == 1 else bitfield_mask.contiguous()
     flags = compressed_mask if compressed_mask.stride(-1) == 1 else compressed_mask.contiguous()
-    num_m, num_n = -(-seqlen_q // BLOCK_M), -(-seqlen_k // BLOCK_N)
-    assert flags.dtype == torch.int8 and flags.shape == (batch, num_m, num_n)
-    plan = BitfieldUtils.plan_for(compressed_mask, bitfield_mask) if view is None else None
 
     seqlen_q_rounded = num_m * BLOCK_M
     lse = torch.empty((batch, nheads, seqlen_q_rounded), device=q.device, dtype=torch.float32)
@@ -590,7 +493,7 @@ def _bitfield_attn_forward(
                 flags.data_ptr(), *_strides3(qk, kk, vk, o),
                 flags.stride(0), flags.stride(1),
                 batch, nheads, nheads_k, dp, float(softmax_scale), _dtype_code(q.dtype),
-                _bias_arg(bias_view), _plan_arg(view.plan), _stream_ptr(q.device),
+                _bias_arg(bias_view), _plan_arg(plan), _stream_ptr(q.device),
             )
     if dp != d:
         o = o[..., :d].contiguous()
@@ -694,32 +597,10 @@ def _bitfield_attn_backward_overwrite(do, q, k, v, o, bitfield_mask, compressed_
     ``BitfieldAttentionFunction.backward`` needs, without the reference's zero-filled fp32
     staging buffers and the final cast (bitfield_attention.py:1248-1266).  Returns None when the
     layout needs the general path (padded head dimension, unaligned views)."""
-    d = q.shape[-1]
-    if d not in _SUPPORTED_HEAD_DIMS:
-        return None
-    if do.stride(-1) != 1 or not _is_kernel_ready(do):
-        do = do.contiguous()
-    if not all(_is_kernel_ready(x) for x in (q, k, v, o)):
-        return None
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    if not all(_is_kernel_ready(x) for x in (dq, dk, dv)):
-        return None
-    lse = lse.contiguous()
     bf = bitfield_mask if bitfield_mask.stride(1) == 1 else bitfield_mask.contiguous()
     flags = compressed_mask if compressed_mask.stride(-1) == 1 else compressed_mask.contiguous()
-    plan = BitfieldUtils.plan_for(compressed_mask, bitfield_mask)
-    delta = torch.empty_like(lse)
-    batch, seqlen_q, nheads, _ = q.shape
-    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, k.shape[1], may_copy=False) if bias is not None else None
-    _launch_bwd_preprocess(o, do, delta)
-
-    def launch(q, k, v, do, lse, delta, dq, dk, dv):
-        _launch_bwd_dkdv(q, k, v, do, lse, delta, dk, dv, bf, flags, softmax_scale, accumulate=False, bias=bias_view, plan=plan)
-        _launch_bwd_dq(q, k, v, do, lse, delta, dq, bf, flags, softmax_scale, accumulate=False, bias=bias_view, plan=plan)
-
-    # (a bias is indexed by absolute head: with one, the heads stay in one run)
-    _backward_in_head_runs(plan, launch, q, k, v, do, lse, delta, dq, dk, dv, d, splittable=bias_view is None)
-    return dq, dk, dv
+    return _host.backward(do, q, k, v, o, lse.contiguous(), None, None, None, False, bf, 0, None, False, flags, bias,
+                          softmax_scale, BitfieldUtils.plan_for(compressed_mask, bitfield_mask))
 
 
 def _bitfield_attn_backward(
@@ -752,8 +633,6 @@ def _bitfield_attn_backward(
     assert dq.stride(-1) == dk.stride(-1) == dv.stride(-1) == 1
     assert dq.dtype == dk.dtype == dv.dtype == torch.float32
     assert q.is_cuda
-    # the reference asserts the unit stride here instead of copying (bitfield_attention.py:1130)
-    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k, may_copy=False) if bias is not None else None
     view = None
     if offsets_q is not None or offsets_k is not None:
         view = _IndexView.get(bitfield_mask, offsets_q, offsets_k)
@@ -761,7 +640,15 @@ def _bitfield_attn_backward(
     else:
         assert seqlen_q == seqlen_k, "without index tensors query and key sequence lengths must match"
     softmax_scale = softmax_scale or 1.0 / math.sqrt(d)
+    assert compressed_mask.shape == (batch, -(-seqlen_q // BLOCK_M), -(-seqlen_k // BLOCK_N))
+    plan = BitfieldUtils.plan_for(compressed_mask, bitfield_mask) if view is None else view.plan
+    if _host.backward(do, q, k, v, o, lse, dq, dk, dv, True, bitfield_mask, view.address if view is not None else 0, None,
+                      False, compressed_mask, bias, softmax_scale, plan) is not None:
+        return
 
+    # the general path: head dims, layouts and biases that have to be brought into the kernels' form first
+    # the reference asserts the unit stride here instead of copying (bitfield_attention.py:1130)
+    bias_view = _BiasView(bias, q, batch, nheads, seqlen_q, seqlen_k, may_copy=False) if bias is not None else None
     dp = _padded_head_dim(d)
     acc = (dq, dk, dv)
     if dp != d:
@@ -774,19 +661,16 @@ def _bitfield_attn_backward(
     if view is not None:
         bf = view
     flags = compressed_mask if compressed_mask.stride(-1) == 1 else compressed_mask.contiguous()
-    assert flags.shape == (batch, -(-seqlen_q // BLOCK_M), -(-seqlen_k // BLOCK_N))
-    plan = BitfieldUtils.plan_for(compressed_mask, bitfield_mask) if view is None else None
     delta = torch.empty_like(lse)
     wq, wk, wv = work
     _launch_bwd_preprocess(ok, gk, delta)
-    the_plan = plan if view is None else view.plan
 
     def launch(q, k, v, do, lse, delta, dq, dk, dv):
         _launch_bwd_dkdv(q, k, v, do, lse, delta, dk, dv, bf, flags, softmax_scale, bias=bias_view, plan=plan)
         _launch_bwd_dq(q, k, v, do, lse, delta, dq, bf, flags, softmax_scale, bias=bias_view, plan=plan)
 
     # (a bias is indexed by absolute head: with one, the heads stay in one run)
-    _backward_in_head_runs(the_plan, launch, qk, kk, vk, gk, lse, delta, wq, wk, wv, dp, splittable=bias_view is None)
+    _backward_in_head_runs(plan, launch, qk, kk, vk, gk, lse, delta, wq, wk, wv, dp, splittable=bias_view is None)
     # the kernels accumulated into `work`; hand the sums back if those were copies
     for dst, mid, w in zip((dq, dk, dv), acc, work):
         if dp != d:
@@ -852,4 +736,10 @@ def bitfield_attn_func(
     bias: Optional[torch.Tensor] = None,
     softmax_scale: Optional[float] = None,
 ) -> torch.Tensor:
+    out = _host.bitfield_attention(q, k, v, bitfield_mask, bias, softmax_scale)
+    if out is not None:
+        return out
     return BitfieldAttentionFunction.apply(q, k, v, bitfield_mask, bias, softmax_scale)
+
+
+_host.setup(_TilePlan, _bam_hip.BamError)

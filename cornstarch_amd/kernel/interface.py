@@ -16,6 +16,7 @@ from torch import nn
 import math
 
 from . import _bam_hip
+from ._bam_hip import host as _host
 from .attention import flash_attn_func
 from .bitfield_attention import _dtype_code, _kernel_ready, _padded_head_dim, _stream_ptr, bitfield_attn_func
 
@@ -60,6 +61,11 @@ def _decode_attention(query, key, value, scaling, dropout, sliding_window, softc
     ``sliding_window`` keys.  Dropout is inactive in eval mode either way.
 
     query (B, Hq, 1, D), key / value (B, Hkv, Sk, D) -> (B, 1, Hq, D) in the dtype of query."""
+    if not dropout and (sliding_window is None or sliding_window > 0) and (softcap is None or softcap >= 0):
+        out = _host.decode(query, key, value, scaling, sliding_window or 0, softcap or 0.0)
+        if out is not None:
+            return out, None
+    # the general path: other layouts and head dims, and what is refused
     batch, nheads, q_len, d = query.shape
     _, nheads_k, seqlen_k, _ = key.shape
     assert q_len == 1

@@ -173,6 +173,17 @@ int64_t bam_plan_workspace_bytes_rect(int B, int Sq, int Sk);
 int bam_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                   int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
                   void* stream);
+/*
+ * The same, and *plan->ds_count reaches the host without a copy: the last launch of the builder stores
+ * (count_tag << 32) | count to *count_host, a word of bam_host_words_alloc (null = as without).  The host may poll the
+ * word for its tag; nothing else tells it that the value has arrived.  (There is a counted form of every plan builder.)
+ */
+int bam_tile_plan_counted(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
+                          int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
+                          uint64_t* count_host, uint32_t count_tag, void* stream);
+/* Pinned, coherent host memory for those words (zero-filled; hipHostMalloc / hipHostFree, so not while capturing). */
+int bam_host_words_alloc(uint64_t** words, int n);
+int bam_host_words_free(uint64_t* words);
 
 /*
  * bam_tile_plan without a workspace argument, for callers that cannot allocate device memory (code under HIP
@@ -204,6 +215,8 @@ int64_t bam_ds_workspace_bytes(int Hq, int64_t pairs);
  */
 int bam_plan_indexed(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
                      void* stream);
+int bam_plan_indexed_counted(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
+                             uint64_t* count_host, uint32_t count_tag, void* stream);
 
 /*
  * Dense bool mask, uint8 (B, S, S) contiguous: the allow rule for every pair
@@ -397,6 +410,9 @@ int bam_bwd_dq_masked(const void* q, const void* k, const void* v, const void* d
 int64_t bam_mask_plan_workspace_bytes(int B, int Sq, int Sk);
 int bam_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m, void* workspace,
                        int64_t workspace_bytes, int B, int Sq, int Sk, bam_plan* plan, void* stream);
+int bam_mask_tile_plan_counted(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m,
+                               void* workspace, int64_t workspace_bytes, int B, int Sq, int Sk, bam_plan* plan,
+                               uint64_t* count_host, uint32_t count_tag, void* stream);
 
 /*
  * Single-token decode step of a model in eval mode: one query row per batch element and head against the whole
@@ -417,6 +433,39 @@ int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_s
                int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
                int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D, float scale,
                int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
+ * Struct form of the attention calls: what bam_fwd*, bam_bwd_preprocess and bam_bwd_dkdv* / bam_bwd_dq* take, in one
+ * host struct, for hosts that fill it once per call instead of passing 40 arguments.  bam_attn_fwd is the forward of any
+ * mask mode; bam_attn_bwd runs the whole backward (delta into `delta`, then dK/dV and dQ), where head_runs > 1 takes the
+ * heads in that many runs of whole kv heads through one dS workspace of a run's size.  Unused fields are zero.
+ */
+#define BAM_MASK_BITFIELD 0 /* bf */
+#define BAM_MASK_INDEXED 1  /* index */
+#define BAM_MASK_DENSE 2    /* mask (null = every pair allowed) */
+typedef struct bam_tensor { /* (B, S, H, D), element strides, unit stride along D */
+    void* ptr;
+    int64_t stride_b, stride_s, stride_h;
+} bam_tensor;
+typedef struct bam_attn {
+    bam_tensor q, k, v, o, dout, dq, dk, dv;
+    float* lse;
+    float* delta;
+    const int64_t* bf;
+    int64_t bf_stride_b;
+    const bam_index_view* index;
+    const uint8_t* mask;
+    const int8_t* flags;
+    int64_t flags_stride_b, flags_stride_m;
+    const bam_bias* bias; /* may be null */
+    const bam_plan* plan; /* may be null; its own ds_workspace is not looked at */
+    void* ds_workspace;   /* bam_attn_bwd: may be null; bam_ds_workspace_bytes(Hq / head_runs, pairs) bytes */
+    int64_t ds_capacity;
+    int32_t mode, B, Sq, Sk, Hq, Hkv, D, dtype, accumulate, head_runs;
+    float scale;
+} bam_attn;
+int bam_attn_fwd(const bam_attn* args, void* stream);
+int bam_attn_bwd(const bam_attn* args, void* stream);
 
 #ifdef __cplusplus
 }
