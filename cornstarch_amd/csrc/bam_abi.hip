@@ -55,13 +55,15 @@ int check_f32_tensor(const char* name, const void* ptr, int64_t sb, int64_t ss, 
     return BAM_OK;
 }
 
-int check_problem(int B, int Sq, int Sk, int Hq, int Hkv, int D, int dtype) {
+// any_dim: the struct form takes every multiple of 8, the older entry points the three head dims they always took
+int check_problem(int B, int Sq, int Sk, int Hq, int Hkv, int D, int dtype, bool any_dim = false) {
     if (B <= 0 || Sq <= 0 || Sk <= 0 || Hq <= 0 || Hkv <= 0)
         return fail(BAM_ERR_INVALID_ARGUMENT, "B, S, Hq, Hkv must be positive (got B %d, Sq %d, Sk %d, Hq %d, Hkv %d)", B,
                     Sq, Sk, Hq, Hkv);
     if (Hq % Hkv) return fail(BAM_ERR_INVALID_ARGUMENT, "Hq (%d) must be a multiple of Hkv (%d)", Hq, Hkv);
-    if (D != 32 && D != 64 && D != 128)
-        return fail(BAM_ERR_UNSUPPORTED, "head dimension %d is not supported (32, 64 or 128)", D);
+    if (any_dim ? (D <= 0 || D > 128 || D % 8) : (D != 32 && D != 64 && D != 128))
+        return fail(BAM_ERR_UNSUPPORTED, "head dimension %d is not supported (%s)", D,
+                    any_dim ? "a multiple of 8 up to 128" : "32, 64 or 128");
     if (dtype != BAM_DTYPE_F16 && dtype != BAM_DTYPE_BF16)
         return fail(BAM_ERR_INVALID_ARGUMENT, "dtype %d is neither BAM_DTYPE_F16 nor BAM_DTYPE_BF16", dtype);
     static_assert(BAM_MAX_SEQLEN == bam::MAX_SEQLEN, "header and kernels disagree on the longest sequence");
@@ -158,7 +160,7 @@ int fill_plan(bam::AttnParams& p, const char* who, const bam_plan* plan, int B, 
         return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan: misaligned group order", who);
     p.group_order = plan->group_order;   // may be null
     // hand-over of dS from dK/dV to dQ: only with a workspace, for the head dim and lengths its kernels cover
-    if (plan->ds_workspace != nullptr && plan->ds_entry != nullptr && plan->ds_tile_base != nullptr && p.D == 128 &&
+    if (plan->ds_workspace != nullptr && plan->ds_entry != nullptr && plan->ds_tile_base != nullptr && p.D > 64 &&
         Sk <= bam::MAX_LIST * 64) {
         if (reinterpret_cast<uintptr_t>(plan->ds_workspace) & 15u)
             return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan: dS workspace is not 16-byte aligned", who);
@@ -199,7 +201,8 @@ void fill_sizes(bam::AttnParams& p, const MaskSource& m, int B, int Hq, int Hkv,
     p.Sk = m.Sk;
     p.Hq = Hq;
     p.Hkv = Hkv;
-    p.D = D;
+    p.D = D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128;
+    p.d = D;
     p.num_m = (m.Sq + 127) / 128;
     p.num_n = (m.Sk + 31) / 32;
     p.num_kt = (m.Sk + 127) / 128;
@@ -210,11 +213,12 @@ void fill_sizes(bam::AttnParams& p, const MaskSource& m, int B, int Hq, int Hkv,
 
 int fwd_impl(const char* who, const void* q, const void* k, const void* v, void* o, float* lse, const MaskSource& m,
              const int8_t* flags, const int64_t* st, int64_t flags_stride_b, int64_t flags_stride_m, int B, int Hq,
-             int Hkv, int D, float scale, int dtype, const bam_bias* bias, const bam_plan* plan, void* stream);
+             int Hkv, int D, float scale, int dtype, const bam_bias* bias, const bam_plan* plan, void* stream,
+             bool any_dim = false);
 int bwd_params(bam::AttnParams& p, const char* who, const void* q, const void* k, const void* v, const void* dout,
                const float* lse, const float* delta, void* dq, void* dk, void* dv, const MaskSource& m,
                const int8_t* flags, const int64_t* st, int B, int Hq, int Hkv, int D, float scale, int dtype,
-               int accumulate, bool need_dq, bool need_dkdv, const bam_bias* bias, const bam_plan* plan);
+               int accumulate, bool need_dq, bool need_dkdv, const bam_bias* bias, const bam_plan* plan, bool any_dim = false);
 
 }  // namespace
 
@@ -228,8 +232,9 @@ namespace {
 
 int fwd_impl(const char* who, const void* q, const void* k, const void* v, void* o, float* lse, const MaskSource& m,
              const int8_t* flags, const int64_t* st, int64_t flags_stride_b, int64_t flags_stride_m, int B, int Hq,
-             int Hkv, int D, float scale, int dtype, const bam_bias* bias, const bam_plan* plan, void* stream) {
-    BAM_TRY(check_problem(B, m.Sq, m.Sk, Hq, Hkv, D, dtype));
+             int Hkv, int D, float scale, int dtype, const bam_bias* bias, const bam_plan* plan, void* stream,
+             bool any_dim) {
+    BAM_TRY(check_problem(B, m.Sq, m.Sk, Hq, Hkv, D, dtype, any_dim));
     BAM_TRY(check_half_tensor("q", q, st[0], st[1], st[2]));
     BAM_TRY(check_half_tensor("k", k, st[3], st[4], st[5]));
     BAM_TRY(check_half_tensor("v", v, st[6], st[7], st[8]));
@@ -256,8 +261,8 @@ int fwd_impl(const char* who, const void* q, const void* k, const void* v, void*
 int bwd_params(bam::AttnParams& p, const char* who, const void* q, const void* k, const void* v, const void* dout,
                const float* lse, const float* delta, void* dq, void* dk, void* dv, const MaskSource& m,
                const int8_t* flags, const int64_t* st, int B, int Hq, int Hkv, int D, float scale, int dtype,
-               int accumulate, bool need_dq, bool need_dkdv, const bam_bias* bias, const bam_plan* plan) {
-    BAM_TRY(check_problem(B, m.Sq, m.Sk, Hq, Hkv, D, dtype));
+               int accumulate, bool need_dq, bool need_dkdv, const bam_bias* bias, const bam_plan* plan, bool any_dim) {
+    BAM_TRY(check_problem(B, m.Sq, m.Sk, Hq, Hkv, D, dtype, any_dim));
     BAM_TRY(check_half_tensor("q", q, st[0], st[1], st[2]));
     BAM_TRY(check_half_tensor("k", k, st[3], st[4], st[5]));
     BAM_TRY(check_half_tensor("v", v, st[6], st[7], st[8]));
@@ -732,14 +737,14 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
     const int64_t st[12] = {a->q.stride_b, a->q.stride_s, a->q.stride_h, a->k.stride_b, a->k.stride_s, a->k.stride_h,
                             a->v.stride_b, a->v.stride_s, a->v.stride_h, a->o.stride_b, a->o.stride_s, a->o.stride_h};
     return fwd_impl("bam_attn_fwd", a->q.ptr, a->k.ptr, a->v.ptr, a->o.ptr, a->lse, m, a->flags, st, a->flags_stride_b,
-                    a->flags_stride_m, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->bias, a->plan, stream);
+                    a->flags_stride_m, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->bias, a->plan, stream, true);
 }
 
 int bam_attn_bwd(const bam_attn* a, void* stream) {
     if (a == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: null pointer");
     MaskSource m;
     BAM_TRY(attn_source(a, m));
-    BAM_TRY(check_problem(a->B, m.Sq, m.Sk, a->Hq, a->Hkv, a->D, a->dtype));
+    BAM_TRY(check_problem(a->B, m.Sq, m.Sk, a->Hq, a->Hkv, a->D, a->dtype, true));
     BAM_TRY(check_half_tensor("o", a->o.ptr, a->o.stride_b, a->o.stride_s, a->o.stride_h));
     BAM_TRY(check_half_tensor("do", a->dout.ptr, a->dout.stride_b, a->dout.stride_s, a->dout.stride_h));
     const int runs = a->head_runs > 1 ? a->head_runs : 1;
@@ -761,7 +766,7 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
     bam::AttnParams all = {};
     BAM_TRY(bwd_params(all, "bam_attn_bwd", a->q.ptr, a->k.ptr, a->v.ptr, a->dout.ptr, a->lse, a->delta, a->dq.ptr, a->dk.ptr,
                        a->dv.ptr, m, a->flags, st, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->accumulate, true, true,
-                       a->bias, nullptr));
+                       a->bias, nullptr, true));
     all.o = {a->o.ptr, a->o.stride_b, a->o.stride_s, a->o.stride_h};
     BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
     // The heads in runs of whole kv heads, every run through the same dS workspace: the launches of a stream run in

@@ -167,15 +167,22 @@ __device__ __forceinline__ float load_bias1(const void* base, int64_t index, boo
 
 // ---------------------------------------------------------------------------------
 // LDS tile layout.  A tile is ROWS x D elements of 2 bytes, stored as 16-byte chunks;
-// chunk c of row r lives at chunk slot  r * (D/8) + (c ^ swz(r)).  The XOR pattern is a
+// chunk c of row r lives at chunk slot  r * (LDS_COLS/8) + (c ^ swz(r)).  The XOR pattern is a
 // one-bit rotation of the 256-byte line number.  Access shapes used by the kernels:
 //   * natural read  : 16 lanes read the same chunk column of 16 consecutive rows (conflict free);
 //   * transposed read (ds_read_b64_tr_b16): 16 lanes read a 4-row x 32-byte block (conflict free
 //     within the 16 lanes; the two blocks of a half wave overlap in two bank groups, which costs
 //     two cycles per instruction, hidden inside the four cycles a wave-wide LDS instruction takes).
+// Head dims.  The kernels are compiled for D = 32, 64, 96 and 128; a call's head dim d is any multiple of 8 up to D.  A
+// row of an LDS tile has room for LDS_COLS<D> elements (a power of two: the swizzle is an XOR over whole rows of chunks).
+// Chunks past d are never zero filled by the tile copies: their lanes fetch chunk 0 of the row again (tile_chunk), and
+// whoever multiplies along the head dim has zeros in the other operand there; columns past d of an output are computed
+// and not stored.  Before, other head dims were padded on the host: three copies of q, k, v and up to 37 launches a step.
+template <int D>
+constexpr int LDS_COLS = D <= 32 ? 32 : D <= 64 ? 64 : 128;
 template <int D>
 __device__ __forceinline__ int swz(int row) {
-    constexpr int NCH = D / 8;                                       // chunks per row: 4, 8, 16
+    constexpr int NCH = LDS_COLS<D> / 8;                             // chunks per row: 4, 8, 16
     constexpr int CB = (NCH == 16) ? 4 : (NCH == 8) ? 3 : 2;         // log2(NCH)
     const int line = (row >> (4 - CB)) & (NCH - 1);
     return ((line << 1) & (NCH - 1)) | (line >> (CB - 1));
@@ -183,7 +190,7 @@ __device__ __forceinline__ int swz(int row) {
 
 template <int D>
 __device__ __forceinline__ int chunk_slot(int row, int c) {
-    return row * (D / 8) + (c ^ swz<D>(row));
+    return row * (LDS_COLS<D> / 8) + (c ^ swz<D>(row));
 }
 
 // Natural MFMA operand: 8 consecutive elements (one chunk) of one row.

@@ -83,7 +83,8 @@ struct AttnParams {
     int64_t row_bits_sb, row_bits_sn;
     const unsigned* col_bits;
     int64_t col_bits_sb, col_bits_ss;
-    int B, Sq, Sk, Hq, Hkv, D;
+    int B, Sq, Sk, Hq, Hkv;
+    int D, d;                  // the D the kernels are compiled for (32, 64, 96, 128) and the head dim (<= D, a multiple of 8)
     int Sq_rounded, num_m, num_n, num_kt;  // ceil(Sq/128)*128, ceil(Sq/128), ceil(Sk/32), ceil(Sk/128)
     int64_t lse_sb;            // batch stride of lse and delta (a run of heads is a view of the tensors of all heads)
     float scale;

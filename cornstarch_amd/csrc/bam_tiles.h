@@ -64,20 +64,22 @@ __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)"
 // checks, so the offsets fit 32 bits.
 template <int D, int ROWS, int THREADS>
 struct TileStage {
-    static constexpr int NCH = D / 8;
+    static constexpr int NCH = LDS_COLS<D> / 8;
     static constexpr int CHUNKS = ROWS * NCH;
     static constexpr int CPT = (CHUNKS + THREADS - 1) / THREADS;
     static constexpr bool EXACT = (CHUNKS % THREADS) == 0;
     unsigned goff[CPT];
     int wave_first;  // first chunk slot this wave fills with instruction 0
 
-    __device__ __forceinline__ void setup(int64_t row_stride_bytes, int tid) {
+    // chunks: how many 16-byte chunks a row has in global memory (d / 8)
+    __device__ __forceinline__ void setup(int64_t row_stride_bytes, int chunks, int tid) {
         wave_first = __builtin_amdgcn_readfirstlane(tid & ~63);
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int id = tid + THREADS * i;
             const int row = id / NCH, pc = id % NCH;
-            goff[i] = (unsigned)(row * row_stride_bytes + (pc ^ swz<D>(row)) * 16);
+            const int c = pc ^ swz<D>(row);
+            goff[i] = (unsigned)(row * row_stride_bytes + (c < chunks ? c : 0) * 16);
         }
     }
     // tile_base: first row of the tile in global memory, tile_lds: lds_addr() of the LDS tile
@@ -116,20 +118,22 @@ struct TileStage {
 // inside one slice and only its (wave-uniform) base pointer depends on which.
 template <int D, int THREADS>
 struct SliceStage {
-    static constexpr int NCH = D / 8;
+    static constexpr int NCH = LDS_COLS<D> / 8;
     static constexpr int CHUNKS = 64 * NCH;
     static constexpr int CPT = (CHUNKS + THREADS - 1) / THREADS;
     static constexpr bool EXACT = (CHUNKS % THREADS) == 0;
     unsigned goff[CPT];
     int wave_first;  // first chunk slot this wave fills with instruction 0
 
-    __device__ __forceinline__ void setup(int64_t row_stride_bytes, int tid) {
+    // chunks: how many 16-byte chunks a row has in global memory (d / 8)
+    __device__ __forceinline__ void setup(int64_t row_stride_bytes, int chunks, int tid) {
         wave_first = __builtin_amdgcn_readfirstlane(tid & ~63);
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int id = tid + THREADS * i;
             const int row = id / NCH, pc = id % NCH;
-            goff[i] = (unsigned)((row & 31) * row_stride_bytes + (pc ^ swz<D>(row)) * 16);
+            const int c = pc ^ swz<D>(row);
+            goff[i] = (unsigned)((row & 31) * row_stride_bytes + (c < chunks ? c : 0) * 16);
         }
     }
     // lo / hi: first row of the two slices in global memory, tile_lds: lds_addr() of the LDS tile (wave-uniform)

@@ -8,7 +8,7 @@ int launch_bwd_dkdv_long(const AttnParams& p, int dtype, hipStream_t stream);  /
 
 template <typename T, int D>
 static int launch_pre_t(const AttnParams& p, hipStream_t stream) {
-    const int64_t threads = (int64_t)p.B * p.Sq * p.Hq * (D / 8);
+    const int64_t threads = (int64_t)p.B * p.Sq * p.Hq * (LDS_COLS<D> / 8);
     const int64_t blocks = (threads + 255) / 256;
     hipLaunchKernelGGL((bwd_preprocess_kernel<T, D>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
     return (int)hipGetLastError();

@@ -71,7 +71,7 @@ __device__ __forceinline__ u32x4 ds_block_read_transposed(const char* block, int
 
 template <typename T, int D>
 __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const AttnParams p) {
-    constexpr int NCH = D / 8, DB = D / 32;
+    constexpr int NCH = LDS_COLS<D> / 8, DB = D / 32;
     __shared__ u32x4 sK[2][DQS_KT * NCH];
     __shared__ u32x4 sDS[DQS_THREADS / 64][2][256];  // per wave and buffer: two 2 KiB blocks (key halves 0 and 1)
     __shared__ int sList[MAX_LIST];
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
     typedef TileStage<D, DQS_KT, DQS_THREADS> Stage;
     constexpr int CPT = Stage::CPT;
     Stage stK;
-    stK.setup(2 * p.k.ss, tid);
+    stK.setup(2 * p.k.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsDS = lds_addr(sDS) + wave * 8192u;
     constexpr unsigned TILE_BYTES = DQS_KT * NCH * 16;
     // records of this q head; record e (a slice x 128-key tile pair) is 8 KiB = four 2 KiB blocks
@@ -260,6 +260,7 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
+                if (32 * db + 8 * grp >= p.d) break;
                 u32x2 w;
                 w[0] = T::pack2(dq[db][4 * grp + 0] * factor, dq[db][4 * grp + 1] * factor);
                 w[1] = T::pack2(dq[db][4 * grp + 2] * factor, dq[db][4 * grp + 3] * factor);
@@ -271,6 +272,7 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
+                if (32 * db + 8 * grp >= p.d) break;
                 const int d0 = 32 * db + 8 * grp + 4 * hi;
                 f32x4 a = *(f32x4*)(dqp + d0);
 #pragma unroll

@@ -1,4 +1,4 @@
-// Backward of bitfield-masked attention: dQ from the dS blocks the dK/dV kernel stored (head dim 128).
+// Backward of bitfield-masked attention: dQ from the dS blocks the dK/dV kernel stored (head dims above 64).
 #include "bwd_dq_saved.h"
 
 namespace bam {
@@ -11,6 +11,7 @@ static int launch_dq_saved_t(const AttnParams& p, hipStream_t stream) {
 }
 
 int launch_bwd_dq_saved(const AttnParams& p, int dtype, hipStream_t stream) {
+    if (p.D == 96) return dtype == 1 ? launch_dq_saved_t<BF16, 96>(p, stream) : launch_dq_saved_t<F16, 96>(p, stream);
     return dtype == 1 ? launch_dq_saved_t<BF16, 128>(p, stream) : launch_dq_saved_t<F16, 128>(p, stream);
 }
 

@@ -17,10 +17,10 @@
 namespace bam {
 
 // ---------------------------------------------------------------------------------------
-// delta[b,h,i] = sum_d o * do   (fp32).  D/8 lanes per row, 16 bytes per lane per tensor.
+// delta[b,h,i] = sum_d o * do   (fp32).  LDS_COLS/8 lanes per row, 16 bytes per lane per tensor.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const AttnParams p) {
-    constexpr int LPR = D / 8;
+    constexpr int LPR = LDS_COLS<D> / 8;
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t row = gid / LPR;
     const int c = (int)(gid % LPR);
@@ -33,10 +33,13 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const AttnParams p)
         const int64_t bi = row / p.Hq;
         i = (int)(bi % p.Sq);
         b = (int)(bi / p.Sq);
-        const u32x4 ov = *(const u32x4*)((const char*)p.o.ptr +
-                                         2 * ((int64_t)b * p.o.sb + (int64_t)i * p.o.ss + (int64_t)h * p.o.sh) + c * 16);
-        const u32x4 gv = *(const u32x4*)((const char*)p.dout.ptr +
-                                         2 * ((int64_t)b * p.dout.sb + (int64_t)i * p.dout.ss + (int64_t)h * p.dout.sh) + c * 16);
+        u32x4 ov = {0u, 0u, 0u, 0u}, gv = {0u, 0u, 0u, 0u};
+        if (8 * c < p.d) {
+            ov = *(const u32x4*)((const char*)p.o.ptr +
+                                 2 * ((int64_t)b * p.o.sb + (int64_t)i * p.o.ss + (int64_t)h * p.o.sh) + c * 16);
+            gv = *(const u32x4*)((const char*)p.dout.ptr +
+                                 2 * ((int64_t)b * p.dout.sb + (int64_t)i * p.dout.ss + (int64_t)h * p.dout.sh) + c * 16);
+        }
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
             acc += T::to_float((unsigned short)(ov[x] & 0xFFFFu)) * T::to_float((unsigned short)(gv[x] & 0xFFFFu));
@@ -75,7 +78,7 @@ constexpr int DKDV_THREADS = 512;
 template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
-    constexpr int NCH = D / 8, KK = D / 16, DB = D / 32;
+    constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     __shared__ u32x4 sK[128 * NCH];
     __shared__ u32x4 sV[128 * NCH];
     __shared__ u32x4 sQ[2][DKDV_QT * NCH];
@@ -125,8 +128,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     // ---- K, V of the tile -> LDS (once) ---------------------------------------------------
     {
         TileStage<D, 128, DKDV_THREADS> stK, stV;
-        stK.setup(2 * p.k.ss, tid);
-        stV.setup(2 * p.v.ss, tid);
+        stK.setup(2 * p.k.ss, p.d / 8, tid);
+        stV.setup(2 * p.v.ss, p.d / 8, tid);
         const char* kb = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh + (int64_t)nt * 128 * p.k.ss);
         const char* vb = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)hk * p.v.sh + (int64_t)nt * 128 * p.v.ss);
         stK.load(kb, sK, Sk - nt * 128, tid);
@@ -157,14 +160,20 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     const float c2 = BIAS ? LOG2E : p.scale * LOG2E;  // with a bias the scores become scale * s + bias first
 
     // Flip the sign of every element of the V tile in LDS (once per workgroup, after the tile has landed and
-    // before anybody reads it; the caller brackets it with workgroup barriers).
+    // before anybody reads it; the caller brackets it with workgroup barriers).  Where the head dim is below D, the
+    // columns past it become zero in K and V: the Q and dO tiles hold other numbers there.
     auto negate_v_tile = [&]() {
 #pragma unroll
         for (int i = 0; i < (128 * NCH) / DKDV_THREADS; ++i) {
-            u32x4 x = sV[tid + DKDV_THREADS * i];
+            const int id = tid + DKDV_THREADS * i;
+            u32x4 x = sV[id];
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[e] ^= 0x80008000u;
-            sV[tid + DKDV_THREADS * i] = x;
+            if (p.d < D) {
+                const u32x4 z = {0u, 0u, 0u, 0u};
+                if (8 * ((id % NCH) ^ swz<D>(id / NCH)) >= p.d) sK[id] = x = z;
+            }
+            sV[id] = x;
         }
     };
     bool v_negated = false;
@@ -190,8 +199,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0);
     static_assert(NLOADS <= 2 * KK, "one copy per MFMA of the S / dP phase");
     Stage stQ, stDO;
-    stQ.setup(2 * p.q.ss, tid);
-    stDO.setup(2 * p.dout.ss, tid);
+    stQ.setup(2 * p.q.ss, p.d / 8, tid);
+    stDO.setup(2 * p.dout.ss, p.d / 8, tid);
     const unsigned ldsQ = lds_addr(sQ), ldsDO = lds_addr(sDO);
     constexpr unsigned TILE_BYTES = DKDV_QT * NCH * 16;
     // small rows of a tile: lse, delta and the two halves of the 64 int64 bitfields, 64 dwords each;
@@ -628,6 +637,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
+                    if (32 * db + 8 * grp >= p.d) break;
                     float a[4], c[4];
 #pragma unroll
                     for (int x = 0; x < 4; ++x) {
@@ -658,6 +668,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
+                    if (32 * db + 8 * grp >= p.d) break;
                     const int d0 = 32 * db + 8 * grp + 4 * hi;
                     f32x4 a = *(f32x4*)(dkp + d0), c = *(f32x4*)(dvp + d0);
 #pragma unroll
@@ -683,9 +694,9 @@ constexpr int DQ_THREADS = 256;
 
 // LONG: as in the dK/dV kernel, for more than MAX_LIST 64-key tiles.
 template <typename T, int D, int MODE, bool BIAS, bool LONG>
-__global__ __launch_bounds__(DQ_THREADS, D == 128 ? 2 : 3) void bwd_dq_kernel(const AttnParams p) {
+__global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
-    constexpr int NCH = D / 8, KK = D / 16, DB = D / 32;
+    constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     __shared__ u32x4 sK[2][DQ_KT * NCH];
     __shared__ u32x4 sV[2][DQ_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf[2][DQ_KT];  // raw bitfields of the tile's keys
@@ -722,7 +733,7 @@ __global__ __launch_bounds__(DQ_THREADS, D == 128 ? 2 : 3) void bwd_dq_kernel(co
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
             u32x4 zq = {0u, 0u, 0u, 0u}, zg = {0u, 0u, 0u, 0u};
-            if (qvalid) {
+            if (qvalid && 16 * kk + 8 * hi < p.d) {
                 zq = *(const u32x4*)(qp + (16 * kk + 8 * hi) * 2);
                 zg = *(const u32x4*)(gp + (16 * kk + 8 * hi) * 2);
             }
@@ -767,8 +778,8 @@ __global__ __launch_bounds__(DQ_THREADS, D == 128 ? 2 : 3) void bwd_dq_kernel(co
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0);
     static_assert(NLOADS <= 2 * KK, "one copy per MFMA of the first S / dP block");
     Stage stK, stV;
-    stK.setup(2 * p.k.ss, tid);
-    stV.setup(2 * p.v.ss, tid);
+    stK.setup(2 * p.k.ss, p.d / 8, tid);
+    stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);
     const unsigned ldsR = lds_addr(sRowBits);
     // DENSE: the packed mask rows of this wave's slice (null: no plan, the mask bytes are read instead)
@@ -998,6 +1009,7 @@ __global__ __launch_bounds__(DQ_THREADS, D == 128 ? 2 : 3) void bwd_dq_kernel(co
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
+                if (32 * db + 8 * grp >= p.d) break;
                 u32x2 w;
                 w[0] = T::pack2(dq[db][4 * grp + 0] * p.scale, dq[db][4 * grp + 1] * p.scale);
                 w[1] = T::pack2(dq[db][4 * grp + 2] * p.scale, dq[db][4 * grp + 3] * p.scale);
@@ -1009,6 +1021,7 @@ __global__ __launch_bounds__(DQ_THREADS, D == 128 ? 2 : 3) void bwd_dq_kernel(co
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
+                if (32 * db + 8 * grp >= p.d) break;
                 const int d0 = 32 * db + 8 * grp + 4 * hi;
                 f32x4 a = *(f32x4*)(dqp + d0);
 #pragma unroll
@@ -1058,10 +1071,12 @@ static int launch_dq_b(const AttnParams& p, hipStream_t stream) {
 #define BAM_DISPATCH(fn)                                       \
     if (dtype == 1) {                                          \
         if (p.D == 128) return fn<BF16, 128>(p, stream);       \
+        if (p.D == 96) return fn<BF16, 96>(p, stream);         \
         if (p.D == 64) return fn<BF16, 64>(p, stream);         \
         return fn<BF16, 32>(p, stream);                        \
     }                                                          \
     if (p.D == 128) return fn<F16, 128>(p, stream);            \
+    if (p.D == 96) return fn<F16, 96>(p, stream);              \
     if (p.D == 64) return fn<F16, 64>(p, stream);              \
     return fn<F16, 32>(p, stream);
 

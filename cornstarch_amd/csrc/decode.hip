@@ -72,8 +72,8 @@ __global__ __launch_bounds__(64, 2) void decode_split_kernel(const DecodeParams 
     const char* kbase = (const char*)p.k + 2 * ((int64_t)b * p.k_sb + (int64_t)hk * p.k_sh);
     const char* vbase = (const char*)p.v + 2 * ((int64_t)b * p.v_sb + (int64_t)hk * p.v_sh);
     TileStage<D, DEC_KT, 64> stK, stV;
-    stK.setup(2 * p.k_ss, lane);
-    stV.setup(2 * p.v_ss, lane);
+    stK.setup(2 * p.k_ss, D / 8, lane);
+    stV.setup(2 * p.v_ss, D / 8, lane);
 
     f32x16 o[DB];
 #pragma unroll

@@ -37,8 +37,8 @@ constexpr int FWD_THREADS = 256;
 // LONG: sequences of more than MAX_LIST 64-key tiles (131072 keys), walked in several passes; the short form has no
 // pass loop at all (a loop around the main loop costs registers and a few per cent).
 template <typename T, int D, int MODE, bool BIAS, bool LONG>
-__global__ __launch_bounds__(FWD_THREADS, D == 128 ? 2 : 3) void fwd_kernel(const AttnParams p) {
-    constexpr int NCH = D / 8, KK = D / 16, DB = D / 32;
+__global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const AttnParams p) {
+    constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     __shared__ u32x4 sK[2][FWD_KT * NCH];
     __shared__ u32x4 sV[2][FWD_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf[2][FWD_KT];  // raw bitfields of the tile's keys
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(FWD_THREADS, D == 128 ? 2 : 3) void fwd_kernel(cons
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
             u32x4 z = {0u, 0u, 0u, 0u};
-            if (qvalid) z = *(const u32x4*)(qp + (16 * kk + 8 * hi) * 2);
+            if (qvalid && 16 * kk + 8 * hi < p.d) z = *(const u32x4*)(qp + (16 * kk + 8 * hi) * 2);
             qreg[kk] = z;
         }
     }
@@ -131,8 +131,8 @@ __global__ __launch_bounds__(FWD_THREADS, D == 128 ? 2 : 3) void fwd_kernel(cons
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (BIAS ? 1 : 0);
     static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the S phase (and at most one behind it)");
     Stage stK, stV;
-    stK.setup(2 * p.k.ss, tid);
-    stV.setup(2 * p.v.ss, tid);
+    stK.setup(2 * p.k.ss, p.d / 8, tid);
+    stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);
     const unsigned ldsR = lds_addr(sRowBits);
     const char* bias_head = BIAS ? (const char*)p.bias + (p.bias_f32 ? 4 : 2) * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh) : nullptr;
@@ -482,6 +482,7 @@ __global__ __launch_bounds__(FWD_THREADS, D == 128 ? 2 : 3) void fwd_kernel(cons
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
+                if (32 * db + 8 * grp >= p.d) break;
                 u32x2 w;
                 w[0] = T::pack2(o[db][4 * grp + 0] * inv, o[db][4 * grp + 1] * inv);
                 w[1] = T::pack2(o[db][4 * grp + 2] * inv, o[db][4 * grp + 3] * inv);
@@ -511,10 +512,12 @@ template <bool LONG>
 static int launch_fwd_all(const AttnParams& p, int dtype, hipStream_t stream) {
     if (dtype == 1) {
         if (p.D == 128) return launch_fwd_t<BF16, 128, LONG>(p, stream);
+        if (p.D == 96) return launch_fwd_t<BF16, 96, LONG>(p, stream);
         if (p.D == 64) return launch_fwd_t<BF16, 64, LONG>(p, stream);
         return launch_fwd_t<BF16, 32, LONG>(p, stream);
     }
     if (p.D == 128) return launch_fwd_t<F16, 128, LONG>(p, stream);
+    if (p.D == 96) return launch_fwd_t<F16, 96, LONG>(p, stream);
     if (p.D == 64) return launch_fwd_t<F16, 64, LONG>(p, stream);
     return launch_fwd_t<F16, 32, LONG>(p, stream);
 }

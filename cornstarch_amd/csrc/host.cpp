@@ -1,6 +1,6 @@
 // Host side of the attention entry points in native code: argument checks, the caches of the last mask's flags and plan,
 // output allocation, the autograd node and the calls into libbam_hip.so.  Python keeps the public functions and whatever
-// is not in the usual form (other layouts, head dims that need padding, error reporting): every function here answers
+// is not in the usual form (other layouts, head dims that are no multiple of 8, error reporting): every function here answers
 // None for those and the caller takes its general path.
 //
 // Why native: a short forward + backward (2 x 283 tokens) kept the GPU busy for 84 us but took 332 us of Python --
@@ -281,7 +281,7 @@ const Cached& mask_flags(const Tensor& mask) {
 }
 
 // ------------------------------------------------------------------ calls
-bool head_dim_ready(int64_t d) { return d == 32 || d == 64 || d == 128; }
+bool head_dim_ready(int64_t d) { return d > 0 && d <= 128 && d % 8 == 0; }
 
 // the kernels' layout rules: unit stride along D, 16-byte aligned rows
 bool rows_ready(const Tensor& t, int64_t elems) {
@@ -384,7 +384,7 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     a.delta = delta.data_ptr<float>();
     a.accumulate = accumulate ? 1 : 0;
     Tensor ws;
-    if (plan && a.D == 128 && a.Sk <= 131072) {
+    if (plan && a.D > 64 && a.Sk <= 131072) {
         optional<py::gil_scoped_release> release;
         if (PyGILState_Check()) release.emplace();
         plan.core->wait_pairs();
@@ -601,7 +601,7 @@ optional<Tensor> decode(const Tensor& q, const Tensor& k, const Tensor& v, optio
     const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3), Hkv = k.size(1), Sk = k.size(2);
     if (!q.is_cuda() || (type != at::kHalf && type != at::kBFloat16) || k.scalar_type() != type || v.scalar_type() != type ||
         k.device() != q.device() || v.device() != q.device() || q.size(2) != 1 || k.sizes() != v.sizes() || k.size(0) != B ||
-        k.size(3) != D || !head_dim_ready(D) || q.numel() == 0 || k.numel() == 0 || Hq % Hkv != 0 || q.stride(3) != 1 ||
+        k.size(3) != D || (D != 32 && D != 64 && D != 128) || q.numel() == 0 || k.numel() == 0 || Hq % Hkv != 0 || q.stride(3) != 1 ||
         !rows_ready(k, 8) || !rows_ready(v, 8) || !plain(q) || !plain(k) || !plain(v))
         return c10::nullopt;
     const c10::DeviceGuard guard(q.device());

@@ -160,7 +160,7 @@ class _TilePlan(_host.PlanCore):
 
     def allocate_ds_workspace(self, nheads: int, head_dim: int, seqlen_k: int) -> Optional[torch.Tensor]:
         """The dS workspace of one backward call, or None where the hand-over does not apply."""
-        if head_dim != 128 or seqlen_k > 131072:
+        if head_dim <= 64 or seqlen_k > 131072:
             return None
         pairs = self.ds_pairs()
         nbytes = nheads * pairs * _DS_RECORD_BYTES
@@ -186,7 +186,7 @@ class _TilePlan(_host.PlanCore):
         dS workspace of one run stays within the limit, and beyond that more runs while a run's workspace is above
         ``_DS_RUN_TARGET`` and its dK/dV launch keeps ``_DS_RUN_MIN_WORKGROUPS`` workgroups.  1: all heads at once
         (also where the hand-over does not apply or no split helps: ``allocate_ds_workspace`` then decides)."""
-        if head_dim != 128 or seqlen_k > 131072 or nheads % nheads_k != 0:
+        if head_dim <= 64 or seqlen_k > 131072 or nheads % nheads_k != 0:
             return 1
         pairs = self.ds_pairs()
         limit = _ds_workspace_limit(self.workspace.device)

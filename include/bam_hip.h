@@ -8,7 +8,7 @@
  *   - q/k/v/o/do/dq/dk/dv are logically (B, S, H, D) with element strides for b, s, h and
  *     unit stride along D; 16-bit tensors need 16-byte aligned rows (pointer % 16 == 0,
  *     strides % 8 == 0), fp32 gradient buffers need pointer % 16 == 0, strides % 4 == 0;
- *   - D is 32, 64 or 128; Hq % Hkv == 0; kv head of q head h is h / (Hq / Hkv);
+ *   - D is 32, 64 or 128 (bam_attn_fwd / bam_attn_bwd: any multiple of 8 up to 128); Hq % Hkv == 0; kv head of q head h is h / (Hq / Hkv);
  *   - dtype: BAM_DTYPE_F16 or BAM_DTYPE_BF16;
  *   - flags: int8 (B, ceil(S/128), ceil(S/32)), unit stride along the last axis,
  *     0 = empty, 1 = partial, 2 = every in-range pair allowed;
@@ -96,7 +96,7 @@ typedef struct bam_bias {
  * dS hand-over.  The reference's backward computes dS once per tile and adds dS k to dq with fp32 atomics
  * (bitfield_attention.py:877-898); the atomic-free split used here (dK/dV kernel, dQ kernel) recomputes S and dP in
  * the dQ kernel.  When the caller provides a workspace (plan->ds_workspace, plan->ds_capacity >= *plan->ds_count,
- * head dim 128, at most 131072 keys), the dK/dV kernel also stores every 32 x 32 block of dS it computes
+ * head dim above 64, at most 131072 keys), the dK/dV kernel also stores every 32 x 32 block of dS it computes
  * (input dtype, as the reference rounds it, :877) and the dQ kernel becomes one GEMM over those blocks: 8 KiB per
  * (q head, pair).  With bam_bwd both kernels run in that order; with the separate entry points bam_bwd_dkdv* must be
  * called before bam_bwd_dq* with the same plan and workspace.  dq is then the sum of the very dS values that went
