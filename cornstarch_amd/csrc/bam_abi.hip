@@ -807,18 +807,21 @@ int bam_host_words_free(uint64_t* words) {
     return e == hipSuccess ? BAM_OK : fail(BAM_ERR_LAUNCH, "bam_host_words_free: %s", hipGetErrorString(e));
 }
 
+// the D the kernels are compiled for
+static int compiled_dim(int d) { return d <= 32 ? 32 : d <= 64 ? 64 : d <= 96 ? 96 : 128; }
+
 int64_t bam_decode_workspace_bytes(int B, int Sk, int Hq, int Hkv, int D, int window) {
-    if (B <= 0 || Sk <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || window < 0) return 0;
-    int nsplit = 1, tps = 1, rgs = 1;
-    bam::decode_split_plan(B, Hq, Hkv, Sk, window, &nsplit, &tps, &rgs);
-    return nsplit > 1 ? (int64_t)B * Hq * nsplit * (D + 2) * 4 : 0;
+    if (B <= 0 || Sk <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || D > 128 || window < 0) return 0;
+    const bam::DecodeSplit s = bam::decode_split(B, Hq, Hkv, Sk, compiled_dim(D), window);
+    return s.parts > 1 ? (int64_t)B * Hq * s.parts * (compiled_dim(D) + 2) * 4 : 0;
 }
 
-int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_stride_b, int64_t q_stride_h,
-               int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
-               int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D, float scale,
-               int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes, void* stream) {
-    BAM_TRY(check_problem(B, 1, Sk, Hq, Hkv, D, dtype));
+static int decode_impl(const void* q, const void* k, const void* v, void* o, int64_t q_stride_b, int64_t q_stride_h,
+                       int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
+                       int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D, float scale,
+                       int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes, uint32_t* counters,
+                       int64_t n_counters, bool any_dim, void* stream) {
+    BAM_TRY(check_problem(B, 1, Sk, Hq, Hkv, D, dtype, any_dim));
     BAM_TRY(check_half_tensor("k", k, k_stride_b, k_stride_s, k_stride_h));
     BAM_TRY(check_half_tensor("v", v, v_stride_b, v_stride_s, v_stride_h));
     if (q == nullptr || o == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_decode: null pointer");
@@ -827,12 +830,12 @@ int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_s
     if (!(scale > 0.f)) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_decode: softmax scale must be > 0 (got %g)", scale);
     if (window < 0) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_decode: window must be >= 0 (0 = none), got %d", window);
     if (!(softcap >= 0.f)) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_decode: softcap must be >= 0 (0 = none), got %g", softcap);
-    if ((int64_t)B * Hq > 0x7FFFFFFFll) return fail(BAM_ERR_UNSUPPORTED, "bam_decode: grid too large");
     bam::DecodeParams p = {};
-    bam::decode_split_plan(B, Hq, Hkv, Sk, window, &p.nsplit, &p.tiles_per_split, &p.row_groups);
-    if ((int64_t)B * p.row_groups > 65535 || Hkv > 65535)
-        return fail(BAM_ERR_UNSUPPORTED, "bam_decode: grid too large (B = %d, Hkv = %d)", B, Hkv);
-    if (p.nsplit > 1) {
+    p.D = compiled_dim(D);
+    p.d = D;
+    const bam::DecodeSplit s = bam::decode_split(B, Hq, Hkv, Sk, p.D, window);
+    if ((int64_t)B * Hq > 0x7FFFFFFFll || s.units * s.parts > 0x7FFFFFFFll) return fail(BAM_ERR_UNSUPPORTED, "bam_decode: grid too large");
+    if (s.parts > 1) {
         const int64_t need = bam_decode_workspace_bytes(B, Sk, Hq, Hkv, D, window);
         if (workspace == nullptr || workspace_bytes < need)
             return fail(BAM_ERR_INVALID_ARGUMENT, "bam_decode: workspace of %lld bytes, %lld needed",
@@ -840,8 +843,19 @@ int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_s
         if (reinterpret_cast<uintptr_t>(workspace) & 15u)
             return fail(BAM_ERR_INVALID_ARGUMENT, "bam_decode: workspace is not 16-byte aligned");
         p.ws_o = (float*)workspace;
-        p.ws_ml = p.ws_o + (int64_t)B * Hq * p.nsplit * D;
+        p.ws_ml = p.ws_o + (int64_t)B * Hq * s.parts * p.D;
+        // The last part merges where that is a short step.  Not in a captured graph: its replays may overlap the caller's
+        // eager calls, and the counters serve one call at a time.
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (counters != nullptr && s.units <= n_counters && s.parts <= 32 &&
+            hipStreamIsCapturing((hipStream_t)stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone)
+            p.counters = counters;
     }
+    p.row_groups = s.row_groups;
+    p.parts = s.parts;
+    p.first = s.first;
+    p.n_tiles = s.n_tiles;
+    p.o_vec = ((reinterpret_cast<uintptr_t>(o) & 7u) == 0 && o_stride_b % 4 == 0 && o_stride_h % 4 == 0) ? 1 : 0;
     p.q = q;
     p.k = k;
     p.v = v;
@@ -860,11 +874,29 @@ int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_s
     p.Sk = Sk;
     p.Hq = Hq;
     p.Hkv = Hkv;
-    p.D = D;
     p.window = window;
     p.scale = scale;
     p.softcap = softcap;
-    return launched(bam::launch_decode(p, dtype, (hipStream_t)stream), "bam_decode");
+    return launched(bam::launch_decode(p, s, dtype, (hipStream_t)stream), "bam_decode");
+}
+
+int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_stride_b, int64_t q_stride_h,
+               int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
+               int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D, float scale,
+               int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes, void* stream) {
+    return decode_impl(q, k, v, o, q_stride_b, q_stride_h, k_stride_b, k_stride_s, k_stride_h, v_stride_b, v_stride_s, v_stride_h,
+                       o_stride_b, o_stride_h, B, Sk, Hq, Hkv, D, scale, dtype, window, softcap, workspace, workspace_bytes,
+                       nullptr, 0, false, stream);
+}
+
+int bam_decode_counted(const void* q, const void* k, const void* v, void* o, int64_t q_stride_b, int64_t q_stride_h,
+                       int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
+                       int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D,
+                       float scale, int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes,
+                       uint32_t* counters, int64_t n_counters, void* stream) {
+    return decode_impl(q, k, v, o, q_stride_b, q_stride_h, k_stride_b, k_stride_s, k_stride_h, v_stride_b, v_stride_s, v_stride_h,
+                       o_stride_b, o_stride_h, B, Sk, Hq, Hkv, D, scale, dtype, window, softcap, workspace, workspace_bytes,
+                       counters, n_counters, true, stream);
 }
 
 int bam_mask_tile_flags(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m, int B,

@@ -95,17 +95,27 @@ struct DecodeParams {
     const void *q, *k, *v;         // q (B, Hq, D): q_sb, q_sh; k / v (B, Sk, Hkv, D): *_sb, *_ss, *_sh
     void* o;                       // (B, Hq, D) in the dtype of q
     int64_t q_sb, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh, o_sb, o_sh;
-    int B, Sk, Hq, Hkv, D;
+    int B, Sk, Hq, Hkv;
+    int D, d;                      // the D the kernel is compiled for and the head dim (a multiple of 8, <= D)
     int window;                    // > 0: only the last `window` keys are attended to
     float scale, softcap;          // softcap > 0: scores become softcap * tanh(score / softcap)
-    // How the keys are split over workgroups (decode_split_plan) and where the splits leave their partial results:
-    // ws_o (B, Hq, nsplit, D) unnormalized outputs, ws_ml (B, Hq, nsplit, 2) maximum (log2 domain) and sum; unused
-    // when nsplit == 1.  row_groups = ceil((Hq / Hkv) / 32): q heads of one kv head per workgroup, 32 at a time.
+    int o_vec;                     // groups of four columns of o are 8-byte aligned
+    // How the tiles are dealt to workgroups (decode_split) and where the parts of a unit leave their partial results:
+    // ws_o (B, Hq, parts, D) unnormalized outputs, ws_ml (B, Hq, parts, 2) maximum (log2 domain) and sum; unused when
+    // parts == 1.  counters (one per unit, zero): the last part to arrive merges; null: a second launch does.
     float* ws_o;
     float* ws_ml;
-    int nsplit, tiles_per_split, row_groups;
+    unsigned* counters;
+    int first, n_tiles;            // first key attended to, 32-key tiles from there
+    int row_groups, parts;
 };
-void decode_split_plan(int B, int Hq, int Hkv, int Sk, int window, int* nsplit, int* tiles_per_split, int* row_groups);
+struct DecodeSplit {
+    int64_t units;                 // B * Hkv * row_groups
+    int row_groups;                // q heads of one kv head, 32 at a time
+    int first, n_tiles;
+    int waves, parts;              // waves of a workgroup, workgroups of a unit
+};
+DecodeSplit decode_split(int B, int Hq, int Hkv, int Sk, int D, int window);
 
 int launch_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                       int64_t flags_stride_m, int B, int S, hipStream_t stream);
@@ -147,7 +157,7 @@ int launch_fwd(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_preprocess(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dkdv(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dq(const AttnParams& p, int dtype, hipStream_t stream);
-int launch_decode(const DecodeParams& p, int dtype, hipStream_t stream);
+int launch_decode(const DecodeParams& p, const DecodeSplit& s, int dtype, hipStream_t stream);
 // dK/dV that also stores dS (p.ds_ws), and the dQ kernel that consumes it; D = 128, plan required
 int launch_bwd_dkdv_save(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dq_saved(const AttnParams& p, int dtype, hipStream_t stream);

@@ -593,6 +593,20 @@ py::tuple index_view(const Tensor& bf, const Tensor& idx_q, const Tensor& idx_k,
     return py::make_tuple(py::make_tuple(bits, pos), plan.py_object());
 }
 
+// Counters of the decode step's merge, zero between calls, one set per stream: the calls of a stream run in order, those
+// of different streams may overlap.  32 KiB per stream that has decoded; given back when the process ends.
+constexpr int64_t kDecodeCounters = 8192;
+std::mutex g_counters_mutex;
+std::vector<std::pair<void*, Tensor>> g_counters;
+uint32_t* decode_counters(const Tensor& like, const Stream& stream) {
+    std::lock_guard<std::mutex> guard(g_counters_mutex);
+    for (const auto& [s, t] : g_counters)
+        if (s == (void*)stream.stream() && t.device() == like.device()) return (uint32_t*)t.data_ptr();
+    if (g_counters.size() >= 64) return nullptr;
+    g_counters.emplace_back((void*)stream.stream(), at::zeros({kDecodeCounters}, like.options().dtype(at::kInt)));
+    return (uint32_t*)g_counters.back().second.data_ptr();
+}
+
 // Decode step: query (B, Hq, 1, D), key / value (B, Hkv, Sk, D) -> (B, 1, Hq, D)
 optional<Tensor> decode(const Tensor& q, const Tensor& k, const Tensor& v, optional<double> scaling, int64_t window,
                         double softcap) {
@@ -601,20 +615,25 @@ optional<Tensor> decode(const Tensor& q, const Tensor& k, const Tensor& v, optio
     const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3), Hkv = k.size(1), Sk = k.size(2);
     if (!q.is_cuda() || (type != at::kHalf && type != at::kBFloat16) || k.scalar_type() != type || v.scalar_type() != type ||
         k.device() != q.device() || v.device() != q.device() || q.size(2) != 1 || k.sizes() != v.sizes() || k.size(0) != B ||
-        k.size(3) != D || (D != 32 && D != 64 && D != 128) || q.numel() == 0 || k.numel() == 0 || Hq % Hkv != 0 || q.stride(3) != 1 ||
+        k.size(3) != D || !head_dim_ready(D) || q.numel() == 0 || k.numel() == 0 || Hq % Hkv != 0 || q.stride(3) != 1 ||
         !rows_ready(k, 8) || !rows_ready(v, 8) || !plain(q) || !plain(k) || !plain(v))
         return c10::nullopt;
     const c10::DeviceGuard guard(q.device());
     const at::NoGradGuard no_grad;
     Tensor out = at::empty({B, 1, Hq, D}, q.options());
     const int64_t bytes = bam_decode_workspace_bytes((int)B, (int)Sk, (int)Hq, (int)Hkv, (int)D, (int)window);
+    const Stream stream = current_stream(q.device());
     Tensor ws;
-    if (bytes > 0) ws = at::empty({bytes}, q.options().dtype(at::kByte));
-    check(bam_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), q.stride(0), q.stride(1), k.stride(0), k.stride(2),
+    uint32_t* counters = nullptr;
+    if (bytes > 0) {
+        ws = at::empty({bytes}, q.options().dtype(at::kByte));
+        counters = decode_counters(q, stream);
+    }
+    check(bam_decode_counted(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), q.stride(0), q.stride(1), k.stride(0), k.stride(2),
                      k.stride(1), v.stride(0), v.stride(2), v.stride(1), Hq * D, D, (int)B, (int)Sk, (int)Hq, (int)Hkv, (int)D,
                      (float)(scaling ? *scaling : 1.0 / std::sqrt((double)D)),
                      type == at::kBFloat16 ? BAM_DTYPE_BF16 : BAM_DTYPE_F16, (int)window, (float)softcap,
-                     bytes > 0 ? ws.data_ptr() : nullptr, bytes, current_stream(q.device()).stream()),
+                     bytes > 0 ? ws.data_ptr() : nullptr, bytes, counters, kDecodeCounters, stream.stream()),
           "bam_decode");
     return out;
 }
@@ -688,7 +707,10 @@ PYBIND11_MODULE(_bam_host, m) {
         Cached gone;
         std::swap(g_mask, gone);
     });
-    m.def("release_host_memory", []() { count_words().release(); });
+    m.def("release_memory", []() {
+        count_words().release();
+        g_counters.clear();
+    });
     // what tells a tensor (and its contents) from another for the caches that live in Python
     m.def("tensor_key", [](const Tensor& t) {
         std::string key;

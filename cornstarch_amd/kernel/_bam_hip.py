@@ -144,6 +144,7 @@ SIGNATURES = {
     "bam_bwd_dq_indexed": [_ptr] * 7 + [_view, _ptr] + [_i64] * 17 + [_int] * 4 + [_f32, _int, _int, _bias, _plan, _ptr],
     "bam_attn_fwd": [_attn, _ptr],
     "bam_attn_bwd": [_attn, _ptr],
+    "bam_decode_counted": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr, _i64, _ptr],
     "bam_decode": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr],
 }
 

@@ -123,7 +123,7 @@ def _release_device_state() -> None:
         pass
     BitfieldUtils.clear_cache()
     _host.forget_mask()
-    _host.release_host_memory()
+    _host.release_memory()
 
 
 atexit.register(_release_device_state)

@@ -433,6 +433,16 @@ int bam_decode(const void* q, const void* k, const void* v, void* o, int64_t q_s
                int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
                int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D, float scale,
                int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes, void* stream);
+/*
+ * The same for head dims of any multiple of 8 up to 128, in one launch where it can: with `counters` (device, n_counters
+ * uint32, all zero; null = as bam_decode) the workgroup that finishes a (batch, kv head) last merges its partial results.
+ * A call leaves the counters zero again; calls that may overlap on the GPU (other streams) need counters of their own.
+ */
+int bam_decode_counted(const void* q, const void* k, const void* v, void* o, int64_t q_stride_b, int64_t q_stride_h,
+                       int64_t k_stride_b, int64_t k_stride_s, int64_t k_stride_h, int64_t v_stride_b, int64_t v_stride_s,
+                       int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h, int B, int Sk, int Hq, int Hkv, int D,
+                       float scale, int dtype, int window, float softcap, void* workspace, int64_t workspace_bytes,
+                       uint32_t* counters, int64_t n_counters, void* stream);
 
 /*
  * Struct form of the attention calls: what bam_fwd*, bam_bwd_preprocess and bam_bwd_dkdv* / bam_bwd_dq* take, in one
