@@ -497,20 +497,38 @@ int bam_plan_indexed(const bam_index_view* iv, void* workspace, int64_t workspac
     return bam_plan_indexed_counted(iv, workspace, workspace_bytes, B, plan, nullptr, 0, stream);
 }
 
-int bam_plan_indexed_counted(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
-                             uint64_t* count_host, uint32_t count_tag, void* stream) {
+static int plan_indexed(const char* who, const bam_index_view* iv, const int64_t* bf, int64_t bf_stride_b, int L,
+                        const int64_t* idx_q, const int64_t* idx_k, void* workspace, int64_t workspace_bytes, int B,
+                        bam_plan* plan, uint64_t* count_host, uint32_t count_tag, void* stream) {
     MaskSource m;
     BAM_TRY(indexed_source(iv, m));
-    if (B <= 0 || m.Sq <= 0 || m.Sk <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_plan_indexed: B, Sq and Sk must be positive");
-    if (B > 65535) return fail(BAM_ERR_UNSUPPORTED, "bam_plan_indexed: B is limited to 65535 (got %d)", B);
+    if (B <= 0 || m.Sq <= 0 || m.Sk <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "%s: B, Sq and Sk must be positive", who);
+    if (B > 65535) return fail(BAM_ERR_UNSUPPORTED, "%s: B is limited to 65535 (got %d)", who, B);
     PlanLayout l;
-    BAM_TRY(place_plan("bam_plan_indexed", workspace, workspace_bytes, B, m.Sq, m.Sk, plan, l));
+    BAM_TRY(place_plan(who, workspace, workspace_bytes, B, m.Sq, m.Sk, plan, l));
     char* w = (char*)workspace;
-    BAM_TRY(launched(bam::launch_indexed_plan(m.bfq, m.bfq_sb, m.bfk, m.bfk_sb, m.posq, m.posk, m.Sq, m.Sk,
-                                              (uint8_t*)(w + l.fine_off), l.fine_sb, l.fine_ss, (int*)(w + l.order_off),
-                                              l.order_sb, (int*)(w + l.count_off), B, (hipStream_t)stream),
-                     "bam_plan_indexed"));
-    return number_pairs("bam_plan_indexed", plan, l, workspace, count_host, count_tag, stream);
+    BAM_TRY(launched(bam::launch_indexed_plan(bf, bf_stride_b, L, idx_q, idx_k, const_cast<int64_t*>(m.bfq), m.bfq_sb,
+                                              const_cast<int64_t*>(m.bfk), m.bfk_sb, const_cast<int*>(m.posq),
+                                              const_cast<int*>(m.posk), m.Sq, m.Sk, (uint8_t*)(w + l.fine_off), l.fine_sb,
+                                              l.fine_ss, (int*)(w + l.order_off), l.order_sb, (int*)(w + l.count_off), B,
+                                              (hipStream_t)stream),
+                     who));
+    return number_pairs(who, plan, l, workspace, count_host, count_tag, stream);
+}
+
+int bam_plan_indexed_counted(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
+                             uint64_t* count_host, uint32_t count_tag, void* stream) {
+    return plan_indexed("bam_plan_indexed", iv, nullptr, 0, 0, nullptr, nullptr, workspace, workspace_bytes, B, plan, count_host,
+                        count_tag, stream);
+}
+
+int bam_gather_plan_indexed(const int64_t* bf, int64_t bf_stride_b, int L, const int64_t* idx_q, const int64_t* idx_k,
+                            const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
+                            uint64_t* count_host, uint32_t count_tag, void* stream) {
+    if (bf == nullptr || idx_q == nullptr || idx_k == nullptr || L <= 0)
+        return fail(BAM_ERR_INVALID_ARGUMENT, "bam_gather_plan_indexed: null pointer or empty sequence");
+    return plan_indexed("bam_gather_plan_indexed", iv, bf, bf_stride_b, L, idx_q, idx_k, workspace, workspace_bytes, B, plan,
+                        count_host, count_tag, stream);
 }
 
 int bam_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m, void* workspace,

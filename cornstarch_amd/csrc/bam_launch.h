@@ -132,10 +132,12 @@ int launch_mask_tile_flags(const uint8_t* mask, int8_t* flags, int64_t flags_str
                            int Sq, int Sk, hipStream_t stream);
 int launch_gather_bitfields(const int64_t* bf, int64_t bf_stride_b, int L, const int64_t* idx, int n, int64_t* out_bits,
                             int64_t out_stride_b, int* out_pos, int B, hipStream_t stream);
-// Plan (fine classes + slice order) of index-tensor attention, from the gathered bitfields and positions.
-int launch_indexed_plan(const int64_t* qbits, int64_t qbits_sb, const int64_t* kbits, int64_t kbits_sb, const int* qpos,
-                        const int* kpos, int Sq, int Sk, uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int* order,
-                        int64_t order_sb, int* pair_count, int B, hipStream_t stream);
+// Plan (fine classes + slice order) of index-tensor attention: from gathered bitfields and positions, or (idx_q, idx_k not
+// null) from the global bitfields bf (B, L) through index tensors, leaving the gathered arrays in qbits .. kpos.
+int launch_indexed_plan(const int64_t* bf, int64_t bf_sb, int L, const int64_t* idx_q, const int64_t* idx_k, int64_t* qbits,
+                        int64_t qbits_sb, int64_t* kbits, int64_t kbits_sb, int* qpos, int* kpos, int Sq, int Sk, uint8_t* fine,
+                        int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B,
+                        hipStream_t stream);
 // Flags plus plan of a materialized bool mask.
 int launch_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m,
                           uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count,

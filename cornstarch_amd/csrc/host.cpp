@@ -573,22 +573,24 @@ py::tuple index_view(const Tensor& bf, const Tensor& idx_q, const Tensor& idx_k,
     int* qp = pos.data_ptr<int>();
     bam_index_view& iv = *reinterpret_cast<bam_index_view*>(view);
     iv = bam_index_view{qb, qb + B * Sq, qp, qp + Sq, Sq, Sk, (int32_t)Sq, (int32_t)Sk};
-    check(bam_gather_bitfields(bf.data_ptr<int64_t>(), bf.stride(0), (int)bf.size(1), idx_q.data_ptr<int64_t>(), (int)Sq, qb, Sq,
-                               qp, (int)B, stream.stream()),
-          "bam_gather_bitfields");
-    check(bam_gather_bitfields(bf.data_ptr<int64_t>(), bf.stride(0), (int)bf.size(1), idx_k.data_ptr<int64_t>(), (int)Sk,
-                               qb + B * Sq, Sk, qp + Sq, (int)B, stream.stream()),
-          "bam_gather_bitfields");
     const int64_t bytes = bam_plan_workspace_bytes_rect((int)B, (int)Sq, (int)Sk);
     Plan plan;
     if (bytes > 0) {
         plan = new_plan();
         PlanCore& c = *plan.core;
         c.prepare(at::empty({bytes}, bf.options().dtype(at::kByte)), stream);
-        const int rc = bam_plan_indexed_counted(&iv, c.workspace.data_ptr(), bytes, (int)B, &c.plan, c.word.at, c.word.tag,
-                                                stream.stream());
+        const int rc = bam_gather_plan_indexed(bf.data_ptr<int64_t>(), bf.stride(0), (int)bf.size(1), idx_q.data_ptr<int64_t>(),
+                                               idx_k.data_ptr<int64_t>(), &iv, c.workspace.data_ptr(), bytes, (int)B, &c.plan,
+                                               c.word.at, c.word.tag, stream.stream());
         if (rc != BAM_OK) c.abandon();
-        check(rc, "bam_plan_indexed");
+        check(rc, "bam_gather_plan_indexed");
+    } else {  // no plan for so many rows
+        check(bam_gather_bitfields(bf.data_ptr<int64_t>(), bf.stride(0), (int)bf.size(1), idx_q.data_ptr<int64_t>(), (int)Sq, qb,
+                                   Sq, qp, (int)B, stream.stream()),
+              "bam_gather_bitfields");
+        check(bam_gather_bitfields(bf.data_ptr<int64_t>(), bf.stride(0), (int)bf.size(1), idx_k.data_ptr<int64_t>(), (int)Sk,
+                                   qb + B * Sq, Sk, qp + Sq, (int)B, stream.stream()),
+              "bam_gather_bitfields");
     }
     return py::make_tuple(py::make_tuple(bits, pos), plan.py_object());
 }

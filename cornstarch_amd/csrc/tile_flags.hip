@@ -3,6 +3,7 @@
 // Reference: cornstarch/kernel/bitfield_attention.py:60-156.
 #include "bam_common.h"
 #include "bam_launch.h"
+#include <type_traits>
 
 namespace bam {
 
@@ -26,31 +27,35 @@ constexpr int FLAG_MAX_BLOCKS_X = 64;  // workgroups per 128-row block; longer r
 // Every slice gets a two-word sort key and is ranked against all others of its sequence (at most
 // MAX_PLAN_SLICES of them); slots past the last slice are set to -1.  The work rides in the launch of the flag
 // kernel, as extra workgroups of its grid (it needs the bitfields only): workgroup `part` of sequence b ranks
-// slices [256 part, +256).
-// Ranks the slices [256 part, +256) of one sequence among all `ns` slices by two-word keys (distinct for distinct
+// slices [64 part, +64).
+// Ranks the slices [64 part, +64) of one sequence among all `ns` slices by two-word keys (distinct for distinct
 // slices; slices >= ns get the largest key) and writes order_row[rank] = slice; the slots past the last slice are set
-// to -1.  `fill(base, sk)` puts the keys of slices [base, base + 256) into sk[2 i], sk[2 i + 1] (all 256 threads take
-// part).  The compares read the keys eight at a time, so that the loop runs at the rate of the LDS and not at its
-// latency.
+// to -1.  `fill(base, sk)` puts the keys of slices [base, min(base + 256, ns)) into sk[2 i], sk[2 i + 1] (all 256 threads
+// take part).  Four threads share a slice and compare it with a quarter of every chunk each, eight keys per step, so that
+// the loop runs at the rate of the LDS and not at its latency.  (With one thread per slice and whole chunks of 256 keys
+// whatever the length, this column of workgroups was what the launch waited for: 11 us of it at 283 tokens.)
+constexpr int RANKED_PER_GROUP = 64;
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 template <typename FillFn>
 __device__ __forceinline__ void slice_order_ranked(FillFn fill, int ns, int slots, int part, int* __restrict__ order_row) {
     __shared__ __attribute__((aligned(16))) unsigned long long sk[2 * 256];
-    const int tid = threadIdx.x, s = part * 256 + tid;
+    const int tid = threadIdx.x, s = part * RANKED_PER_GROUP + (tid >> 2), sub = tid & 3;
     unsigned long long my1 = 0, my2 = 0;
     int rank = 0;
-    // this workgroup's own slices first (their keys are what the others are compared with), then the other chunks
-    const int nchunks = (ns + 255) / 256;
+    // the chunk that holds this workgroup's own slices first (their keys are what the others are compared with)
+    const int own = part * RANKED_PER_GROUP / 256, nchunks = max(own + 1, (ns + 255) / 256);
     for (int c = 0; c < nchunks; ++c) {
-        const int base = 256 * (c == 0 ? part : c <= part ? c - 1 : c);
+        const int base = 256 * (c == 0 ? own : c <= own ? c - 1 : c), n = min(256, ns - base);
         __syncthreads();
         fill(base, sk);
+        // the last step of eight reads past the last key
+        if (tid < 32 && n + tid < 256 && n + tid < ((max(n, 0) + 31) & ~31)) sk[2 * (n + tid)] = sk[2 * (n + tid) + 1] = ~0ull;
         __syncthreads();
         if (c == 0) {
-            my1 = sk[2 * tid];
-            my2 = sk[2 * tid + 1];
+            my1 = sk[2 * (s & 255)];
+            my2 = sk[2 * (s & 255) + 1];
         }
-        for (int j0 = 0; j0 < 256; j0 += 8) {  // entries past the last slice hold the largest key: never smaller
+        for (int j0 = 8 * sub; j0 < n; j0 += 32) {  // entries past the last slice hold the largest key: never smaller
             u64x2 o[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) o[u] = *(const u64x2*)&sk[2 * (j0 + u)];
@@ -58,6 +63,9 @@ __device__ __forceinline__ void slice_order_ranked(FillFn fill, int ns, int slot
             for (int u = 0; u < 8; ++u) rank += (o[u][0] < my1 || (o[u][0] == my1 && o[u][1] < my2)) ? 1 : 0;
         }
     }
+    rank += __shfl_xor(rank, 1);
+    rank += __shfl_xor(rank, 2);
+    if (sub != 0) return;
     if (s < ns)
         order_row[rank] = s;
     else if (s < slots)
@@ -80,22 +88,24 @@ __device__ __forceinline__ void slice_keys_chunk(const int64_t* __restrict__ row
                                                  unsigned long long* sk) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t M = (((int64_t)1) << 62) - 1;
-#pragma unroll 4
-    for (int pass = 0; pass < 16; ++pass) {
-        const int local = 64 * wave + 4 * pass + (lane >> 4);  // slice within the chunk
-        const int s = base + local;
-        const int i = s * 32 + 2 * (lane & 15);
-        const int64_t f0 = i < S ? row[i] : 0, f1 = i + 1 < S ? row[i + 1] : 0;
-        const uint64_t f = (uint64_t)(f0 | f1);
-        const unsigned lo = row_or((unsigned)f), hi = row_or((unsigned)(f >> 32));
-        if ((lane & 15) == 0) {
-            const bool text = (lo & 1u) != 0;
-            const unsigned long long sig = (((unsigned long long)hi << 32) | lo) & (unsigned long long)M;
-            unsigned long long k1 = text ? 0ull : (1ull << 62) | sig;
-            unsigned long long k2 = text ? (unsigned long long)(ns - 1 - s) : (unsigned long long)s;
-            if (s >= ns) k1 = k2 = ~0ull;
-            sk[2 * local] = k1;
-            sk[2 * local + 1] = k2;
+    const int n = min(256, ns - base);
+    for (int s0 = 0; s0 < n; s0 += 128) {  // eight slices per 16 lanes at a time: one memory latency for 128 slices
+        uint64_t f[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = (base + s0 + 16 * u + 4 * wave + (lane >> 4)) * 32 + 2 * (lane & 15);
+            f[u] = (uint64_t)((i < S ? row[i] : 0) | (i + 1 < S ? row[i + 1] : 0));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int local = s0 + 16 * u + 4 * wave + (lane >> 4), s = base + local;  // local: slice within the chunk
+            const unsigned lo = row_or((unsigned)f[u]), hi = row_or((unsigned)(f[u] >> 32));
+            if ((lane & 15) == 0 && local < n) {
+                const bool text = (lo & 1u) != 0;
+                const unsigned long long sig = (((unsigned long long)hi << 32) | lo) & (unsigned long long)M;
+                sk[2 * local] = text ? 0ull : (1ull << 62) | sig;
+                sk[2 * local + 1] = text ? (unsigned long long)(ns - 1 - s) : (unsigned long long)s;
+            }
         }
     }
 }
@@ -110,30 +120,66 @@ __device__ __forceinline__ void slice_order_part(const int64_t* __restrict__ row
 // The same ordering idea for index-tensor attention, where a local row's position is pos[row]: slices holding a
 // text row first, by descending largest position; then modality-only slices grouped by the OR of their bitfields,
 // by ascending smallest position.  The slice number in the low bits keeps the keys distinct whatever the positions.
-__device__ __forceinline__ void slice_sort_key_indexed(const int64_t* __restrict__ bits, const int* __restrict__ pos,
-                                                       int S, int ns, int s, unsigned long long& k1,
-                                                       unsigned long long& k2) {
-    k1 = ~0ull;
-    k2 = ~0ull;
-    if (s >= ns) return;
+__device__ __forceinline__ int row_max(int x) {  // over the 16 lanes of a DPP row, result in every lane
+    x = max(x, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false));
+    x = max(x, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false));
+    x = max(x, __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false));
+    return max(x, __builtin_amdgcn_mov_dpp(x, 0x140, 0xF, 0xF, false));
+}
+// Bitfields and positions of the local rows (or keys): gathered arrays, or -- for the launch that does the gathering --
+// the global bitfields seen through an index tensor.
+struct GatheredRows {
+    const int64_t* bits;
+    const int* positions;
+    __device__ __forceinline__ void get(int i, int64_t& f, int& pos) const {
+        f = bits[i];
+        pos = positions[i];
+    }
+};
+struct IndexedRows {
+    const int64_t* bf;
+    const int64_t* idx;
+    int L;
+    __device__ __forceinline__ void get(int i, int64_t& f, int& pos) const {
+        const int64_t p = idx[i];
+        f = (p >= 0 && p < L) ? bf[p] : 0;
+        pos = (int)(p < 0 ? 0 : p > 0x7FFFFFFE ? 0x7FFFFFFE : p);
+    }
+};
+
+template <typename Rows>
+__device__ __forceinline__ void slice_keys_chunk_indexed(const Rows& rows, int S, int ns, int base, unsigned long long* sk) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t M = (((int64_t)1) << 62) - 1;
-    int64_t sig = 0;
-    bool text = false;
-    int pmax = 0, pmin = 0x7FFFFFFF;
+    const int n = min(256, ns - base);
+    for (int s0 = 0; s0 < n; s0 += 64) {
+        int64_t f[4][2];
+        int p[4][2];
 #pragma unroll
-    for (int r = 0; r < 32; ++r) {
-        const int i = s * 32 + r;
-        const int64_t f = i < S ? bits[i] : 0;
-        const int q = i < S ? pos[i] : 0;
-        sig |= f & M;
-        text |= (f & 1) != 0;
-        if (i < S) {
-            pmax = max(pmax, q);
-            pmin = min(pmin, q);
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                const int i = (base + s0 + 16 * u + 4 * wave + (lane >> 4)) * 32 + 2 * (lane & 15) + x;
+                f[u][x] = 0;
+                p[u][x] = -1;  // no such row
+                if (i < S) rows.get(i, f[u][x], p[u][x]);
+            }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int local = s0 + 16 * u + 4 * wave + (lane >> 4), s = base + local;
+            const uint64_t both = (uint64_t)(f[u][0] | f[u][1]);
+            const unsigned lo = row_or((unsigned)both), hi = row_or((unsigned)(both >> 32));
+            const int hi_pos = max(0, row_max(max(p[u][0], p[u][1])));
+            const int first = p[u][0] < 0 ? 0x7FFFFFFF : p[u][1] < 0 ? p[u][0] : min(p[u][0], p[u][1]);
+            const int lo_pos = -row_max(-first);
+            if ((lane & 15) == 0 && local < n) {
+                const bool text = (lo & 1u) != 0;
+                const unsigned long long sig = (((unsigned long long)hi << 32) | lo) & (unsigned long long)M;
+                sk[2 * local] = text ? 0ull : (1ull << 62) | sig;
+                sk[2 * local + 1] = ((unsigned long long)(text ? 0x7FFFFFFF - hi_pos : lo_pos) << 20) | (unsigned long long)s;
+            }
         }
     }
-    k1 = text ? 0ull : (1ull << 62) | (unsigned long long)sig;
-    k2 = ((unsigned long long)(text ? 0x7FFFFFFF - pmax : pmin) << 20) | (unsigned long long)s;
 }
 
 // FINE: also write the class of every 32-row x 32-column tile (the four row slices of each flag tile) to
@@ -153,7 +199,7 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void tile_flags_kernel(const int64
         *pair_count = 0;
     if (FINE && (int)blockIdx.x >= flag_blocks_x) {  // the workgroups that sort the slices (see slice_order_part)
         const int part = blockIdx.y;
-        if (part * 256 < 4 * (int)gridDim.y)
+        if (part * RANKED_PER_GROUP < 4 * (int)gridDim.y)
             slice_order_part(bf + (int64_t)blockIdx.z * bf_stride_b, S, part, order + (int64_t)blockIdx.z * order_sb);
         return;
     }
@@ -165,13 +211,24 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void tile_flags_kernel(const int64
     const int b = blockIdx.z, m = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t* row = bf + (int64_t)b * bf_stride_b;
+    // the key bitfields of both tiles of this wave, requested together (one memory latency instead of one per tile), and
+    // for the first group before the workgroup waits for its row bitfields
+    const int half = lane >> 5, l32 = lane & 31;
+    int64_t kfs[FLAG_TILES_PER_WAVE];
+    auto request_keys = [&](int bx) {
+#pragma unroll
+        for (int t = 0; t < FLAG_TILES_PER_WAVE; ++t) {
+            const int j = (bx * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + t) * BLOCK_N + l32;
+            kfs[t] = (j < S) ? row[j] : 0;
+        }
+    };
+    request_keys(blockIdx.x);
     if (tid < BLOCK_M) {
         const int i = m * BLOCK_M + tid;
         q_bits[tid] = (i < S) ? row[i] : 0;  // out-of-range positions read 0 (reference :86-87)
     }
     __syncthreads();
     const int rows_in_range = min(BLOCK_M, S - m * BLOCK_M);
-    const int half = lane >> 5, l32 = lane & 31;
     // Runs of equal bitfields inside each of the four 32-row slices: bit r of slice_starts[w] = row r starts a run
     // (rows past the end of the sequence read 0 and make a run of their own).  The count of a column over a run
     // follows from one evaluation of the bit test, so a tile costs one evaluation per run, not one per row.
@@ -194,13 +251,7 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void tile_flags_kernel(const int64
         if (tid < 5 * FLAG_COLS_PER_BLOCK) s_out[0][tid] = 0;
         __syncthreads();
         static_assert(FLAG_TILES_PER_WAVE == 2, "the counting path gives each half of a wave one tile");
-        // the key bitfields of both tiles of this wave, requested together (one memory latency instead of one per tile)
-        int64_t kfs[FLAG_TILES_PER_WAVE];
-#pragma unroll
-        for (int t = 0; t < FLAG_TILES_PER_WAVE; ++t) {
-            const int j = (bx * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + t) * BLOCK_N + l32;
-            kfs[t] = (j < S) ? row[j] : 0;
-        }
+        if (it > 0) request_keys(bx);
         bool counted[FLAG_TILES_PER_WAVE];  // wave-uniform: the tile still needs the counting path
 #pragma unroll
         for (int t = 0; t < FLAG_TILES_PER_WAVE; ++t) {
@@ -390,70 +441,104 @@ int launch_flag_row_workloads(const int8_t* flags, int64_t flags_stride_b, int64
     return (int)hipGetLastError();
 }
 
-// Plan for index-tensor attention: the class of every 32-row x 32-key tile of the LOCAL score matrix (rows and keys
-// are gathered subsets of a global sequence: bits / positions per local row and key, as bam_gather_bitfields
-// delivers them) and a slice order.  Brute force over the pairs of each tile, same wave layout as the flag kernel:
-// lane = key column (lane & 31) x 64-row half (lane >> 5).  The extra column of workgroups ranks the slices.
+// Plan for index-tensor attention: the class of every 32-row x 32-key tile of the LOCAL score matrix (rows and keys are
+// subsets of a global sequence) and a slice order.  Same counting as the flag kernel: a run is a stretch of rows of one
+// slice with equal bitfields at consecutive positions, and a column's count over a run follows from one evaluation of the
+// bit test.  The extra column of workgroups ranks the slices.
+// GATHER: rows and keys are read through index tensors, and the gathered bitfields and positions are left in out_* for the
+// attention kernels (restates the index branch of the reference's mask block, bitfield_attention.py:71-87): the
+// workgroups of column 0 write the rows, those of row 0 the keys.  One launch instead of three: with every pair evaluated and
+// two gathers before it, 4096 rows against 8192 keys took 45 us; now 8.
+template <bool GATHER>
 __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
-    const int64_t* __restrict__ qbits, int64_t qbits_sb, const int64_t* __restrict__ kbits, int64_t kbits_sb,
-    const int* __restrict__ qpos, const int* __restrict__ kpos, int Sq, int Sk, int num_n, uint8_t* __restrict__ fine,
-    int64_t fine_sb, int64_t fine_ss, int* __restrict__ order, int64_t order_sb, int flag_blocks_x,
-    int* __restrict__ pair_count) {
+    const int64_t* __restrict__ bf, int64_t bf_sb, int L, const int64_t* __restrict__ idx_q, const int64_t* __restrict__ idx_k,
+    int64_t* __restrict__ qbits, int64_t qbits_sb, int64_t* __restrict__ kbits, int64_t kbits_sb, int* __restrict__ qpos,
+    int* __restrict__ kpos, int Sq, int Sk, int num_n, uint8_t* __restrict__ fine, int64_t fine_sb, int64_t fine_ss,
+    int* __restrict__ order, int64_t order_sb, int flag_blocks_x, int* __restrict__ pair_count) {
+    typedef typename std::conditional<GATHER, IndexedRows, GatheredRows>::type Rows;
     const int b = blockIdx.z;
-    const int64_t* qrow = qbits + (int64_t)b * qbits_sb;
+    Rows q_rows, k_rows;
+    if constexpr (GATHER) {
+        q_rows = IndexedRows{bf + (int64_t)b * bf_sb, idx_q, L};
+        k_rows = IndexedRows{bf + (int64_t)b * bf_sb, idx_k, L};
+    } else {
+        q_rows = GatheredRows{qbits + (int64_t)b * qbits_sb, qpos};
+        k_rows = GatheredRows{kbits + (int64_t)b * kbits_sb, kpos};
+    }
     if (pair_count != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) *pair_count = 0;
     if ((int)blockIdx.x >= flag_blocks_x) {
         const int part = blockIdx.y;
         const int ns = (Sq + 31) / 32, slots = 4 * (int)gridDim.y;
-        if (part * 256 < slots)
-            slice_order_ranked(
-                [&](int base, unsigned long long* sk) {
-                    slice_sort_key_indexed(qrow, qpos, Sq, ns, base + (int)threadIdx.x, sk[2 * threadIdx.x], sk[2 * threadIdx.x + 1]);
-                },
-                ns, slots, part, order + (int64_t)b * order_sb);
+        if (part * RANKED_PER_GROUP < slots)
+            slice_order_ranked([&](int base, unsigned long long* sk) { slice_keys_chunk_indexed(q_rows, Sq, ns, base, sk); }, ns,
+                               slots, part, order + (int64_t)b * order_sb);
         return;
     }
     __shared__ int64_t q_bits[BLOCK_M];
     __shared__ int q_pos[BLOCK_M];
     __shared__ __attribute__((aligned(8))) uint8_t s_out[4][FLAG_COLS_PER_BLOCK];
     const int m = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
+    // lanes [0, 32) own the columns of the wave's first tile, lanes [32, 64) those of the second
+    static_assert(FLAG_TILES_PER_WAVE == 2, "each half of a wave takes one tile");
+    const int n = blockIdx.x * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + half, j = n * BLOCK_N + l32;
+    int64_t kf = 0;
+    int kp = 0;
+    if (j < Sk) {
+        k_rows.get(j, kf, kp);
+        if (GATHER && m == 0) {
+            kbits[(int64_t)b * kbits_sb + j] = kf;
+            if (b == 0) kpos[j] = kp;
+        }
+    }
     if (tid < 4 * FLAG_COLS_PER_BLOCK) s_out[0][tid] = 0;
     if (tid < BLOCK_M) {
         const int i = m * BLOCK_M + tid;
-        q_bits[tid] = (i < Sq) ? qrow[i] : 0;
-        q_pos[tid] = (i < Sq) ? qpos[i] : 0;
+        int64_t f = 0;
+        int pos = 0;
+        if (i < Sq) {
+            q_rows.get(i, f, pos);
+            if (GATHER && blockIdx.x == 0) {
+                qbits[(int64_t)b * qbits_sb + i] = f;
+                if (b == 0) qpos[i] = pos;
+            }
+        }
+        q_bits[tid] = f;  // rows past the end carry no bits: they see nothing
+        q_pos[tid] = pos;
     }
     __syncthreads();
-    const int64_t* krow = kbits + (int64_t)b * kbits_sb;
+    const int64_t M = (((int64_t)1) << 62) - 1;
+    const int64_t kb = kf & M;
+    int cnt[4];
 #pragma unroll
-    for (int t = 0; t < FLAG_TILES_PER_WAVE; ++t) {
-        const int n = blockIdx.x * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + t;
-        if (n >= num_n) break;  // wave-uniform
-        const int j = n * BLOCK_N + (lane & 31);
-        const int64_t kf = (j < Sk) ? krow[j] : 0;
-        const int64_t kp = (j < Sk) ? kpos[j] : 0;
-        int cnt_a = 0, cnt_b = 0;  // rows [64 half, +32) and [64 half + 32, +32)
-#pragma unroll 8
-        for (int r = 0; r < 32; ++r) {
-            const int ri = half * 64 + r;
-            cnt_a += allow_rule(q_bits[ri], kf, q_pos[ri], kp) ? 1 : 0;
-            cnt_b += allow_rule(q_bits[ri + 32], kf, q_pos[ri + 32], kp) ? 1 : 0;
-        }
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) {
-            cnt_a += __shfl_xor(cnt_a, off);
-            cnt_b += __shfl_xor(cnt_b, off);
-        }
-        const int cols_in_range = min(BLOCK_N, Sk - n * BLOCK_N);
-        const int col = wave * FLAG_TILES_PER_WAVE + t;
-        if ((lane & 31) == 0) {
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-                const int w = 2 * half + x, c = x ? cnt_b : cnt_a;
-                const int rows = max(0, min(32, Sq - (m * BLOCK_M + 32 * w)));
-                s_out[w][col] = (uint8_t)(c == 0 ? 0 : c == rows * cols_in_range ? 2 : 1);
+    for (int w = 0; w < 4; ++w) {
+        const int r = 32 * w + l32, before = 32 * w + max(l32, 1) - 1;
+        unsigned starts = (unsigned)__ballot(l32 == 0 || q_bits[r] != q_bits[before] || q_pos[r] != q_pos[before] + 1);
+        int c = 0;
+        while (starts != 0u) {  // wave-uniform
+            const int a = __builtin_ctz(starts);
+            starts &= starts - 1u;
+            const int e = starts != 0u ? __builtin_ctz(starts) : 32;  // the run is rows [a, e) of the slice
+            const int64_t qf = q_bits[32 * w + a], qb = qf & M, p0 = q_pos[32 * w + a];
+            if (qf & 1) {  // text rows: those at or after the key's position
+                const int64_t seen = p0 + (e - a) - (kp > p0 ? (int64_t)kp : p0);
+                c += (qb & kb) != 0 && seen > 0 ? (int)seen : 0;
+            } else {
+                c += (qb == kb && qb != 0) ? e - a : 0;
             }
+        }
+        cnt[w] = c;
+    }
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) cnt[w] += __shfl_xor(cnt[w], off);
+    if (l32 == 0 && n < num_n) {
+        const int cols_in_range = min(BLOCK_N, Sk - n * BLOCK_N), col = wave * FLAG_TILES_PER_WAVE + half;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int rows = max(0, min(32, Sq - (m * BLOCK_M + 32 * w)));
+            s_out[w][col] = (uint8_t)(cnt[w] == 0 ? 0 : cnt[w] == rows * cols_in_range ? 2 : 1);
         }
     }
     __syncthreads();
@@ -465,14 +550,21 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
     }
 }
 
-int launch_indexed_plan(const int64_t* qbits, int64_t qbits_sb, const int64_t* kbits, int64_t kbits_sb, const int* qpos,
-                        const int* kpos, int Sq, int Sk, uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int* order,
-                        int64_t order_sb, int* pair_count, int B, hipStream_t stream) {
+int launch_indexed_plan(const int64_t* bf, int64_t bf_sb, int L, const int64_t* idx_q, const int64_t* idx_k, int64_t* qbits,
+                        int64_t qbits_sb, int64_t* kbits, int64_t kbits_sb, int* qpos, int* kpos, int Sq, int Sk, uint8_t* fine,
+                        int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B,
+                        hipStream_t stream) {
     const int num_m = (Sq + BLOCK_M - 1) / BLOCK_M, num_n = (Sk + BLOCK_N - 1) / BLOCK_N;
     const int flag_blocks_x = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
     dim3 grid(flag_blocks_x + 1, num_m, B);
-    hipLaunchKernelGGL(indexed_plan_kernel, grid, dim3(FLAG_WAVES * 64), 0, stream, qbits, qbits_sb, kbits, kbits_sb, qpos,
-                       kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb, flag_blocks_x, pair_count);
+    if (idx_q != nullptr)
+        hipLaunchKernelGGL(indexed_plan_kernel<true>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_sb, L, idx_q, idx_k, qbits,
+                           qbits_sb, kbits, kbits_sb, qpos, kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb,
+                           flag_blocks_x, pair_count);
+    else
+        hipLaunchKernelGGL(indexed_plan_kernel<false>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_sb, L, idx_q, idx_k, qbits,
+                           qbits_sb, kbits, kbits_sb, qpos, kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb,
+                           flag_blocks_x, pair_count);
     return (int)hipGetLastError();
 }
 
@@ -809,6 +901,129 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__
     if (sub == 0 && i < n_tiles) tile_order[rank] = i;
 }
 
+// Both launches in one, for plans of up to SMALL_PLAN_WORDS (slice, 128-key tile) pairs (at 16384 the two are as fast): every workgroup computes the
+// counts of ALL tiles (or of all groups) for itself -- a few thousand four-byte words out of L2, a dozen per thread --
+// and so knows its own base and rank without waiting for anybody.  At 3001 tokens the two launches took 9.4 us and a gap.
+// Tiles take their blocks of numbers in the order of their codes.
+constexpr int SMALL_PLAN_WORDS = 10240, SMALL_PLAN_ITEMS = 1024, SMALL_PLAN_THREADS = 1024;
+__global__ __launch_bounds__(SMALL_PLAN_THREADS) void small_plan_kernel(
+    const uint8_t* __restrict__ fine, int64_t fine_sb, int64_t fine_ss, int B, int num_m, int nkt, int num_n,
+    int* __restrict__ entry, int64_t entry_sb, int* __restrict__ tile_base, int* __restrict__ count,
+    int* __restrict__ tile_order, const int* __restrict__ order, int64_t order_sb, int* __restrict__ group_order,
+    long long* __restrict__ row_workloads, unsigned long long* __restrict__ count_host, unsigned long long count_tag) {
+    __shared__ __attribute__((aligned(16))) int s_cnt[SMALL_PLAN_ITEMS];
+    __shared__ int s_sum[SMALL_PLAN_THREADS / 64], s_rank[SMALL_PLAN_THREADS / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int slots = 4 * num_m, n_tiles = B * nkt, n_groups = B * num_m;
+    const int role = blockIdx.x;
+    // how many counts are larger than count i, or equal and of a lower code, among n counts: the rank of item i
+    auto before_me = [&](int j, int i, int mine) { return (s_cnt[j] > mine) | ((s_cnt[j] == mine) & (j < i)); };
+
+    if (role < n_tiles) {  // ---- one key tile
+        for (int j = tid; j < n_tiles; j += SMALL_PLAN_THREADS) s_cnt[j] = 0;
+        __syncthreads();
+        const int words = B * slots * nkt;
+        for (int w = tid; w < words; w += SMALL_PLAN_THREADS) {
+            const int t = w % nkt, row = w / nkt, b = row / slots, sl = row - b * slots;
+            const int cols = min(4, num_n - 4 * t);  // 32-key columns of the tile that exist
+            const unsigned valid = cols == 4 ? ~0u : (1u << (8 * cols)) - 1u;
+            const unsigned cls = *(const unsigned*)(fine + (int64_t)b * fine_sb + (int64_t)sl * fine_ss + 4 * t);
+            if ((cls & valid) != 0) atomicAdd(&s_cnt[b * nkt + t], 1);
+        }
+        __syncthreads();
+        const int mine = s_cnt[role];
+        int below = 0, rank = 0;  // pairs of the tiles in front of this one, tiles with more pairs
+        for (int j = tid; j < n_tiles; j += SMALL_PLAN_THREADS) {
+            below += j < role ? s_cnt[j] : 0;
+            rank += before_me(j, role, mine);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            below += __shfl_xor(below, off);
+            rank += __shfl_xor(rank, off);
+        }
+        if (lane == 0) {
+            s_sum[wave] = below;
+            s_rank[wave] = rank;
+        }
+        __syncthreads();
+        int base = 0, place = 0;
+        for (int w = 0; w < SMALL_PLAN_THREADS / 64; ++w) {
+            base += s_sum[w];
+            place += s_rank[w];
+        }
+        if (tid == 0) {
+            tile_base[role] = base;
+            if (tile_order != nullptr) tile_order[place] = role;
+            if (role == n_tiles - 1) {
+                *count = base + mine;
+                if (count_host != nullptr)
+                    __hip_atomic_store(count_host, count_tag | (unsigned)(base + mine), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+        // number this tile's slices, ascending
+        const int b = role / nkt, t = role - b * nkt, cols = min(4, num_n - 4 * t);
+        const unsigned valid = cols == 4 ? ~0u : (1u << (8 * cols)) - 1u;
+        const uint8_t* col = fine + (int64_t)b * fine_sb + 4 * t;
+        int* out = entry + (int64_t)b * entry_sb + t;
+        for (int s0 = 0; s0 < slots; s0 += SMALL_PLAN_THREADS) {
+            const int sl = s0 + tid;
+            const bool h = sl < slots && (*(const unsigned*)(col + (int64_t)sl * fine_ss) & valid) != 0;
+            const unsigned long long bal = __ballot(h);
+            __syncthreads();  // s_sum is free
+            if (lane == 0) s_sum[wave] = __popcll(bal);
+            __syncthreads();
+            int front = 0, all = 0;
+            for (int w = 0; w < SMALL_PLAN_THREADS / 64; ++w) {
+                if (w < wave) front += s_sum[w];
+                all += s_sum[w];
+            }
+            if (sl < slots) out[(int64_t)sl * nkt] = h ? base + front + __popcll(bal & ((1ull << lane) - 1ull)) : -1;
+            base += all;
+        }
+        return;
+    }
+    const int group_blocks = group_order != nullptr ? (n_groups + 63) / 64 : 0, gb = role - n_tiles;
+    if (gb < group_blocks) {  // ---- 64 groups of four slices, 16 threads each
+        for (int j = tid; j < n_groups; j += SMALL_PLAN_THREADS) s_cnt[j] = 0;
+        __syncthreads();
+        const int nkt64 = (num_n + 1) / 2;
+        for (int w = tid; w < n_groups * nkt64; w += SMALL_PLAN_THREADS) {
+            const int g = w / nkt64, kt = w - g * nkt64, b = g / num_m;
+            const int* ord = order + (int64_t)b * order_sb + 4 * (g - b * num_m);
+            const unsigned valid = 2 * kt + 1 < num_n ? 0xFFFFu : 0xFFu;
+            unsigned any = 0;
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                if (ord[x] >= 0) any |= *(const uint16_t*)(fine + (int64_t)b * fine_sb + (int64_t)ord[x] * fine_ss + 2 * kt);
+            if ((any & valid) != 0) atomicAdd(&s_cnt[g], 1);
+        }
+        __syncthreads();
+        const int g = 64 * gb + (tid >> 4), sub = tid & 15;
+        int rank = 0;
+        if (g < n_groups) {
+            const int mine = s_cnt[g];
+            for (int j = sub; j < n_groups; j += 16) rank += before_me(j, g, mine);
+        }
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) rank += __shfl_xor(rank, off);
+        if (g < n_groups && sub == 0) group_order[rank] = g;
+        return;
+    }
+    // ---- 16 row blocks, one per wave: their non-empty 128 x 32 tiles over the whole batch
+    const int m = 16 * (gb - group_blocks) + wave;
+    if (m >= num_m) return;
+    int tiles = 0;
+    for (int b = 0; b < B; ++b) {
+        const uint8_t* rows = fine + (int64_t)b * fine_sb + (int64_t)(4 * m) * fine_ss;
+        for (int n = lane; n < num_n; n += 64)
+            tiles += (rows[n] | rows[fine_ss + n] | rows[2 * fine_ss + n] | rows[3 * fine_ss + n]) != 0 ? 1 : 0;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) tiles += __shfl_xor(tiles, off);
+    if (lane == 0) row_workloads[m] = tiles;
+}
+
 int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int B, int Sq, int Sk, int* entry,
                       int64_t entry_sb, int* tile_base, int* count, int* tile_count, int* tile_order, const int* order,
                       int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, uint64_t* count_host,
@@ -816,6 +1031,14 @@ int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int
     const int num_m = (Sq + BLOCK_M - 1) / BLOCK_M;
     const int slots = 4 * num_m, nkt = (Sk + 127) / 128, num_n = (Sk + BLOCK_N - 1) / BLOCK_N;
     const int n_tiles = nkt * B, n_groups = num_m * B;
+    if (B <= SMALL_PLAN_ITEMS && (int64_t)n_tiles * slots <= SMALL_PLAN_WORDS && n_tiles <= SMALL_PLAN_ITEMS &&
+        n_groups <= SMALL_PLAN_ITEMS && tile_count != nullptr && (group_order == nullptr || order != nullptr)) {
+        const int blocks = n_tiles + (group_order != nullptr ? (n_groups + 63) / 64 : 0) + (row_workloads != nullptr ? (num_m + 15) / 16 : 0);
+        hipLaunchKernelGGL(small_plan_kernel, dim3(blocks), dim3(SMALL_PLAN_THREADS), 0, stream, fine, fine_sb, fine_ss, B, num_m,
+                           nkt, num_n, entry, entry_sb, tile_base, count, tile_order, order, order_sb, group_order,
+                           (long long*)row_workloads, (unsigned long long*)count_host, (unsigned long long)count_tag << 32);
+        return (int)hipGetLastError();
+    }
     if (n_tiles > DS_MAX_ORDERED_TILES || tile_count == nullptr) tile_order = nullptr;
     if (n_groups > DS_MAX_ORDERED_TILES || group_count == nullptr || order == nullptr) group_order = nullptr;
     const int group_blocks = group_order != nullptr ? num_m : 0;
@@ -850,8 +1073,8 @@ int launch_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int6
     const int num_m = (S + BLOCK_M - 1) / BLOCK_M, num_n = (S + BLOCK_N - 1) / BLOCK_N;
     const int flag_groups = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
     const int flag_blocks_x = min(flag_groups, FLAG_MAX_BLOCKS_X);
-    // one more column of workgroups: (flag_blocks_x, part, b) ranks 256 slices; 4 num_m slots need
-    // ceil(4 num_m / 256) <= num_m parts
+    // one more column of workgroups: (flag_blocks_x, part, b) ranks 64 slices; 4 num_m slots need
+    // ceil(4 num_m / 64) <= num_m parts
     dim3 grid(flag_blocks_x + 1, num_m, B);
     hipLaunchKernelGGL(tile_flags_kernel<true>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_stride_b, flags,
                        flags_stride_b, flags_stride_m, S, num_n, fine, fine_sb, fine_ss, order, order_sb, flag_blocks_x,

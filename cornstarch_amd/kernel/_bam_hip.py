@@ -138,6 +138,7 @@ SIGNATURES = {
     "bam_flag_row_workloads": [_ptr, _i64, _i64, _int, _int, _int, _ptr, _ptr],
     "bam_gather_bitfields": [_ptr, _i64, _int, _ptr, _int, _ptr, _i64, _ptr, _int, _ptr],
     "bam_plan_indexed": [_view, _ptr, _i64, _int, _plan, _ptr],
+    "bam_gather_plan_indexed": [_ptr, _i64, _int, _ptr, _ptr, _view, _ptr, _i64, _int, _plan, _ptr, _u32, _ptr],
     "bam_plan_indexed_counted": [_view, _ptr, _i64, _int, _plan, _ptr, _u32, _ptr],
     "bam_fwd_indexed": [_ptr] * 5 + [_view, _ptr] + [_i64] * 14 + [_int] * 4 + [_f32, _int, _bias, _plan, _ptr],
     "bam_bwd_dkdv_indexed": [_ptr] * 8 + [_view, _ptr] + [_i64] * 20 + [_int] * 4 + [_f32, _int, _int, _bias, _plan, _ptr],

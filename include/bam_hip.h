@@ -217,6 +217,10 @@ int bam_plan_indexed(const bam_index_view* iv, void* workspace, int64_t workspac
                      void* stream);
 int bam_plan_indexed_counted(const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
                              uint64_t* count_host, uint32_t count_tag, void* stream);
+/* bam_gather_bitfields for rows and keys and bam_plan_indexed_counted in one: WRITES the arrays the view points at. */
+int bam_gather_plan_indexed(const int64_t* bf, int64_t bf_stride_b, int L, const int64_t* idx_q, const int64_t* idx_k,
+                            const bam_index_view* iv, void* workspace, int64_t workspace_bytes, int B, bam_plan* plan,
+                            uint64_t* count_host, uint32_t count_tag, void* stream);
 
 /*
  * Dense bool mask, uint8 (B, S, S) contiguous: the allow rule for every pair
