@@ -694,7 +694,7 @@ constexpr int DQ_THREADS = 256;
 
 // LONG: as in the dK/dV kernel, for more than MAX_LIST 64-key tiles.
 template <typename T, int D, int MODE, bool BIAS, bool LONG>
-__global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(const AttnParams p) {
+__global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS ? 2 : 3) void bwd_dq_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     __shared__ u32x4 sK[2][DQ_KT * NCH];
@@ -705,6 +705,8 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
     __shared__ int sCount;
     // DENSE with packed mask bits: per wave, the words of its 32 rows for the tile's two 32-key blocks
     __shared__ unsigned sRowBits[DENSE ? 2 : 1][4][DENSE ? 64 : 1];
+    // BIAS in its per-key form: the 64 values of the tile (raw words; 16-bit elements fill half)
+    __shared__ __attribute__((aligned(16))) unsigned sBias[BIAS ? 2 : 1][BIAS ? 64 : 1];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
@@ -761,7 +763,14 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
     f32x16 zero16;
 #pragma unroll
     for (int i = 0; i < 16; ++i) zero16[i] = 0.f;
-    const float c2 = BIAS ? LOG2E : p.scale * LOG2E;  // with a bias the scores become scale * s + bias first
+    // A per-key bias whose groups of four keys are aligned, in-range accesses travels with the tile copies, and with bf16
+    // operands it is added by one more MFMA of the S phase, as in the forward.  (Read from global memory inside the loop,
+    // every group of four waited, through the in-order vmcnt, for all tile copies in flight: 2 x 2048 tokens, 16 heads,
+    // D 64: 75 us, now 63.)
+    const bool bias_lds = BIAS && p.bias_sm == 0 && p.bias_vec != 0;
+    const bool bias_fold = bias_lds && std::is_same<T, BF16>::value;
+    const float c2 = (BIAS && !bias_fold) ? LOG2E : p.scale * LOG2E;  // otherwise the scores become scale * s + bias first
+    const float inv_scale = 1.f / p.scale;
     const char* bias_row = nullptr;  // this lane's row of the bias
     if (BIAS)
         bias_row = (const char*)p.bias + (p.bias_f32 ? 4 : 2) * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh +
@@ -774,9 +783,9 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
 
     typedef TileStage<D, DQ_KT, DQ_THREADS> Stage;
     constexpr int CPT = Stage::CPT;
-    // copy instructions per wave and tile: K, V, the key bitfields and (IDX) the key positions
-    constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0);
-    static_assert(NLOADS <= 2 * KK, "one copy per MFMA of the first S / dP block");
+    // copy instructions per wave and tile: K, V, the key bitfields, (IDX) the key positions and (BIAS) the bias values
+    constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (BIAS ? 1 : 0);
+    static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the first S / dP block (and at most one behind it)");
     Stage stK, stV;
     stK.setup(2 * p.k.ss, p.d / 8, tid);
     stV.setup(2 * p.v.ss, p.d / 8, tid);
@@ -787,6 +796,9 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
                                      ? p.row_bits + (int64_t)b * p.row_bits_sb + (slice < 0 ? 0 : slice) * 32
                                      : nullptr;
     const unsigned row_bits_voff = DENSE ? (unsigned)(hi * (int)p.row_bits_sn * 4 + l32 * 4) : 0u;
+    const char* bias_head = BIAS ? (const char*)p.bias + (p.bias_f32 ? 4 : 2) * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh) : nullptr;
+    const unsigned bias_voff = (unsigned)((p.bias_f32 ? lane : (lane & 31)) * 4);
+    const int bias_tile_bytes = DQ_KT * (p.bias_f32 ? 4 : 2);
     constexpr unsigned TILE_BYTES = DQ_KT * NCH * 16, BITS_BYTES = DQ_KT * 8;
     // copy instruction j of full tile kt into buffer buf (key bitfields: 64 dwords per wave, waves 2, 3
     // repeat what waves 0, 1 write, so that every wave issues the same number of copies)
@@ -803,8 +815,10 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
                 dma_b32(bfrow + kt * DQ_KT, (unsigned)((wave & 1) * 256 + lane * 4), ldsB + buf * BITS_BYTES + (wave & 1) * 256u);
             }
         }
-        else  // 64 positions; every wave writes the same values
+        else if (IDX && j == 2 * CPT + 1)  // 64 positions; every wave writes the same values
             dma_b32(p.posk + kt * DQ_KT, (unsigned)(lane * 4), ldsP + buf * (DQ_KT * 4u));
+        else if (bias_lds)  // BIAS: the tile's 64 bias values; every wave writes the same values
+            dma_b32(bias_head + (int64_t)kt * bias_tile_bytes, bias_voff, lds_addr(sBias) + buf * 256u);
     };
 
     // One 64-key tile held in buffer `cur`; with PREFETCH the copies of tile kt_next into the other buffer
@@ -846,6 +860,12 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
         for (int kb = 0; kb < 2; ++kb) {
             // ---- S^T = K Q^T and dP^T = V dO^T : 32 keys x 32 queries, two accumulator chains
             f32x16 s, dp;
+            u32x4 bias_a = {0u, 0u, 0u, 0u};  // bias_fold: this lane's key of the block, as an operand
+            if (BIAS && PREFETCH && bias_fold && hi == 0) {
+                const float bv = p.bias_f32 ? ((const float*)sBias[cur])[32 * kb + l32]
+                                            : T::to_float(((const unsigned short*)sBias[cur])[32 * kb + l32]);
+                bias_a = split3_operand<T>(bv * inv_scale);
+            }
             {
                 constexpr int NOP = 2 * KK, AHEAD = 4;  // operand j: K chunk (j even) or V chunk (j odd) of k-slice j / 2
                 u32x4 a[NOP];
@@ -862,14 +882,43 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 ? 2 : 3) void bwd_dq_kernel(cons
                         s = T::mfma(a[j], qreg[j >> 1], j < 2 ? zero16 : s);
                     if (PREFETCH && kb == 0 && j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
                 }
+                if (PREFETCH && kb == 0) {
+#pragma unroll
+                    for (int j = NOP; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
+                }
+                if (BIAS && PREFETCH && bias_fold) {
+                    const u32x4 z = {0u, 0u, 0u, 0u};
+                    s = T::mfma(bias_a, hi == 0 ? ones3_operand<T>() : z, s);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (BIAS) {
+            if (BIAS && PREFETCH && bias_fold) {
+                // (added by the MFMA above)
+            } else if (BIAS && PREFETCH && bias_lds) {  // (the ragged last tile is staged without the bias)
+#pragma unroll
+                for (int grp = 0; grp < 4; ++grp) {
+                    const int koff = 32 * kb + 8 * grp + 4 * hi;
+                    f32x4 b4;
+                    if (p.bias_f32) {
+                        b4 = *(const f32x4*)&sBias[cur][koff];
+                    } else {
+                        const u32x2 w = *(const u32x2*)((const char*)sBias[cur] + 2 * koff);
+                        b4[0] = T::to_float((unsigned short)(w[0] & 0xFFFFu));
+                        b4[1] = T::to_float((unsigned short)(w[0] >> 16));
+                        b4[2] = T::to_float((unsigned short)(w[1] & 0xFFFFu));
+                        b4[3] = T::to_float((unsigned short)(w[1] >> 16));
+                    }
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) s[4 * grp + x] = fmaf(s[4 * grp + x], p.scale, b4[x]);
+                }
+            } else if (BIAS) {
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
                     const f32x4 b4 = load_bias4<T>(bias_row, kt * DQ_KT + 32 * kb + 8 * grp + 4 * hi, Sk, p.bias_f32 != 0, p.bias_vec != 0);
 #pragma unroll
-                    for (int x = 0; x < 4; ++x) s[4 * grp + x] = fmaf(s[4 * grp + x], p.scale, b4[x]);
+                    for (int x = 0; x < 4; ++x)
+                        s[4 * grp + x] = bias_fold ? fmaf(b4[x], inv_scale, s[4 * grp + x])  // (c2 holds the scale)
+                                                   : fmaf(s[4 * grp + x], p.scale, b4[x]);
                 }
             }
 #pragma unroll
