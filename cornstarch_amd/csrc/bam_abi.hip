@@ -786,7 +786,9 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
                        a->dv.ptr, m, a->flags, st, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->accumulate, true, true,
                        a->bias, nullptr, true));
     all.o = {a->o.ptr, a->o.stride_b, a->o.stride_s, a->o.stride_h};
-    BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
+    // head dims up to 64: the dQ kernel runs first and computes delta on the way; above, dK/dV needs it first
+    const bool dq_first = all.D <= 64;
+    if (!dq_first) BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
     // The heads in runs of whole kv heads, every run through the same dS workspace: the launches of a stream run in
     // order, so a run's dQ kernel has read the workspace before the next run's dK/dV kernel writes it.
     for (int r = 0; r < runs; ++r) {
@@ -804,6 +806,11 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         p.Hq = hq;
         p.Hkv = hk;
         if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
+        if (dq_first) {
+            BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
+            BAM_TRY(launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+            continue;
+        }
         BAM_TRY(launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
         BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
     }
