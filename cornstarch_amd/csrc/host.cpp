@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <sched.h>
 
@@ -39,6 +40,7 @@ void check(int rc, const char* what) {
 
 typedef c10::hip::HIPStream Stream;
 Stream current_stream(c10::Device device) { return c10::hip::getCurrentHIPStream(device.index()); }
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
 // ------------------------------------------------------------------ pair counts
 // The number of pairs of a plan is device data; the last launch of the plan builder stores it, under a tag, to a word of
@@ -118,7 +120,10 @@ struct PlanCore {
     ~PlanCore() {
         if (word.at != nullptr) count_words().give_back(word, pairs.load() >= 0);
     }
+    // Not while capturing: every replay would store to the word again, whoever owns it by then, and the caches would hold
+    // a plan that nothing has computed yet.  A plan built before the capture is used in it like any other.
     void prepare(Tensor ws, Stream s) {
+        if (capturing()) throw BamFailure("a plan cannot be built while a graph is captured: run the call once before");
         workspace = std::move(ws);
         stream = s;
         word = count_words().take();
@@ -600,7 +605,10 @@ py::tuple index_view(const Tensor& bf, const Tensor& idx_q, const Tensor& idx_k,
 constexpr int64_t kDecodeCounters = 8192;
 std::mutex g_counters_mutex;
 std::vector<std::pair<void*, Tensor>> g_counters;
+// None while capturing: the library does not use them there, and a set made then would live in the graph's memory and be
+// cleared by its replays.
 uint32_t* decode_counters(const Tensor& like, const Stream& stream) {
+    if (capturing()) return nullptr;
     std::lock_guard<std::mutex> guard(g_counters_mutex);
     for (const auto& [s, t] : g_counters)
         if (s == (void*)stream.stream() && t.device() == like.device()) return (uint32_t*)t.data_ptr();

@@ -200,6 +200,8 @@ def call(name: str, *args) -> None:
 
 def _load_host():
     """The native host layer (csrc/host.cpp), which calls the library above."""
+    import torch  # noqa: F401  (its libraries first: the host layer is linked against them)
+
     try:
         from cornstarch_amd import _bam_host
     except ImportError as e:

@@ -11,6 +11,7 @@ import torch
 
 from cornstarch_amd.kernel import _bam_hip
 from cornstarch_amd.kernel import bitfield_attention as BA
+from cornstarch_amd.kernel.interface import bitfield_attention_forward
 from tests.helpers import random_bitfield
 
 pytestmark = pytest.mark.gpu
@@ -127,3 +128,50 @@ def test_a_recorded_step_replays_bit_for_bit(B, S, Hq, Hkv, D):
         assert torch.equal(replayed[1], o.detach())
         for a, b in zip(replayed[3:], (dq, dk, dv)):
             assert torch.equal(a, b)
+
+
+def test_decode_first_seen_in_a_capture_leaves_eager_calls_alone():
+    """A stream's merge counters are never made by a capture: replays and eager calls on the capture stream agree."""
+    torch.manual_seed(3)
+    q, k, v = (torch.randn(1, h, s, 128, device=dev(), dtype=torch.bfloat16) for h, s in ((8, 1), (2, 2100), (2, 2100)))
+    module = torch.nn.Module().eval()
+    want = bitfield_attention_forward(module, q, k, v, None)[0]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = bitfield_attention_forward(module, q, k, v, None)[0]
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            eager = bitfield_attention_forward(module, q, k, v, None)[0]
+        torch.cuda.synchronize()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (eager.float() - want.float()).abs().max() == 0
+        # two launches merge the same partial results here: equal up to the rounding of the output
+        assert (out.float() - want.float()).abs().max() <= 2.0 ** -8 * want.float().abs().max()
+
+
+def test_a_plan_is_not_built_by_a_capture():
+    """A replay would store the pair count to a word that has another owner by then: refused before anything is launched."""
+    q, k, v = (torch.randn(1, 200, 2, 64, device=dev(), dtype=torch.bfloat16) for _ in range(3))
+    bf = torch.full((1, 200), (1 << 62) | 1, dtype=torch.int64, device=dev())
+    BA.BitfieldUtils.clear_cache()
+    want = BA.bitfield_attn_func(q, k, v, bf)  # also loads the code objects
+    BA.BitfieldUtils.clear_cache()
+    torch.cuda.synchronize()
+    with pytest.raises(_bam_hip.BamError, match="captured"):
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            BA.bitfield_attn_func(q, k, v, bf)
+    torch.cuda.synchronize()
+    BA.bitfield_attn_func(q, k, v, bf)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = BA.bitfield_attn_func(q, k, v, bf)  # with the plan built before
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    BA.BitfieldUtils.clear_cache()
