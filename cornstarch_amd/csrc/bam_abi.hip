@@ -318,7 +318,7 @@ extern "C" {
 
 const char* bam_last_error(void) { return g_error; }
 
-int bam_abi_version(void) { return 11; }
+int bam_abi_version(void) { return 12; }
 
 int bam_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                    int64_t flags_stride_m, int B, int S, void* stream) {
@@ -758,6 +758,30 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
                     a->flags_stride_m, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->bias, a->plan, stream, true);
 }
 
+// How many workgroups share the q heads of a kv head in dK/dV.  One workgroup per (key tile, kv head) walks all of them one
+// after the other, so calls with grouped heads leave most compute units without one until the sequence is long.  As many
+// parts as keep the launch within one workgroup per compute unit (beyond that the parts queue behind each other).  Whole
+// training step, bf16, D 64, one part -> parts: 1 x 1024 tokens, 32 / 8 heads 139 -> 98 us; 1 x 2048, 32 / 4 heads
+// 363 -> 183; 1 x 4000, 16 / 4 heads 401 -> 286.  The price is a launch (4 us), an allocation and their host work, so at
+// least 32 steps over a pair of slices have to go: 4 x 400 tokens, 6 / 1 heads, D 40 (35 steps) 94 -> 58 to 98 us with the
+// speed of the host; 512 tokens, 16 / 4 heads (24 steps) 83 -> 95, 2 x 283, 6 / 2 heads (10 steps) 86 -> 91.
+static int dkdv_parts(const bam_attn* a) {
+    if (a->D > 64 || a->head_runs > 1 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32) return 1;
+    const int G = a->Hq / a->Hkv, pairs = (a->Sq + 63) / 64;
+    const int64_t units = (int64_t)a->B * a->Hkv * ((a->Sk + 127) / 128);
+    for (int parts = G; parts > 1; --parts)
+        if (G % parts == 0 && units * parts <= 256) return (int64_t)(G - G / parts) * pairs >= 32 ? parts : 1;
+    return 1;
+}
+static int64_t dkdv_part_floats(const bam_attn* a, int parts) { return (int64_t)a->B * a->Sk * a->Hkv * parts * a->D; }
+
+int bam_attn_bwd_parts(const bam_attn* a, int64_t* bytes) {
+    if (a == nullptr || bytes == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd_parts: null pointer");
+    const int parts = dkdv_parts(a);
+    *bytes = parts > 1 ? 2 * 4 * dkdv_part_floats(a, parts) : 0;
+    return BAM_OK;
+}
+
 int bam_attn_bwd(const bam_attn* a, void* stream) {
     if (a == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: null pointer");
     MaskSource m;
@@ -808,6 +832,24 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
         if (dq_first) {
             BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
+            const int parts = a->parts_workspace != nullptr ? dkdv_parts(a) : 1;
+            if (parts > 1) {
+                const int64_t floats = dkdv_part_floats(a, parts);
+                if (a->parts_bytes < 2 * 4 * floats || (reinterpret_cast<uintptr_t>(a->parts_workspace) & 15u))
+                    return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: parts workspace of %lld bytes, %lld needed, 16-byte aligned",
+                                (long long)a->parts_bytes, (long long)(2 * 4 * floats));
+                bam::AttnParams part = p;
+                const int64_t sh = a->D, ss = sh * p.Hkv * parts, sb = ss * p.Sk;
+                float* ws = (float*)a->parts_workspace;
+                part.dk = {ws, sb, ss, sh};
+                part.dv = {ws + floats, sb, ss, sh};
+                part.grad_typed = 2;
+                part.kv_parts = parts;
+                part.Hkv = p.Hkv * parts;
+                BAM_TRY(launched(launch_dkdv(part, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+                BAM_TRY(launched(bam::launch_sum_parts(p, ws, ws + floats, parts, a->dtype, (hipStream_t)stream), "bam_attn_bwd (sum)"));
+                continue;
+            }
             BAM_TRY(launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
             continue;
         }

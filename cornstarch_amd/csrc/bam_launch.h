@@ -29,7 +29,10 @@ struct Tensor4 {  // logical (B, S, H, D), unit stride along D, strides in eleme
 struct AttnParams {
     Tensor4 q, k, v, o, dout;  // 16-bit tensors
     Tensor4 dq, dk, dv;        // gradients: fp32 accumulated into, or (grad_typed) input dtype, overwritten
-    int grad_typed;
+    int grad_typed;            // 2 (dK/dV parts): fp32, overwritten
+    // dK/dV at head dims up to 64: the q heads of a kv head are dealt to this many workgroups; Hkv counts the parts then,
+    // k and v are those of kv head (part / kv_parts) and dk / dv hold one fp32 sum per part.  0 or 1: one part.
+    int kv_parts;
     float* lse;                // (B, Hq, Sq_rounded)
     float* delta;              // (B, Hq, Sq_rounded)
     // Bitfields of the query rows (B, Sq) and of the keys (B, Sk), and their global positions.  Plain
@@ -159,6 +162,8 @@ int launch_fwd(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_preprocess(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dkdv(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dq(const AttnParams& p, int dtype, hipStream_t stream);
+// dk, dv of p from the parts that a dK/dV launch with kv_parts left at `parts_dk` and `parts_dv` (contiguous).
+int launch_sum_parts(const AttnParams& p, const float* parts_dk, const float* parts_dv, int parts, int dtype, hipStream_t stream);
 int launch_decode(const DecodeParams& p, const DecodeSplit& s, int dtype, hipStream_t stream);
 // dK/dV that also stores dS (p.ds_ws), and the dQ kernel that consumes it; D = 128, plan required
 int launch_bwd_dkdv_save(const AttnParams& p, int dtype, hipStream_t stream);

@@ -111,6 +111,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 
     const int unit = blockIdx.x;
     const int hk = unit % p.Hkv;
+    constexpr bool PARTS = D <= 64 && !LONG && !SAVE;  // (a kv head's q heads may be dealt to several workgroups)
+    const int kv_head = PARTS && p.kv_parts > 1 ? hk / p.kv_parts : hk;
     int ub = unit / p.Hkv;  // position of the (batch, key tile) in the order of falling work
     {
         // The hardware deals the workgroups of an XCD to its four shader engines in turn and launches them strictly
@@ -139,8 +141,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         TileStage<D, 128, DKDV_THREADS> stK, stV;
         stK.setup(2 * p.k.ss, p.d / 8, tid);
         stV.setup(2 * p.v.ss, p.d / 8, tid);
-        const char* kb = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh + (int64_t)nt * 128 * p.k.ss);
-        const char* vb = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)hk * p.v.sh + (int64_t)nt * 128 * p.v.ss);
+        const char* kb = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)kv_head * p.k.sh + (int64_t)nt * 128 * p.k.ss);
+        const char* vb = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)kv_head * p.v.sh + (int64_t)nt * 128 * p.v.ss);
         stK.load(kb, sK, Sk - nt * 128, tid);
         stV.load(vb, sV, Sk - nt * 128, tid);
     }
@@ -639,6 +641,29 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 }
         }
         __syncthreads();
+        if (PARTS && p.grad_typed == 2) {
+            if (st == 0 && kvalid) {
+                float* dkp = (float*)p.dk.ptr + ((int64_t)b * p.dk.sb + (int64_t)key * p.dk.ss + (int64_t)hk * p.dk.sh);
+                float* dvp = (float*)p.dv.ptr + ((int64_t)b * p.dv.sb + (int64_t)key * p.dv.ss + (int64_t)hk * p.dv.sh);
+#pragma unroll
+                for (int db = 0; db < DB; ++db)
+#pragma unroll
+                    for (int grp = 0; grp < 4; ++grp) {
+                        if (32 * db + 8 * grp >= p.d) break;
+                        f32x4 a, c;
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            const int i = 4 * grp + x;
+                            a[x] = (dk[db][i] + park[(db * 16 + i) * 64 + lane]) * -p.scale;
+                            c[x] = dv[db][i] + park[((DB + db) * 16 + i) * 64 + lane];
+                        }
+                        const int d0 = 32 * db + 8 * grp + 4 * hi;
+                        *(f32x4*)(dkp + d0) = a;
+                        *(f32x4*)(dvp + d0) = c;
+                    }
+            }
+            return;
+        }
         if (st == 0 && kvalid) {
             char* dkp = (char*)p.dk.ptr + 2 * ((int64_t)b * p.dk.sb + (int64_t)key * p.dk.ss + (int64_t)hk * p.dk.sh);
             char* dvp = (char*)p.dv.ptr + 2 * ((int64_t)b * p.dv.sb + (int64_t)key * p.dv.ss + (int64_t)hk * p.dv.sh);

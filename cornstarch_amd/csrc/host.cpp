@@ -403,6 +403,12 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
             a.ds_capacity = plan.core->pairs.load();
         }
     }
+    Tensor parts;  // (given back to the caching allocator on return: the launches that use it are on the current stream)
+    check(bam_attn_bwd_parts(&a, &a.parts_bytes), "bam_attn_bwd_parts");
+    if (a.parts_bytes > 0) {
+        parts = at::empty({a.parts_bytes}, q.options().dtype(at::kByte));
+        a.parts_workspace = parts.data_ptr();
+    }
     check(bam_attn_bwd(&a, current_stream(q.device()).stream()), "bam_attn_bwd");
 }
 

@@ -15,7 +15,7 @@ BAM_DTYPE_F16 = 0
 BAM_DTYPE_BF16 = 1
 BAM_MAX_SEQLEN = 4194304
 BAM_STATIC_PLAN_BYTES = 8 << 20
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -106,6 +106,8 @@ class Attn(ctypes.Structure):
         ("ds_capacity", ctypes.c_int64),
         *((name, ctypes.c_int32) for name in ("mode", "B", "Sq", "Sk", "Hq", "Hkv", "D", "dtype", "accumulate", "head_runs")),
         ("scale", ctypes.c_float),
+        ("parts_workspace", ctypes.c_void_p),
+        ("parts_bytes", ctypes.c_int64),
     ]
 
 
@@ -145,6 +147,7 @@ SIGNATURES = {
     "bam_bwd_dq_indexed": [_ptr] * 7 + [_view, _ptr] + [_i64] * 17 + [_int] * 4 + [_f32, _int, _int, _bias, _plan, _ptr],
     "bam_attn_fwd": [_attn, _ptr],
     "bam_attn_bwd": [_attn, _ptr],
+    "bam_attn_bwd_parts": [_attn, _ptr],
     "bam_decode_counted": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr, _i64, _ptr],
     "bam_decode": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr],
 }

@@ -477,9 +477,14 @@ typedef struct bam_attn {
     int64_t ds_capacity;
     int32_t mode, B, Sq, Sk, Hq, Hkv, D, dtype, accumulate, head_runs;
     float scale;
+    void* parts_workspace; /* bam_attn_bwd: may be null; bam_attn_bwd_parts bytes, 16-byte aligned */
+    int64_t parts_bytes;
 } bam_attn;
 int bam_attn_fwd(const bam_attn* args, void* stream);
 int bam_attn_bwd(const bam_attn* args, void* stream);
+/* Bytes of scratch with which bam_attn_bwd deals the q heads of a kv head to several workgroups of its dK/dV launch and sums
+ * their parts (0: this call would not).  Looks at the sizes and head_runs only. */
+int bam_attn_bwd_parts(const bam_attn* args, int64_t* bytes);
 
 #ifdef __cplusplus
 }
