@@ -762,11 +762,12 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
 // after the other, so calls with grouped heads leave most compute units without one until the sequence is long.  As many
 // parts as keep the launch within one workgroup per compute unit (beyond that the parts queue behind each other).  Whole
 // training step, bf16, D 64, one part -> parts: 1 x 1024 tokens, 32 / 8 heads 139 -> 98 us; 1 x 2048, 32 / 4 heads
-// 363 -> 183; 1 x 4000, 16 / 4 heads 401 -> 286.  The price is a launch (4 us), an allocation and their host work, so at
+// 363 -> 183; 1 x 4000, 16 / 4 heads 401 -> 286; D 128: 1 x 700, 16 / 4 heads 138 -> 105; 1 x 1024, 32 / 8 heads
+// 180 -> 117; 1 x 3000, 16 / 4 heads 456 -> 319.  The price is a launch (4 us), an allocation and their host work, so at
 // least 32 steps over a pair of slices have to go: 4 x 400 tokens, 6 / 1 heads, D 40 (35 steps) 94 -> 58 to 98 us with the
 // speed of the host; 512 tokens, 16 / 4 heads (24 steps) 83 -> 95, 2 x 283, 6 / 2 heads (10 steps) 86 -> 91.
 static int dkdv_parts(const bam_attn* a) {
-    if (a->D > 64 || a->head_runs > 1 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32) return 1;
+    if (a->head_runs > 1 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32) return 1;
     const int G = a->Hq / a->Hkv, pairs = (a->Sq + 63) / 64;
     const int64_t units = (int64_t)a->B * a->Hkv * ((a->Sk + 127) / 128);
     for (int parts = G; parts > 1; --parts)
@@ -813,6 +814,24 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
     // head dims up to 64: the dQ kernel runs first and computes delta on the way; above, dK/dV needs it first
     const bool dq_first = all.D <= 64;
     if (!dq_first) BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
+    const int parts = a->parts_workspace != nullptr ? dkdv_parts(a) : 1;
+    auto dkdv = [&](const bam::AttnParams& p) -> int {
+        if (parts == 1) return launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)");
+        const int64_t floats = dkdv_part_floats(a, parts);
+        if (a->parts_bytes < 2 * 4 * floats || (reinterpret_cast<uintptr_t>(a->parts_workspace) & 15u))
+            return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: parts workspace of %lld bytes, %lld needed, 16-byte aligned",
+                        (long long)a->parts_bytes, (long long)(2 * 4 * floats));
+        bam::AttnParams part = p;
+        const int64_t sh = a->D, ss = sh * p.Hkv * parts, sb = ss * p.Sk;
+        float* ws = (float*)a->parts_workspace;
+        part.dk = {ws, sb, ss, sh};
+        part.dv = {ws + floats, sb, ss, sh};
+        part.grad_typed = 2;
+        part.kv_parts = parts;
+        part.Hkv = p.Hkv * parts;
+        BAM_TRY(launched(launch_dkdv(part, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+        return launched(bam::launch_sum_parts(p, ws, ws + floats, parts, a->dtype, (hipStream_t)stream), "bam_attn_bwd (sum)");
+    };
     // The heads in runs of whole kv heads, every run through the same dS workspace: the launches of a stream run in
     // order, so a run's dQ kernel has read the workspace before the next run's dK/dV kernel writes it.
     for (int r = 0; r < runs; ++r) {
@@ -832,28 +851,10 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
         if (dq_first) {
             BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
-            const int parts = a->parts_workspace != nullptr ? dkdv_parts(a) : 1;
-            if (parts > 1) {
-                const int64_t floats = dkdv_part_floats(a, parts);
-                if (a->parts_bytes < 2 * 4 * floats || (reinterpret_cast<uintptr_t>(a->parts_workspace) & 15u))
-                    return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: parts workspace of %lld bytes, %lld needed, 16-byte aligned",
-                                (long long)a->parts_bytes, (long long)(2 * 4 * floats));
-                bam::AttnParams part = p;
-                const int64_t sh = a->D, ss = sh * p.Hkv * parts, sb = ss * p.Sk;
-                float* ws = (float*)a->parts_workspace;
-                part.dk = {ws, sb, ss, sh};
-                part.dv = {ws + floats, sb, ss, sh};
-                part.grad_typed = 2;
-                part.kv_parts = parts;
-                part.Hkv = p.Hkv * parts;
-                BAM_TRY(launched(launch_dkdv(part, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
-                BAM_TRY(launched(bam::launch_sum_parts(p, ws, ws + floats, parts, a->dtype, (hipStream_t)stream), "bam_attn_bwd (sum)"));
-                continue;
-            }
-            BAM_TRY(launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+            BAM_TRY(dkdv(p));
             continue;
         }
-        BAM_TRY(launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+        BAM_TRY(dkdv(p));
         BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
     }
     return BAM_OK;

@@ -30,7 +30,7 @@ struct AttnParams {
     Tensor4 q, k, v, o, dout;  // 16-bit tensors
     Tensor4 dq, dk, dv;        // gradients: fp32 accumulated into, or (grad_typed) input dtype, overwritten
     int grad_typed;            // 2 (dK/dV parts): fp32, overwritten
-    // dK/dV at head dims up to 64: the q heads of a kv head are dealt to this many workgroups; Hkv counts the parts then,
+    // dK/dV: the q heads of a kv head are dealt to this many workgroups; Hkv counts the parts then,
     // k and v are those of kv head (part / kv_parts) and dk / dv hold one fp32 sum per part.  0 or 1: one part.
     int kv_parts;
     float* lse;                // (B, Hq, Sq_rounded)

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 
     const int unit = blockIdx.x;
     const int hk = unit % p.Hkv;
-    constexpr bool PARTS = D <= 64 && !LONG && !SAVE;  // (a kv head's q heads may be dealt to several workgroups)
+    constexpr bool PARTS = !LONG;  // (a kv head's q heads may be dealt to several workgroups)
     const int kv_head = PARTS && p.kv_parts > 1 ? hk / p.kv_parts : hk;
     int ub = unit / p.Hkv;  // position of the (batch, key tile) in the order of falling work
     {
