@@ -840,6 +840,7 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         skip(p.q, hq, 2);
         skip(p.k, hk, 2);
         skip(p.v, hk, 2);
+        skip(p.o, hq, 2);  // (up to head dim 64 the dQ kernel computes delta from it)
         skip(p.dout, hq, 2);
         skip(p.dq, hq, gsz);
         skip(p.dk, hk, gsz);
