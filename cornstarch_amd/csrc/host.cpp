@@ -418,6 +418,9 @@ struct AttentionBackward : public torch::autograd::Node {
     SavedVariable q, k, v, o, lse, bias, mask, flags;  // mask: the bitfields, or the materialized mask
     Plan plan;
     int mode = BAM_MASK_BITFIELD;
+    bool has_bias = false;
+    at::ScalarType type = at::kHalf;  // of q
+    int64_t Sk = 0, Hkv = 0;
     double scale = 0;
 
     std::string name() const override { return "BitfieldAttentionFunctionBackward"; }
@@ -428,20 +431,51 @@ struct AttentionBackward : public torch::autograd::Node {
     variable_list apply(variable_list&& grads) override {
         if (!grads[0].defined()) return variable_list(3);
         const at::NoGradGuard no_grad;
-        const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack(),
-                     bias_ = bias.unpack(), mask_ = mask.unpack(), flags_ = flags.unpack();
+        Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack(),
+               bias_ = bias.unpack(), mask_ = mask.unpack(), flags_ = flags.unpack();
         Tensor dout = grads[0];
-        if (dout.scalar_type() != q_.scalar_type()) dout = dout.to(q_.scalar_type());
+        if (dout.scalar_type() != type) dout = dout.to(type);
         if (!rows_ready(dout, 8)) dout = dout.contiguous();
+        // What the forward saved has been through the user's saved-tensor hooks, if there are any.  Another layout is copied
+        // into the kernels' form; with another shape, type or device the kernels would compute something else.
+        const int64_t B = dout.size(0), Sq = dout.size(1), Hq = dout.size(2), D = dout.size(3);
+        auto expect = [&](const Tensor& t, at::ScalarType st, at::IntArrayRef sizes, const char* what) {
+            if (!t.defined() || t.device() != dout.device() || t.scalar_type() != st || t.sizes() != sizes || !plain(t))
+                throw BamFailure(std::string("the saved ") + what + " came back from its hooks with another shape, type or device");
+        };
+        auto expect_rows = [&](Tensor& t, at::IntArrayRef sizes, const char* what) {
+            expect(t, type, sizes, what);
+            if (!rows_ready(t, 8)) t = t.contiguous();
+        };
+        expect_rows(q_, dout.sizes(), "q");
+        expect_rows(k_, {B, Sk, Hkv, D}, "k");
+        expect_rows(v_, {B, Sk, Hkv, D}, "v");
+        expect_rows(o_, dout.sizes(), "o");
+        expect(lse_, at::kFloat, {B, Hq, (Sq + 127) / 128 * 128}, "lse");
+        lse_ = lse_.contiguous();
+        expect(flags_, at::kChar, {B, (Sq + 127) / 128, (Sk + 31) / 32}, "flags");
+        if (flags_.stride(2) != 1) flags_ = flags_.contiguous();
+        if (mode == BAM_MASK_BITFIELD) {
+            expect(mask_, at::kLong, {B, Sk}, "mask");
+            if (mask_.stride(1) != 1) mask_ = mask_.contiguous();
+        } else {
+            expect(mask_, at::kBool, {B, Sq, Sk}, "mask");
+            mask_ = mask_.contiguous();
+        }
         Tensor dq = at::empty_like(q_), dk = at::empty_like(k_), dv = at::empty_like(v_);
         Call c;
         bam_bias desc;
         c.mode = mode;
         c.bf = mode == BAM_MASK_BITFIELD ? &mask_ : nullptr;
-        c.mask = mode == BAM_MASK_DENSE && mask_.defined() ? &mask_ : nullptr;
+        c.mask = mode == BAM_MASK_DENSE ? &mask_ : nullptr;
         c.flags = &flags_;
         c.scale = scale;
-        if (bias_.defined() && make_bias(bias_, q_, k_.size(1), desc)) c.bias = &desc;
+        if (has_bias) {
+            if (bias_.defined() && bias_.dim() == 4 && bias_.stride(3) != 1) bias_ = bias_.contiguous();
+            if (!bias_.defined() || !make_bias(bias_, q_, Sk, desc))
+                throw BamFailure("the saved bias came back from its hooks with another shape, type or device");
+            c.bias = &desc;
+        }
         run_backward(c, plan, dout, q_, k_, v_, o_, lse_, dq, dk, dv, false);
         return {dq, dk, dv};
     }
@@ -459,10 +493,14 @@ Tensor attention(Call c, const Plan& plan, const Tensor& q, const Tensor& k, con
         node->v = torch::autograd::SavedVariable(v, false);
         node->lse = torch::autograd::SavedVariable(lse, false);
         if (bias) node->bias = torch::autograd::SavedVariable(*bias, false);
-        if (mask.defined()) node->mask = torch::autograd::SavedVariable(mask, false);
+        node->has_bias = (bool)bias;
+        node->mask = torch::autograd::SavedVariable(mask, false);
         node->flags = torch::autograd::SavedVariable(*c.flags, false);
         node->plan = plan;
         node->mode = c.mode;
+        node->type = q.scalar_type();
+        node->Sk = k.size(1);
+        node->Hkv = k.size(2);
         node->scale = c.scale;
         torch::autograd::set_history(o, node);
         node->o = torch::autograd::SavedVariable(o, true);

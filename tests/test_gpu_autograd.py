@@ -1,0 +1,99 @@
+"""The native autograd node under saved-tensor hooks."""
+
+import pytest
+import torch
+
+from cornstarch_amd.kernel import attention as A
+from cornstarch_amd.kernel import bitfield_attention as BA
+from tests.helpers import random_bitfield
+
+pytestmark = pytest.mark.gpu
+
+
+class Problem:
+    def __init__(self, B=2, S=200, Hq=4, Hkv=2, D=64, dtype=torch.bfloat16, bias=False):
+        dev = torch.device("cuda:0")
+        g = torch.Generator(device=dev).manual_seed(S + D)
+        self.q, self.k, self.v, self.do = (torch.randn(B, S, H, D, generator=g, device=dev).to(dtype).requires_grad_(n < 3)
+                                           for n, H in enumerate((Hq, Hkv, Hkv, Hq)))
+        self.bf = random_bitfield(B, S, seed=S, pad=3).to(dev)
+        self.bias = torch.randn(1, Hq, 1, S, generator=g, device=dev) if bias else None
+        BA.BitfieldUtils.clear_cache()
+
+    @property
+    def inputs(self):
+        return self.q, self.k, self.v
+
+    def forward(self, q=None, k=None, v=None):
+        return BA.bitfield_attn_func(*(x if x is not None else y for x, y in zip((q, k, v), self.inputs)), self.bf, self.bias)
+
+    def grads(self, o=None, **kw):
+        return torch.autograd.grad(self.forward() if o is None else o, self.inputs, self.do, **kw)
+
+
+def same(xs, ys):
+    return all(torch.equal(x, y) for x, y in zip(xs, ys))
+
+
+def wide(t):
+    """The same values with another layout: twice the stride along the last dimension."""
+    return torch.stack((t, t), -1).flatten(-2)[..., ::2]
+
+
+def hooks(change):
+    return torch.autograd.graph.saved_tensors_hooks(lambda t: t, change)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bias", [False, True])
+def test_saved_tensor_hooks_that_move_or_lay_out_the_tensors(D, bias):
+    p = Problem(D=D, bias=bias)
+    want = p.grads()
+    with torch.autograd.graph.save_on_cpu():
+        o = p.forward()
+    assert same(p.grads(o), want)
+    for change in (torch.clone, wide):
+        with hooks(change):
+            o = p.forward()
+        assert same(p.grads(o), want), change
+    mask = BA.materialize_bitfield_mask(p.bf)
+    if not bias:
+        want = torch.autograd.grad(A.flash_attn_func(*p.inputs, mask=mask), p.inputs, p.do)
+        for change in (torch.clone, wide):
+            with hooks(change):
+                o = A.flash_attn_func(*p.inputs, mask=mask)
+            assert same(torch.autograd.grad(o, p.inputs, p.do), want), change
+
+
+def test_a_bias_that_comes_back_in_another_type_is_an_error_and_not_ignored():
+    p = Problem(bias=True)
+    with hooks(lambda t: t.double() if t.shape == p.bias.shape else t):
+        o = p.forward()
+    with pytest.raises(RuntimeError, match="bias"):
+        p.grads(o)
+
+
+# (tests of what else a hook may hand back, each refused on the host before anything is launched)
+@pytest.mark.parametrize("which,change", [
+    ("q", lambda t: t.float()), ("k", lambda t: t[:, :-1]), ("v", lambda t: t.cpu()), ("o", lambda t: t[..., :32]),
+    ("lse", lambda t: t.half()), ("lse", lambda t: t[:, :, :-1]), ("mask", lambda t: t.int()), ("mask", lambda t: t[:, :-1]),
+    ("flags", lambda t: t[:, :, :-1]), ("flags", lambda t: t.float()), ("bias", lambda t: t[..., :-1]), ("bias", lambda t: t.cpu()),
+])
+def test_a_tensor_that_comes_back_as_something_else_is_an_error(which, change):
+    p = Problem(Hkv=4, bias=True)
+    order = ["q", "k", "v", "lse", "bias", "mask", "flags", "o"]  # as the node packs them
+    packed = []
+
+    def pack(t):
+        packed.append(t)
+        return len(packed) - 1, t
+
+    def unpack(x):
+        n, t = x
+        return change(t) if order[n] == which else t
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        o = p.forward()
+    assert len(packed) == len(order)
+    with pytest.raises(RuntimeError, match=which):
+        p.grads(o)
