@@ -10,6 +10,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/Exceptions.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
@@ -428,7 +429,29 @@ struct AttentionBackward : public torch::autograd::Node {
         for (SavedVariable* s : {&q, &k, &v, &o, &lse, &bias, &mask, &flags}) s->reset_data();
         plan = Plan();
     }
+    // A C++ exception reaches the caller of the engine as a plain RuntimeError (this module's translator is not on that way);
+    // a Python error passes through it as what it is.
     variable_list apply(variable_list&& grads) override {
+        try {
+            return compute(std::move(grads));
+        } catch (const BamFailure& e) {
+            py::gil_scoped_acquire gil;
+            PyErr_SetString(g_error_type, e.what());
+            raise_python_error();
+        } catch (py::error_already_set& e) {
+            py::gil_scoped_acquire gil;
+            e.restore();
+            raise_python_error();
+        }
+    }
+
+private:
+    [[noreturn]] static void raise_python_error() {
+        python_error e;
+        e.persist();
+        throw e;
+    }
+    variable_list compute(variable_list&& grads) {
         if (!grads[0].defined()) return variable_list(3);
         const at::NoGradGuard no_grad;
         Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack(),

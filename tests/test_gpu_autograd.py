@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from cornstarch_amd.kernel import _bam_hip
 from cornstarch_amd.kernel import attention as A
 from cornstarch_amd.kernel import bitfield_attention as BA
 from tests.helpers import random_bitfield
@@ -95,5 +96,16 @@ def test_a_tensor_that_comes_back_as_something_else_is_an_error(which, change):
     with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
         o = p.forward()
     assert len(packed) == len(order)
-    with pytest.raises(RuntimeError, match=which):
+    with pytest.raises(_bam_hip.BamError, match=which):  # (the library's own error, also out of the engine)
+        p.grads(o)
+
+
+def test_a_python_error_inside_the_backward_reaches_the_caller_as_it_is(monkeypatch):
+    def no_workspace(*args):
+        raise KeyError("no workspace today")
+
+    p = Problem(D=128)
+    o = p.forward()
+    monkeypatch.setattr(BA._TilePlan, "backward_workspace", no_workspace)
+    with pytest.raises(KeyError, match="no workspace today"):
         p.grads(o)
