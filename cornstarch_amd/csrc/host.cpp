@@ -426,6 +426,7 @@ struct AttentionBackward : public torch::autograd::Node {
 
     std::string name() const override { return "BitfieldAttentionFunctionBackward"; }
     void release_variables() override {
+        const std::lock_guard<std::mutex> lock(mutex_);
         for (SavedVariable* s : {&q, &k, &v, &o, &lse, &bias, &mask, &flags}) s->reset_data();
         plan = Plan();
     }
@@ -454,8 +455,14 @@ private:
     variable_list compute(variable_list&& grads) {
         if (!grads[0].defined()) return variable_list(3);
         const at::NoGradGuard no_grad;
-        Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack(),
-               bias_ = bias.unpack(), mask_ = mask.unpack(), flags_ = flags.unpack();
+        Tensor q_, k_, v_, o_, lse_, bias_, mask_, flags_;
+        Plan plan_;
+        {  // (another thread's backward through the same graph may be releasing them)
+            const std::lock_guard<std::mutex> lock(mutex_);
+            q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(shared_from_this()), lse_ = lse.unpack();
+            bias_ = bias.unpack(), mask_ = mask.unpack(), flags_ = flags.unpack();
+            plan_ = plan;
+        }
         Tensor dout = grads[0];
         if (dout.scalar_type() != type) dout = dout.to(type);
         if (!rows_ready(dout, 8)) dout = dout.contiguous();
@@ -499,7 +506,7 @@ private:
                 throw BamFailure("the saved bias came back from its hooks with another shape, type or device");
             c.bias = &desc;
         }
-        run_backward(c, plan, dout, q_, k_, v_, o_, lse_, dq, dk, dv, false);
+        run_backward(c, plan_, dout, q_, k_, v_, o_, lse_, dq, dk, dv, false);
         return {dq, dk, dv};
     }
 };

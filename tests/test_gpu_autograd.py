@@ -1,5 +1,7 @@
 """The native autograd node under saved-tensor hooks."""
 
+import threading
+
 import pytest
 import torch
 
@@ -109,3 +111,46 @@ def test_a_python_error_inside_the_backward_reaches_the_caller_as_it_is(monkeypa
     monkeypatch.setattr(BA._TilePlan, "backward_workspace", no_workspace)
     with pytest.raises(KeyError, match="no workspace today"):
         p.grads(o)
+
+
+def test_threads_that_run_the_backward_of_one_graph():
+    p = Problem(D=128)
+    o = p.forward()
+    want = p.grads(o, retain_graph=True)
+    got, go = {}, threading.Barrier(4)
+
+    def work(n):
+        go.wait()
+        got[n] = [p.grads(o, retain_graph=True) for _ in range(5)]
+
+    threads = [threading.Thread(target=work, args=(n,)) for n in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert all(same(x, want) for n in range(4) for x in got[n])
+
+
+def test_threads_of_which_one_may_free_the_graph():
+    # every backward either gives the gradients or says that the graph has been freed
+    p = Problem(D=128)
+    want = p.grads()
+    for _ in range(20):
+        o, go, got = p.forward(), threading.Barrier(4), {}
+
+        def work(n):
+            go.wait()
+            try:
+                got[n] = p.grads(o, retain_graph=n != 0)
+            except RuntimeError as e:
+                got[n] = e
+
+        threads = [threading.Thread(target=work, args=(n,)) for n in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        for x in got.values():
+            assert "second time" in str(x) if isinstance(x, RuntimeError) else same(x, want)
