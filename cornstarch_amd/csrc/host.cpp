@@ -199,8 +199,15 @@ void store(Cached& slot, const Tensor& owner, const Tensor& flags, Plan plan) {
     fresh.flags = flags;
     fresh.version = owner._version();
     fresh.plan = std::move(plan);
-    std::swap(slot, fresh);  // the old entry goes after the new one is in place: its end may run Python code
+    std::swap(slot, fresh);  // the old entry goes after the new one is in place: its end may run Python code, which may call here
 }
+
+// What the caller of a lookup works with: a copy, as the entry itself may be replaced whenever Python code can run (the end
+// of the entry it replaced, a garbage collection), by another thread or by a finalizer of this one.
+struct Flags {
+    Tensor flags;
+    Plan plan;
+};
 
 bool plain(const Tensor& t) {  // an ordinary tensor: no subclass, no functorch wrapper, no forward-mode tangent
     return !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
@@ -214,8 +221,8 @@ bool bitfield_ready(const Tensor& bf) {
 }
 
 // flags (and plan, up to 131072 tokens) of an int64 (B, S) mask on the GPU
-const Cached& bitfield_flags(const Tensor& mask) {
-    if (g_bitfield.hit(mask)) return g_bitfield;
+Flags bitfield_flags(const Tensor& mask) {
+    if (g_bitfield.hit(mask)) return {g_bitfield.flags, g_bitfield.plan};
     const Tensor bf = mask.stride(1) == 1 ? mask : mask.contiguous();
     const c10::DeviceGuard guard(bf.device());
     const int64_t B = bf.size(0), S = bf.size(1);
@@ -239,8 +246,8 @@ const Cached& bitfield_flags(const Tensor& mask) {
                              (int)B, (int)S, stream.stream()),
               "bam_tile_flags");
     }
-    store(g_bitfield, mask, flags, std::move(plan));
-    return g_bitfield;
+    store(g_bitfield, mask, flags, plan);
+    return {flags, plan};
 }
 
 bool mask_ready(const Tensor& mask, int64_t B, int64_t Sq, int64_t Sk) {
@@ -250,8 +257,8 @@ bool mask_ready(const Tensor& mask, int64_t B, int64_t Sq, int64_t Sk) {
 }
 
 // the same for a materialized mask that satisfies mask_ready
-const Cached& mask_flags(const Tensor& mask) {
-    if (g_mask.hit(mask)) return g_mask;
+Flags mask_flags(const Tensor& mask) {
+    if (g_mask.hit(mask)) return {g_mask.flags, g_mask.plan};
     const c10::DeviceGuard guard(mask.device());
     const int64_t B = mask.size(0), Sq = mask.size(1), Sk = mask.size(2);
     const Stream stream = current_stream(mask.device());
@@ -282,8 +289,8 @@ const Cached& mask_flags(const Tensor& mask) {
                                   stream.stream()),
               "bam_mask_tile_flags");
     }
-    store(g_mask, mask, flags, std::move(plan));
-    return g_mask;
+    store(g_mask, mask, flags, plan);
+    return {flags, plan};
 }
 
 // ------------------------------------------------------------------ calls
@@ -554,9 +561,7 @@ optional<Tensor> bitfield_attention(const Tensor& q, const Tensor& k, const Tens
         if (!make_bias(*bias, q, k.size(1), desc)) return c10::nullopt;
         c.bias = &desc;
     }
-    const Cached& cached = bitfield_flags(bf);
-    const Tensor flags = cached.flags;
-    const Plan plan = cached.plan;
+    const auto [flags, plan] = bitfield_flags(bf);
     if (plan && plan.core->flags.unsafeGetTensorImpl() != flags.unsafeGetTensorImpl()) return c10::nullopt;
     c.bf = &bf;
     c.flags = &flags;
@@ -575,9 +580,7 @@ optional<Tensor> masked_attention(const Tensor& q, const Tensor& k, const Tensor
         if (!make_bias(*bias, q, k.size(1), desc)) return c10::nullopt;
         c.bias = &desc;
     }
-    const Cached& cached = mask_flags(mask);
-    const Tensor flags = cached.flags;
-    const Plan plan = cached.plan;
+    const auto [flags, plan] = mask_flags(mask);
     c.mode = BAM_MASK_DENSE;
     c.mask = &mask;
     c.flags = &flags;
@@ -760,8 +763,8 @@ PYBIND11_MODULE(_bam_host, m) {
     m.def("bitfield_flags_general", [](const Tensor& bf) { return bitfield_flags(bf).flags; });
     m.def("mask_flags", [](const Tensor& mask, int64_t B, int64_t Sq, int64_t Sk) -> py::object {
         if (!mask_ready(mask, B, Sq, Sk)) return py::none();
-        const Cached& c = mask_flags(mask);
-        return py::make_tuple(c.flags, c.plan.py_object());
+        const Flags f = mask_flags(mask);
+        return py::make_tuple(f.flags, f.plan.py_object());
     });
     // the plan cached with these very flags, if `bf` is still the unchanged mask they were computed from
     m.def("plan_for", [](const Tensor& flags, const Tensor& bf) -> py::object {
@@ -772,7 +775,8 @@ PYBIND11_MODULE(_bam_host, m) {
         return c.plan.py_object();
     });
     m.def("cached_bitfield_flags", []() -> py::object {
-        return g_bitfield.flags.defined() ? py::cast(g_bitfield.flags) : py::none();
+        const Tensor flags = g_bitfield.flags;
+        return flags.defined() ? py::cast(flags) : py::none();
     });
     m.def("cached_bitfield_plan", []() { return g_bitfield.plan.py_object(); });
     m.def("set_cached_bitfield_flags", [](optional<Tensor> flags) {

@@ -3,6 +3,7 @@ against a brute-force classification of the oracle's mask, and the attention res
 
 import ctypes
 import math
+import weakref
 
 import pytest
 import torch
@@ -275,6 +276,30 @@ def test_two_host_threads_with_different_masks_share_the_caches():
     for th in threads:
         th.join()
     assert not errors, errors
+    BA.BitfieldUtils.clear_cache()
+
+
+def test_a_mask_whose_end_looks_up_other_flags():
+    # the cache lets go of the previous mask when it takes a new one; a finalizer of that mask may itself use the cache
+    old, new, other = (random_bitfield(1, S, seed=S) for S in (500, 300, 200))
+    newd, otherd = new.to(dev()), other.to(dev())
+    g = torch.Generator().manual_seed(0)
+    q, k, v = ((torch.randn(1, 300, H, 64, generator=g) * 0.5).bfloat16().to(dev()) for H in (4, 2, 2))
+    BA.BitfieldUtils.clear_cache()
+    want = BA.bitfield_attn_func(q, k, v, newd)
+    seen = []
+
+    def remember():
+        mask = old.to(dev())
+        BA.BitfieldUtils.clear_cache()
+        BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(mask)
+        weakref.finalize(mask, lambda: seen.append(BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(otherd)))
+
+    remember()
+    got = BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(newd)
+    assert len(seen) == 1 and torch.equal(got.cpu(), O.tile_flags(new)) and torch.equal(seen[0].cpu(), O.tile_flags(other))
+    remember()
+    assert torch.equal(BA.bitfield_attn_func(q, k, v, newd), want) and len(seen) == 2
     BA.BitfieldUtils.clear_cache()
 
 
