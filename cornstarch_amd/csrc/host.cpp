@@ -185,7 +185,7 @@ struct Cached {
     uint32_t version = 0;
     Plan plan;
     bool hit(const Tensor& t) const {
-        return owner.defined() && flags.defined() && owner.data_ptr() == t.data_ptr() && owner.sizes() == t.sizes() &&
+        return !t.is_inference() && owner.defined() && flags.defined() && owner.data_ptr() == t.data_ptr() && owner.sizes() == t.sizes() &&
                owner_strides == t.strides() && version == t._version() && owner.device() == t.device();
     }
     std::vector<int64_t> owner_strides;  // (the owner's own may be changed in place)
@@ -193,6 +193,7 @@ struct Cached {
 Cached g_bitfield, g_mask;
 
 void store(Cached& slot, const Tensor& owner, const Tensor& flags, Plan plan) {
+    if (owner.is_inference()) return;  // no version counter: nothing would tell that it has been written to
     Cached fresh;
     fresh.owner = owner;
     fresh.owner_strides = owner.strides().vec();
@@ -227,6 +228,7 @@ Flags bitfield_flags(const Tensor& mask) {
     const c10::DeviceGuard guard(bf.device());
     const int64_t B = bf.size(0), S = bf.size(1);
     const Stream stream = current_stream(bf.device());
+    const c10::InferenceMode ordinary(false);  // (an entry made in inference mode also serves calls outside)
     Tensor flags = at::empty({B, (S + 127) / 128, (S + 31) / 32}, bf.options().dtype(at::kChar));
     const int64_t bytes = bam_plan_workspace_bytes((int)B, (int)S);
     Plan plan;
@@ -262,6 +264,7 @@ Flags mask_flags(const Tensor& mask) {
     const c10::DeviceGuard guard(mask.device());
     const int64_t B = mask.size(0), Sq = mask.size(1), Sk = mask.size(2);
     const Stream stream = current_stream(mask.device());
+    const c10::InferenceMode ordinary(false);
     Tensor flags = at::empty({B, (Sq + 127) / 128, (Sk + 31) / 32}, mask.options().dtype(at::kChar));
     const int64_t bytes = bam_mask_plan_workspace_bytes((int)B, (int)Sq, (int)Sk);
     Plan plan;

@@ -154,3 +154,29 @@ def test_threads_of_which_one_may_free_the_graph():
         torch.cuda.synchronize()
         for x in got.values():
             assert "second time" in str(x) if isinstance(x, RuntimeError) else same(x, want)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_inference_mode(masked):
+    p = Problem()
+
+    def forward(q, k, v, bf):
+        return A.flash_attn_func(q, k, v, mask=BA.materialize_bitfield_mask(bf)) if masked else BA.bitfield_attn_func(q, k, v, bf)
+
+    want = forward(*p.inputs, p.bf).detach()
+    BA.BitfieldUtils.clear_cache()
+    A._MaskPlan.forget()
+    with torch.inference_mode():
+        first = forward(*(x.detach() for x in p.inputs), p.bf)
+        # inputs made in inference mode, a mask without a version counter among them
+        copies = [x.detach().clone() for x in (*p.inputs, p.bf)]
+        second = forward(*copies)
+        copies[3].fill_(p.bf[0, 0])  # written to: nothing of the last call is left
+        third = forward(*copies)
+    assert first.is_inference() and torch.equal(first, want) and torch.equal(second, want)
+    # what the first call left in the cache serves training as well
+    got = torch.autograd.grad(forward(*p.inputs, p.bf), p.inputs, p.do)
+    BA.BitfieldUtils.clear_cache()
+    assert same(got, torch.autograd.grad(forward(*p.inputs, p.bf), p.inputs, p.do))
+    assert torch.equal(third, forward(*p.inputs, torch.full_like(p.bf, int(p.bf[0, 0]))))
+    BA.BitfieldUtils.clear_cache()
