@@ -1,9 +1,12 @@
-"""The native autograd node under saved-tensor hooks."""
+"""The native autograd node under what a training program does around it: saved-tensor hooks, activation checkpointing, graphs
+kept or freed, gradients of some inputs only, tensor subclasses, inference mode, and the transforms it has no rule for."""
 
 import threading
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
+from torch.utils.checkpoint import checkpoint
 
 from cornstarch_amd.kernel import _bam_hip
 from cornstarch_amd.kernel import attention as A
@@ -156,6 +159,64 @@ def test_threads_of_which_one_may_free_the_graph():
             assert "second time" in str(x) if isinstance(x, RuntimeError) else same(x, want)
 
 
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_activation_checkpointing(reentrant):
+    p = Problem(D=128)
+    want = p.grads()
+    o = checkpoint(p.forward, *p.inputs, use_reentrant=reentrant)
+    if reentrant:  # (its backward only runs through backward())
+        o.backward(p.do)
+        got = [x.grad for x in p.inputs]
+    else:
+        got = p.grads(o)
+    assert same(got, want)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_graph_is_kept_or_freed(D):
+    p = Problem(D=D)
+    o = p.forward()
+    first = p.grads(o, retain_graph=True)
+    assert same(p.grads(o), first)
+    with pytest.raises(RuntimeError, match="second time"):
+        p.grads(o)
+    # no second derivative: the gradients are constants
+    assert not any(x.requires_grad for x in p.grads(create_graph=True))
+
+
+def test_inputs_changed_after_the_forward_are_noticed():
+    for name in ("q", "bf"):
+        p = Problem()
+        o = p.forward()
+        with torch.no_grad():
+            getattr(p, name).add_(0)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            p.grads(o)
+
+
+def test_gradients_of_some_inputs_only():
+    p = Problem(D=128)
+    want = p.grads()
+    for n in range(3):
+        inputs = [x if n == m else x.detach() for m, x in enumerate(p.inputs)]
+        (got,) = torch.autograd.grad(p.forward(*inputs), (p.inputs[n],), p.do)
+        assert torch.equal(got, want[n])
+    # an input that is the output of other operations, and one tensor in two roles
+    x = p.k.detach().clone().requires_grad_(True)
+    (got,) = torch.autograd.grad(p.forward(p.q.detach(), x * 1.0, x), (x,), p.do)
+    o = p.forward(p.q.detach(), p.k, p.k)
+    (both,) = torch.autograd.grad(o, (p.k,), p.do)
+    assert torch.equal(got, both)
+
+
+def test_no_graph_without_gradients():
+    p = Problem()
+    want = p.forward().detach()
+    with torch.no_grad():
+        assert p.forward().grad_fn is None
+    assert p.forward(*(x.detach() for x in p.inputs)).grad_fn is None
+
+
 @pytest.mark.parametrize("masked", [False, True])
 def test_inference_mode(masked):
     p = Problem()
@@ -180,3 +241,28 @@ def test_inference_mode(masked):
     assert same(got, torch.autograd.grad(forward(*p.inputs, p.bf), p.inputs, p.do))
     assert torch.equal(third, forward(*p.inputs, torch.full_like(p.bf, int(p.bf[0, 0]))))
     BA.BitfieldUtils.clear_cache()
+
+
+def test_tensor_subclasses():
+    class Named(torch.Tensor):
+        pass
+
+    p = Problem()
+    want = p.grads()
+    named = [x.detach().as_subclass(Named).requires_grad_(True) for x in p.inputs]
+    got = torch.autograd.grad(p.forward(*named), named, p.do)
+    assert same(got, want)
+    parameters = [torch.nn.Parameter(x.detach()) for x in p.inputs]
+    assert same(torch.autograd.grad(p.forward(*parameters), parameters, p.do), want)
+
+
+def test_transforms_without_a_rule_are_refused():
+    p = Problem(Hkv=4)
+    q, k, v = (x.detach() for x in p.inputs)
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: p.forward(x, k, v).float().sum())(q)
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda x: p.forward(x, k, v))(torch.stack((q, q)))
+    with fwAD.dual_level():
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            p.forward(fwAD.make_dual(q, torch.ones_like(q)), k, v)
