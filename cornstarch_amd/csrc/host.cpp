@@ -417,8 +417,11 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     Tensor parts;  // (given back to the caching allocator on return: the launches that use it are on the current stream)
     check(bam_attn_bwd_parts(&a, &a.parts_bytes), "bam_attn_bwd_parts");
     if (a.parts_bytes > 0) {
-        parts = at::empty({a.parts_bytes}, q.options().dtype(at::kByte));
-        a.parts_workspace = parts.data_ptr();
+        try {
+            parts = at::empty({a.parts_bytes}, q.options().dtype(at::kByte));
+            a.parts_workspace = parts.data_ptr();
+        } catch (const c10::OutOfMemoryError&) {  // no room for it right now: one part, as without a workspace
+        }
     }
     check(bam_attn_bwd(&a, current_stream(q.device()).stream()), "bam_attn_bwd");
 }

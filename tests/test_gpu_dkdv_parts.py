@@ -49,3 +49,39 @@ def test_parts_against_the_oracle(B, S, Hq, Hkv, D, bias):
         err = (a - 1.0 - t.float()).abs() - t.float().abs() * 2.0 ** -8 - 2.0 ** -22
         assert err.max().item() <= 0
     BA.BitfieldUtils.clear_cache()
+
+
+def test_without_room_for_the_parts_the_backward_runs_in_one_part():
+    B, S, Hq, Hkv, D = 1, 512, 8, 1, 64  # 8 parts: 2 MiB, a segment of its own; everything else comes from smaller ones
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(0)
+    q, k, v, do = (torch.randn(B, S, H, D, generator=g, device=dev).bfloat16().requires_grad_(n < 3)
+                   for n, H in enumerate((Hq, Hkv, Hkv, Hq)))
+    bf = random_bitfield(B, S, seed=1).to(dev)
+    BA.BitfieldUtils.clear_cache()
+    want = torch.autograd.grad(BA.bitfield_attn_func(q, k, v, bf), (q, k, v), do)
+    o = BA.bitfield_attn_func(q, k, v, bf)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    small = [torch.empty(1 << 19, dtype=torch.uint8, device=dev) for _ in range(8)]  # room for the gradients
+    total = torch.cuda.get_device_properties(dev).total_memory
+    hold = []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved(dev) / total)
+        while True:  # what is left of larger segments
+            try:
+                hold.append(torch.empty(2 << 20, dtype=torch.uint8, device=dev))
+            except torch.cuda.OutOfMemoryError:
+                break
+        small = small[:1]  # (keeps their segment)
+        got = torch.autograd.grad(o, (q, k, v), do)
+        torch.cuda.synchronize()
+        with pytest.raises(torch.cuda.OutOfMemoryError):  # there was no room indeed
+            torch.empty(2 << 20, dtype=torch.uint8, device=dev)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        del hold, small
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):  # the same sums in another order, rounded to bf16 once
+        assert ((a.float() - b.float()).norm() / b.float().norm()).item() <= 2.0 ** -8
+    BA.BitfieldUtils.clear_cache()
