@@ -144,3 +144,26 @@ def test_training_mode_takes_the_bitfield_path_and_bad_arguments_are_refused():
         _bam_hip.call("bam_decode", q.data_ptr(), kt.data_ptr(), vt.data_ptr(), o.data_ptr(), q.stride(0), q.stride(1),
                       kt.stride(0), kt.stride(1), kt.stride(2), vt.stride(0), vt.stride(1), vt.stride(2), o.stride(0),
                       o.stride(1), 1, 8, 4, 2, 64, 0.125, BA._dtype_code(q.dtype), -1, 0.0, None, 0, BA._stream_ptr(dev()))
+
+
+@pytest.mark.parametrize("cap", [1e4, 1e6, float(2 ** 30)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_step_scores_far_below_the_cap_keep_their_precision(cap, D):
+    # Two keys with values +1 and -1: the output is tanh((s0 - s1) / 2), so an error e of a capped score shows as up to e / 2.
+    # Bound: the second weight (at most 1) and the output are rounded to fp16, 2^-11 each, and the scores are sums in fp32 of a
+    # few units, about 1e-6.
+    B, Hq = 16, 8
+    q, k, v = inputs(B, Hq, Hq, 2, D, torch.float16, seed=D, std=1.0)
+    v[:, :, 0], v[:, :, 1] = 1.0, -1.0
+    got = decode(q, k, v, softcap=cap).double()[:, 0, :, 0]
+    s = (q.double() @ k.double().transpose(2, 3))[:, :, 0] / math.sqrt(D)
+    s = cap * torch.tanh(s / cap)
+    want = torch.tanh((s[..., 0] - s[..., 1]) / 2)
+    assert (got - want).abs().max().item() <= 2 * 2.0 ** -11 + 1e-5
+
+
+def test_decode_step_with_scores_of_zero_under_the_smallest_cap():
+    q, k, v = inputs(2, 4, 2, 50, 64, torch.bfloat16)
+    got = decode(torch.zeros_like(q), k, v, softcap=1e-40)  # 1 / cap is not a finite float
+    want = v.float().mean(dim=2).repeat_interleave(2, dim=1)[:, None]
+    assert (got.float() - want).abs().max().item() <= 2.0 ** -9 + 50 * 2.0 ** -24  # |v| below 2: the output is rounded to bf16
