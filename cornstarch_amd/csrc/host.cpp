@@ -689,9 +689,9 @@ constexpr int64_t kDecodeCounters = 8192;
 std::mutex g_counters_mutex;
 std::vector<std::pair<void*, Tensor>> g_counters;
 // None while capturing: the library does not use them there, and a set made then would live in the graph's memory and be
-// cleared by its replays.
+// cleared by its replays.  None on hipStreamPerThread: one handle, another stream in each thread.
 uint32_t* decode_counters(const Tensor& like, const Stream& stream) {
-    if (capturing()) return nullptr;
+    if (capturing() || stream.stream() == hipStreamPerThread) return nullptr;
     std::lock_guard<std::mutex> guard(g_counters_mutex);
     for (const auto& [s, t] : g_counters)
         if (s == (void*)stream.stream() && t.device() == like.device()) return (uint32_t*)t.data_ptr();
@@ -801,6 +801,7 @@ PYBIND11_MODULE(_bam_host, m) {
         Cached gone;
         std::swap(g_mask, gone);
     });
+    m.def("decode_counter_sets", []() { return g_counters.size(); });
     m.def("release_memory", []() {
         count_words().release();
         g_counters.clear();

@@ -49,3 +49,19 @@ def test_pieces_and_merges(B, Hq, Hkv, Sk, D, dtype):
                           BA._stream_ptr(d))
             torch.cuda.synchronize()
             assert (out.float().cpu() - want).abs().max().item() <= 2e-2
+
+
+def test_the_stream_that_has_one_handle_for_all_threads():
+    # hipStreamPerThread: no counters are kept for it, the second launch merges
+    d = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(0)
+    q, k, v = ((torch.randn(s, generator=g) * 0.5).bfloat16() for s in ((2, 8, 1, 64), (2, 2, 1999, 64), (2, 2, 1999, 64)))
+    qd, kd, vd = (t.to(d) for t in (q, k, v))
+    want = O.decode_step(q, k, v)
+    before = _bam_hip.host.decode_counter_sets()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.ExternalStream(2)):
+        out = interface.bitfield_attention_forward(torch.nn.Module().eval(), qd, kd, vd, None)[0]
+    torch.cuda.synchronize()
+    assert (out.float().cpu() - want).abs().max().item() <= 2e-2
+    assert _bam_hip.host.decode_counter_sets() == before
