@@ -943,7 +943,6 @@ static int decode_impl(const void* q, const void* k, const void* v, void* o, int
     p.Sk = Sk;
     p.Hq = Hq;
     p.Hkv = Hkv;
-    p.window = window;
     p.scale = scale;
     p.softcap = softcap;
     return launched(bam::launch_decode(p, s, dtype, (hipStream_t)stream), "bam_decode");

@@ -100,7 +100,6 @@ struct DecodeParams {
     int64_t q_sb, q_sh, k_sb, k_ss, k_sh, v_sb, v_ss, v_sh, o_sb, o_sh;
     int B, Sk, Hq, Hkv;
     int D, d;                      // the D the kernel is compiled for and the head dim (a multiple of 8, <= D)
-    int window;                    // > 0: only the last `window` keys are attended to
     float scale, softcap;          // softcap > 0: scores become softcap * tanh(score / softcap)
     int o_vec;                     // groups of four columns of o are 8-byte aligned
     // How the tiles are dealt to workgroups (decode_split) and where the parts of a unit leave their partial results:
