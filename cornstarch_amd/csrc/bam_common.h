@@ -175,8 +175,9 @@ __device__ __forceinline__ float load_bias1(const void* base, int64_t index, boo
 //     two cycles per instruction, hidden inside the four cycles a wave-wide LDS instruction takes).
 // Head dims.  The kernels are compiled for D = 32, 64, 96 and 128; a call's head dim d is any multiple of 8 up to D.  A
 // row of an LDS tile has room for LDS_COLS<D> elements (a power of two: the swizzle is an XOR over whole rows of chunks).
-// Chunks past d are never zero filled by the tile copies: their lanes fetch chunk 0 of the row again (tile_chunk), and
-// whoever multiplies along the head dim has zeros in the other operand there; columns past d of an output are computed
+// Chunks past d hold zeros where the tile copies put them (the K tiles of the forward, dQ and the decode step: ZERO_PAD) and
+// chunk 0 of the row again in the other tiles; whoever multiplies along the head dim has zeros in the other operand there,
+// and columns past d of an output are computed
 // and not stored.  Before, other head dims were padded on the host: three copies of q, k, v and up to 37 launches a step.
 template <int D>
 constexpr int LDS_COLS = D <= 32 ? 32 : D <= 64 ? 64 : 128;

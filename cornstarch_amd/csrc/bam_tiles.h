@@ -37,6 +37,19 @@ __device__ __forceinline__ void dma_b128_stream(const void* sbase, unsigned voff
                  "n"(SITE)
                  : "memory");
 }
+// The 16-byte copy through a buffer descriptor over [base, base + DMA_RANGE): a lane whose offset lies beyond reads nothing
+// and the hardware writes zeros to its LDS slot.  The descriptor's last two words stay in registers over the loop; K tiles
+// copied this way instead of by dma_b128, whole step: 1 x 8192 tokens, D 128 no change (1903 / 1904 us), 8 x 4096, D 64
+// 1142 / 1147, decode of 8 x 8192 keys 48.7 / 48.7.
+constexpr unsigned DMA_RANGE = 0x80000000u, DMA_ZERO = 0xC0000000u;  // (room below for 31 rows of 2^24 bytes: decode steps back)
+template <int SITE = 0>
+__device__ __forceinline__ void dma_b128_ranged(const void* sbase, unsigned voff, unsigned lds_base) {
+    const unsigned long long base = reinterpret_cast<unsigned long long>(sbase);  // (48 bits: no stride in the second word)
+    const u32x4 desc = {(unsigned)base, (unsigned)(base >> 32), DMA_RANGE, 0x00020000u};
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds ; site %3" ::"v"(voff), "s"(desc), "{m0}"(lds_base),
+                 "n"(SITE)
+                 : "memory");
+}
 template <int SITE = 0>
 __device__ __forceinline__ void dma_b32(const void* sbase, unsigned voff, unsigned lds_base) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1 ; site %3" ::"v"(voff), "s"(sbase), "{m0}"(lds_base),
@@ -62,7 +75,10 @@ __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)"
 // The last, ragged tile of a sequence takes the synchronous path (`load_ragged`), which
 // zero-fills the rows past the end.  Row strides are limited to 2^23 elements by the host
 // checks, so the offsets fit 32 bits.
-template <int D, int ROWS, int THREADS>
+// ZERO_PAD: chunks past the head dim become zero in LDS (whoever multiplies along the head dim has zeros in the other operand
+// there, but zero times an infinity of chunk 0 would be a NaN in the score of a key whose weight is 0); otherwise their lanes
+// fetch chunk 0 again.
+template <int D, int ROWS, int THREADS, bool ZERO_PAD = false>
 struct TileStage {
     static constexpr int NCH = LDS_COLS<D> / 8;
     static constexpr int CHUNKS = ROWS * NCH;
@@ -79,15 +95,21 @@ struct TileStage {
             const int id = tid + THREADS * i;
             const int row = id / NCH, pc = id % NCH;
             const int c = pc ^ swz<D>(row);
-            goff[i] = (unsigned)(row * row_stride_bytes + (c < chunks ? c : 0) * 16);
+            goff[i] = ZERO_PAD && c >= chunks ? DMA_ZERO : (unsigned)(row * row_stride_bytes + (c < chunks ? c : 0) * 16);
         }
     }
     // tile_base: first row of the tile in global memory, tile_lds: lds_addr() of the LDS tile
     // (both wave-uniform)
     template <int SITE = 0>
     __device__ __forceinline__ void issue(int i, const char* tile_base, unsigned tile_lds) const {
-        if (EXACT || wave_first + THREADS * i < CHUNKS)
-            dma_b128<SITE>(tile_base, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
+        if (EXACT || wave_first + THREADS * i < CHUNKS) copy<SITE>(tile_base, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
+    }
+    template <int SITE = 0>
+    static __device__ __forceinline__ void copy(const char* base, unsigned voff, unsigned lds_base) {
+        if (ZERO_PAD)
+            dma_b128_ranged<SITE>(base, voff, lds_base);
+        else
+            dma_b128<SITE>(base, voff, lds_base);
     }
     __device__ __forceinline__ void load_full(const char* tile_base, unsigned tile_lds) const {
 #pragma unroll
@@ -99,7 +121,7 @@ struct TileStage {
         for (int i = 0; i < CPT; ++i) {
             const int id = tid + THREADS * i;
             u32x4 z = {0u, 0u, 0u, 0u};
-            if ((EXACT || id < CHUNKS) && id / NCH < rows_valid) z = *(const u32x4*)(tile_base + goff[i]);
+            if ((EXACT || id < CHUNKS) && id / NCH < rows_valid && !(ZERO_PAD && goff[i] == DMA_ZERO)) z = *(const u32x4*)(tile_base + goff[i]);
             if (EXACT || id < CHUNKS) tile[id] = z;
         }
     }

@@ -835,7 +835,8 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS ? 2 : 3) void bwd_dq_ker
     // copy instructions per wave and tile: K, V, the key bitfields, (IDX) the key positions and (BIAS) the bias values
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (BIAS ? 1 : 0);
     static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the first S / dP block (and at most one behind it)");
-    Stage stK, stV;
+    TileStage<D, DQ_KT, DQ_THREADS, true> stK;
+    Stage stV;
     stK.setup(2 * p.k.ss, p.d / 8, tid);
     stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);

@@ -122,7 +122,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 1 ? 2 : 1) void decode_kernel(
     u32x4* const sV = sTiles[wave] + DEC_K_BUFS * TILE;
     const bool q_aligned = ((reinterpret_cast<uintptr_t>(p.q) | (uintptr_t)(2 * p.q_sb) | (uintptr_t)(2 * p.q_sh)) & 15u) == 0;
     const float inv_cap = p.softcap > 0.f ? fminf(1.f / p.softcap, FLT_MAX) : 0.f;  // (finite: a score of 0 stays 0)
-    TileStage<D, DEC_KT, 64> stK, stV;
+    TileStage<D, DEC_KT, 64, true> stK;
+    TileStage<D, DEC_KT, 64> stV;
     constexpr int CPT = TileStage<D, DEC_KT, 64>::CPT;
     stK.setup(2 * p.k_ss, chunks, lane);
     stV.setup(2 * p.v_ss, chunks, lane);
@@ -176,8 +177,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 1 ? 2 : 1) void decode_kernel(
 #pragma unroll
             for (int i = 0; i < CPT; ++i) {
                 const int over = max(0, (lane + 64 * i) / NCH - (nvalid - 1));  // rows this lane has to go back
-                dma_b128<3>(kt, stK.goff[i] - (unsigned)(over * (int)(2 * p.k_ss)), lk + 1024u * i);
-                dma_b128<4>(vt, stV.goff[i] - (unsigned)(over * (int)(2 * p.v_ss)), lv + 1024u * i);
+                stK.template copy<3>(kt, stK.goff[i] - (unsigned)(over * (int)(2 * p.k_ss)), lk + 1024u * i);
+                stV.template copy<4>(vt, stV.goff[i] - (unsigned)(over * (int)(2 * p.v_ss)), lv + 1024u * i);
             }
         }
     };

@@ -130,7 +130,8 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
     // (IDX) the key positions
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (BIAS ? 1 : 0);
     static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the S phase (and at most one behind it)");
-    Stage stK, stV;
+    TileStage<D, FWD_KT, FWD_THREADS, true> stK;
+    Stage stV;
     stK.setup(2 * p.k.ss, p.d / 8, tid);
     stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);

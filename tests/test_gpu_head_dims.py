@@ -2,11 +2,16 @@
 gradients written in the input dtype and gradients accumulated in fp32, with and without the dS hand-over (head dims
 above 64), against the fp32 oracle at the bars of the other parity tests."""
 
+import ctypes
+
 import pytest
 import torch
 
+from cornstarch_amd.kernel import attention as A
 from cornstarch_amd.kernel import bitfield_attention as BA
+from cornstarch_amd.kernel import interface
 from oracle import bam_oracle as O
+from tests import lds_fill
 from tests.helpers import random_bitfield, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -41,4 +46,66 @@ def test_head_dims_between_the_compiled_ones(dtype, D, B, S, Hq, Hkv):
         for a, b, w in zip(typed, acc, want):
             assert a.shape == w.shape and torch.isfinite(a).all()
             assert rel_l2(a.float().cpu(), w) <= 5e-2 and rel_l2(b.cpu() - 1, w) <= 5e-2
+    BA.BitfieldUtils.clear_cache()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [8, 24, 32, 40, 56, 64, 72, 96, 104, 128])
+def test_an_infinity_in_a_key_gives_its_scores_and_nothing_else(dtype, D):
+    # a key with -inf in one column and queries that are positive there: every score of it is -inf and its weight is 0,
+    # also where the tiles have columns past the head dim.  Lengths with and without a ragged last tile.
+    d = torch.device("cuda:0")
+    for S in (64, 200):
+        g = torch.Generator().manual_seed(D + S)
+        q, k, v = ((torch.randn(1, S, H, D, generator=g) * 0.5).to(dtype) for H in (4, 2, 2))
+        bf = torch.full((1, S), (1 << 62) | 1 | 2, dtype=torch.int64)
+        col, keys = 3, torch.tensor([5, 41, S - 2])
+        q[..., col] = q[..., col].abs() + 0.5
+        k[:, keys, :, col] = -float("inf")
+        want, _ = O.attention_forward(q, k, v, bf)
+        assert torch.isfinite(want).all()
+        BA.BitfieldUtils.clear_cache()
+        qd, kd, vd, bfd = (t.to(d) for t in (q, k, v, bf))
+        o = BA.bitfield_attn_func(qd, kd, vd, bfd)
+        mask = torch.ones(S, S, dtype=torch.bool, device=d).tril()[None]
+        for got in (o, A.flash_attn_func(qd, kd, vd, mask=mask)):
+            assert (got.float().cpu() - want).abs().max().item() <= 2e-2
+        # the decode step: one query against the same keys
+        out, _ = interface.bitfield_attention_forward(torch.nn.Module().eval(), qd[:, -1:].transpose(1, 2), kd.transpose(1, 2),
+                                                      vd.transpose(1, 2), None)
+        assert (out[:, 0].float().cpu() - want[:, -1]).abs().max().item() <= 2e-2
+    BA.BitfieldUtils.clear_cache()
+
+
+@pytest.mark.parametrize("D", [24, 40, 56, 72, 104])
+def test_columns_past_the_head_dim_do_not_come_from_lds_leftovers(D):
+    # after the LDS of every compute unit was filled with NaN patterns: same bits as undisturbed
+    d = torch.device("cuda:0")
+    fill, sink = lds_fill.load(), torch.zeros(4, dtype=torch.int32, device=d)
+    g = torch.Generator().manual_seed(D)
+    q, k, v, do = ((torch.randn(2, 200, H, D, generator=g) * 0.5).bfloat16().to(d) for H in (4, 2, 2, 4))
+    bf = random_bitfield(2, 200, seed=D, pad=3).to(d)
+    BA.BitfieldUtils.clear_cache()
+    flags = BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(bf)
+    module = torch.nn.Module().eval()
+
+    def run(disturb):
+        def poison():
+            if disturb:
+                assert fill.lds_fill(ctypes.c_void_p(sink.data_ptr()), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+
+        acc = [torch.zeros(t.shape, dtype=torch.float32, device=d) for t in (q, k, v)]
+        poison()
+        o, lse, scale = BA._bitfield_attn_forward(q, k, v, bf, flags)
+        poison()
+        BA._bitfield_attn_backward(do, q, k, v, o, bf, flags, lse, *acc, softmax_scale=scale)
+        poison()
+        step = interface.bitfield_attention_forward(module, q[:, -1:].transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), None)[0]
+        torch.cuda.synchronize()
+        return o, *acc, step
+
+    want = run(False)
+    assert all(torch.isfinite(t).all() for t in want)
+    for _ in range(4):
+        assert all(torch.equal(a, b) for a, b in zip(run(True), want))
     BA.BitfieldUtils.clear_cache()
