@@ -124,14 +124,13 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
     const int64_t k_ts = 2 * p.k.ss * FWD_KT, v_ts = 2 * p.v.ss * FWD_KT;  // bytes per tile
     const int64_t* bfrow = p.bfk + (int64_t)b * p.bfk_sb;
 
-    typedef TileStage<D, FWD_KT, FWD_THREADS> Stage;
+    typedef TileStage<D, FWD_KT, FWD_THREADS, true> Stage;  // (V only to copy both tiles alike, see dma_b128_ranged)
     constexpr int CPT = Stage::CPT;
     // copy instructions per wave and tile: K, V, the key bitfields (DENSE: the mask bits of the wave's rows) and
     // (IDX) the key positions
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (BIAS ? 1 : 0);
     static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the S phase (and at most one behind it)");
-    TileStage<D, FWD_KT, FWD_THREADS, true> stK;
-    Stage stV;
+    Stage stK, stV;
     stK.setup(2 * p.k.ss, p.d / 8, tid);
     stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);
