@@ -7,7 +7,7 @@ int launch_bwd_dq_long(const AttnParams& p, int dtype, hipStream_t stream);  // 
 
 template <typename T, int D>
 static int launch_dq_t(const AttnParams& p, hipStream_t stream) {
-    return p.bias != nullptr ? launch_dq_b<T, D, true, false>(p, stream) : launch_dq_b<T, D, false, false>(p, stream);
+    return launch_dq_b<T, D, false>(p, stream);
 }
 
 int launch_bwd_dq(const AttnParams& p, int dtype, hipStream_t stream) {

@@ -726,9 +726,17 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 constexpr int DQ_KT = 64;
 constexpr int DQ_THREADS = 256;
 
+// Forms of a bias: read from global memory group by group, or (one row of keys, its groups of four aligned) copied with the
+// tiles.  The second takes a wave per SIMD of the head dims up to 64 (26 spilled registers otherwise), the first keeps it.  As
+// one kernel with two waves the matrix form lost and both paid for the choice in the loop; dQ, 2 x 2048 tokens, 16 heads, bf16,
+// one kernel -> two: matrix D 32 104.6 -> 96.6 us, D 64 108.0 -> 108.0, fp32 matrix D 32 92.8 -> 85.6, D 64 99.0 -> 97.1; one
+// row of keys D 32 47.2 -> 43.1, D 64 59.9 -> 57.0; 2047 tokens (unaligned rows) D 32 88.8 -> 81.9, D 64 104.6 -> 103.1.
+constexpr int BIAS_NONE = 0, BIAS_READ = 1, BIAS_TILES = 2;
+
 // LONG: as in the dK/dV kernel, for more than MAX_LIST 64-key tiles.
-template <typename T, int D, int MODE, bool BIAS, bool LONG>
-__global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS ? 2 : 3) void bwd_dq_kernel(const AttnParams p) {
+template <typename T, int D, int MODE, int BIAS_FORM, bool LONG>
+__global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 : 3) void bwd_dq_kernel(const AttnParams p) {
+    constexpr bool BIAS = BIAS_FORM != BIAS_NONE, bias_lds = BIAS_FORM == BIAS_TILES;
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     __shared__ u32x4 sK[2][DQ_KT * NCH];
@@ -740,7 +748,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS ? 2 : 3) void bwd_dq_ker
     // DENSE with packed mask bits: per wave, the words of its 32 rows for the tile's two 32-key blocks
     __shared__ unsigned sRowBits[DENSE ? 2 : 1][4][DENSE ? 64 : 1];
     // BIAS in its per-key form: the 64 values of the tile (raw words; 16-bit elements fill half)
-    __shared__ __attribute__((aligned(16))) unsigned sBias[BIAS ? 2 : 1][BIAS ? 64 : 1];
+    __shared__ __attribute__((aligned(16))) unsigned sBias[bias_lds ? 2 : 1][bias_lds ? 64 : 1];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
@@ -816,8 +824,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS ? 2 : 3) void bwd_dq_ker
     // operands it is added by one more MFMA of the S phase, as in the forward.  (Read from global memory inside the loop,
     // every group of four waited, through the in-order vmcnt, for all tile copies in flight: 2 x 2048 tokens, 16 heads,
     // D 64: 75 us, now 63.)
-    const bool bias_lds = BIAS && p.bias_sm == 0 && p.bias_vec != 0;
-    const bool bias_fold = bias_lds && std::is_same<T, BF16>::value;
+    constexpr bool bias_fold = bias_lds && std::is_same<T, BF16>::value;
     const float c2 = (BIAS && !bias_fold) ? LOG2E : p.scale * LOG2E;  // otherwise the scores become scale * s + bias first
     const float inv_scale = 1.f / p.scale;
     const char* bias_row = nullptr;  // this lane's row of the bias
@@ -832,8 +839,8 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS ? 2 : 3) void bwd_dq_ker
 
     typedef TileStage<D, DQ_KT, DQ_THREADS> Stage;
     constexpr int CPT = Stage::CPT;
-    // copy instructions per wave and tile: K, V, the key bitfields, (IDX) the key positions and (BIAS) the bias values
-    constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (BIAS ? 1 : 0);
+    // copy instructions per wave and tile: K, V, the key bitfields, (IDX) the key positions and (BIAS_TILES) the bias values
+    constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (bias_lds ? 1 : 0);
     static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the first S / dP block (and at most one behind it)");
     TileStage<D, DQ_KT, DQ_THREADS, true> stK;
     Stage stV;
@@ -1154,8 +1161,8 @@ static int launch_dkdv_save_b(const AttnParams& p, hipStream_t stream) {
         hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     return (int)hipGetLastError();
 }
-template <typename T, int D, bool BIAS, bool LONG>
-static int launch_dq_b(const AttnParams& p, hipStream_t stream) {
+template <typename T, int D, int BIAS, bool LONG>
+static int launch_dq_f(const AttnParams& p, hipStream_t stream) {
     const int blocks = p.num_m * p.B * p.Hq;
     if (p.mask_mode == MASK_INDEXED)
         hipLaunchKernelGGL((bwd_dq_kernel<T, D, MASK_INDEXED, BIAS, LONG>), dim3(blocks), dim3(DQ_THREADS), 0, stream, p);
@@ -1164,6 +1171,11 @@ static int launch_dq_b(const AttnParams& p, hipStream_t stream) {
     else
         hipLaunchKernelGGL((bwd_dq_kernel<T, D, MASK_BITFIELD, BIAS, LONG>), dim3(blocks), dim3(DQ_THREADS), 0, stream, p);
     return (int)hipGetLastError();
+}
+template <typename T, int D, bool LONG>
+static int launch_dq_b(const AttnParams& p, hipStream_t stream) {
+    if (p.bias == nullptr) return launch_dq_f<T, D, BIAS_NONE, LONG>(p, stream);
+    return p.bias_sm == 0 && p.bias_vec ? launch_dq_f<T, D, BIAS_TILES, LONG>(p, stream) : launch_dq_f<T, D, BIAS_READ, LONG>(p, stream);
 }
 
 // fn<T, D>(p, stream) for the element type and head dimension of the call

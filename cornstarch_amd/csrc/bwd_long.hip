@@ -10,7 +10,7 @@ static int launch_dkdv_long_t(const AttnParams& p, hipStream_t stream) {
 }
 template <typename T, int D>
 static int launch_dq_long_t(const AttnParams& p, hipStream_t stream) {
-    return p.bias != nullptr ? launch_dq_b<T, D, true, true>(p, stream) : launch_dq_b<T, D, false, true>(p, stream);
+    return launch_dq_b<T, D, true>(p, stream);
 }
 
 int launch_bwd_dkdv_long(const AttnParams& p, int dtype, hipStream_t stream) { BAM_DISPATCH(launch_dkdv_long_t) }
