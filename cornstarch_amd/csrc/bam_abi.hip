@@ -763,7 +763,7 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
 // parts as keep the launch within one workgroup per compute unit (beyond that the parts queue behind each other).  Whole
 // training step, bf16, D 64, one part -> parts: 1 x 1024 tokens, 32 / 8 heads 139 -> 98 us; 1 x 2048, 32 / 4 heads
 // 363 -> 183; 1 x 4000, 16 / 4 heads 401 -> 286; D 128: 1 x 700, 16 / 4 heads 138 -> 105; 1 x 1024, 32 / 8 heads
-// 180 -> 117; 1 x 3000, 16 / 4 heads 456 -> 319.  The price is a launch (4 us), an allocation and their host work, so at
+// 180 -> 117; 1 x 3000, 16 / 4 heads 456 -> 319.  The price is a launch (4 to 6 us), an allocation and their host work, so at
 // least 32 steps over a pair of slices have to go: 4 x 400 tokens, 6 / 1 heads, D 40 (35 steps) 94 -> 58 to 98 us with the
 // speed of the host; 512 tokens, 16 / 4 heads (24 steps) 83 -> 95, 2 x 283, 6 / 2 heads (10 steps) 86 -> 91.
 static int dkdv_parts(const bam_attn* a) {

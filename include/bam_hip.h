@@ -451,8 +451,9 @@ int bam_decode_counted(const void* q, const void* k, const void* v, void* o, int
 /*
  * Struct form of the attention calls: what bam_fwd*, bam_bwd_preprocess and bam_bwd_dkdv* / bam_bwd_dq* take, in one
  * host struct, for hosts that fill it once per call instead of passing 40 arguments.  bam_attn_fwd is the forward of any
- * mask mode; bam_attn_bwd runs the whole backward (delta into `delta`, then dK/dV and dQ), where head_runs > 1 takes the
- * heads in that many runs of whole kv heads through one dS workspace of a run's size.  Unused fields are zero.
+ * mask mode; bam_attn_bwd runs the whole backward (delta into `delta`, dK/dV and dQ, in the order the head dim asks for), where
+ * head_runs > 1 takes the heads in that many runs of whole kv heads, through one dS workspace of a run's size if there is one.
+ * Unused fields are zero.
  */
 #define BAM_MASK_BITFIELD 0 /* bf */
 #define BAM_MASK_INDEXED 1  /* index */

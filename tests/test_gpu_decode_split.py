@@ -16,9 +16,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,Sk,D", [
-    (10, 8, 8, 2100, 128),   # 80 units: pieces along the line of all tiles
+    (10, 8, 8, 2100, 128),   # 80 units: 3 workgroups of four waves each
     (7, 6, 3, 517, 64), (3, 4, 1, 4001, 32), (1, 8, 2, 129, 96), (33, 16, 8, 97, 128), (2, 70, 2, 1025, 128),
-    (300, 2, 1, 700, 128),   # more units than workgroups: a workgroup walks several
+    (300, 2, 1, 700, 128),   # more units than compute units: two workgroups of one wave each
     (2, 8, 2, 333, 8), (2, 8, 2, 1333, 40), (1, 6, 2, 2003, 80), (1, 4, 4, 65, 120),
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
