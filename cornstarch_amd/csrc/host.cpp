@@ -450,7 +450,7 @@ struct AttentionBackward : public torch::autograd::Node {
             return compute(std::move(grads));
         } catch (const BamFailure& e) {
             py::gil_scoped_acquire gil;
-            PyErr_SetString(g_error_type, e.what());
+            PyErr_SetString(g_error_type != nullptr ? g_error_type : PyExc_RuntimeError, e.what());
             raise_python_error();
         } catch (py::error_already_set& e) {
             py::gil_scoped_acquire gil;
@@ -488,7 +488,7 @@ private:
         };
         auto expect_rows = [&](Tensor& t, at::IntArrayRef sizes, const char* what) {
             expect(t, type, sizes, what);
-            if (!rows_ready(t, 8)) t = t.contiguous();
+            if (!rows_ready(t, 8)) t = t.clone(at::MemoryFormat::Contiguous);  // (also where only the address is not aligned)
         };
         expect_rows(q_, dout.sizes(), "q");
         expect_rows(k_, {B, Sk, Hkv, D}, "k");
@@ -503,7 +503,8 @@ private:
             if (mask_.stride(1) != 1) mask_ = mask_.contiguous();
         } else {
             expect(mask_, at::kBool, {B, Sq, Sk}, "mask");
-            mask_ = mask_.contiguous();
+            if (!mask_.is_contiguous() || (reinterpret_cast<uintptr_t>(mask_.data_ptr()) & 3) != 0)
+                mask_ = mask_.clone(at::MemoryFormat::Contiguous);
         }
         Tensor dq = at::empty_like(q_), dk = at::empty_like(k_), dv = at::empty_like(v_);
         Call c;

@@ -46,6 +46,12 @@ def wide(t):
     return torch.stack((t, t), -1).flatten(-2)[..., ::2]
 
 
+def shifted(t):
+    """The same values at an address that is a multiple of the element size and of nothing more."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    return flat[1:].view(t.shape).copy_(t)
+
+
 def hooks(change):
     return torch.autograd.graph.saved_tensors_hooks(lambda t: t, change)
 
@@ -58,14 +64,14 @@ def test_saved_tensor_hooks_that_move_or_lay_out_the_tensors(D, bias):
     with torch.autograd.graph.save_on_cpu():
         o = p.forward()
     assert same(p.grads(o), want)
-    for change in (torch.clone, wide):
+    for change in (torch.clone, wide, shifted):
         with hooks(change):
             o = p.forward()
         assert same(p.grads(o), want), change
     mask = BA.materialize_bitfield_mask(p.bf)
     if not bias:
         want = torch.autograd.grad(A.flash_attn_func(*p.inputs, mask=mask), p.inputs, p.do)
-        for change in (torch.clone, wide):
+        for change in (torch.clone, wide, shifted):
             with hooks(change):
                 o = A.flash_attn_func(*p.inputs, mask=mask)
             assert same(torch.autograd.grad(o, p.inputs, p.do), want), change
@@ -266,3 +272,6 @@ def test_transforms_without_a_rule_are_refused():
     with fwAD.dual_level():
         with pytest.raises((RuntimeError, NotImplementedError)):
             p.forward(fwAD.make_dual(q, torch.ones_like(q)), k, v)
+    o = p.forward()
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(o, p.inputs, torch.stack((p.do, p.do)), is_grads_batched=True)
