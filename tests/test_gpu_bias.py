@@ -193,3 +193,28 @@ def test_bias_argument_checks():
     out = BA.bitfield_attn_func(q, k, v, bf, bt)
     assert (out.float() - BA.bitfield_attn_func(q, k, v, bf).float()).abs().max().item() <= 4e-3
     BA.BitfieldUtils.clear_cache()
+
+
+@pytest.mark.parametrize("S", [131072 + 4096 + 56, 131072 + 4096 + 57], ids=["aligned", "unaligned"])
+def test_a_bias_over_several_passes_equals_one_more_column_of_q_and_k(S):
+    # a bias per key is what a column of ones in q and bias / scale in k adds; the values are exact in bf16.  Both sides
+    # differ in the rounding of fp32 scores only, which now and then turns a probability's rounding to bf16 (2^-9) around.
+    D, scale, d = 24, 0.125, dev()
+    g = torch.Generator(device=d).manual_seed(S)
+    q, k, v, do = ((torch.randn(1, S, H, D, generator=g, device=d) * 0.5).bfloat16() for H in (2, 1, 1, 2))
+    bias = torch.randint(-32, 32, (1, 1, 1, S), generator=g, device=d) / 16.0
+    bf = torch.full((1, S), (1 << 62) | 1 | 2, dtype=torch.int64, device=d)
+    bf[0, 1000:5000] = 2
+    bf[0, S - 3000 :] = 4
+    got_in = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    o = BA.bitfield_attn_func(*got_in, bf, bias, scale)
+    got = torch.autograd.grad(o, got_in, do)
+    pad = torch.nn.functional.pad
+    q2, k2, v2, do2 = (pad(t, (0, 8)) for t in (q, k, v, do))
+    q2[..., D], k2[..., D] = 1.0, (bias / scale).reshape(1, S, 1)
+    want_in = [t.requires_grad_(True) for t in (q2, k2, v2)]
+    o2 = BA.bitfield_attn_func(*want_in, bf, None, scale)
+    want = torch.autograd.grad(o2, want_in, do2)
+    for a, b in zip((o, *got), (o2, *want)):
+        assert torch.isfinite(a).all() and rel_l2(a.float(), b[..., :D].float()) <= 2e-3
+    BA.BitfieldUtils.clear_cache()
