@@ -74,6 +74,17 @@ def test_an_infinity_in_a_key_gives_its_scores_and_nothing_else(dtype, D):
         out, _ = interface.bitfield_attention_forward(torch.nn.Module().eval(), qd[:, -1:].transpose(1, 2), kd.transpose(1, 2),
                                                       vd.transpose(1, 2), None)
         assert (out[:, 0].float().cpu() - want[:, -1]).abs().max().item() <= 2e-2
+        # gradients: dS of those keys is 0, so only the column of dq that multiplies it by the infinity is not a number.  (Whole
+        # tiles of rows only: the zero rows past the end of a ragged one make NaN of a key's infinity in dk and dv.)
+        if S % 64:
+            continue
+        do = torch.randn(1, S, 4, D, generator=g).to(dtype)
+        inputs = [t.clone().requires_grad_(True) for t in (qd, kd, vd)]
+        dq, dk, dv = torch.autograd.grad(BA.bitfield_attn_func(*inputs, bfd), inputs, do.to(d))
+        rest = [c for c in range(D) if c != col]
+        wq, wk, wv = O.attention_backward(q, k, v, bf, do)
+        for a, b in ((dq[..., rest], wq[..., rest]), (dk, wk), (dv, wv)):
+            assert torch.isfinite(b).all() and torch.isfinite(a).all() and rel_l2(a.float().cpu(), b) <= 5e-2
     BA.BitfieldUtils.clear_cache()
 
 
