@@ -153,7 +153,7 @@ struct PlanCore {
 // A Python object held by native state that may be destroyed on any thread.
 std::shared_ptr<PyObject> hold(const py::object& o) {
     return std::shared_ptr<PyObject>(py::object(o).release().ptr(), [](PyObject* p) {
-        if (!Py_IsInitialized()) return;
+        if (!Py_IsInitialized() || _Py_IsFinalizing()) return;  // (a thread that asks for the lock then is ended where it stands)
         py::gil_scoped_acquire gil;
         Py_DECREF(p);
     });
