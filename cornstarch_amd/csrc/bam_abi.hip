@@ -161,7 +161,7 @@ int fill_plan(bam::AttnParams& p, const char* who, const bam_plan* plan, int B, 
     p.group_order = plan->group_order;   // may be null
     // hand-over of dS from dK/dV to dQ: only with a workspace, for the head dim and lengths its kernels cover
     if (plan->ds_workspace != nullptr && plan->ds_entry != nullptr && plan->ds_tile_base != nullptr && p.D > 64 &&
-        Sk <= bam::MAX_LIST * 64) {
+        Sk <= bam::MAX_LIST * 64 && !bam::dkdv_far(p)) {
         if (reinterpret_cast<uintptr_t>(plan->ds_workspace) & 15u)
             return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan: dS workspace is not 16-byte aligned", who);
         if (plan->ds_capacity <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan: dS workspace without a capacity", who);
@@ -768,6 +768,9 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
 // speed of the host; 512 tokens, 16 / 4 heads (24 steps) 83 -> 95, 2 x 283, 6 / 2 heads (10 steps) 86 -> 91.
 static int dkdv_parts(const bam_attn* a) {
     if (a->head_runs > 1 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32) return 1;
+    if (bam::far_rows(a->q.stride_s, a->Sq, a->D) || bam::far_rows(a->dout.stride_s, a->Sq, a->D) ||
+        bam::far_rows(a->k.stride_s, a->Sk, a->D) || bam::far_rows(a->v.stride_s, a->Sk, a->D))
+        return 1;  // (the instantiation for such rows has no parts)
     const int G = a->Hq / a->Hkv, pairs = (a->Sq + 63) / 64;
     const int64_t units = (int64_t)a->B * a->Hkv * ((a->Sk + 127) / 128);
     for (int parts = G; parts > 1; --parts)

@@ -93,6 +93,14 @@ struct AttnParams {
     float scale;
 };
 
+// The rows of one head span 2^31 bytes or more: beyond the 32-bit tile offsets of the kernels for sequences of ordinary length;
+// the instantiations that walk sequences in passes take such calls.
+inline bool far_rows(int64_t stride_s, int rows, int d) { return ((int64_t)(rows - 1) * stride_s + d) * 2 >= (1ll << 31); }
+inline bool far_rows(const Tensor4& t, int rows, int d) { return far_rows(t.ss, rows, d); }
+inline bool dkdv_far(const AttnParams& p) {
+    return far_rows(p.q, p.Sq, p.d) || far_rows(p.dout, p.Sq, p.d) || far_rows(p.k, p.Sk, p.d) || far_rows(p.v, p.Sk, p.d);
+}
+
 // Single-token decode step (one query row per batch element and head, no mask); strides in elements.
 struct DecodeParams {
     const void *q, *k, *v;         // q (B, Hq, D): q_sb, q_sh; k / v (B, Sk, Hkv, D): *_sb, *_ss, *_sh

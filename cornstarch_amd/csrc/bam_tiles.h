@@ -58,6 +58,70 @@ __device__ __forceinline__ void dma_b32(const void* sbase, unsigned voff, unsign
                  : "memory");
 }
 
+// Consecutive rows of one head of one sequence (or of any array) that tiles are copied from: a buffer descriptor over exactly
+// these rows, and where a tile starts in it.  Whatever a copy addresses past the last row becomes zeros in LDS (the hardware's
+// range check covers the scalar offset too), so the tile that holds the end of a sequence is copied like any other.  The
+// descriptor stays in scalar registers over the key loop and a tile costs one 32-bit product: with a 64-bit base per tile and
+// the end of the sequence staged by a second instance of the loop body, dK/dV at D = 128 needed 88 bytes of scratch per lane.
+// (Where rows overlap in memory -- a stride below the row's own bytes, 0 for a broadcast -- rows past the end may repeat bytes of
+// the rows before them instead.)
+// FAR: views of 2^31 bytes and more; the descriptor is built per tile around a 64-bit base.
+constexpr unsigned BUFFER_WORD3 = 0x00020000u;
+struct TileSrc {
+    u32x4 desc;
+    unsigned off;  // bytes, wave-uniform
+};
+template <bool FAR>
+struct RowView {
+    u32x4 desc;
+    unsigned stride;  // bytes from row to row, below 2^24 by the host checks
+    int rows;
+    unsigned row_bytes;
+
+    __device__ __forceinline__ static u32x4 describe(const void* ptr, unsigned range) {
+        const unsigned long long base = reinterpret_cast<unsigned long long>(ptr);  // (48 bits: no stride in the second word)
+        return u32x4{(unsigned)base, (unsigned)(base >> 32), range, BUFFER_WORD3};
+    }
+    __device__ __forceinline__ void init(const void* ptr, int64_t stride_bytes, int n_rows, int bytes_per_row) {
+        stride = (unsigned)stride_bytes;
+        rows = n_rows;
+        row_bytes = (unsigned)bytes_per_row;
+        desc = describe(ptr, (unsigned)(n_rows - 1) * stride + row_bytes);
+    }
+    // moves the view to another head of the same tensor
+    __device__ __forceinline__ void move(int64_t bytes) {
+        const unsigned long long base = (((unsigned long long)desc[1] << 32) | desc[0]) + (unsigned long long)bytes;
+        desc[0] = (unsigned)base;
+        desc[1] = (unsigned)(base >> 32);
+    }
+    __device__ __forceinline__ TileSrc at(int row) const {
+        if (!FAR) return TileSrc{desc, (unsigned)row * stride};
+        const unsigned long long base = (((unsigned long long)desc[1] << 32) | desc[0]) + (uint64_t)(unsigned)row * stride;
+        const int left = rows - row;  // (a tile has up to 128 rows)
+        return TileSrc{u32x4{(unsigned)base, (unsigned)(base >> 32), left >= 128 ? DMA_RANGE : (unsigned)(left - 1) * stride + row_bytes, BUFFER_WORD3}, 0u};
+    }
+};
+// Lane l fetches 16 (4) bytes at src + voff and the hardware writes them to LDS byte address lds_base + 16 l (4 l).
+// WAIT: wait states in front of the copy, less one.  A scalar register that a vector instruction has written (the reload of a
+// spilled one) must not be read by a memory instruction within five wait states, and the compiler does not look into an asm
+// statement.  Instantiations whose scalar registers spill in the loop pass 4 (COPY_WAIT); the others need the one state after
+// the write of M0: waiting five everywhere costs 1 to 2.5 % of every kernel (forward + backward of 1 x 8192 tokens, 32 / 8
+// heads, D 128: 1769 -> 1791 us).  tests/test_copy_hazard.py looks at every copy of the built library.
+template <int WAIT>
+__device__ __forceinline__ void copy_b128(const TileSrc& src, unsigned voff, unsigned lds_base) {
+    asm volatile("s_nop %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(src.desc), "s"(src.off),
+                 "{m0}"(lds_base), "n"(WAIT)
+                 : "memory");
+}
+template <int WAIT>
+__device__ __forceinline__ void copy_b32(const TileSrc& src, unsigned voff, unsigned lds_base) {
+    asm volatile("s_nop %4\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(src.desc), "s"(src.off),
+                 "{m0}"(lds_base), "n"(WAIT)
+                 : "memory");
+}
+template <int MODE, bool BIAS, bool LONG>
+constexpr int COPY_WAIT = LONG || (BIAS && MODE == MASK_INDEXED) ? 4 : 0;
+
 // All direct global-to-LDS copies this wave has issued have landed (pair with a barrier).
 __device__ __forceinline__ void wait_async() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
@@ -73,9 +137,7 @@ __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)"
 // XOR swizzle is applied on the SOURCE side -- lane `id` fetches the chunk that belongs in
 // slot `id`.  `setup` fixes those source offsets once per kernel; `issue(i, ...)` emits copy
 // instruction i of CPT so that callers can spread a tile's copies between other work.
-// The last, ragged tile of a sequence takes the synchronous path (`load_ragged`), which
-// zero-fills the rows past the end.  Row strides are limited to 2^23 elements by the host
-// checks, so the offsets fit 32 bits.
+// Row strides are limited to 2^23 elements by the host checks, so the offsets fit 32 bits.
 // ZERO_PAD: chunks past the head dim become zero in LDS (whoever multiplies along the head dim has zeros in the other operand
 // there, but zero times an infinity of chunk 0 would be a NaN in the score of a key whose weight is 0); otherwise their lanes
 // fetch chunk 0 again.
@@ -112,26 +174,18 @@ struct TileStage {
         else
             dma_b128<SITE>(base, voff, lds_base);
     }
+    template <int WAIT>
+    __device__ __forceinline__ void issue(int i, const TileSrc& src, unsigned tile_lds) const {
+        if (EXACT || wave_first + THREADS * i < CHUNKS) copy_b128<WAIT>(src, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
+    }
     __device__ __forceinline__ void load_full(const char* tile_base, unsigned tile_lds) const {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) issue(i, tile_base, tile_lds);
     }
-    // synchronous, zero-filling copy of a tile with only rows_valid (< ROWS) rows in range
-    __device__ __forceinline__ void load_ragged(const char* tile_base, u32x4* tile, int rows_valid, int tid) const {
+    template <int WAIT>
+    __device__ __forceinline__ void load(const TileSrc& src, unsigned tile_lds) const {
 #pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int id = tid + THREADS * i;
-            u32x4 z = {0u, 0u, 0u, 0u};
-            if ((EXACT || id < CHUNKS) && id / NCH < rows_valid && !(ZERO_PAD && goff[i] == DMA_ZERO)) z = *(const u32x4*)(tile_base + goff[i]);
-            if (EXACT || id < CHUNKS) tile[id] = z;
-        }
-    }
-    // tile_base / rows_valid wave-uniform
-    __device__ __forceinline__ void load(const char* tile_base, u32x4* tile, int rows_valid, int tid) const {
-        if (rows_valid >= ROWS)
-            load_full(tile_base, lds_addr(tile));
-        else
-            load_ragged(tile_base, tile, rows_valid, tid);
+        for (int i = 0; i < CPT; ++i) issue<WAIT>(i, src, tile_lds);
     }
 };
 
@@ -159,14 +213,6 @@ struct SliceStage {
             goff[i] = (unsigned)((row & 31) * row_stride_bytes + (c < chunks ? c : 0) * 16);
         }
     }
-    // lo / hi: first row of the two slices in global memory, tile_lds: lds_addr() of the LDS tile (wave-uniform)
-    template <int SITE = 0>
-    __device__ __forceinline__ void issue(int i, const char* lo, const char* hi, unsigned tile_lds) const {
-        if (EXACT || wave_first + THREADS * i < CHUNKS) {
-            const bool upper = (wave_first + THREADS * i) / NCH >= 32;
-            dma_b128<SITE>(upper ? hi : lo, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
-        }
-    }
     // Does copy instruction i of this wave fill LDS rows 32..63 (slice `hi`)?  Wave-uniform, and a compile-time
     // constant where every instruction covers whole 32-row halves (D = 128 with 512 threads).
     __device__ __forceinline__ bool upper(int i) const {
@@ -174,32 +220,13 @@ struct SliceStage {
         if ((THREADS * i) / NCH >= 32) return true;
         return (wave_first + THREADS * i) / NCH >= 32;
     }
-    // As issue(), with the slice's base pointer already chosen by the caller (see upper()).
-    template <int SITE = 0>
-    __device__ __forceinline__ void issue_from(int i, const char* slice_base, unsigned tile_lds) const {
+    // Copy instruction i from the first row of the slice it belongs to (see upper()).
+    template <int WAIT>
+    __device__ __forceinline__ void issue_from(int i, const TileSrc& slice, unsigned tile_lds) const {
         if (EXACT || wave_first + THREADS * i < CHUNKS)
-            dma_b128<SITE>(slice_base, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
-    }
-    // synchronous, zero-filling copy of ONE slice with only rows_valid (<= 32) rows in range into LDS rows
-    // [0, 32); rows [32, 64) are zeroed
-    __device__ __forceinline__ void load_ragged(const char* slice_base, u32x4* tile, int rows_valid, int tid) const {
-#pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int id = tid + THREADS * i;
-            u32x4 z = {0u, 0u, 0u, 0u};
-            if ((EXACT || id < CHUNKS) && id / NCH < rows_valid) z = *(const u32x4*)(slice_base + goff[i]);
-            if (EXACT || id < CHUNKS) tile[id] = z;
-        }
+            copy_b128<WAIT>(slice, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
     }
 };
-
-// One wave copies `DWORDS` consecutive dwords (a multiple of 64) global -> LDS asynchronously.
-template <int DWORDS>
-__device__ __forceinline__ void copy_dwords_async(const void* src, void* dst_lds, int lane) {
-    const unsigned dst = lds_addr(dst_lds);
-#pragma unroll
-    for (int i = 0; i < DWORDS / 64; ++i) dma_b32(src, (unsigned)(lane * 4 + 256 * i), dst + 256u * i);
-}
 
 // The 32-row slice each of the four waves of a forward / dQ workgroup works on, and the row of tile classes
 // (one byte per 32-key column tile: 0 empty, 1 partial, 2 full) that says which keys that slice needs.
@@ -285,8 +312,9 @@ __device__ __forceinline__ void build_slice_list(const AttnParams& p, int b, int
                                   : p.flags + (int64_t)b * p.flags_sb + (int64_t)(s >> 2) * p.flags_sm + 4 * nt;
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                const int fw = (4 * nt + w < p.num_n) ? f[w] : 0;
-                packed |= (fw & 3) << (2 * w);
+                int fw = (4 * nt + w < p.num_n) ? f[w] & 3 : 0;
+                if ((s + 1) * 32 > p.Sq) fw = min(fw, 1);  // rows past the end have to be masked out
+                packed |= fw << (2 * w);
             }
         }
         const unsigned long long bal = __ballot(packed != 0);

@@ -51,7 +51,7 @@ static int launch_dkdv_t(const AttnParams& p, hipStream_t stream) {
 
 int launch_bwd_preprocess(const AttnParams& p, int dtype, hipStream_t stream) { BAM_DISPATCH(launch_pre_t) }
 int launch_bwd_dkdv(const AttnParams& p, int dtype, hipStream_t stream) {
-    if (p.Sq > MAX_SLICE_LIST * 32) return launch_bwd_dkdv_long(p, dtype, stream);
+    if (p.Sq > MAX_SLICE_LIST * 32 || dkdv_far(p)) return launch_bwd_dkdv_long(p, dtype, stream);
     BAM_DISPATCH(launch_dkdv_t)
 }
 

@@ -11,7 +11,7 @@ static int launch_dq_t(const AttnParams& p, hipStream_t stream) {
 }
 
 int launch_bwd_dq(const AttnParams& p, int dtype, hipStream_t stream) {
-    if (p.Sk > MAX_LIST * DQ_KT) return launch_bwd_dq_long(p, dtype, stream);
+    if (p.Sk > MAX_LIST * DQ_KT || far_rows(p.k, p.Sk, p.d) || far_rows(p.v, p.Sk, p.d)) return launch_bwd_dq_long(p, dtype, stream);
     BAM_DISPATCH(launch_dq_t)
 }
 

@@ -107,8 +107,8 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
 #pragma unroll
         for (int i = 0; i < 16; ++i) dq[db][i] = 0.f;
 
-    const char* kbase = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh);
-    const int64_t k_ts = 2 * p.k.ss * DQS_KT;  // bytes per tile
+    RowView<false> k_rows;
+    k_rows.init((const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh), 2 * p.k.ss, Sk, 2 * p.d);
     typedef TileStage<D, DQS_KT, DQS_THREADS> Stage;
     constexpr int CPT = Stage::CPT;
     Stage stK;
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
     // copy of the K tile of list entry `entry` into buffer buf (shared by the four waves)
     auto issue_k = [&](int entry, int buf) {
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) stK.issue(j, kbase + (entry >> 16) * k_ts, ldsK + buf * TILE_BYTES);
+        for (int j = 0; j < CPT; ++j) stK.template issue<0>(j, k_rows.at((entry >> 16) * DQS_KT), ldsK + buf * TILE_BYTES);
     };
     // copies of this wave's dS blocks of tile `entry` (record e), the halves that have work, into its buffer buf;
     // returns the number of copy instructions issued (wave-uniform)
@@ -191,14 +191,9 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
     };
 
     __syncthreads();
-    const int n_all = sCount;
-    // A tile that holds the end of a sequence whose length is not a multiple of 64 is always the last entry of the
-    // list; its K rows are staged synchronously (zero fill past the end) after the main loop.
-    const bool ragged = (Sk & (DQS_KT - 1)) != 0 && n_all > 0 &&
-                        (__builtin_amdgcn_readfirstlane(sList[n_all > 0 ? n_all - 1 : 0]) >> 16) == ((Sk - 1) >> 6);
-    const int n = n_all - (ragged ? 1 : 0);
+    const int n = sCount;
     if (n > 0) {
-        load_entries(0, n_all);
+        load_entries(0, n);
         int entry = __builtin_amdgcn_readfirstlane(sList[0]);
         int next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
         issue_k(entry, 0);
@@ -214,7 +209,7 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
             const int i2 = it + 2;
             int entry2 = -1, e2 = 0;
             if (i2 < n) {
-                if ((i2 & 63) == 0) load_entries(i2, n_all);
+                if ((i2 & 63) == 0) load_entries(i2, n);
                 entry2 = __builtin_amdgcn_readfirstlane(sList[i2]);
                 e2 = __builtin_amdgcn_readlane(ent_vec, i2 & 63);
             }
@@ -231,27 +226,6 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
             __syncthreads();
         }
     }
-    if (ragged) {
-        const int entry = __builtin_amdgcn_readfirstlane(sList[n_all - 1]);
-        const int kt = entry >> 16, rows = Sk - kt * DQS_KT;
-        __syncthreads();
-        stK.load_ragged(kbase + kt * k_ts, sK[0], rows, tid);
-        const int c = (entry >> (4 * wave)) & 15;
-        if (c != 0) {
-            const int e = entry_row[kt >> 1];
-            const char* rec = ds_head + ((int64_t)e << 13) + (kt & 1) * 4096;
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-                if ((c >> (2 * kb)) & 3) {
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        sDS[wave][0][kb * 128 + j * 64 + lane] = *(const u32x4*)(rec + kb * 2048 + j * 1024 + lane * 16);
-                }
-        }
-        __syncthreads();
-        tile_step(0, entry, -1, 0);
-    }
-
     // ---- epilogue: dq holds -dQ / scale (C fragment: lane = query column, registers = head dims 8 g + 4 hi + x)
     const float factor = -p.scale;
     if (qvalid && p.grad_typed) {

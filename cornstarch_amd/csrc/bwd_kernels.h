@@ -88,6 +88,7 @@ template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
+    constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
     __shared__ u32x4 sK[128 * NCH];
     __shared__ u32x4 sV[128 * NCH];
     __shared__ u32x4 sQ[2][DKDV_QT * NCH];
@@ -141,10 +142,11 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         TileStage<D, 128, DKDV_THREADS> stK, stV;
         stK.setup(2 * p.k.ss, p.d / 8, tid);
         stV.setup(2 * p.v.ss, p.d / 8, tid);
-        const char* kb = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)kv_head * p.k.sh + (int64_t)nt * 128 * p.k.ss);
-        const char* vb = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)kv_head * p.v.sh + (int64_t)nt * 128 * p.v.ss);
-        stK.load(kb, sK, Sk - nt * 128, tid);
-        stV.load(vb, sV, Sk - nt * 128, tid);
+        RowView<LONG> rows;
+        rows.init((const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)kv_head * p.k.sh), 2 * p.k.ss, Sk, 2 * p.d);
+        stK.template load<WAIT>(rows.at(nt * 128), lds_addr(sK));
+        rows.init((const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)kv_head * p.v.sh), 2 * p.v.ss, Sk, 2 * p.d);
+        stV.template load<WAIT>(rows.at(nt * 128), lds_addr(sV));
     }
     const int key = nt * 128 + kg * 32 + l32;
     const bool kvalid = key < Sk;
@@ -227,76 +229,75 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                                            : lds_addr(sQbf) + (small - 2) * 256u;
     const unsigned smallBytes = small < 2 ? DKDV_QT * 4u : DENSE ? 2 * 128 * 4u : DKDV_QT * 8u;  // per buffer
     // Where the copies of a tile read.  The scalar unit is shared by the whole compute unit, so the address
-    // arithmetic is kept short: per-head base pointers are carried along and bumped when the head changes, row
-    // offsets are 32 x 32 -> 64 bit unsigned products (rows < 2^22, row strides < 2^25 bytes by the host checks).
-    struct HeadBase {
-        const char* q;      // first row of the head in q
-        const char* g;      // ... in dout
-        const char* small;  // this wave's small row: lse / delta of the head, or the bitfields (head independent)
+    // arithmetic is kept short: descriptors of the head in work are carried along and moved when the head changes, a slice
+    // costs one 32-bit product.  The slice that holds the end of the sequence is copied like the others: its rows past the
+    // end are zeros, with an empty bitfield, and the list never calls such a slice "full".
+    struct HeadViews {
+        RowView<LONG> q, g;    // rows of the head in q and dout
+        RowView<false> small;  // this wave's small row: lse / delta of the head, or the bitfields (head independent)
     };
-    const unsigned q_rs = (unsigned)(2 * p.q.ss), g_rs = (unsigned)(2 * p.dout.ss);  // row strides in bytes
     const int64_t small_head_step = small < 2 ? (int64_t)p.Sq_rounded * 4 : 0;
-    auto head_base = [&](int h) {
-        HeadBase hb;
-        hb.q = (const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)h * p.q.sh);
-        hb.g = (const char*)p.dout.ptr + 2 * ((int64_t)b * p.dout.sb + (int64_t)h * p.dout.sh);
-        hb.small = small == 0   ? (const char*)(p.lse + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded)
-                   : small == 1 ? (const char*)(p.delta + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded)
-                   : DENSE      ? (const char*)(p.col_bits + (int64_t)b * p.col_bits_sb + nt * 128 + (small - 2) * 64)
-                                : (const char*)bfrow;
-        return hb;
+    auto head_views = [&](int h) {
+        HeadViews hv;
+        hv.q.init((const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)h * p.q.sh), 2 * p.q.ss, Sq, 2 * p.d);
+        hv.g.init((const char*)p.dout.ptr + 2 * ((int64_t)b * p.dout.sb + (int64_t)h * p.dout.sh), 2 * p.dout.ss, Sq, 2 * p.d);
+        if (small < 2)
+            hv.small.init((small == 0 ? p.lse : p.delta) + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded, 4, Sq, 4);
+        else if (DENSE)  // (one row per slice)
+            hv.small.init(p.col_bits + (int64_t)b * p.col_bits_sb + nt * 128 + (small - 2) * 64, p.col_bits_ss * 4, (Sq + 31) >> 5, 256);
+        else
+            hv.small.init(bfrow, 8, Sq, 8);
+        return hv;
     };
-    auto next_head = [&](HeadBase& hb) {
-        hb.q += 2 * (int64_t)p.q.sh;
-        hb.g += 2 * (int64_t)p.dout.sh;
-        hb.small += small_head_step;
+    auto next_head = [&](HeadViews& hv) {
+        hv.q.move(2 * (int64_t)p.q.sh);
+        hv.g.move(2 * (int64_t)p.dout.sh);
+        hv.small.move(small_head_step);
     };
+    RowView<false> pos_rows;
+    if (IDX) pos_rows.init(p.posq, 4, Sq, 4);
     // lanes 32..63 of a copy of 2 x 32 consecutive floats / ints take the second slice: their byte offset moves
     // from "the rows after the first slice" to it
     const unsigned upper_lanes = lane >= 32 ? 0xFFFFFFFFu : 0u;
     struct TileSource {
-        const char* q[CPT];
-        const char* g[CPT];
-        const char* small;
-        const int* pos;
+        TileSrc q[CPT], g[CPT], small, pos;
         unsigned small_voff, pos_voff;
     };
     // the 64-row tile made of the slices starting at rows row_lo (LDS rows 0..31) and row_hi (LDS rows 32..63)
-    auto tile_source = [&](const HeadBase& hb, int row_lo, int row_hi) {
+    auto tile_source = [&](const HeadViews& hv, int row_lo, int row_hi) {
         TileSource t;
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
-            const unsigned row = (unsigned)(stQ.upper(i) ? row_hi : row_lo);
-            t.q[i] = hb.q + (uint64_t)row * q_rs;
-            t.g[i] = hb.g + (uint64_t)row * g_rs;
+            const int row = stQ.upper(i) ? row_hi : row_lo;
+            t.q[i] = hv.q.at(row);
+            t.g[i] = hv.g.at(row);
         }
         // lse / delta (small < 2): 32 floats of each slice.  Bitfields: 32 int64 = 64 dwords of slice lo
-        // (small == 2) or hi (small == 3).
-        const unsigned srow = (unsigned)(small == 3 ? row_hi : row_lo);
-        if (DENSE && small >= 2)  // the words of the slice this wave's row stream works on
-            t.small = hb.small + (uint64_t)((unsigned)(st ? row_hi : row_lo) >> 5) * (uint64_t)(p.col_bits_ss * 4);
+        // (small == 2) or hi (small == 3).  DENSE: the words of the slice this wave's row stream works on
+        if (DENSE && small >= 2)
+            t.small = hv.small.at((st ? row_hi : row_lo) >> 5);
         else
-            t.small = hb.small + (small < 2 ? srow * 4u : srow * 8u);
+            t.small = hv.small.at(small == 3 ? row_hi : row_lo);
         const unsigned shift = (unsigned)((row_hi - row_lo - 32) * 4);
         t.pos_voff = (unsigned)(lane * 4) + (shift & upper_lanes);
         t.small_voff = small < 2 ? t.pos_voff : (unsigned)(lane * 4);
-        t.pos = IDX ? p.posq + row_lo : nullptr;
+        if (IDX) t.pos = pos_rows.at(row_lo);
         return t;
     };
     // copy instruction j of a tile into buffer buf
     auto issue_copy = [&](int j, const TileSource& t, int buf) {
         if (j < CPT)
-            stQ.issue_from(j, t.q[j], ldsQ + buf * TILE_BYTES);
+            stQ.template issue_from<WAIT>(j, t.q[j], ldsQ + buf * TILE_BYTES);
         else if (j < 2 * CPT)
-            stDO.issue_from(j - CPT, t.g[j - CPT], ldsDO + buf * TILE_BYTES);
+            stDO.template issue_from<WAIT>(j - CPT, t.g[j - CPT], ldsDO + buf * TILE_BYTES);
         else if (j == 2 * CPT)
-            dma_b32(t.small, t.small_voff, ldsSmall + buf * smallBytes);
+            copy_b32<WAIT>(t.small, t.small_voff, ldsSmall + buf * smallBytes);
         else  // 2 x 32 row positions; every wave writes the same values
-            dma_b32(t.pos, t.pos_voff, lds_addr(sQpos) + buf * (DKDV_QT * 4u));
+            copy_b32<WAIT>(t.pos, t.pos_voff, lds_addr(sQpos) + buf * (DKDV_QT * 4u));
     };
 
     // One 64-row tile held in buffer cur against this wave's 32 keys; the wave's 32 rows sit at sequence
-    // rows myrow0.. and its class for them is cls.  With PREFETCH the copies of the next tile into the other buffer
+    // rows myrow0.. and its class for them is cls.  The copies of the next tile into the other buffer
     // are issued one per MFMA of the S / dP phase, or back to back when this wave has nothing to compute.
     const int qr = 32 * st;  // this wave's rows inside the 64-row tile
     // The wave's flag class is extracted with a per-lane copy of the key group number on purpose: a branch
@@ -321,13 +322,10 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     };
     // ds_pos: position of the wave's slice in the slice list.
     // returns true when the wave has issued its two dS stores (they may stay in flight over the end of the iteration)
-    auto tile_step = [&](auto prefetch, int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next) -> bool {
-        constexpr bool PREFETCH = decltype(prefetch)::value;
+    auto tile_step = [&](int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next) -> bool {
         if (cls == 0) {
-            if (PREFETCH) {
 #pragma unroll
-                for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, cur ^ 1);
-            }
+            for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, cur ^ 1);
             return false;
         }
         const int ds_e = ds_base + ds_pos;
@@ -368,7 +366,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                     dp = T::mfma(a[j], bb[j], dp);
                 else
                     s = T::mfma(a[j], bb[j], j < 2 ? zero16 : s);
-                if (PREFETCH && j < NLOADS) issue_copy(j, next, cur ^ 1);
+                if (j < NLOADS) issue_copy(j, next, cur ^ 1);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -515,12 +513,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     // of its own; dK and dV live in registers and simply carry over.
     for (int s_end = ns_total;;) {
         __syncthreads();
-        const int n_all = sCount;
-        // The last slice of a sequence whose length is not a multiple of 32 (always the last list entry) is
-        // staged synchronously, with neutral values for the rows past the end, after the main loop.
-        const bool ragged = (Sq & 31) != 0 && n_all > 0 &&
-                            (__builtin_amdgcn_readfirstlane(sList[n_all > 0 ? n_all - 1 : 0]) >> 8) == ((Sq - 1) >> 5);
-        const int n = n_all - (ragged ? 1 : 0);
+        const int n = sCount;
         // Main loop: the listed slices are taken in pairs from the END of the list (the workgroups of one kv head
         // that are resident together then read the same Q / dO rows at about the same time, and all but the first
         // of them find them in L2); pair r = entries n - 2 - 2 r (row stream 0) and n - 1 - 2 r (row stream 1).
@@ -531,20 +524,20 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         if (total > 0) {
             auto entry_hi = [&](int r) { return sList[n - 1 - 2 * r]; };
             auto entry_lo = [&](int r) { return sList[n - 2 - 2 * r]; };  // entry -1 where the count is odd
-            // current tile (g_cur, entries e_*), next tile (g_nxt, r_nxt, entries n_*, head base hb_nxt); past the
+            // current tile (g_cur, entries e_*), next tile (g_nxt, r_nxt, entries n_*, head views hv_nxt); past the
             // last tile "next" keeps walking through pairs of the last head, whose copies nobody reads
             int g_cur = 0, g_nxt = 0, r_nxt = 0, r_cur = 0;
-            HeadBase hb_nxt = head_base(hk * G);
+            HeadViews hv_nxt = head_views(hk * G);
             int e_lo = __builtin_amdgcn_readfirstlane(entry_lo(0)), e_hi = __builtin_amdgcn_readfirstlane(entry_hi(0));
             {
-                const TileSource first = tile_source(hb_nxt, (e_lo >> 8) * 32, (e_hi >> 8) * 32);
+                const TileSource first = tile_source(hv_nxt, (e_lo >> 8) * 32, (e_hi >> 8) * 32);
 #pragma unroll
                 for (int j = 0; j < NLOADS; ++j) issue_copy(j, first, 0);
             }
             auto advance = [&]() {
                 if (++r_nxt == npairs) {
                     r_nxt = 0;
-                    if (++g_nxt < G) next_head(hb_nxt);
+                    if (++g_nxt < G) next_head(hv_nxt);
                 }
             };
             advance();
@@ -562,10 +555,10 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 // pair after next: its list entries are requested now and picked up at the end of the iteration
                 const int r_aft = r_nxt + 1 == npairs ? 0 : r_nxt + 1;
                 const int a_lo = entry_lo(r_aft), a_hi = entry_hi(r_aft);
-                const TileSource next = tile_source(hb_nxt, (n_lo >> 8) * 32, (n_hi >> 8) * 32);
+                const TileSource next = tile_source(hv_nxt, (n_lo >> 8) * 32, (n_hi >> 8) * 32);
                 const int mine = st ? e_hi : e_lo;
                 fetch_bias_key(hk * G + g_cur);
-                const bool stored = tile_step(std::true_type{}, cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur,
+                const bool stored = tile_step(cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur,
                                               (mine >> 8) * 32, n - 2 - 2 * r_cur + st, next);
                 g_cur = g_nxt;
                 r_cur = r_nxt;
@@ -580,38 +573,6 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 else
                     wait_async();
                 __syncthreads();
-            }
-        }
-        if (ragged) {
-            wait_async();  // K, V of the tile, in case the main loop had nothing to do
-            if (!v_negated) {
-                __syncthreads();
-                negate_v_tile();
-                v_negated = true;  // (the barrier at the top of the loop below publishes it)
-            }
-            const int entry = __builtin_amdgcn_readfirstlane(sList[n_all - 1]);
-            const int row0 = (entry >> 8) * 32;
-            const int rows = Sq - row0;  // rows of the slice inside the sequence (1..31)
-            for (int g = 0; g < G; ++g) {
-                const int h = hk * G + g;
-                __syncthreads();  // everybody is done with buffer 0
-                stQ.load_ragged((const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)h * p.q.sh + (int64_t)row0 * p.q.ss), sQ[0], rows, tid);
-                stDO.load_ragged((const char*)p.dout.ptr + 2 * ((int64_t)b * p.dout.sb + (int64_t)h * p.dout.sh + (int64_t)row0 * p.dout.ss), sDO[0], rows, tid);
-                if (tid < DKDV_QT) {
-                    const int64_t off = (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + row0;
-                    const bool ok = tid < rows;
-                    sLse[0][tid] = ok ? p.lse[off + tid] : INFINITY;  // lse = +inf gives P = 0
-                    sDelta[0][tid] = ok ? p.delta[off + tid] : 0.f;
-                    if (!DENSE) sQbf[0][tid] = ok ? bfrow[row0 + tid] : 0;
-                    if (IDX) sQpos[0][tid] = ok ? p.posq[row0 + tid] : 0;
-                }
-                if (col_bits_on && tid < 128)  // the slice sits in row stream 0
-                    sColBits[0][0][tid] = p.col_bits[(int64_t)b * p.col_bits_sb + (int64_t)(row0 >> 5) * p.col_bits_ss + nt * 128 + tid];
-                __syncthreads();
-                load_kv_operands();
-                fetch_bias_key(h);
-                // the slice sits in LDS rows 0..31: row stream 0 computes it, row stream 1 has nothing to do
-                tile_step(std::false_type{}, 0, st ? 0 : (entry >> (2 * kg_lane)) & 3, h, row0, n_all - 1, TileSource{});
             }
         }
         if (!LONG) break;
@@ -739,6 +700,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
     constexpr bool BIAS = BIAS_FORM != BIAS_NONE, bias_lds = BIAS_FORM == BIAS_TILES;
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
+    constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
     __shared__ u32x4 sK[2][DQ_KT * NCH];
     __shared__ u32x4 sV[2][DQ_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf[2][DQ_KT];  // raw bitfields of the tile's keys
@@ -832,18 +794,20 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
         bias_row = (const char*)p.bias + (p.bias_f32 ? 4 : 2) * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh +
                                                                 (int64_t)(qvalid ? qrow : 0) * p.bias_sm);
 
-    const char* kbase = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh);
-    const char* vbase = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)hk * p.v.sh);
-    const int64_t k_ts = 2 * p.k.ss * DQ_KT, v_ts = 2 * p.v.ss * DQ_KT;  // bytes per tile
-    const int64_t* bfrow = p.bfk + (int64_t)b * p.bfk_sb;
+    RowView<LONG> k_rows, v_rows;
+    RowView<false> bf_rows, pos_rows, bias_rows;  // key bitfields, (IDX) positions, per-key bias
+    k_rows.init((const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh), 2 * p.k.ss, Sk, 2 * p.d);
+    v_rows.init((const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)hk * p.v.sh), 2 * p.v.ss, Sk, 2 * p.d);
+    if (!DENSE) bf_rows.init(p.bfk + (int64_t)b * p.bfk_sb, 8, Sk, 8);
+    if (IDX) pos_rows.init(p.posk, 4, Sk, 4);
 
-    typedef TileStage<D, DQ_KT, DQ_THREADS> Stage;
+    typedef TileStage<D, DQ_KT, DQ_THREADS, true> Stage;
     constexpr int CPT = Stage::CPT;
     // copy instructions per wave and tile: K, V, the key bitfields, (IDX) the key positions and (BIAS_TILES) the bias values
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0) + (bias_lds ? 1 : 0);
     static_assert(NLOADS <= 2 * KK + 1, "one copy per MFMA of the first S / dP block (and at most one behind it)");
-    TileStage<D, DQ_KT, DQ_THREADS, true> stK;
-    Stage stV;
+    Stage stK;
+    TileStage<D, DQ_KT, DQ_THREADS> stV;
     stK.setup(2 * p.k.ss, p.d / 8, tid);
     stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);
@@ -853,43 +817,43 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
                                      ? p.row_bits + (int64_t)b * p.row_bits_sb + (slice < 0 ? 0 : slice) * 32
                                      : nullptr;
     const unsigned row_bits_voff = DENSE ? (unsigned)(hi * (int)p.row_bits_sn * 4 + l32 * 4) : 0u;
-    const char* bias_head = BIAS ? (const char*)p.bias + (p.bias_f32 ? 4 : 2) * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh) : nullptr;
+    if (bias_lds) {
+        const int esz = p.bias_f32 ? 4 : 2;
+        bias_rows.init((const char*)p.bias + esz * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh), esz, Sk, esz);
+    }
     const unsigned bias_voff = (unsigned)((p.bias_f32 ? lane : (lane & 31)) * 4);
-    const int bias_tile_bytes = DQ_KT * (p.bias_f32 ? 4 : 2);
     constexpr unsigned TILE_BYTES = DQ_KT * NCH * 16, BITS_BYTES = DQ_KT * 8;
-    // copy instruction j of full tile kt into buffer buf (key bitfields: 64 dwords per wave, waves 2, 3
+    // copy instruction j of tile kt into buffer buf (key bitfields: 64 dwords per wave, waves 2, 3
     // repeat what waves 0, 1 write, so that every wave issues the same number of copies)
     auto issue_copy = [&](int j, int kt, int buf) {
+        const int row = kt * DQ_KT;
         if (j < CPT)
-            stK.issue(j, kbase + kt * k_ts, ldsK + buf * TILE_BYTES);
+            stK.template issue<WAIT>(j, k_rows.at(row), ldsK + buf * TILE_BYTES);
         else if (j < 2 * CPT)
-            stV.issue(j - CPT, vbase + kt * v_ts, ldsV + buf * TILE_BYTES);
+            stV.template issue<WAIT>(j - CPT, v_rows.at(row), ldsV + buf * TILE_BYTES);
         else if (j == 2 * CPT) {
             if (DENSE) {  // lanes 0..31: block 2 kt, lanes 32..63: block 2 kt + 1, rows of this wave's slice
                 if (row_bits_w != nullptr)
                     dma_b32(row_bits_w + (int64_t)(2 * kt) * p.row_bits_sn, row_bits_voff, ldsR + (unsigned)(buf * 4 + wave) * 256u);
             } else {
-                dma_b32(bfrow + kt * DQ_KT, (unsigned)((wave & 1) * 256 + lane * 4), ldsB + buf * BITS_BYTES + (wave & 1) * 256u);
+                copy_b32<WAIT>(bf_rows.at(row), (unsigned)((wave & 1) * 256 + lane * 4), ldsB + buf * BITS_BYTES + (wave & 1) * 256u);
             }
         }
         else if (IDX && j == 2 * CPT + 1)  // 64 positions; every wave writes the same values
-            dma_b32(p.posk + kt * DQ_KT, (unsigned)(lane * 4), ldsP + buf * (DQ_KT * 4u));
+            copy_b32<WAIT>(pos_rows.at(row), (unsigned)(lane * 4), ldsP + buf * (DQ_KT * 4u));
         else if (bias_lds)  // BIAS: the tile's 64 bias values; every wave writes the same values
-            dma_b32(bias_head + (int64_t)kt * bias_tile_bytes, bias_voff, lds_addr(sBias) + buf * 256u);
+            copy_b32<WAIT>(bias_rows.at(row), bias_voff, lds_addr(sBias) + buf * 256u);
     };
 
-    // One 64-key tile held in buffer `cur`; with PREFETCH the copies of tile kt_next into the other buffer
+    // One 64-key tile held in buffer `cur`; the copies of tile kt_next into the other buffer
     // are issued one per MFMA of the first S / dP block.
-    auto tile_step = [&](auto prefetch, int cur, int entry, int kt_next) {
-        constexpr bool PREFETCH = decltype(prefetch)::value;
+    auto tile_step = [&](int cur, int entry, int kt_next) {
         // (the class is extracted with a per-lane copy of the wave number on purpose: a skip branch the compiler
         // can prove wave-uniform makes it restructure the loop around it at the price of ~90 spilled registers)
         const int kt = entry >> 8, cls = (entry >> (2 * wave_lane)) & 3;
         if (cls == 0) {  // nothing for this wave's slice in the tile: only keep the copies of the next one going
-            if (PREFETCH) {
 #pragma unroll
-                for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
-            }
+            for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
             return;
         }
         const u32x4* tK = sK[cur];
@@ -918,7 +882,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
             // ---- S^T = K Q^T and dP^T = V dO^T : 32 keys x 32 queries, two accumulator chains
             f32x16 s, dp;
             u32x4 bias_a = {0u, 0u, 0u, 0u};  // bias_fold: this lane's key of the block, as an operand
-            if (BIAS && PREFETCH && bias_fold && hi == 0) {
+            if (BIAS && bias_fold && hi == 0) {
                 const float bv = p.bias_f32 ? ((const float*)sBias[cur])[32 * kb + l32]
                                             : T::to_float(((const unsigned short*)sBias[cur])[32 * kb + l32]);
                 bias_a = split3_operand<T>(bv * inv_scale);
@@ -937,21 +901,21 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
                         dp = T::mfma(a[j], greg[j >> 1], j < 2 ? zero16 : dp);
                     else
                         s = T::mfma(a[j], qreg[j >> 1], j < 2 ? zero16 : s);
-                    if (PREFETCH && kb == 0 && j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
+                    if (kb == 0 && j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
                 }
-                if (PREFETCH && kb == 0) {
+                if (kb == 0) {
 #pragma unroll
                     for (int j = NOP; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
                 }
-                if (BIAS && PREFETCH && bias_fold) {
+                if (BIAS && bias_fold) {
                     const u32x4 z = {0u, 0u, 0u, 0u};
                     s = T::mfma(bias_a, hi == 0 ? ones3_operand<T>() : z, s);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (BIAS && PREFETCH && bias_fold) {
+            if (BIAS && bias_fold) {
                 // (added by the MFMA above)
-            } else if (BIAS && PREFETCH && bias_lds) {  // (the ragged last tile is staged without the bias)
+            } else if (BIAS && bias_lds) {
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
                     const int koff = 32 * kb + 8 * grp + 4 * hi;
@@ -1063,12 +1027,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
     const int nkt_total = (Sk + DQ_KT - 1) / DQ_KT;
     for (int kt_begin = 0;;) {
         __syncthreads();
-        const int n_all = sCount;
-        // A tile that holds the end of a sequence whose length is not a multiple of 64 is always the last
-        // entry of the list; it is staged synchronously (zero fill past the end) after the main loop.
-        const bool ragged = (Sk & (DQ_KT - 1)) != 0 && n_all > 0 &&
-                            (__builtin_amdgcn_readfirstlane(sList[n_all > 0 ? n_all - 1 : 0]) >> 8) == ((Sk - 1) >> 6);
-        const int n = n_all - (ragged ? 1 : 0);
+        const int n = sCount;
         if (n > 0) {
             int entry = __builtin_amdgcn_readfirstlane(sList[0]);
             int next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
@@ -1081,26 +1040,12 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
                 // entry after next, requested now and picked up at the end of the iteration; past the end of the
                 // list the last tile is simply copied again (into the buffer nobody reads any more)
                 const int after = sList[it + 2 < n ? it + 2 : n - 1];
-                tile_step(std::true_type{}, cur, entry, next >> 8);
+                tile_step(cur, entry, next >> 8);
                 entry = next;
                 next = __builtin_amdgcn_readfirstlane(after);
                 wait_async();
                 __syncthreads();
             }
-        }
-        if (ragged) {
-            const int entry = __builtin_amdgcn_readfirstlane(sList[n_all - 1]);
-            const int kt = entry >> 8, rows = Sk - kt * DQ_KT;
-            stK.load_ragged(kbase + kt * k_ts, sK[0], rows, tid);
-            stV.load_ragged(vbase + kt * v_ts, sV[0], rows, tid);
-            if (!DENSE && tid < DQ_KT) {
-                sKbf[0][tid] = (tid < rows) ? bfrow[kt * DQ_KT + tid] : 0;
-                if (IDX) sKpos[0][tid] = (tid < rows) ? p.posk[kt * DQ_KT + tid] : 0;
-            }
-            if (DENSE && row_bits_w != nullptr)
-                sRowBits[0][wave][lane] = row_bits_w[(int64_t)(2 * kt + hi) * p.row_bits_sn + l32];
-            __syncthreads();
-            tile_step(std::false_type{}, 0, entry, 0);
         }
         if (!LONG) break;
         kt_begin += MAX_LIST;

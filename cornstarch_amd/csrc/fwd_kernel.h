@@ -39,6 +39,7 @@ constexpr int FWD_THREADS = 256;
 template <typename T, int D, int MODE, bool BIAS, bool LONG>
 __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const AttnParams p) {
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
+    constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
     __shared__ u32x4 sK[2][FWD_KT * NCH];
     __shared__ u32x4 sV[2][FWD_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf[2][FWD_KT];  // raw bitfields of the tile's keys
@@ -119,12 +120,14 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
 #pragma unroll
     for (int i = 0; i < 16; ++i) zero16[i] = 0.f;
 
-    const char* kbase = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh);
-    const char* vbase = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)hk * p.v.sh);
-    const int64_t k_ts = 2 * p.k.ss * FWD_KT, v_ts = 2 * p.v.ss * FWD_KT;  // bytes per tile
-    const int64_t* bfrow = p.bfk + (int64_t)b * p.bfk_sb;
+    RowView<LONG> k_rows, v_rows;
+    RowView<false> bf_rows, pos_rows, bias_rows;  // key bitfields, (IDX) positions, per-key bias
+    k_rows.init((const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)hk * p.k.sh), 2 * p.k.ss, Sk, 2 * p.d);
+    v_rows.init((const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)hk * p.v.sh), 2 * p.v.ss, Sk, 2 * p.d);
+    if (!DENSE) bf_rows.init(p.bfk + (int64_t)b * p.bfk_sb, 8, Sk, 8);
+    if (IDX) pos_rows.init(p.posk, 4, Sk, 4);
 
-    typedef TileStage<D, FWD_KT, FWD_THREADS, true> Stage;  // (V only to copy both tiles alike, see dma_b128_ranged)
+    typedef TileStage<D, FWD_KT, FWD_THREADS, true> Stage;
     constexpr int CPT = Stage::CPT;
     // copy instructions per wave and tile: K, V, the key bitfields (DENSE: the mask bits of the wave's rows) and
     // (IDX) the key positions
@@ -135,49 +138,49 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
     stV.setup(2 * p.v.ss, p.d / 8, tid);
     const unsigned ldsK = lds_addr(sK), ldsV = lds_addr(sV), ldsB = lds_addr(sKbf), ldsP = lds_addr(sKpos);
     const unsigned ldsR = lds_addr(sRowBits);
-    const char* bias_head = BIAS ? (const char*)p.bias + (p.bias_f32 ? 4 : 2) * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh) : nullptr;
+    if (BIAS) {
+        const int esz = p.bias_f32 ? 4 : 2;
+        bias_rows.init((const char*)p.bias + esz * ((int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh), esz, Sk, esz);
+    }
     const unsigned bias_voff = (unsigned)((p.bias_f32 ? lane : (lane & 31)) * 4);
-    const int bias_tile_bytes = FWD_KT * (p.bias_f32 ? 4 : 2);
     // DENSE: the packed mask rows of this wave's slice (null: no plan, the mask bytes are read instead)
     const unsigned* row_bits_w = (DENSE && p.row_bits != nullptr)
                                      ? p.row_bits + (int64_t)b * p.row_bits_sb + (slice < 0 ? 0 : slice) * 32
                                      : nullptr;
     const unsigned row_bits_voff = DENSE ? (unsigned)(hi * (int)p.row_bits_sn * 4 + l32 * 4) : 0u;
     constexpr unsigned TILE_BYTES = FWD_KT * NCH * 16, BITS_BYTES = FWD_KT * 8;
-    // Copy instruction j (0 <= j < NLOADS) of full tile kt into buffer buf.  The 128 dwords of key
+    // Copy instruction j (0 <= j < NLOADS) of tile kt into buffer buf.  The 128 dwords of key
     // bitfields are copied 64 dwords per wave (waves 2, 3 repeat what waves 0, 1 write), so that every
     // wave issues the same number of copies.
     auto issue_copy = [&](int j, int kt, int buf) {
+        const int row = kt * FWD_KT;
         if (j < CPT)
-            stK.issue(j, kbase + kt * k_ts, ldsK + buf * TILE_BYTES);
+            stK.template issue<WAIT>(j, k_rows.at(row), ldsK + buf * TILE_BYTES);
         else if (j < 2 * CPT)
-            stV.issue(j - CPT, vbase + kt * v_ts, ldsV + buf * TILE_BYTES);
+            stV.template issue<WAIT>(j - CPT, v_rows.at(row), ldsV + buf * TILE_BYTES);
         else if (j == 2 * CPT) {
             if (DENSE) {  // lanes 0..31: block 2 kt, lanes 32..63: block 2 kt + 1, rows of this wave's slice
                 if (row_bits_w != nullptr)
                     dma_b32(row_bits_w + (int64_t)(2 * kt) * p.row_bits_sn, row_bits_voff, ldsR + (unsigned)(buf * 4 + wave) * 256u);
             } else {
-                dma_b32(bfrow + kt * FWD_KT, (unsigned)((wave & 1) * 256 + lane * 4), ldsB + buf * BITS_BYTES + (wave & 1) * 256u);
+                copy_b32<WAIT>(bf_rows.at(row), (unsigned)((wave & 1) * 256 + lane * 4), ldsB + buf * BITS_BYTES + (wave & 1) * 256u);
             }
         }
         else if (IDX && j == 2 * CPT + 1)  // 64 positions; every wave writes the same values
-            dma_b32(p.posk + kt * FWD_KT, (unsigned)(lane * 4), ldsP + buf * (FWD_KT * 4u));
+            copy_b32<WAIT>(pos_rows.at(row), (unsigned)(lane * 4), ldsP + buf * (FWD_KT * 4u));
         else if (bias_lds)  // BIAS: the tile's 64 bias values; every wave writes the same values
-            dma_b32(bias_head + (int64_t)kt * bias_tile_bytes, bias_voff, lds_addr(sBias) + buf * 256u);
+            copy_b32<WAIT>(bias_rows.at(row), bias_voff, lds_addr(sBias) + buf * 256u);
     };
 
-    // One 64-key tile held in buffer `cur`.  With PREFETCH the copies of tile `kt_next` into the other
+    // One 64-key tile held in buffer `cur`.  The copies of tile `kt_next` into the other
     // buffer are issued one per MFMA of the S phase, where the wave has nothing else to wait for.
-    auto tile_step = [&](auto prefetch, int cur, int entry, int kt_next) {
-        constexpr bool PREFETCH = decltype(prefetch)::value;
+    auto tile_step = [&](int cur, int entry, int kt_next) {
         // (the class is extracted with a per-lane copy of the wave number on purpose: with a skip branch the
         // compiler can prove wave-uniform it lays the loop out around that branch and the kernel loses ~8 %)
         const int kt = entry >> 8, cls = (entry >> (2 * wave_lane)) & 3;
         if (cls == 0) {  // nothing for this wave's slice in the tile: only keep the copies of the next one going
-            if (PREFETCH) {
 #pragma unroll
-                for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
-            }
+            for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
             return;
         }
         const u32x4* tK = sK[cur];
@@ -190,7 +193,7 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
         // wave's next MFMA is picked first and the MFMA pipe does not idle behind a queue of VALU instructions)
         f32x16 s[2];
         u32x4 bias_a[2];  // bias_fold: this lane's key of either 32-key block, as an operand (keys are the rows of S^T)
-        if (BIAS && PREFETCH && bias_fold) {
+        if (BIAS && bias_fold) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
                 const float bv = p.bias_f32 ? ((const float*)sBias[cur])[32 * kb + l32]
@@ -211,13 +214,11 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
                 if (j + AHEAD < NOP)
                     ka[j + AHEAD] = lds_read_chunk<D>(tK, 32 * ((j + AHEAD) & 1) + l32, 2 * ((j + AHEAD) >> 1) + hi);
                 s[j & 1] = T::mfma(ka[j], qreg[j >> 1], j < 2 ? zero16 : s[j & 1]);
-                if (PREFETCH && j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
+                if (j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
             }
-            if (PREFETCH) {
 #pragma unroll
-                for (int j = NOP; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
-            }
-            if (BIAS && PREFETCH && bias_fold) {
+            for (int j = NOP; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
+            if (BIAS && bias_fold) {
                 const u32x4 z = {0u, 0u, 0u, 0u};
                 const u32x4 ones = hi == 0 ? ones3_operand<T>() : z;
                 s[0] = T::mfma(bias_a[0], ones, s[0]);
@@ -227,9 +228,9 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
         }
         __builtin_amdgcn_s_setprio(0);
 
-        if (BIAS && PREFETCH && bias_fold) {
+        if (BIAS && bias_fold) {
             // (added by the MFMA above)
-        } else if (BIAS && PREFETCH && bias_lds) {  // (the ragged last tile is staged without the bias)
+        } else if (BIAS && bias_lds) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -420,12 +421,7 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
     const int nkt_total = (Sk + FWD_KT - 1) / FWD_KT;
     for (int kt_begin = 0;;) {
         __syncthreads();
-        const int n_all = sCount;
-        // A tile that holds the end of a sequence whose length is not a multiple of 64 is always the last
-        // entry of the list; it is staged synchronously (zero fill past the end) after the main loop.
-        const bool ragged = (Sk & (FWD_KT - 1)) != 0 && n_all > 0 &&
-                            (__builtin_amdgcn_readfirstlane(sList[n_all > 0 ? n_all - 1 : 0]) >> 8) == ((Sk - 1) >> 6);
-        const int n = n_all - (ragged ? 1 : 0);
+        const int n = sCount;
         if (n > 0) {
             int entry = __builtin_amdgcn_readfirstlane(sList[0]);
             int next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
@@ -438,26 +434,12 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
                 // entry after next, requested now and picked up at the end of the iteration; past the end of the
                 // list the last tile is simply copied again (into the buffer nobody reads any more)
                 const int after = sList[it + 2 < n ? it + 2 : n - 1];
-                tile_step(std::true_type{}, cur, entry, next >> 8);
+                tile_step(cur, entry, next >> 8);
                 entry = next;
                 next = __builtin_amdgcn_readfirstlane(after);
                 wait_async();
                 __syncthreads();
             }
-        }
-        if (ragged) {
-            const int entry = __builtin_amdgcn_readfirstlane(sList[n_all - 1]);
-            const int kt = entry >> 8, rows = Sk - kt * FWD_KT;
-            stK.load_ragged(kbase + kt * k_ts, sK[0], rows, tid);
-            stV.load_ragged(vbase + kt * v_ts, sV[0], rows, tid);
-            if (!DENSE && tid < FWD_KT) {
-                sKbf[0][tid] = (tid < rows) ? bfrow[kt * FWD_KT + tid] : 0;
-                if (IDX) sKpos[0][tid] = (tid < rows) ? p.posk[kt * FWD_KT + tid] : 0;
-            }
-            if (DENSE && row_bits_w != nullptr)
-                sRowBits[0][wave][lane] = row_bits_w[(int64_t)(2 * kt + hi) * p.row_bits_sn + l32];
-            __syncthreads();
-            tile_step(std::false_type{}, 0, entry, 0);
         }
         if (!LONG) break;
         kt_begin += MAX_LIST;
