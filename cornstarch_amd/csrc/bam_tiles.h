@@ -267,10 +267,14 @@ __device__ __forceinline__ WaveSlices pick_wave_slices(const AttnParams& p, int 
 // A tile is "full" for a slice only when both of its 32-column classes say so AND it has no column past
 // the end of the sequence (those columns must still be masked out of the softmax).
 // Executed by wave 0; the caller synchronizes before reading.
+// STREAMS = 2: the even and the odd tiles make a list each (the second at list + MAX_LIST / 2, its length in count_out[1]).  Which
+// list a tile is in does not depend on what else is listed, so a row's result does not depend on its neighbours or the plan.
+template <int STREAMS = 1>
 __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int num_n, int S, int lane, int kt_begin,
                                                     int* list, int* count_out) {
     const int nkt = min((S + 63) >> 6, kt_begin + MAX_LIST);
-    int count = 0;
+    int count[STREAMS] = {};
+    const int mine = STREAMS > 1 ? lane & 1 : 0;  // (kt_begin is even)
     for (int base = kt_begin; base < nkt; base += 64) {
         const int kt = base + lane;
         int packed = 0;
@@ -286,11 +290,17 @@ __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int nu
                 packed |= cls << (2 * x);
             }
         }
-        const unsigned long long bal = __ballot(packed != 0);
-        if (packed) list[count + __popcll(bal & ((1ull << lane) - 1ull))] = (kt << 8) | packed;
-        count += __popcll(bal);
+        unsigned long long bal = __ballot(packed != 0), own = bal;
+        if (STREAMS > 1) own &= mine ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull;
+        const int at = (mine ? MAX_LIST / 2 + count[STREAMS - 1] : count[0]) + __popcll(own & ((1ull << lane) - 1ull));
+        if (packed) list[at] = (kt << 8) | packed;
+#pragma unroll
+        for (int x = 0; x < STREAMS; ++x)
+            count[x] += __popcll(STREAMS == 1 ? bal : bal & (x ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull));
     }
-    if (lane == 0) *count_out = count;
+#pragma unroll
+    for (int x = 0; x < STREAMS; ++x)
+        if (lane == 0) count_out[x] = count[x];
     wait_lds();
 }
 

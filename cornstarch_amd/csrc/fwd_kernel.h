@@ -36,23 +36,32 @@ constexpr int FWD_THREADS = 256;
 // BIAS: an additive bias p.bias (reference bitfield_attention.py:410-434) is added to scale * q.k.
 // LONG: sequences of more than MAX_LIST 64-key tiles (131072 keys), walked in several passes; the short form has no
 // pass loop at all (a loop around the main loop costs registers and a few per cent).
-template <typename T, int D, int MODE, bool BIAS, bool LONG>
-__global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const AttnParams p) {
+// STREAMS: how many tiles of the list are in work at a time, each by four waves of its own on the same four slices.
+template <typename T, int D, int MODE, bool BIAS, bool LONG, int STREAMS>
+__global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 3) void fwd_kernel(const AttnParams p) {
+    static_assert(STREAMS == 1 || !LONG, "streams and passes are not combined");
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
-    __shared__ u32x4 sK[2][FWD_KT * NCH];
-    __shared__ u32x4 sV[2][FWD_KT * NCH];
-    __shared__ __attribute__((aligned(16))) int64_t sKbf[2][FWD_KT];  // raw bitfields of the tile's keys
-    __shared__ __attribute__((aligned(16))) int sKpos[2][FWD_KT];     // their global positions (IDX only)
+    __shared__ u32x4 sK_all[STREAMS][2][FWD_KT * NCH];
+    __shared__ u32x4 sV_all[STREAMS][2][FWD_KT * NCH];
+    __shared__ __attribute__((aligned(16))) int64_t sKbf_all[STREAMS][2][FWD_KT];  // raw bitfields of the tile's keys
+    __shared__ __attribute__((aligned(16))) int sKpos_all[STREAMS][2][FWD_KT];     // their global positions (IDX only)
     __shared__ int sList[MAX_LIST];
-    __shared__ int sCount;
+    __shared__ int sCount[STREAMS];
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     // DENSE with packed mask bits: per wave, the words of its 32 rows for the tile's two 32-key blocks
-    __shared__ unsigned sRowBits[DENSE ? 2 : 1][4][DENSE ? 64 : 1];
+    __shared__ unsigned sRowBits_all[STREAMS][DENSE ? 2 : 1][4][DENSE ? 64 : 1];
     // BIAS in its per-key ("vector") form: the 64 values of the tile (raw words; 16-bit elements fill half)
-    __shared__ __attribute__((aligned(16))) unsigned sBias[BIAS ? 2 : 1][BIAS ? 64 : 1];
+    __shared__ __attribute__((aligned(16))) unsigned sBias_all[STREAMS][BIAS ? 2 : 1][BIAS ? 64 : 1];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // (tid and wave: inside the stream)
+    const int tid = threadIdx.x % FWD_THREADS, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int stream = STREAMS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / FWD_THREADS) : 0;
+    auto &sK = sK_all[stream], &sV = sV_all[stream];
+    auto& sKbf = sKbf_all[stream];
+    auto& sKpos = sKpos_all[stream];
+    auto& sRowBits = sRowBits_all[stream];
+    auto& sBias = sBias_all[stream];
     const int hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
     const int wave_lane = tid >> 6;
     const int Sq = p.Sq, Sk = p.Sk;
@@ -69,7 +78,7 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
     const int h = hk * G + g;
     const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
 
-    if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, 0, sList, &sCount);  // first pass (usually the only one)
+    if (wave == 0 && stream == 0) build_key_tile_list<STREAMS>(ws, p.num_n, Sk, lane, 0, sList, sCount);  // first pass (usually the only one)
 
     // ---- per-lane query state -------------------------------------------------------
     const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
@@ -421,19 +430,26 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
     const int nkt_total = (Sk + FWD_KT - 1) / FWD_KT;
     for (int kt_begin = 0;;) {
         __syncthreads();
-        const int n = sCount;
-        if (n > 0) {
-            int entry = __builtin_amdgcn_readfirstlane(sList[0]);
-            int next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
+        // With two streams, one takes the even tiles and the other the odd ones.  Past the end of its list a stream copies its
+        // last tile again, for nobody to read or, where the other list is longer, with all classes cleared.
+        const int n = sCount[stream], rounds = STREAMS > 1 ? max(n, sCount[STREAMS - 1 - stream]) : n;
+        if (rounds > 0) {
+            const int* const list = sList + stream * (MAX_LIST / 2);
+            auto list_at = [&](int i) {
+                if (STREAMS == 1) return list[i < n ? i : n - 1];
+                const int e = list[i < n ? i : max(n - 1, 0)];
+                return i < n ? e : n > 0 ? e & ~0xFF : 0;
+            };
+            int entry = __builtin_amdgcn_readfirstlane(list_at(0));
+            int next = __builtin_amdgcn_readfirstlane(list_at(1));
     #pragma unroll
             for (int j = 0; j < NLOADS; ++j) issue_copy(j, entry >> 8, 0);
             wait_async();
             __syncthreads();
-            for (int it = 0; it < n; ++it) {
+            for (int it = 0; it < rounds; ++it) {
                 const int cur = it & 1;
-                // entry after next, requested now and picked up at the end of the iteration; past the end of the
-                // list the last tile is simply copied again (into the buffer nobody reads any more)
-                const int after = sList[it + 2 < n ? it + 2 : n - 1];
+                // entry after next, requested now and picked up at the end of the iteration
+                const int after = list_at(it + 2);
                 tile_step(cur, entry, next >> 8);
                 entry = next;
                 next = __builtin_amdgcn_readfirstlane(after);
@@ -445,46 +461,96 @@ __global__ __launch_bounds__(FWD_THREADS, D > 64 ? 2 : 3) void fwd_kernel(const 
         kt_begin += MAX_LIST;
         if (kt_begin >= nkt_total) break;
         __syncthreads();  // everybody has read the list of the pass that just ended
-        if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, kt_begin, sList, &sCount);
+        if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, kt_begin, sList, sCount);
     }
 
     // ---- epilogue: normalize, write O (q dtype) and LSE (natural log) -------------------
-    const float ltot = half_swap_sum(l_i);
+    float ltot = half_swap_sum(l_i), mine = 1.f, theirs = 0.f;
+    // With two streams, a row's two partial results meet through the tile arrays, which nobody reads any more: each stream
+    // hands over the columns that the other one finishes.
+    constexpr int DB0 = STREAMS > 1 ? (DB + 1) / 2 : DB;  // stream 0 finishes the column blocks below DB0, stream 1 the others
+    f32x4* const park = (f32x4*)sK_all + wave * (DB * 4 * 64);
+    float* const park_ml = (float*)sV_all;
+    if constexpr (STREAMS > 1) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            if ((db < DB0) == (stream == 1)) {
+#pragma unroll
+                for (int grp = 0; grp < 4; ++grp)
+                    park[(4 * db + grp) * 64 + lane] = f32x4{o[db][4 * grp], o[db][4 * grp + 1], o[db][4 * grp + 2], o[db][4 * grp + 3]};
+            }
+        park_ml[(8 * stream + 2 * wave) * 64 + lane] = m_i;
+        park_ml[(8 * stream + 2 * wave + 1) * 64 + lane] = ltot;
+        __syncthreads();
+        const float m_other = park_ml[(8 * (1 - stream) + 2 * wave) * 64 + lane];
+        const float l_other = park_ml[(8 * (1 - stream) + 2 * wave + 1) * 64 + lane];
+        const float m = fmaxf(m_i, m_other), muse = m == -INFINITY ? 0.f : m;
+        mine = __builtin_amdgcn_exp2f((m_i - muse) * c2);  // 0 for a stream that has seen no key of this row
+        theirs = __builtin_amdgcn_exp2f((m_other - muse) * c2);
+        ltot = stream == 0 ? fmaf(ltot, mine, l_other * theirs) : fmaf(l_other, theirs, ltot * mine);
+        m_i = m;
+    }
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-    if (hi == 0 && slice >= 0)
+    if (stream == 0 && hi == 0 && slice >= 0)
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] =
             ltot > 0.f ? (m_i * c2 + __builtin_amdgcn_logf(ltot)) * LN2 : -INFINITY;
     // A wave without a slice (plan: slot 4 grp + wave of the order lies past the last slice) owns the 32 padding rows
     // of that slot, so that every row of the rounded lse is written whether or not a plan is given.
-    if (hi == 0 && slice < 0 && 32 * (4 * grp + wave) + 31 < p.Sq_rounded)
+    if (stream == 0 && hi == 0 && slice < 0 && 32 * (4 * grp + wave) + 31 < p.Sq_rounded)
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + 32 * (4 * grp + wave) + l32] = -INFINITY;
     if (qvalid) {
         char* op = (char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db) {
+            if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
                 if (32 * db + 8 * grp >= p.d) break;
+                float x[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] = o[db][4 * grp + i];
+                if constexpr (STREAMS > 1) {
+                    const f32x4 other = park[(4 * db + grp) * 64 + lane];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[i] = fmaf(x[i], mine, other[i] * theirs);
+                }
                 u32x2 w;
-                w[0] = T::pack2(o[db][4 * grp + 0] * inv, o[db][4 * grp + 1] * inv);
-                w[1] = T::pack2(o[db][4 * grp + 2] * inv, o[db][4 * grp + 3] * inv);
+                w[0] = T::pack2(x[0] * inv, x[1] * inv);
+                w[1] = T::pack2(x[2] * inv, x[3] * inv);
                 *(u32x2*)(op + (32 * db + 8 * grp + 4 * hi) * 2) = w;
             }
+        }
     }
 }
 
 
 // Launches every (mask mode, bias) instantiation of one (element type, head dim, LONG) combination.
+template <typename T, int D, bool BIAS, bool LONG, int STREAMS>
+static int launch_fwd_s(const AttnParams& p, hipStream_t stream) {
+    const int blocks = p.num_m * p.B * p.Hq, threads = FWD_THREADS * STREAMS;
+    if (p.mask_mode == MASK_INDEXED)
+        hipLaunchKernelGGL((fwd_kernel<T, D, MASK_INDEXED, BIAS, LONG, STREAMS>), dim3(blocks), dim3(threads), 0, stream, p);
+    else if (p.mask_mode == MASK_DENSE)
+        hipLaunchKernelGGL((fwd_kernel<T, D, MASK_DENSE, BIAS, LONG, STREAMS>), dim3(blocks), dim3(threads), 0, stream, p);
+    else
+        hipLaunchKernelGGL((fwd_kernel<T, D, MASK_BITFIELD, BIAS, LONG, STREAMS>), dim3(blocks), dim3(threads), 0, stream, p);
+    return (int)hipGetLastError();
+}
+// Two streams halve the chain of tiles a workgroup walks and double the waves of a compute unit that has one workgroup; the price
+// is a workgroup that fills the unit (D = 64 and above), so that nothing runs beside its first loads and its stores.  Forward
+// kernel alone, bf16, one stream -> two, 32 / 8 heads (8 / 8 where marked *): D 128: 200 tokens * 15.9 -> 14.5 us, 1000 * 30.2 ->
+// 25.2, 1024 (256 workgroups) 31.8 -> 27.3, 2 x 700 (384) 31.0 -> 30.7, 2048 (512) 57.5 -> 57.2, 3001 (768) 88 -> 103; D 64:
+// 1000 * 24.1 -> 19.2, 2 x 700 24.2 -> 22.0, 2048 43.4 -> 40.9, 3001 62 -> 69.  At D = 32 two such workgroups fit a unit: 2048
+// 37.8 -> 28.2, 3001 52.4 -> 40.7, 4096 (1024) 69 -> 61, but with short lists 8 x 300 (768) 16.0 -> 19.5, 4 x 1024 27.8 -> 30.4.
+static bool fwd_two_streams(const AttnParams& p) {
+    const int64_t units = (int64_t)p.num_m * p.B * p.Hq;
+    return units <= (p.D > 64 ? 256 : 512) || (p.D <= 32 && units <= 1024 && p.Sk >= 2560);
+}
 template <typename T, int D, bool BIAS, bool LONG>
 static int launch_fwd_b(const AttnParams& p, hipStream_t stream) {
-    const int blocks = p.num_m * p.B * p.Hq;
-    if (p.mask_mode == MASK_INDEXED)
-        hipLaunchKernelGGL((fwd_kernel<T, D, MASK_INDEXED, BIAS, LONG>), dim3(blocks), dim3(FWD_THREADS), 0, stream, p);
-    else if (p.mask_mode == MASK_DENSE)
-        hipLaunchKernelGGL((fwd_kernel<T, D, MASK_DENSE, BIAS, LONG>), dim3(blocks), dim3(FWD_THREADS), 0, stream, p);
-    else
-        hipLaunchKernelGGL((fwd_kernel<T, D, MASK_BITFIELD, BIAS, LONG>), dim3(blocks), dim3(FWD_THREADS), 0, stream, p);
-    return (int)hipGetLastError();
+    if constexpr (!LONG)
+        if (fwd_two_streams(p)) return launch_fwd_s<T, D, BIAS, false, 2>(p, stream);
+    return launch_fwd_s<T, D, BIAS, LONG, 1>(p, stream);
 }
 template <typename T, int D, bool LONG>
 static int launch_fwd_t(const AttnParams& p, hipStream_t stream) {

@@ -1,0 +1,38 @@
+"""The forward with few workgroups walks two tiles at a time and merges two partial results per row.  Every sequence of a batch
+that is large enough to go tile by tile, against the same sequence by itself."""
+
+import pytest
+import torch
+
+from cornstarch_amd.kernel import bitfield_attention as BA
+from tests.helpers import random_bitfield, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("D", [32, 40, 64, 96, 128])
+@pytest.mark.parametrize("S", [1, 64, 65, 130, 200, 257])  # lists of 1 to 5 tiles, odd and even
+def test_a_sequence_of_a_large_batch_equals_the_sequence_alone(S, D, biased):
+    Hq, Hkv = 8, 2
+    B = 1024 // (Hq * ((S + 127) // 128)) + 1  # more than 1024 workgroups
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v = ((torch.randn(B, S, H, D, generator=g, device="cuda")).bfloat16() for H in (Hq, Hkv, Hkv))
+    bf = random_bitfield(B, S, seed=S, pad=S // 9).cuda()
+    bias = torch.randn(1, Hq, 1, S, generator=g, device="cuda") if biased else None
+
+    def forward(rows):
+        BA.BitfieldUtils.clear_cache()
+        flags = BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(bf[rows])
+        return BA._bitfield_attn_forward(q[rows], k[rows], v[rows], bf[rows], flags, bias=bias)[:2]
+
+    o, lse = forward(slice(None))
+    for b in (0, B // 2, B - 1):
+        o1, lse1 = forward(slice(b, b + 1))
+        # probabilities are rounded to bf16 against another running maximum: 2^-9 each, over at least one key; the sums of the
+        # rounded ones (the lse) differ by no more than that
+        assert rel_l2(o1[0].float(), o[b].float()) <= 2.0**-8
+        live = torch.isfinite(lse[b])
+        assert torch.equal(live, torch.isfinite(lse1[0])) and (lse1[0] - lse[b])[live].abs().max().item() <= 2.0**-8
+        assert torch.isfinite(o1).all() and torch.equal(lse[b][~live], lse1[0][~live])
+    BA.BitfieldUtils.clear_cache()
