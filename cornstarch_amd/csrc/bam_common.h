@@ -252,6 +252,31 @@ __device__ __forceinline__ float half_swap_sum(float x) {
     return a + b;
 }
 
+// Two neighbouring groups of four columns each, packed to 16 bits (a: columns 4 hi .. of group A, b: of group B): the lane ends
+// up with the eight columns of group A (lower half wave) or B (upper half wave), to be stored as one 16-byte chunk.  Half the
+// store instructions, each with whole 32-byte sectors, of storing eight bytes per lane and group.
+__device__ __forceinline__ u32x4 pair_columns(u32x2 a, u32x2 b) {
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
+                 : "+v"(a[0]), "+v"(a[1]), "+v"(b[0]), "+v"(b[1]));
+    return u32x4{a[0], a[1], b[0], b[1]};
+}
+// One 32-column block (C fragment: registers = columns 8 g + 4 hi + x) of a row in the 16-bit type: the block's columns that
+// exist, `left` of them (a multiple of 8).  value(i): register i, already scaled.
+template <typename T, typename F>
+__device__ __forceinline__ void store_block16(char* dst, int left, int hi, F value) {
+#pragma unroll
+    for (int gp = 0; gp < 2; ++gp) {
+        u32x2 w[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int i = 4 * (2 * gp + x);
+            w[x] = u32x2{T::pack2(value(i), value(i + 1)), T::pack2(value(i + 2), value(i + 3))};
+        }
+        const u32x4 chunk = pair_columns(w[0], w[1]);
+        if (8 * (2 * gp + hi) < left) *(u32x4*)(dst + 16 * (2 * gp + hi)) = chunk;
+    }
+}
+
 // Scheduling hint: interleave `n` MFMAs with the LDS reads that feed them so that reads run
 // `ahead` operands in front of their MFMA (reads_per_op LDS instructions per operand).  Must
 // follow, in the same basic block, the n operand reads and the n MFMAs it orders.

@@ -119,8 +119,8 @@ __device__ __forceinline__ void copy_b32(const TileSrc& src, unsigned voff, unsi
                  "{m0}"(lds_base), "n"(WAIT)
                  : "memory");
 }
-template <int MODE, bool BIAS, bool LONG>
-constexpr int COPY_WAIT = LONG || (BIAS && MODE == MASK_INDEXED) ? 4 : 0;
+template <bool BIAS, bool LONG>
+constexpr int COPY_WAIT = LONG || BIAS ? 4 : 0;
 
 // All direct global-to-LDS copies this wave has issued have landed (pair with a barrier).
 __device__ __forceinline__ void wait_async() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -227,6 +227,16 @@ struct SliceStage {
             copy_b128<WAIT>(slice, goff[i], tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
     }
 };
+
+// Workgroup barrier that publishes LDS writes and leaves loads from memory in flight (the compiler's own barrier waits for them).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// The arrival of a load is pinned where this stands.  Left alone, the compiler waits for it at its first use inside the key
+// loop, with a vmcnt that also (and every time round) drains the tile copies it does not know about.
+template <int N>
+__device__ __forceinline__ void arrived(u32x4 (&regs)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(regs[i]));
+}
 
 // The 32-row slice each of the four waves of a forward / dQ workgroup works on, and the row of tile classes
 // (one byte per 32-key column tile: 0 empty, 1 partial, 2 full) that says which keys that slice needs.

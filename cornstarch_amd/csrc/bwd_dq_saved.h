@@ -232,14 +232,7 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
         char* dqp = (char*)p.dq.ptr + 2 * ((int64_t)b * p.dq.sb + (int64_t)qrow * p.dq.ss + (int64_t)h * p.dq.sh);
 #pragma unroll
         for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int grp = 0; grp < 4; ++grp) {
-                if (32 * db + 8 * grp >= p.d) break;
-                u32x2 w;
-                w[0] = T::pack2(dq[db][4 * grp + 0] * factor, dq[db][4 * grp + 1] * factor);
-                w[1] = T::pack2(dq[db][4 * grp + 2] * factor, dq[db][4 * grp + 3] * factor);
-                *(u32x2*)(dqp + (32 * db + 8 * grp + 4 * hi) * 2) = w;
-            }
+            store_block16<T>(dqp + 64 * db, p.d - 32 * db, hi, [&](int i) { return dq[db][i] * factor; });
     } else if (qvalid) {
         float* dqp = (float*)p.dq.ptr + ((int64_t)b * p.dq.sb + (int64_t)qrow * p.dq.ss + (int64_t)h * p.dq.sh);
 #pragma unroll

@@ -88,7 +88,7 @@ template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
-    constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
+    constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
     __shared__ u32x4 sK[128 * NCH];
     __shared__ u32x4 sV[128 * NCH];
     __shared__ u32x4 sQ[2][DKDV_QT * NCH];
@@ -134,9 +134,6 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     }
 
     const int ns_total = (Sq + 31) >> 5;
-    // first pass (usually the only one): the last MAX_SLICE_LIST slices
-    if (wave == 0) build_slice_list(p, b, nt, lane, max(0, ns_total - MAX_SLICE_LIST), ns_total, sList, &sCount);
-
     // ---- K, V of the tile -> LDS (once) ---------------------------------------------------
     {
         TileStage<D, 128, DKDV_THREADS> stK, stV;
@@ -155,9 +152,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     int kpos = (IDX && kvalid) ? p.posk[key] : key;  // global position of this lane's key
     unsigned klo = (unsigned)(kf & 0xFFFFFFFFll);
     unsigned khi = (unsigned)((uint64_t)kf >> 32);
-    // Pin the arrival of this load here.  Left alone, the compiler waits for it at the first use inside the
-    // main loop, with a vmcnt that also (and every time round) drains the tile copies it does not know about.
-    asm volatile("" : "+v"(klo), "+v"(khi), "+v"(kpos));
+    // first pass (usually the only one): the last MAX_SLICE_LIST slices
+    if (wave == 0) build_slice_list(p, b, nt, lane, max(0, ns_total - MAX_SLICE_LIST), ns_total, sList, &sCount);
 
     f32x16 dk[DB], dv[DB];
 #pragma unroll
@@ -512,7 +508,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     // Sequences of more than MAX_SLICE_LIST slices are walked in several passes, from the end, each with a list
     // of its own; dK and dV live in registers and simply carry over.
     for (int s_end = ns_total;;) {
-        __syncthreads();
+        lds_barrier();
         const int n = sCount;
         // Main loop: the listed slices are taken in pairs from the END of the list (the workgroups of one kv head
         // that are resident together then read the same Q / dO rows at about the same time, and all but the first
@@ -543,6 +539,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             advance();
             int n_lo = __builtin_amdgcn_readfirstlane(entry_lo(r_nxt)), n_hi = __builtin_amdgcn_readfirstlane(entry_hi(r_nxt));
             wait_async();
+            asm volatile("" : "+v"(klo), "+v"(khi), "+v"(kpos));  // (see arrived())
             __syncthreads();
             if (!v_negated) {  // K, V and the first tile have landed
                 negate_v_tile();
@@ -585,99 +582,52 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     wait_async();
     __syncthreads();
 
-    // ---- epilogue.  The two waves of a key group hold partial sums.
-    if (p.grad_typed) {
-        // Overwrite mode: dk/dv have the input dtype.  The K, V, Q, dO tiles are dead now; the
-        // stream-1 wave of key group kg parks its partial sums in tile array number kg (exactly
-        // the right size: 2 * D/32 * 16 floats per lane), its stream-0 partner adds its own and
-        // stores the converted result.
-        float* park = (float*)(kg == 0 ? sK : kg == 1 ? sV : kg == 2 ? &sQ[0][0] : &sDO[0][0]);
-        if (st == 1) {
+    // ---- epilogue.  The two waves of a key group hold partial sums of dK and dV.  The K, V, Q and dO tiles are dead now: through
+    // tile array number kg (exactly the right size) the row stream 0 wave hands its dV over and the stream 1 wave its dK; then
+    // the one finishes dK, the other dV.  This workgroup is the sole owner of these rows.
+    f32x4* const park = (f32x4*)(kg == 0 ? sK : kg == 1 ? sV : kg == 2 ? &sQ[0][0] : &sDO[0][0]);
+    auto hand_over = [&](const f32x16 (&acc)[DB], int half) {
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    park[(db * 16 + i) * 64 + lane] = dk[db][i];
-                    park[((DB + db) * 16 + i) * 64 + lane] = dv[db][i];
-                }
-        }
-        __syncthreads();
-        if (PARTS && p.grad_typed == 2) {
-            if (st == 0 && kvalid) {
-                float* dkp = (float*)p.dk.ptr + ((int64_t)b * p.dk.sb + (int64_t)key * p.dk.ss + (int64_t)hk * p.dk.sh);
-                float* dvp = (float*)p.dv.ptr + ((int64_t)b * p.dv.sb + (int64_t)key * p.dv.ss + (int64_t)hk * p.dv.sh);
+            for (int grp = 0; grp < 4; ++grp)
+                park[((half * DB + db) * 4 + grp) * 64 + lane] =
+                    f32x4{acc[db][4 * grp], acc[db][4 * grp + 1], acc[db][4 * grp + 2], acc[db][4 * grp + 3]};
+    };
+    auto finish = [&](const f32x16 (&acc)[DB], int half, float factor, const Tensor4& t) {
+        const int64_t at = (int64_t)b * t.sb + (int64_t)key * t.ss + (int64_t)hk * t.sh;
 #pragma unroll
-                for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db) {
+            f32x16 x = acc[db];
 #pragma unroll
-                    for (int grp = 0; grp < 4; ++grp) {
-                        if (32 * db + 8 * grp >= p.d) break;
-                        f32x4 a, c;
+            for (int grp = 0; grp < 4; ++grp) {
+                const f32x4 other = park[((half * DB + db) * 4 + grp) * 64 + lane];
 #pragma unroll
-                        for (int x = 0; x < 4; ++x) {
-                            const int i = 4 * grp + x;
-                            a[x] = (dk[db][i] + park[(db * 16 + i) * 64 + lane]) * -p.scale;
-                            c[x] = dv[db][i] + park[((DB + db) * 16 + i) * 64 + lane];
-                        }
-                        const int d0 = 32 * db + 8 * grp + 4 * hi;
-                        *(f32x4*)(dkp + d0) = a;
-                        *(f32x4*)(dvp + d0) = c;
-                    }
+                for (int i = 0; i < 4; ++i) x[4 * grp + i] = (x[4 * grp + i] + other[i]) * factor;
             }
-            return;
+            if (p.grad_typed == 1) {  // overwrite mode: the input dtype
+                store_block16<T>((char*)t.ptr + 2 * (at + 32 * db), p.d - 32 * db, hi, [&](int i) { return x[i]; });
+                continue;
+            }
+#pragma unroll
+            for (int grp = 0; grp < 4; ++grp) {
+                if (32 * db + 8 * grp >= p.d) break;
+                f32x4* dst = (f32x4*)((float*)t.ptr + at + 32 * db + 8 * grp + 4 * hi);
+                const f32x4 y = {x[4 * grp], x[4 * grp + 1], x[4 * grp + 2], x[4 * grp + 3]};
+                *dst = PARTS && p.grad_typed == 2 ? y : *dst + y;
+            }
         }
-        if (st == 0 && kvalid) {
-            char* dkp = (char*)p.dk.ptr + 2 * ((int64_t)b * p.dk.sb + (int64_t)key * p.dk.ss + (int64_t)hk * p.dk.sh);
-            char* dvp = (char*)p.dv.ptr + 2 * ((int64_t)b * p.dv.sb + (int64_t)key * p.dv.ss + (int64_t)hk * p.dv.sh);
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int grp = 0; grp < 4; ++grp) {
-                    if (32 * db + 8 * grp >= p.d) break;
-                    float a[4], c[4];
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        const int i = 4 * grp + x;
-                        a[x] = (dk[db][i] + park[(db * 16 + i) * 64 + lane]) * -p.scale;  // dk holds -dK / scale
-                        c[x] = dv[db][i] + park[((DB + db) * 16 + i) * 64 + lane];
-                    }
-                    const int d0 = 32 * db + 8 * grp + 4 * hi;
-                    u32x2 wk, wv;
-                    wk[0] = T::pack2(a[0], a[1]);
-                    wk[1] = T::pack2(a[2], a[3]);
-                    wv[0] = T::pack2(c[0], c[1]);
-                    wv[1] = T::pack2(c[2], c[3]);
-                    *(u32x2*)(dkp + d0 * 2) = wk;
-                    *(u32x2*)(dvp + d0 * 2) = wv;
-                }
-        }
-        return;
-    }
-    // Accumulate mode: both waves add to the caller's fp32 buffers in turn (this workgroup is
-    // the sole owner of these rows).
-    float* dkp = (float*)p.dk.ptr + ((int64_t)b * p.dk.sb + (int64_t)key * p.dk.ss + (int64_t)hk * p.dk.sh);
-    float* dvp = (float*)p.dv.ptr + ((int64_t)b * p.dv.sb + (int64_t)key * p.dv.ss + (int64_t)hk * p.dv.sh);
-#pragma unroll
-    for (int turn = 0; turn < 2; ++turn) {
-        if (st == turn && kvalid) {
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int grp = 0; grp < 4; ++grp) {
-                    if (32 * db + 8 * grp >= p.d) break;
-                    const int d0 = 32 * db + 8 * grp + 4 * hi;
-                    f32x4 a = *(f32x4*)(dkp + d0), c = *(f32x4*)(dvp + d0);
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        a[x] = fmaf(dk[db][4 * grp + x], -p.scale, a[x]);  // dk holds -dK / scale
-                        c[x] += dv[db][4 * grp + x];
-                    }
-                    *(f32x4*)(dkp + d0) = a;
-                    *(f32x4*)(dvp + d0) = c;
-                }
-        }
-        __threadfence_block();
-        __syncthreads();
-    }
+    };
+    if (st == 0)
+        hand_over(dv, 1);
+    else
+        hand_over(dk, 0);
+    __syncthreads();
+    if (!kvalid) return;
+    if (st == 0)
+        finish(dk, 0, -p.scale, p.dk);  // (dk holds -dK / scale)
+    else
+        finish(dv, 1, 1.f, p.dv);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -700,7 +650,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
     constexpr bool BIAS = BIAS_FORM != BIAS_NONE, bias_lds = BIAS_FORM == BIAS_TILES;
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
-    constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
+    constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
     __shared__ u32x4 sK[2][DQ_KT * NCH];
     __shared__ u32x4 sV[2][DQ_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf[2][DQ_KT];  // raw bitfields of the tile's keys
@@ -754,25 +704,38 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
         lse_row = p.lse[off];
         if (D > 64 || p.o.ptr == nullptr) dlt = p.delta[off];
     }
+    u32x4 oreg[D <= 64 ? KK : 1];
+    const bool sums_delta = D <= 64 && p.o.ptr != nullptr;
+    if (sums_delta) {
+        const char* op = (const char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
+#pragma unroll
+        for (int kk = 0; kk < (D <= 64 ? KK : 1); ++kk) {
+            u32x4 zo = {0u, 0u, 0u, 0u};
+            if (qvalid && 16 * kk + 8 * hi < p.d) zo = *(const u32x4*)(op + (16 * kk + 8 * hi) * 2);
+            oreg[kk] = zo;
+        }
+    }
+    const int qpos = (IDX && qvalid) ? p.posq[qrow] : qrow;
+    // (the row loads above are in flight while wave 0 reads the class rows and the first tile is on its way)
+    if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, 0, sList, &sCount);  // first pass (usually the only one)
+    QueryBits qb = {};
+    float lse2 = INFINITY;
     // With o given, this launch also is the delta pre-pass: it runs in front of the dK/dV kernel, has the rows of dO in
     // registers and covers every row once; a launch and a second reading of dO less (2 x 283 tokens: 3.4 us; 8 x 4096
     // tokens, 16 heads, D 64: 25 us for reading both).  Sums as the pre-pass does: chunk pairs, then the two half waves.
-    if (D <= 64 && p.o.ptr != nullptr) {
-        const char* op = (const char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
-        float part[KK];
+    auto rows_arrived = [&]() {
+        arrived(qreg);
+        arrived(greg);
+        if (sums_delta) {
+            float part[KK];
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            u32x4 zo = {0u, 0u, 0u, 0u};
-            if (qvalid && 16 * kk + 8 * hi < p.d) zo = *(const u32x4*)(op + (16 * kk + 8 * hi) * 2);
-            part[kk] = chunk_dot<T>(zo, greg[kk]);
+            for (int kk = 0; kk < (D <= 64 ? KK : 1); ++kk) part[kk] = chunk_dot<T>(oreg[kk], greg[kk]);
+            dlt = half_swap_sum(KK == 4 ? (part[0] + part[2]) + (part[1] + part[KK - 1]) : part[0] + part[1]);
+            if (qvalid && hi == 0) p.delta[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] = dlt;
         }
-        dlt = half_swap_sum(KK == 4 ? (part[0] + part[2]) + (part[1] + part[KK - 1]) : part[0] + part[1]);
-        if (qvalid && hi == 0) p.delta[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] = dlt;
-    }
-    // (the row loads above are in flight while wave 0 reads the class rows)
-    if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, 0, sList, &sCount);  // first pass (usually the only one)
-    const QueryBits qb = make_query_bits(qf, (IDX && qvalid) ? p.posq[qrow] : qrow);
-    const float lse2 = (!qvalid || lse_row == -INFINITY) ? INFINITY : lse_row * LOG2E;
+        qb = make_query_bits(qf, qpos);
+        lse2 = (!qvalid || lse_row == -INFINITY) ? INFINITY : lse_row * LOG2E;
+    };
 
     f32x16 dq[DB];
 #pragma unroll
@@ -1026,13 +989,17 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
     // Sequences of more than MAX_LIST 64-key tiles are walked in several passes, each with a list of its own.
     const int nkt_total = (Sk + DQ_KT - 1) / DQ_KT;
     for (int kt_begin = 0;;) {
-        __syncthreads();
+        lds_barrier();
         const int n = sCount;
+        int entry = 0, next = 0;
         if (n > 0) {
-            int entry = __builtin_amdgcn_readfirstlane(sList[0]);
-            int next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
+            entry = __builtin_amdgcn_readfirstlane(sList[0]);
+            next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
     #pragma unroll
             for (int j = 0; j < NLOADS; ++j) issue_copy(j, entry >> 8, 0);
+        }
+        if (!LONG || kt_begin == 0) rows_arrived();  // (also where there is no tile: somebody needs delta)
+        if (n > 0) {
             wait_async();
             __syncthreads();
             for (int it = 0; it < n; ++it) {
@@ -1058,14 +1025,7 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
         char* dqp = (char*)p.dq.ptr + 2 * ((int64_t)b * p.dq.sb + (int64_t)qrow * p.dq.ss + (int64_t)h * p.dq.sh);
 #pragma unroll
         for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int grp = 0; grp < 4; ++grp) {
-                if (32 * db + 8 * grp >= p.d) break;
-                u32x2 w;
-                w[0] = T::pack2(dq[db][4 * grp + 0] * p.scale, dq[db][4 * grp + 1] * p.scale);
-                w[1] = T::pack2(dq[db][4 * grp + 2] * p.scale, dq[db][4 * grp + 3] * p.scale);
-                *(u32x2*)(dqp + (32 * db + 8 * grp + 4 * hi) * 2) = w;
-            }
+            store_block16<T>(dqp + 64 * db, p.d - 32 * db, hi, [&](int i) { return dq[db][i] * p.scale; });
     } else if (qvalid) {
         float* dqp = (float*)p.dq.ptr + ((int64_t)b * p.dq.sb + (int64_t)qrow * p.dq.ss + (int64_t)h * p.dq.sh);
 #pragma unroll

@@ -41,7 +41,7 @@ template <typename T, int D, int MODE, bool BIAS, bool LONG, int STREAMS>
 __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 3) void fwd_kernel(const AttnParams p) {
     static_assert(STREAMS == 1 || !LONG, "streams and passes are not combined");
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
-    constexpr int WAIT = COPY_WAIT<MODE, BIAS, LONG>;
+    constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
     __shared__ u32x4 sK_all[STREAMS][2][FWD_KT * NCH];
     __shared__ u32x4 sV_all[STREAMS][2][FWD_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf_all[STREAMS][2][FWD_KT];  // raw bitfields of the tile's keys
@@ -78,8 +78,6 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     const int h = hk * G + g;
     const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
 
-    if (wave == 0 && stream == 0) build_key_tile_list<STREAMS>(ws, p.num_n, Sk, lane, 0, sList, sCount);  // first pass (usually the only one)
-
     // ---- per-lane query state -------------------------------------------------------
     const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
     const int qrow = (slice < 0 ? 0 : slice) * 32 + l32;
@@ -94,8 +92,11 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             qreg[kk] = z;
         }
     }
-    const int64_t qf = (!DENSE && qvalid) ? p.bfq[(int64_t)b * p.bfq_sb + qrow] : 0;
-    const QueryBits qb = make_query_bits(qf, (IDX && qvalid) ? p.posq[qrow] : qrow);
+    int64_t qf = (!DENSE && qvalid) ? p.bfq[(int64_t)b * p.bfq_sb + qrow] : 0;
+    int qpos = (IDX && qvalid) ? p.posq[qrow] : qrow;
+    QueryBits qb = {};  // of qf and qpos, once they have arrived
+    // (the row loads above are in flight while the class rows are read and the first tile is on its way)
+    if (wave == 0 && stream == 0) build_key_tile_list<STREAMS>(ws, p.num_n, Sk, lane, 0, sList, sCount);  // first pass (usually the only one)
 
     f32x16 o[DB];
 #pragma unroll
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     // softmax state lives in registers and simply carries over.
     const int nkt_total = (Sk + FWD_KT - 1) / FWD_KT;
     for (int kt_begin = 0;;) {
-        __syncthreads();
+        lds_barrier();
         // With two streams, one takes the even tiles and the other the odd ones.  Past the end of its list a stream copies its
         // last tile again, for nobody to read or, where the other list is longer, with all classes cleared.
         const int n = sCount[stream], rounds = STREAMS > 1 ? max(n, sCount[STREAMS - 1 - stream]) : n;
@@ -445,6 +446,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     #pragma unroll
             for (int j = 0; j < NLOADS; ++j) issue_copy(j, entry >> 8, 0);
             wait_async();
+            arrived(qreg);
+            if (!LONG || kt_begin == 0) qb = make_query_bits(qf, qpos);
             __syncthreads();
             for (int it = 0; it < rounds; ++it) {
                 const int cur = it & 1;
@@ -503,22 +506,16 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
+            f32x16 x = o[db];
+            if constexpr (STREAMS > 1) {
 #pragma unroll
-            for (int grp = 0; grp < 4; ++grp) {
-                if (32 * db + 8 * grp >= p.d) break;
-                float x[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) x[i] = o[db][4 * grp + i];
-                if constexpr (STREAMS > 1) {
+                for (int grp = 0; grp < 4; ++grp) {
                     const f32x4 other = park[(4 * db + grp) * 64 + lane];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) x[i] = fmaf(x[i], mine, other[i] * theirs);
+                    for (int i = 0; i < 4; ++i) x[4 * grp + i] = fmaf(x[4 * grp + i], mine, other[i] * theirs);
                 }
-                u32x2 w;
-                w[0] = T::pack2(x[0] * inv, x[1] * inv);
-                w[1] = T::pack2(x[2] * inv, x[3] * inv);
-                *(u32x2*)(op + (32 * db + 8 * grp + 4 * hi) * 2) = w;
             }
+            store_block16<T>(op + 64 * db, p.d - 32 * db, hi, [&](int i) { return x[i] * inv; });
         }
     }
 }
