@@ -140,6 +140,18 @@ int fill_plan(bam::AttnParams& p, const char* who, const bam_plan* plan, int B, 
     if (plan->B != B || plan->Sq != Sq || plan->Sk != Sk)
         return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan was built for B = %d, Sq = %d, Sk = %d, not B = %d, Sq = %d, Sk = %d",
                     who, plan->B, plan->Sq, plan->Sk, B, Sq, Sk);
+    if (plan->rows != nullptr) {
+        if (p.mask_mode != bam::MASK_BITFIELD)
+            return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan: sorted rows are for bitfield attention only", who);
+        if (plan->rows_bits == nullptr || plan->rows_moved == nullptr || (reinterpret_cast<uintptr_t>(plan->rows_moved) & 3u) || (reinterpret_cast<uintptr_t>(plan->rows) & 3u) || (reinterpret_cast<uintptr_t>(plan->rows_bits) & 7u))
+            return fail(BAM_ERR_INVALID_ARGUMENT, "%s: plan: null or misaligned array of sorted rows", who);
+        if (bam::dkdv_far(p)) return BAM_OK;  // such rows are not gathered: from the flags alone
+        p.rows = plan->rows;
+        p.rows_bits = plan->rows_bits;
+        p.rows_sb = plan->rows_stride_b;
+        p.rows_moved = plan->rows_moved;
+        p.rows_known = plan->rows_known;
+    }
     if (plan->generation != 0) {  // laid out in the built-in array of bam_tile_plan_static
         int dev = -1;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices ||
@@ -318,7 +330,7 @@ extern "C" {
 
 const char* bam_last_error(void) { return g_error; }
 
-int bam_abi_version(void) { return 12; }
+int bam_abi_version(void) { return 13; }
 
 int bam_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                    int64_t flags_stride_m, int B, int S, void* stream) {
@@ -337,6 +349,7 @@ struct PlanLayout {
     int64_t fine_ss, fine_sb, order_sb, entry_sb, fine_off, order_off, entry_off, base_off, count_off, bytes;
     int64_t row_sn, row_sb, col_ss, col_sb, row_off, col_off, bytes_with_bits, tile_count_off, tile_order_off;
     int64_t group_count_off, group_order_off, row_workloads_off;
+    int64_t rows_sb, rows_off, rows_bits_off, rows_moved_off, bytes_with_rows;
 };
 PlanLayout plan_layout(int B, int Sq, int Sk) {
     const int64_t num_m = (Sq + 127) / 128, num_n = (Sk + 31) / 32, slots = 4 * num_m;
@@ -365,6 +378,12 @@ PlanLayout plan_layout(int B, int Sq, int Sk) {
     l.row_off = l.bytes;
     l.col_off = l.row_off + up(B * l.row_sb * 4, 256);
     l.bytes_with_bits = l.col_off + up(B * l.col_sb * 4, 256);
+    // the sorted rows of bam_tile_plan_sorted_counted
+    l.rows_sb = num_m * 128;
+    l.rows_off = l.bytes;
+    l.rows_bits_off = l.rows_off + up(B * l.rows_sb * 4, 256);
+    l.rows_moved_off = l.rows_bits_off + up(B * l.rows_sb * 8, 256);
+    l.bytes_with_rows = l.rows_moved_off + up(B * 4, 256);
     return l;
 }
 }  // namespace
@@ -372,6 +391,12 @@ PlanLayout plan_layout(int B, int Sq, int Sk) {
 int64_t bam_plan_workspace_bytes_rect(int B, int Sq, int Sk) {
     if (B <= 0 || Sq <= 0 || Sk <= 0 || (Sq + 31) / 32 > bam::MAX_PLAN_SLICES || Sk > BAM_MAX_SEQLEN) return 0;
     return plan_layout(B, Sq, Sk).bytes;
+}
+
+int bam_sorted_plan_workspace_bytes(int B, int S, int64_t* bytes) {
+    if (bytes == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_sorted_plan_workspace_bytes: null pointer");
+    *bytes = bam_plan_workspace_bytes_rect(B, S, S) == 0 ? 0 : plan_layout(B, S, S).bytes_with_rows;
+    return BAM_OK;
 }
 
 int64_t bam_plan_workspace_bytes(int B, int S) { return bam_plan_workspace_bytes_rect(B, S, S); }
@@ -384,9 +409,10 @@ int64_t bam_mask_plan_workspace_bytes(int B, int Sq, int Sk) {
 namespace {
 // Checks the workspace and lays the plan's arrays out in it.
 int place_plan(const char* who, void* workspace, int64_t workspace_bytes, int B, int Sq, int Sk, bam_plan* plan,
-               PlanLayout& l, bool with_bits = false) {
+               PlanLayout& l, bool with_bits = false, bool with_rows = false) {
     if (workspace == nullptr || plan == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
-    const int64_t need = with_bits ? bam_mask_plan_workspace_bytes(B, Sq, Sk) : bam_plan_workspace_bytes_rect(B, Sq, Sk);
+    int64_t need = with_bits ? bam_mask_plan_workspace_bytes(B, Sq, Sk) : bam_plan_workspace_bytes_rect(B, Sq, Sk);
+    if (with_rows) BAM_TRY(bam_sorted_plan_workspace_bytes(B, Sq, &need));
     if (need == 0) return fail(BAM_ERR_UNSUPPORTED, "%s: no plan is built for Sq = %d, Sk = %d", who, Sq, Sk);
     if (workspace_bytes < need)
         return fail(BAM_ERR_INVALID_ARGUMENT, "%s: workspace of %lld bytes, %lld needed", who, (long long)workspace_bytes,
@@ -406,7 +432,13 @@ int place_plan(const char* who, void* workspace, int64_t workspace_bytes, int B,
     plan->ds_count = (const int32_t*)(w + l.count_off);
     plan->ds_tile_order = (int64_t)B * ((Sk + 127) / 128) <= bam::MAX_RANKED ? (const int32_t*)(w + l.tile_order_off) : nullptr;
     plan->group_order = (int64_t)B * ((Sq + 127) / 128) <= bam::MAX_RANKED ? (const int32_t*)(w + l.group_order_off) : nullptr;
-    plan->row_workloads = (const int64_t*)(w + l.row_workloads_off);
+    plan->row_workloads = with_rows ? nullptr : (const int64_t*)(w + l.row_workloads_off);
+    plan->rows = with_rows ? (const int32_t*)(w + l.rows_off) : nullptr;
+    plan->rows_bits = with_rows ? (const int64_t*)(w + l.rows_bits_off) : nullptr;
+    plan->rows_stride_b = with_rows ? l.rows_sb : 0;
+    plan->rows_moved = with_rows ? (const int32_t*)(w + l.rows_moved_off) : nullptr;
+    plan->rows_known = BAM_ROWS_UNKNOWN;
+    plan->reserved = 0;
     plan->ds_workspace = nullptr;
     plan->ds_capacity = 0;
     plan->row_bits = with_bits ? (const uint32_t*)(w + l.row_off) : nullptr;
@@ -433,7 +465,7 @@ int number_pairs(const char* who, const bam_plan* plan, const PlanLayout& l, voi
                                            const_cast<int*>(plan->ds_tile_order), plan->order, plan->order_stride_b,
                                            (int*)((char*)workspace + l.group_count_off),
                                            const_cast<int*>(plan->group_order),
-                                           const_cast<int64_t*>(plan->row_workloads), count_host, count_tag,
+                                           const_cast<int64_t*>(plan->row_workloads), plan->rows_moved, count_host, count_tag,
                                            (hipStream_t)stream),
                     who);
 }
@@ -462,6 +494,27 @@ int bam_tile_plan_counted(const int64_t* bf, int64_t bf_stride_b, int8_t* flags,
                                            (int*)(w + l.count_off), B, S, (hipStream_t)stream),
                      "bam_tile_plan"));
     return number_pairs("bam_tile_plan", plan, l, workspace, count_host, count_tag, stream);
+}
+
+int bam_tile_plan_sorted_counted(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
+                                 int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
+                                 uint64_t* count_host, uint32_t count_tag, void* stream) {
+    const char* who = "bam_tile_plan_sorted_counted";
+    if (bf == nullptr || flags == nullptr || workspace == nullptr || plan == nullptr)
+        return fail(BAM_ERR_INVALID_ARGUMENT, "%s: null pointer", who);
+    if (B <= 0 || S <= 0) return fail(BAM_ERR_INVALID_ARGUMENT, "%s: B and S must be positive", who);
+    if (B > 65535) return fail(BAM_ERR_UNSUPPORTED, "%s: grid too large (B = %d, S = %d)", who, B, S);
+    if ((int64_t)B * ((S + 31) / 32) * ((S + 127) / 128) >= 1ll << 30)
+        return fail(BAM_ERR_UNSUPPORTED, "%s: too many pairs of slices and key tiles (B = %d, S = %d)", who, B, S);
+    PlanLayout l;
+    BAM_TRY(place_plan(who, workspace, workspace_bytes, B, S, S, plan, l, false, true));
+    char* w = (char*)workspace;
+    BAM_TRY(launched(bam::launch_tile_flags(bf, bf_stride_b, flags, flags_stride_b, flags_stride_m, B, S, (hipStream_t)stream), who));
+    BAM_TRY(launched(bam::launch_sorted_plan(bf, bf_stride_b, (int*)(w + l.rows_off), (int64_t*)(w + l.rows_bits_off), l.rows_sb,
+                                             (int*)(w + l.rows_moved_off), (uint8_t*)(w + l.fine_off), l.fine_sb, l.fine_ss, (int*)(w + l.order_off), l.order_sb,
+                                             (int*)(w + l.count_off), B, S, (hipStream_t)stream),
+                     who));
+    return number_pairs(who, plan, l, workspace, count_host, count_tag, stream);
 }
 
 int bam_tile_plan_static(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,

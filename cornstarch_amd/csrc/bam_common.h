@@ -70,6 +70,12 @@ __device__ __forceinline__ bool allow_bits(const QueryBits& q, unsigned klo, uns
 }
 
 // ---------------------------------------------------------------------------------
+// An entry of a plan's slice order: the slice, and whether its rows have been moved (AttnParams::rows).  -1: no slice.
+constexpr int ORDER_MOVED = 1 << 30;
+__device__ __forceinline__ int order_slice(int code) { return code < 0 ? -1 : code & ~ORDER_MOVED; }
+__device__ __forceinline__ bool order_moved(int code) { return code >= ORDER_MOVED; }
+
+// ---------------------------------------------------------------------------------
 // Element types: raw 16-byte operands, MFMA and float -> T conversion.
 struct BF16 {
     static __device__ __forceinline__ f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {

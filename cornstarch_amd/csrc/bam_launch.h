@@ -8,6 +8,7 @@ namespace bam {
 // Where the allow / deny decision of a (query, key) pair comes from.
 constexpr int MASK_BITFIELD = 0;  // bitfield rule, position = row / column number
 constexpr int MASK_INDEXED = 1;   // bitfield rule on gathered bitfields and explicit global positions
+constexpr int MASK_SORTED = 3;    // (dK/dV only) MASK_BITFIELD with the rows in the order of a plan, see AttnParams::rows
 constexpr int MASK_DENSE = 2;     // a materialized bool mask (B, Sq, Sk), one byte per pair (or none: all pairs allowed)
 
 // A workgroup lists its 64-key tiles (forward, dQ) or its 32-row slices (dK/dV) in LDS, this many at a time;
@@ -56,12 +57,20 @@ struct AttnParams {
     const int8_t* flags;       // (B, num_m, num_n)
     int64_t flags_sb, flags_sm;
     // Optional plan (null = none; every mask mode has a builder of its own).  fine: class 0 / 1 / 2 of every 32-row x 32-key
-    // tile, (B, 4 * num_m, fine_ss) bytes; order: the 32-row slices of each sequence sorted so that four
+    // tile, (B, 4 * num_m, fine_ss) bytes; order (see order_slice): the 32-row slices of each sequence sorted so that four
     // neighbours need about the same keys, heaviest first, (B, 4 * num_m) ints, -1 = no slice.
     const uint8_t* fine;
     int64_t fine_sb, fine_ss;
     const int* order;
     int64_t order_sb;
+    // Optional (plan of bitfield attention): the query rows sorted so that every slice holds rows that see the same keys.
+    // Slice s is then the rows rows[32 s ..] instead of 32 s ..; rows_bits are the bitfields in that order.  Both (B,
+    // Sq_rounded), entries past the last row Sq and 0.  null = natural order.
+    const int* rows;
+    const int64_t* rows_bits;
+    int64_t rows_sb;
+    int rows_known;            // BAM_ROWS_*: what the host knows of rows_moved
+    const int* rows_moved;     // (B): whether the sequence's rows are in another than their natural order
     // Optional hand-over of dS from the dK/dV kernel to the dQ kernel (needs the plan; null = none).  ds_entry:
     // number of every (slice, 128-key tile) pair that has work, (B, 4 * num_m, num_kt) ints, -1 = none.  ds_ws: one
     // 8 KiB record per (q head, pair), record (h, e) at ((h * ds_capacity + e) * 8 KiB); inside it four 2 KiB blocks,
@@ -134,6 +143,10 @@ int launch_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int
 int launch_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                      int64_t flags_stride_m, uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int* order,
                      int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream);
+// Sorted rows (see AttnParams::rows; S_rounded entries per sequence), and flags-free plan over them: fine and order.
+int launch_sorted_plan(const int64_t* bf, int64_t bf_stride_b, int* rows, int64_t* rows_bits, int64_t rows_sb, int* rows_moved, uint8_t* fine,
+                       int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B, int S,
+                       hipStream_t stream);
 int launch_materialize_mask(const int64_t* bf, int64_t bf_stride_b, uint8_t* out, int B, int S,
                             hipStream_t stream);
 int launch_flag_row_workloads(const int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m, int B, int num_m,
@@ -160,11 +173,12 @@ int launch_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stri
 // be null, and no order is written beyond MAX_RANKED tiles.  The same for the groups of four slices in the plan's slice
 // order (order, order_sb): group_count (B * num_m) scratch, group_order (B * num_m) = the groups by falling number of
 // 64-key tiles they visit.  row_workloads (num_m int64, or null): per 128-row block, the number of its 128 x 32 tiles
-// with an allowed pair, summed over the batch.  count_host (pinned host memory, or null): receives count_tag << 32 | count.
+// with an allowed pair, summed over the batch.  count_host (pinned host memory, or null): receives count_tag << 32 | count,
+// and with rows_moved (sorted rows, or null) in bits 31 and 30 whether rows of some sequence have been moved, or left.
 int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int B, int Sq, int Sk, int* entry,
                       int64_t entry_sb, int* tile_base, int* count, int* tile_count, int* tile_order, const int* order,
-                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, uint64_t* count_host,
-                      uint32_t count_tag, hipStream_t stream);
+                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, const int* rows_moved,
+                      uint64_t* count_host, uint32_t count_tag, hipStream_t stream);
 int launch_fwd(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_preprocess(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dkdv(const AttnParams& p, int dtype, hipStream_t stream);

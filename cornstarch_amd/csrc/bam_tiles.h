@@ -220,6 +220,14 @@ struct SliceStage {
         if ((THREADS * i) / NCH >= 32) return true;
         return (wave_first + THREADS * i) / NCH >= 32;
     }
+    // Which row of the 64-row tile this lane copies with instruction i, and that copy with an offset of the caller's (sorted
+    // rows: any row of the head; `setup` with a row stride of 0 leaves the offset inside a row in goff).
+    static __device__ __forceinline__ int row(int i, int tid) { return (tid + THREADS * i) / NCH; }
+    template <int WAIT>
+    __device__ __forceinline__ void issue_gather(int i, const u32x4& desc, unsigned voff, unsigned tile_lds) const {
+        if (EXACT || wave_first + THREADS * i < CHUNKS)
+            copy_b128<WAIT>(TileSrc{desc, 0u}, voff, tile_lds + (unsigned)(THREADS * i + wave_first) * 16u);
+    }
     // Copy instruction i from the first row of the slice it belongs to (see upper()).
     template <int WAIT>
     __device__ __forceinline__ void issue_from(int i, const TileSrc& slice, unsigned tile_lds) const {
@@ -244,16 +252,24 @@ __device__ __forceinline__ void arrived(u32x4 (&regs)[N]) {
 // with one, group `grp` takes the next four slices of the sorted order and every slice has a class row of its own.
 struct WaveSlices {
     int slice[4];             // -1: no slice (the wave idles through the key loop)
+    bool moved;               // the rows of the slices are those of AttnParams::rows
     const int8_t* cls_row[4]; // null where slice is -1
 };
 
+// The query row at a place of the slice order's slices: the place itself, or with sorted rows whatever row was sorted there.
+__device__ __forceinline__ int row_of_slot(const AttnParams& p, const WaveSlices& ws, int b, int slot, bool valid) {
+    return ws.moved && valid ? p.rows[(int64_t)b * p.rows_sb + slot] : slot;
+}
+
 __device__ __forceinline__ WaveSlices pick_wave_slices(const AttnParams& p, int b, int grp) {
     WaveSlices w;
+    w.moved = false;
     if (p.fine != nullptr) {
         const int* ord = p.order + (int64_t)b * p.order_sb + 4 * grp;
+        w.moved = order_moved(ord[0]);  // (a group has a first slice)
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-            w.slice[x] = ord[x];
+            w.slice[x] = order_slice(ord[x]);
             w.cls_row[x] = w.slice[x] >= 0
                                ? (const int8_t*)p.fine + (int64_t)b * p.fine_sb + (int64_t)w.slice[x] * p.fine_ss
                                : nullptr;

@@ -98,8 +98,9 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
 
     const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
     // column n of a dS block holds query row 8 * ((n & 15) >> 2) + 4 * (n >> 4) + (n & 3) of the slice
-    const int qrow = (slice < 0 ? 0 : slice) * 32 + 8 * ((l32 & 15) >> 2) + 4 * (l32 >> 4) + (l32 & 3);
-    const bool qvalid = slice >= 0 && qrow < Sq;
+    const int slot = (slice < 0 ? 0 : slice) * 32 + 8 * ((l32 & 15) >> 2) + 4 * (l32 >> 4) + (l32 & 3);
+    const bool qvalid = slice >= 0 && slot < Sq;
+    const int qrow = row_of_slot(p, ws, b, slot, qvalid);
 
     f32x16 dq[DB];
 #pragma unroll

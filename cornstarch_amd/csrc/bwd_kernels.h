@@ -11,6 +11,7 @@
 #pragma once
 #include "bam_common.h"
 #include "bam_launch.h"
+#include "../../include/bam_hip.h"
 #include "bam_tiles.h"
 #include <type_traits>
 
@@ -86,7 +87,9 @@ constexpr int DKDV_THREADS = 512;
 // the dQ kernel of bwd_dq_saved.h picks it up instead of recomputing S and dP.  Record and block layout: AttnParams.
 template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
-    constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE;
+    constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
+    constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
+    static_assert(!(SORTED && LONG), "no plan for so many rows");
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
     __shared__ u32x4 sK[128 * NCH];
@@ -96,7 +99,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     __shared__ __attribute__((aligned(16))) float sLse[2][DKDV_QT];      // natural-log lse of the rows
     __shared__ __attribute__((aligned(16))) float sDelta[2][DKDV_QT];
     __shared__ __attribute__((aligned(16))) int64_t sQbf[2][DKDV_QT];    // raw bitfields of the rows
-    __shared__ __attribute__((aligned(16))) int sQpos[2][DKDV_QT];       // their global positions (IDX only)
+    // their positions (ROW_POS).  SORTED: a tile's rows are gathered, so their numbers have to be here a tile earlier
+    __shared__ __attribute__((aligned(16))) int sQpos[SORTED ? 3 : 2][DKDV_QT];
     __shared__ __attribute__((aligned(16))) unsigned sWq[DKDV_THREADS / 64][5][32];  // per-wave rule constants
     // DENSE with packed mask bits: for the two slices of the tile, one word per key of the workgroup's 128 keys
     __shared__ unsigned sColBits[MODE == MASK_DENSE ? 2 : 1][2][MODE == MASK_DENSE ? 128 : 1];
@@ -133,6 +137,9 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         nt = code - b * p.num_kt;
     }
 
+    // With sorted rows there are two launches: this one is for the sequences whose rows have been moved, or for the others.
+    if ((SORTED || MODE == MASK_BITFIELD) && p.rows_moved != nullptr && (p.rows_moved[b] != 0) != SORTED) return;
+
     const int ns_total = (Sq + 31) >> 5;
     // ---- K, V of the tile -> LDS (once) ---------------------------------------------------
     {
@@ -147,7 +154,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     }
     const int key = nt * 128 + kg * 32 + l32;
     const bool kvalid = key < Sk;
-    const int64_t* bfrow = p.bfq + (int64_t)b * p.bfq_sb;  // bitfields of the query rows
+    // bitfields of the query rows
+    const int64_t* bfrow = SORTED ? p.rows_bits + (int64_t)b * p.rows_sb : p.bfq + (int64_t)b * p.bfq_sb;
     const int64_t kf = (!DENSE && kvalid) ? p.bfk[(int64_t)b * p.bfk_sb + key] : 0;
     int kpos = (IDX && kvalid) ? p.posk[key] : key;  // global position of this lane's key
     unsigned klo = (unsigned)(kf & 0xFFFFFFFFll);
@@ -204,12 +212,12 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 
     typedef SliceStage<D, DKDV_THREADS> Stage;
     constexpr int CPT = Stage::CPT;
-    // copy instructions per wave and tile: Q, dO, one of the four small rows and (IDX) the row positions
+    // copy instructions per wave and tile: Q, dO, one of the small rows and (IDX) the row positions
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0);
     static_assert(NLOADS <= 2 * KK, "one copy per MFMA of the S / dP phase");
     Stage stQ, stDO;
-    stQ.setup(2 * p.q.ss, p.d / 8, tid);
-    stDO.setup(2 * p.dout.ss, p.d / 8, tid);
+    stQ.setup(SORTED ? 0 : 2 * p.q.ss, p.d / 8, tid);
+    stDO.setup(SORTED ? 0 : 2 * p.dout.ss, p.d / 8, tid);
     const unsigned ldsQ = lds_addr(sQ), ldsDO = lds_addr(sDO);
     constexpr unsigned TILE_BYTES = DKDV_QT * NCH * 16;
     // small rows of a tile: lse, delta and the two halves of the 64 int64 bitfields, 64 dwords each;
@@ -218,12 +226,14 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     // (DENSE: rows 2 and 3 are the packed mask words of keys 0..63 / 64..127 of the tile, for the slice of the
     // copying wave's row stream; without packed bits, waves 2, 3, 6, 7 repeat lse / delta instead)
     const bool col_bits_on = DENSE && p.col_bits != nullptr;
-    const int small = (DENSE && !col_bits_on) ? (wave & 1) : (wave & 3);
+    // (SORTED: waves 4..7 copy the row numbers of the tile behind, row 4)
+    const int small = (DENSE && !col_bits_on) ? (wave & 1) : SORTED ? min(wave, 4) : (wave & 3);
     const unsigned ldsSmall = small == 0   ? lds_addr(sLse)
                               : small == 1 ? lds_addr(sDelta)
+                              : SORTED && small == 4 ? lds_addr(sQpos)
                               : DENSE      ? lds_addr(sColBits) + (unsigned)(st * 128 + (small - 2) * 64) * 4u
                                            : lds_addr(sQbf) + (small - 2) * 256u;
-    const unsigned smallBytes = small < 2 ? DKDV_QT * 4u : DENSE ? 2 * 128 * 4u : DKDV_QT * 8u;  // per buffer
+    const unsigned smallBytes = small < 2 || (SORTED && small == 4) ? DKDV_QT * 4u : DENSE ? 2 * 128 * 4u : DKDV_QT * 8u;  // per buffer
     // Where the copies of a tile read.  The scalar unit is shared by the whole compute unit, so the address
     // arithmetic is kept short: descriptors of the head in work are carried along and moved when the head changes, a slice
     // costs one 32-bit product.  The slice that holds the end of the sequence is copied like the others: its rows past the
@@ -243,6 +253,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             hv.small.init(p.col_bits + (int64_t)b * p.col_bits_sb + nt * 128 + (small - 2) * 64, p.col_bits_ss * 4, (Sq + 31) >> 5, 256);
         else
             hv.small.init(bfrow, 8, Sq, 8);
+        if (SORTED && small == 4) hv.small.init(p.rows + (int64_t)b * p.rows_sb, 4, p.Sq_rounded, 4);
         return hv;
     };
     auto next_head = [&](HeadViews& hv) {
@@ -258,6 +269,33 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     struct TileSource {
         TileSrc q[CPT], g[CPT], small, pos;
         unsigned small_voff, pos_voff;
+        unsigned q_voff[SORTED ? CPT : 1], g_voff[SORTED ? CPT : 1];
+    };
+    const unsigned q_rs = (unsigned)(2 * p.q.ss), g_rs = (unsigned)(2 * p.dout.ss);  // row strides in bytes
+    // SORTED: the row numbers of a tile (waves 4..7)
+    auto numbers_of = [&](TileSource& t, const HeadViews& hv, int row_lo, int row_hi) {
+        t.small = hv.small.at(row_lo);
+        t.small_voff = (unsigned)(lane * 4) + ((unsigned)((row_hi - row_lo - 32) * 4) & upper_lanes);
+    };
+    const int from_lo = __builtin_amdgcn_readfirstlane(small == 2 ? -1 : 0), from_hi = __builtin_amdgcn_readfirstlane(small == 3 ? -1 : 0),
+              from_aft = __builtin_amdgcn_readfirstlane(small == 4 ? -1 : 0);
+    // SORTED: the tile whose 64 row numbers are at pos; the rows past the last one are numbered Sq, beyond every descriptor.
+    // (rows below 2^17, strides below 2^24 and products below 2^31: 24-bit products give the offsets).  aft_lo, aft_hi: the
+    // slices of the tile behind it.
+    auto gathered_source = [&](const HeadViews& hv, const int* pos, int row_lo, int row_hi, int aft_lo, int aft_hi) {
+        TileSource t;
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            const unsigned r = (unsigned)pos[Stage::row(i, tid) & (DKDV_QT - 1)];
+            t.q[i].desc = hv.q.desc;
+            t.g[i].desc = hv.g.desc;
+            t.q_voff[SORTED ? i : 0] = __umul24(r, q_rs) + stQ.goff[i];
+            t.g_voff[SORTED ? i : 0] = __umul24(r, g_rs) + stDO.goff[i];
+        }
+        t.small = hv.small.at((row_lo & from_lo) | (row_hi & from_hi) | (aft_lo & from_aft));
+        const unsigned shift = (unsigned)((aft_hi - aft_lo - 32) * 4) & (unsigned)from_aft;
+        t.small_voff = small < 2 ? 4u * (unsigned)pos[lane] : (unsigned)(lane * 4) + (shift & upper_lanes);
+        return t;
     };
     // the 64-row tile made of the slices starting at rows row_lo (LDS rows 0..31) and row_hi (LDS rows 32..63)
     auto tile_source = [&](const HeadViews& hv, int row_lo, int row_hi) {
@@ -281,15 +319,19 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         return t;
     };
     // copy instruction j of a tile into buffer buf
-    auto issue_copy = [&](int j, const TileSource& t, int buf) {
-        if (j < CPT)
+    auto issue_copy = [&](int j, const TileSource& t, int buf, int pos_buf) {
+        if (SORTED && j < CPT)
+            stQ.template issue_gather<WAIT>(j, t.q[j].desc, t.q_voff[j], ldsQ + buf * TILE_BYTES);
+        else if (SORTED && j < 2 * CPT)
+            stDO.template issue_gather<WAIT>(j - CPT, t.g[j - CPT].desc, t.g_voff[j - CPT], ldsDO + buf * TILE_BYTES);
+        else if (j < CPT)
             stQ.template issue_from<WAIT>(j, t.q[j], ldsQ + buf * TILE_BYTES);
         else if (j < 2 * CPT)
             stDO.template issue_from<WAIT>(j - CPT, t.g[j - CPT], ldsDO + buf * TILE_BYTES);
         else if (j == 2 * CPT)
-            copy_b32<WAIT>(t.small, t.small_voff, ldsSmall + buf * smallBytes);
+            copy_b32<WAIT>(t.small, t.small_voff, ldsSmall + (SORTED ? (pos_buf & from_aft) | (buf & ~from_aft) : buf) * smallBytes);
         else  // 2 x 32 row positions; every wave writes the same values
-            copy_b32<WAIT>(t.pos, t.pos_voff, lds_addr(sQpos) + buf * (DKDV_QT * 4u));
+            copy_b32<WAIT>(t.pos, t.pos_voff, lds_addr(sQpos) + pos_buf * (DKDV_QT * 4u));
     };
 
     // One 64-row tile held in buffer cur against this wave's 32 keys; the wave's 32 rows sit at sequence
@@ -318,10 +360,11 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     };
     // ds_pos: position of the wave's slice in the slice list.
     // returns true when the wave has issued its two dS stores (they may stay in flight over the end of the iteration)
-    auto tile_step = [&](int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next) -> bool {
+    // pos_cur, pos_nxt: the buffers of the tile's positions and of those that are copied now
+    auto tile_step = [&](int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int pos_cur, int pos_nxt) -> bool {
         if (cls == 0) {
 #pragma unroll
-            for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, cur ^ 1);
+            for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, cur ^ 1, pos_nxt);
             return false;
         }
         const int ds_e = ds_base + ds_pos;
@@ -335,6 +378,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         f32x16 s, dp;
         {
             constexpr int NOP = 2 * KK, AHEAD = 3;  // MFMA j: S (j even) or dP (j odd), k-slice j / 2
+            constexpr int FIRST = SORTED ? (NOP - NLOADS < 4 ? NOP - NLOADS : 4) : 0;  // the copies start behind MFMA FIRST - 1
             u32x4 a[NOP], bb[NOP];
             a[0] = lds_read_chunk<D>(tQ, qr + l32, hi);  // the operands of the first MFMA go first
             bb[0] = KV_REGS ? kfrag[0] : lds_read_chunk<D>(sK, 32 * kg + l32, hi);
@@ -362,7 +406,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                     dp = T::mfma(a[j], bb[j], dp);
                 else
                     s = T::mfma(a[j], bb[j], j < 2 ? zero16 : s);
-                if (j < NLOADS) issue_copy(j, next, cur ^ 1);
+                if (j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, cur ^ 1, pos_nxt);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -378,7 +422,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             const int64_t col = (int64_t)b * p.bias_sb + (int64_t)h_cur * p.bias_sh + key;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const int row = myrow0 + 8 * (i >> 2) + 4 * hi + (i & 3);
+                const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
+                const int row = SORTED ? sQpos[pos_cur][qr + r] : myrow0 + r;
                 float bv = 0.f;
                 if (kvalid && row < Sq) bv = load_bias1<T>(p.bias, col + (int64_t)row * p.bias_sm, p.bias_f32 != 0);
                 s[i] = fmaf(s[i], p.scale, bv);
@@ -415,8 +460,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             const unsigned flo = __builtin_amdgcn_readfirstlane(mlo), fhi = __builtin_amdgcn_readfirstlane(mhi);
             bool uniform = (mlo == flo) & (mhi == fhi);
             int qpos0 = myrow0;  // position of this wave's first row
-            if (IDX) {              // ... and the 32 rows must sit at consecutive positions
-                const int rel0 = sQpos[cur][qr + l32] - l32;
+            if (ROW_POS) {          // ... and the 32 rows must sit at consecutive positions
+                const int rel0 = sQpos[pos_cur][qr + l32] - l32;
                 qpos0 = __builtin_amdgcn_readfirstlane(rel0);
                 uniform &= rel0 == qpos0;
             }
@@ -431,7 +476,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 // rule constants of this wave's 32 rows, derived once per row (lane r < 32 takes row r) and
                 // handed to all lanes through a wave-private LDS scratch
                 {
-                    const QueryBits qb = make_query_bits(mine, IDX ? sQpos[cur][qr + l32] : myrow0 + l32);
+                    const QueryBits qb = make_query_bits(mine, ROW_POS ? sQpos[pos_cur][qr + l32] : myrow0 + l32);
                     if (hi == 0) {
                         sWq[wave][0][l32] = qb.a_lo;
                         sWq[wave][1][l32] = qb.a_hi;
@@ -525,10 +570,27 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             int g_cur = 0, g_nxt = 0, r_nxt = 0, r_cur = 0;
             HeadViews hv_nxt = head_views(hk * G);
             int e_lo = __builtin_amdgcn_readfirstlane(entry_lo(0)), e_hi = __builtin_amdgcn_readfirstlane(entry_hi(0));
-            {
+            int a_lo = 0, a_hi = 0;  // SORTED: the entries of the tile after next
+            auto after = [&](int r) { return r + 1 == npairs ? 0 : r + 1; };
+            if constexpr (!SORTED) {
                 const TileSource first = tile_source(hv_nxt, (e_lo >> 8) * 32, (e_hi >> 8) * 32);
 #pragma unroll
-                for (int j = 0; j < NLOADS; ++j) issue_copy(j, first, 0);
+                for (int j = 0; j < NLOADS; ++j) issue_copy(j, first, 0, 0);
+            } else {  // the row numbers of the first two tiles, then the first tile
+                const int r1 = after(0);
+                const int lo1 = (__builtin_amdgcn_readfirstlane(entry_lo(r1)) >> 8) * 32, hi1 = (__builtin_amdgcn_readfirstlane(entry_hi(r1)) >> 8) * 32;
+                if (small == 4) {
+                    TileSource numbers;
+                    numbers_of(numbers, hv_nxt, (e_lo >> 8) * 32, (e_hi >> 8) * 32);
+                    issue_copy(2 * CPT, numbers, 0, 0);
+                }
+                wait_async();
+                __syncthreads();
+                const TileSource first = gathered_source(hv_nxt, sQpos[0], (e_lo >> 8) * 32, (e_hi >> 8) * 32, lo1, hi1);
+#pragma unroll
+                for (int j = 0; j < NLOADS; ++j) issue_copy(j, first, 0, 1);
+                a_lo = __builtin_amdgcn_readfirstlane(entry_lo(after(r1)));
+                a_hi = __builtin_amdgcn_readfirstlane(entry_hi(after(r1)));
             }
             auto advance = [&]() {
                 if (++r_nxt == npairs) {
@@ -547,23 +609,36 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 __syncthreads();
             }
             load_kv_operands();
+            int pos_cur = 0;  // SORTED: it % 3
             for (int it = 0; it < total; ++it) {
                 const int cur = it & 1;
-                // pair after next: its list entries are requested now and picked up at the end of the iteration
-                const int r_aft = r_nxt + 1 == npairs ? 0 : r_nxt + 1;
-                const int a_lo = entry_lo(r_aft), a_hi = entry_hi(r_aft);
-                const TileSource next = tile_source(hv_nxt, (n_lo >> 8) * 32, (n_hi >> 8) * 32);
+                // pair after next (SORTED: the one behind it): its list entries are requested now and picked up at the end of
+                // the iteration
+                const int r_req = SORTED ? after(after(r_nxt)) : after(r_nxt);
+                const int x_lo = entry_lo(r_req), x_hi = entry_hi(r_req);
+                TileSource next;
+                const int p1 = SORTED ? (pos_cur == 2 ? 0 : pos_cur + 1) : cur ^ 1, p2 = SORTED ? (pos_cur == 0 ? 2 : pos_cur - 1) : cur ^ 1;
+                if constexpr (SORTED) {
+                    next = gathered_source(hv_nxt, sQpos[p1], (n_lo >> 8) * 32, (n_hi >> 8) * 32, (a_lo >> 8) * 32, (a_hi >> 8) * 32);
+                } else {
+                    next = tile_source(hv_nxt, (n_lo >> 8) * 32, (n_hi >> 8) * 32);
+                }
                 const int mine = st ? e_hi : e_lo;
                 fetch_bias_key(hk * G + g_cur);
-                const bool stored = tile_step(cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur,
-                                              (mine >> 8) * 32, n - 2 - 2 * r_cur + st, next);
+                const bool stored = tile_step(cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur, (mine >> 8) * 32, n - 2 - 2 * r_cur + st,
+                                              next, SORTED ? pos_cur : cur, p2);
                 g_cur = g_nxt;
                 r_cur = r_nxt;
                 e_lo = n_lo;
                 e_hi = n_hi;
                 advance();
-                n_lo = __builtin_amdgcn_readfirstlane(a_lo);
-                n_hi = __builtin_amdgcn_readfirstlane(a_hi);
+                n_lo = SORTED ? a_lo : __builtin_amdgcn_readfirstlane(x_lo);
+                n_hi = SORTED ? a_hi : __builtin_amdgcn_readfirstlane(x_hi);
+                if (SORTED) {
+                    a_lo = __builtin_amdgcn_readfirstlane(x_lo);
+                    a_hi = __builtin_amdgcn_readfirstlane(x_hi);
+                    pos_cur = p1;
+                }
                 // the copies of the next tile must have landed; the two dS stores, issued after them, may stay in flight
                 if (SAVE && stored)
                     asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
@@ -680,8 +755,9 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
     const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
 
     const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
-    const int qrow = (slice < 0 ? 0 : slice) * 32 + l32;
-    const bool qvalid = slice >= 0 && qrow < Sq;
+    const int slot = (slice < 0 ? 0 : slice) * 32 + l32;
+    const bool qvalid = slice >= 0 && slot < Sq;
+    const int qrow = row_of_slot(p, ws, b, slot, qvalid);
     u32x4 qreg[KK], greg[KK];
     {
         const char* qp = (const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)qrow * p.q.ss + (int64_t)h * p.q.sh);
@@ -1044,6 +1120,11 @@ __global__ __launch_bounds__(DQ_THREADS, D > 64 || BIAS_FORM == BIAS_TILES ? 2 :
 
 
 // ---------------------------------------------------------------------------------------
+// Sorted rows: dK/dV of sequences whose rows have been moved and of the others are different instantiations.  As long as the host
+// has not seen the plan builder's count word both are launched, and the workgroups of the wrong one end at once (a launch of 2048
+// such workgroups: 16 us, their LDS keeps them from running beside each other).
+inline bool rows_may_be_moved(const AttnParams& p) { return p.rows != nullptr && p.rows_known != BAM_ROWS_LEFT; }
+inline bool rows_may_be_left(const AttnParams& p) { return p.rows == nullptr || p.rows_known != BAM_ROWS_MOVED; }
 template <typename T, int D, bool BIAS, bool LONG>
 static int launch_dkdv_b(const AttnParams& p, hipStream_t stream) {
     const int blocks = p.num_kt * p.B * p.Hkv;  // one workgroup per 128-key tile
@@ -1051,8 +1132,14 @@ static int launch_dkdv_b(const AttnParams& p, hipStream_t stream) {
         hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     else if (p.mask_mode == MASK_DENSE)
         hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_DENSE, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-    else
-        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+    else {
+        if constexpr (!LONG) {  // (beyond, there are no sorted rows)
+            if (rows_may_be_moved(p))
+                hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_SORTED, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+        }
+        if (LONG || rows_may_be_left(p))
+            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+    }
     return (int)hipGetLastError();
 }
 template <typename T, int D, bool BIAS>
@@ -1062,8 +1149,12 @@ static int launch_dkdv_save_b(const AttnParams& p, hipStream_t stream) {
         hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     else if (p.mask_mode == MASK_DENSE)
         hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_DENSE, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-    else
-        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+    else {
+        if (rows_may_be_moved(p))
+            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_SORTED, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+        if (rows_may_be_left(p))
+            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+    }
     return (int)hipGetLastError();
 }
 template <typename T, int D, int BIAS, bool LONG>

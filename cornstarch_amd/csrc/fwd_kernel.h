@@ -80,8 +80,9 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
 
     // ---- per-lane query state -------------------------------------------------------
     const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
-    const int qrow = (slice < 0 ? 0 : slice) * 32 + l32;
-    const bool qvalid = slice >= 0 && qrow < Sq;
+    const int slot = (slice < 0 ? 0 : slice) * 32 + l32;
+    const bool qvalid = slice >= 0 && slot < Sq;
+    const int qrow = row_of_slot(p, ws, b, slot, qvalid);
     u32x4 qreg[KK];
     {
         const char* qp = (const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)qrow * p.q.ss + (int64_t)h * p.q.sh);

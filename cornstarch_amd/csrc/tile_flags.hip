@@ -37,7 +37,7 @@ constexpr int FLAG_MAX_BLOCKS_X = 64;  // workgroups per 128-row block; longer r
 constexpr int RANKED_PER_GROUP = 64;
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 template <typename FillFn>
-__device__ __forceinline__ void slice_order_ranked(FillFn fill, int ns, int slots, int part, int* __restrict__ order_row) {
+__device__ __forceinline__ void slice_order_ranked(FillFn fill, int ns, int slots, int part, int* __restrict__ order_row, int mark = 0) {
     __shared__ __attribute__((aligned(16))) unsigned long long sk[2 * 256];
     const int tid = threadIdx.x, s = part * RANKED_PER_GROUP + (tid >> 2), sub = tid & 3;
     unsigned long long my1 = 0, my2 = 0;
@@ -67,7 +67,7 @@ __device__ __forceinline__ void slice_order_ranked(FillFn fill, int ns, int slot
     rank += __shfl_xor(rank, 2);
     if (sub != 0) return;
     if (s < ns)
-        order_row[rank] = s;
+        order_row[rank] = s | mark;
     else if (s < slots)
         order_row[s] = -1;
 }
@@ -133,7 +133,7 @@ struct GatheredRows {
     const int* positions;
     __device__ __forceinline__ void get(int i, int64_t& f, int& pos) const {
         f = bits[i];
-        pos = positions[i];
+        pos = positions != nullptr ? positions[i] : i;
     }
 };
 struct IndexedRows {
@@ -453,8 +453,8 @@ template <bool GATHER>
 __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
     const int64_t* __restrict__ bf, int64_t bf_sb, int L, const int64_t* __restrict__ idx_q, const int64_t* __restrict__ idx_k,
     int64_t* __restrict__ qbits, int64_t qbits_sb, int64_t* __restrict__ kbits, int64_t kbits_sb, int* __restrict__ qpos,
-    int* __restrict__ kpos, int Sq, int Sk, int num_n, uint8_t* __restrict__ fine, int64_t fine_sb, int64_t fine_ss,
-    int* __restrict__ order, int64_t order_sb, int flag_blocks_x, int* __restrict__ pair_count) {
+    int64_t qpos_sb, int* __restrict__ kpos, int Sq, int Sk, int num_n, uint8_t* __restrict__ fine, int64_t fine_sb,
+    int64_t fine_ss, int* __restrict__ order, int64_t order_sb, int flag_blocks_x, int flag_groups, const int* __restrict__ rows_moved, int* __restrict__ pair_count) {
     typedef typename std::conditional<GATHER, IndexedRows, GatheredRows>::type Rows;
     const int b = blockIdx.z;
     Rows q_rows, k_rows;
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
         q_rows = IndexedRows{bf + (int64_t)b * bf_sb, idx_q, L};
         k_rows = IndexedRows{bf + (int64_t)b * bf_sb, idx_k, L};
     } else {
-        q_rows = GatheredRows{qbits + (int64_t)b * qbits_sb, qpos};
+        q_rows = GatheredRows{qbits + (int64_t)b * qbits_sb, qpos + (int64_t)b * qpos_sb};
         k_rows = GatheredRows{kbits + (int64_t)b * kbits_sb, kpos};
     }
     if (pair_count != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) *pair_count = 0;
@@ -471,27 +471,32 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
         const int ns = (Sq + 31) / 32, slots = 4 * (int)gridDim.y;
         if (part * RANKED_PER_GROUP < slots)
             slice_order_ranked([&](int base, unsigned long long* sk) { slice_keys_chunk_indexed(q_rows, Sq, ns, base, sk); }, ns,
-                               slots, part, order + (int64_t)b * order_sb);
+                               slots, part, order + (int64_t)b * order_sb,
+                               rows_moved != nullptr && rows_moved[b] != 0 ? ORDER_MOVED : 0);
         return;
     }
     __shared__ int64_t q_bits[BLOCK_M];
     __shared__ int q_pos[BLOCK_M];
-    __shared__ __attribute__((aligned(8))) uint8_t s_out[4][FLAG_COLS_PER_BLOCK];
+    __shared__ __attribute__((aligned(8))) uint8_t s_out_buf[2][4][FLAG_COLS_PER_BLOCK];
     const int m = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
     // lanes [0, 32) own the columns of the wave's first tile, lanes [32, 64) those of the second
     static_assert(FLAG_TILES_PER_WAVE == 2, "each half of a wave takes one tile");
-    const int n = blockIdx.x * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + half, j = n * BLOCK_N + l32;
     int64_t kf = 0;
     int kp = 0;
-    if (j < Sk) {
-        k_rows.get(j, kf, kp);
-        if (GATHER && m == 0) {
-            kbits[(int64_t)b * kbits_sb + j] = kf;
-            if (b == 0) kpos[j] = kp;
+    auto request_keys = [&](int bx) {
+        const int j = (bx * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + half) * BLOCK_N + l32;
+        kf = 0;
+        kp = 0;
+        if (j < Sk) {
+            k_rows.get(j, kf, kp);
+            if (GATHER && m == 0) {
+                kbits[(int64_t)b * kbits_sb + j] = kf;
+                if (b == 0) kpos[j] = kp;
+            }
         }
-    }
-    if (tid < 4 * FLAG_COLS_PER_BLOCK) s_out[0][tid] = 0;
+    };
+    request_keys(blockIdx.x);
     if (tid < BLOCK_M) {
         const int i = m * BLOCK_M + tid;
         int64_t f = 0;
@@ -508,45 +513,75 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
     }
     __syncthreads();
     const int64_t M = (((int64_t)1) << 62) - 1;
-    const int64_t kb = kf & M;
-    int cnt[4];
+    unsigned slice_starts[4];
+    bool one_run = (m + 1) * BLOCK_M <= Sq;  // every slice is one run of rows at consecutive positions
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const int r = 32 * w + l32, before = 32 * w + max(l32, 1) - 1;
-        unsigned starts = (unsigned)__ballot(l32 == 0 || q_bits[r] != q_bits[before] || q_pos[r] != q_pos[before] + 1);
-        int c = 0;
-        while (starts != 0u) {  // wave-uniform
-            const int a = __builtin_ctz(starts);
-            starts &= starts - 1u;
-            const int e = starts != 0u ? __builtin_ctz(starts) : 32;  // the run is rows [a, e) of the slice
-            const int64_t qf = q_bits[32 * w + a], qb = qf & M, p0 = q_pos[32 * w + a];
-            if (qf & 1) {  // text rows: those at or after the key's position
-                const int64_t seen = p0 + (e - a) - (kp > p0 ? (int64_t)kp : p0);
-                c += (qb & kb) != 0 && seen > 0 ? (int)seen : 0;
-            } else {
-                c += (qb == kb && qb != 0) ? e - a : 0;
+        slice_starts[w] = (unsigned)__ballot(l32 == 0 || q_bits[r] != q_bits[before] || q_pos[r] != q_pos[before] + 1);
+        one_run &= slice_starts[w] == 1u;
+    }
+    // A workgroup takes the groups of eight column tiles blockIdx.x, blockIdx.x + flag_blocks_x, ...
+    int it = 0;
+    for (int bx = blockIdx.x; bx < flag_groups; bx += flag_blocks_x, ++it) {
+        uint8_t (*s_out)[FLAG_COLS_PER_BLOCK] = s_out_buf[it & 1];
+        if (it > 0) request_keys(bx);
+        const int n = bx * FLAG_COLS_PER_BLOCK + wave * FLAG_TILES_PER_WAVE + half, col = wave * FLAG_TILES_PER_WAVE + half;
+        const int64_t kb = kf & M;
+        // keys of one bitfield at consecutive positions, all of them there: with such rows the classes follow from the ends
+        const int64_t k0 = __shfl(kf, lane & 32);
+        const int p0 = __shfl(kp, lane & 32);
+        const bool closed = one_run && (__all((kf == k0 && kp == p0 + l32 && (n + 1) * BLOCK_N <= Sk)) != 0);
+        if (closed) {
+            if (l32 < 4) {
+                const int64_t qf = q_bits[32 * l32], qb = qf & M, r0 = q_pos[32 * l32];
+                const int64_t first = p0, last = (int64_t)p0 + BLOCK_N - 1;
+                uint8_t c;
+                if (qf & 1)
+                    c = (qb & kb) == 0 || r0 + 31 < first ? 0 : r0 >= last ? 2 : 1;
+                else
+                    c = qb == kb && qb != 0 ? 2 : 0;
+                s_out[l32][col] = c;
+            }
+        } else {
+            int cnt[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                unsigned starts = slice_starts[w];
+                int c = 0;
+                while (starts != 0u) {  // wave-uniform
+                    const int a = __builtin_ctz(starts);
+                    starts &= starts - 1u;
+                    const int e = starts != 0u ? __builtin_ctz(starts) : 32;  // the run is rows [a, e) of the slice
+                    const int64_t qf = q_bits[32 * w + a], qb = qf & M, first = q_pos[32 * w + a];
+                    if (qf & 1) {  // text rows: those at or after the key's position
+                        const int64_t seen = first + (e - a) - (kp > first ? (int64_t)kp : first);
+                        c += (qb & kb) != 0 && seen > 0 ? (int)seen : 0;
+                    } else {
+                        c += (qb == kb && qb != 0) ? e - a : 0;
+                    }
+                }
+                cnt[w] = c;
+            }
+#pragma unroll
+            for (int off = 16; off > 0; off >>= 1)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) cnt[w] += __shfl_xor(cnt[w], off);
+            if (l32 == 0) {
+                const int cols_in_range = max(0, min(BLOCK_N, Sk - n * BLOCK_N));
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const int rows = max(0, min(32, Sq - (m * BLOCK_M + 32 * w)));
+                    s_out[w][col] = (uint8_t)(cnt[w] == 0 ? 0 : cnt[w] == rows * cols_in_range ? 2 : 1);
+                }
             }
         }
-        cnt[w] = c;
-    }
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) cnt[w] += __shfl_xor(cnt[w], off);
-    if (l32 == 0 && n < num_n) {
-        const int cols_in_range = min(BLOCK_N, Sk - n * BLOCK_N), col = wave * FLAG_TILES_PER_WAVE + half;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int rows = max(0, min(32, Sq - (m * BLOCK_M + 32 * w)));
-            s_out[w][col] = (uint8_t)(cnt[w] == 0 ? 0 : cnt[w] == rows * cols_in_range ? 2 : 1);
+        __syncthreads();
+        if (tid < 4) {
+            static_assert(FLAG_COLS_PER_BLOCK == 8, "one 64-bit word per row");
+            *(unsigned long long*)(fine + (int64_t)b * fine_sb + (int64_t)(4 * m + tid) * fine_ss + bx * FLAG_COLS_PER_BLOCK) =
+                *(const unsigned long long*)s_out[tid];
         }
-    }
-    __syncthreads();
-    const int n0 = blockIdx.x * FLAG_COLS_PER_BLOCK;
-    if (tid < 4) {
-        static_assert(FLAG_COLS_PER_BLOCK == 8, "one 64-bit word per row");
-        *(unsigned long long*)(fine + (int64_t)b * fine_sb + (int64_t)(4 * m + tid) * fine_ss + n0) =
-            *(const unsigned long long*)s_out[tid];
     }
 }
 
@@ -555,16 +590,17 @@ int launch_indexed_plan(const int64_t* bf, int64_t bf_sb, int L, const int64_t* 
                         int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B,
                         hipStream_t stream) {
     const int num_m = (Sq + BLOCK_M - 1) / BLOCK_M, num_n = (Sk + BLOCK_N - 1) / BLOCK_N;
-    const int flag_blocks_x = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
+    const int flag_groups = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
+    const int flag_blocks_x = min(flag_groups, FLAG_MAX_BLOCKS_X);
     dim3 grid(flag_blocks_x + 1, num_m, B);
     if (idx_q != nullptr)
         hipLaunchKernelGGL(indexed_plan_kernel<true>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_sb, L, idx_q, idx_k, qbits,
-                           qbits_sb, kbits, kbits_sb, qpos, kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb,
-                           flag_blocks_x, pair_count);
+                           qbits_sb, kbits, kbits_sb, qpos, (int64_t)0, kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb,
+                           flag_blocks_x, flag_groups, (const int*)nullptr, pair_count);
     else
         hipLaunchKernelGGL(indexed_plan_kernel<false>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_sb, L, idx_q, idx_k, qbits,
-                           qbits_sb, kbits, kbits_sb, qpos, kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb,
-                           flag_blocks_x, pair_count);
+                           qbits_sb, kbits, kbits_sb, qpos, (int64_t)0, kpos, Sq, Sk, num_n, fine, fine_sb, fine_ss, order, order_sb,
+                           flag_blocks_x, flag_groups, (const int*)nullptr, pair_count);
     return (int)hipGetLastError();
 }
 
@@ -796,7 +832,7 @@ __global__ __launch_bounds__(DS_NUM_THREADS) void ds_entries_kernel(const uint8_
         const int* ord = order + (int64_t)b * order_sb + 4 * grp;
         const uint8_t* rows[4];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) rows[x] = ord[x] >= 0 ? fine + (int64_t)b * fine_sb + (int64_t)ord[x] * fine_ss : nullptr;
+        for (int x = 0; x < 4; ++x) rows[x] = ord[x] >= 0 ? fine + (int64_t)b * fine_sb + (int64_t)order_slice(ord[x]) * fine_ss : nullptr;
         int visits = 0;
         for (int kt = tid; 2 * kt < num_n; kt += DS_NUM_THREADS) {
             unsigned any = 0;
@@ -870,11 +906,22 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__
                                                          const int* __restrict__ group_count, int n_groups,
                                                          int* __restrict__ group_order, const int* __restrict__ count,
                                                          unsigned long long* __restrict__ count_host,
-                                                         unsigned long long count_tag) {
+                                                         unsigned long long count_tag, const int* __restrict__ rows_moved, int B) {
     __shared__ __attribute__((aligned(16))) int s_cnt[DS_MAX_ORDERED_TILES];
     const int tid = threadIdx.x;
-    if (count_host != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0)
-        __hip_atomic_store(count_host, count_tag | (unsigned)*count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (count_host != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid < 64) {
+        unsigned moved = 0;  // with sorted rows: whether some sequence's rows have been moved (bit 31), or left (bit 30)
+        if (rows_moved != nullptr) {
+            int some = 0, left = 0;
+            for (int b = tid; b < B; b += 64) {
+                some |= rows_moved[b] != 0;
+                left |= rows_moved[b] == 0;
+            }
+            moved = (__any(some) ? 1u << 31 : 0u) | (__any(left) ? 1u << 30 : 0u);
+        }
+        if (tid == 0)
+            __hip_atomic_store(count_host, count_tag | moved | (unsigned)*count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     if (blockIdx.y == 1) {
         tile_count = group_count;
         n_tiles = n_groups;
@@ -995,7 +1042,7 @@ __global__ __launch_bounds__(SMALL_PLAN_THREADS) void small_plan_kernel(
             unsigned any = 0;
 #pragma unroll
             for (int x = 0; x < 4; ++x)
-                if (ord[x] >= 0) any |= *(const uint16_t*)(fine + (int64_t)b * fine_sb + (int64_t)ord[x] * fine_ss + 2 * kt);
+                if (ord[x] >= 0) any |= *(const uint16_t*)(fine + (int64_t)b * fine_sb + (int64_t)order_slice(ord[x]) * fine_ss + 2 * kt);
             if ((any & valid) != 0) atomicAdd(&s_cnt[g], 1);
         }
         __syncthreads();
@@ -1026,8 +1073,8 @@ __global__ __launch_bounds__(SMALL_PLAN_THREADS) void small_plan_kernel(
 
 int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int B, int Sq, int Sk, int* entry,
                       int64_t entry_sb, int* tile_base, int* count, int* tile_count, int* tile_order, const int* order,
-                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, uint64_t* count_host,
-                      uint32_t count_tag, hipStream_t stream) {
+                      int64_t order_sb, int* group_count, int* group_order, int64_t* row_workloads, const int* rows_moved,
+                      uint64_t* count_host, uint32_t count_tag, hipStream_t stream) {
     const int num_m = (Sq + BLOCK_M - 1) / BLOCK_M;
     const int slots = 4 * num_m, nkt = (Sk + 127) / 128, num_n = (Sk + BLOCK_N - 1) / BLOCK_N;
     const int n_tiles = nkt * B, n_groups = num_m * B;
@@ -1050,7 +1097,7 @@ int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int
         const int nt = tile_order != nullptr ? n_tiles : 0, ng = group_order != nullptr ? n_groups : 0;
         hipLaunchKernelGGL(tile_order_kernel, dim3(max(1, (max(nt, ng) + 63) / 64), group_order != nullptr ? 2 : 1), dim3(256), 0,
                            stream, tile_count, nt, tile_order, group_count, ng, group_order, count,
-                           (unsigned long long*)count_host, (unsigned long long)count_tag << 32);
+                           (unsigned long long*)count_host, (unsigned long long)count_tag << 32, rows_moved, B);
     }
     return (int)hipGetLastError();
 }
@@ -1079,6 +1126,119 @@ int launch_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int6
     hipLaunchKernelGGL(tile_flags_kernel<true>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_stride_b, flags,
                        flags_stride_b, flags_stride_m, S, num_n, fine, fine_sb, fine_ss, order, order_sb, flag_blocks_x,
                        flag_groups, pair_count);
+    return (int)hipGetLastError();
+}
+
+// Sorts the rows of every sequence (whose slices are mixed enough) for launch_sorted_plan: text rows by position, then the modality rows grouped by their
+// bitfield, by position inside a group, then padding.  A counting sort over 64 classes; different bitfields may share a class (only
+// the packing of the slices suffers).  A workgroup places 1024 rows; it counts the classes of all rows for itself (512 KiB of
+// bitfields out of L2 for 65536 rows, eight loads in flight per thread) instead of waiting for the others.
+// Rows are only moved where at least one slice in SORT_MIXED holds text and modality rows: dK/dV gathers moved rows one by one,
+// which costs it 3 %.  Training step, 32 / 8 heads, D 128, natural -> sorted: 65536 tokens, 200 segments (20 % of the slices
+// mixed) 64.3 -> 48.2 ms; 8192 tokens, 30 segments (23 %) 1.87 -> 1.68 ms, 4 segments (3 %) 1.717 -> 1.722 ms; 16384 tokens, 4
+// segments (1.6 %) 7.36 -> 7.46 ms.
+constexpr int SORT_CHUNK = 1024, SORT_CLASSES = 64, SORT_MIXED = 32;
+__device__ __forceinline__ int sort_class(int64_t f) {
+    const uint64_t bits = (uint64_t)f & ((1ull << 62) - 1ull);
+    if (bits & 1) return 0;
+    if (bits == 0) return SORT_CLASSES - 1;
+    if ((bits & (bits - 1)) == 0) return 1 + (__ffsll((long long)bits) - 1) % (SORT_CLASSES - 2);
+    return 1 + (int)((bits * 0x9E3779B97F4A7C15ull) >> 40) % (SORT_CLASSES - 2);
+}
+__global__ __launch_bounds__(SORT_CHUNK) void sort_rows_kernel(const int64_t* __restrict__ bf, int64_t bf_sb, int S, int S_rounded,
+                                                              int* __restrict__ rows, int64_t* __restrict__ rows_bits,
+                                                              int64_t rows_sb, int* __restrict__ rows_moved,
+                                                              int* __restrict__ pair_count) {
+    __shared__ int s_mixed;
+    __shared__ int s_total[SORT_CLASSES], s_before[SORT_CLASSES], s_base[SORT_CLASSES];
+    __shared__ int s_wave[SORT_CHUNK / 64][SORT_CLASSES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.y;
+    const int first = blockIdx.x * SORT_CHUNK;
+    if (pair_count != nullptr && blockIdx.x == 0 && b == 0 && tid == 0) *pair_count = 0;
+    const int64_t* row = bf + (int64_t)b * bf_sb;
+    if (tid < SORT_CLASSES) s_total[tid] = s_before[tid] = 0;
+    if (tid == 0) s_mixed = 0;
+    s_wave[wave][lane] = 0;
+    __syncthreads();
+    int mixed = 0;  // slices (in natural order) that hold text and modality rows, among those this wave has looked at
+    // every class of the wave's 64 rows at once: add(class, count, this lane's number among the earlier ones)
+    auto classes = [&](int cls, auto add) {
+        unsigned long long left = __ballot(cls >= 0);
+        while (left != 0) {  // wave-uniform
+            const int c = __builtin_amdgcn_readlane(cls, __builtin_ctzll(left));
+            const unsigned long long same = __ballot(cls == c);
+            add(c, same);
+            left &= ~same;
+        }
+    };
+    constexpr int AHEAD = 8;
+    for (int i0 = 0; i0 < S; i0 += AHEAD * SORT_CHUNK) {
+        int64_t f[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int i = i0 + u * SORT_CHUNK + tid;
+            f[u] = i < S ? row[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int chunk = i0 + u * SORT_CHUNK, i = chunk + tid;
+            const int cls = i < S ? sort_class(f[u]) : -1;
+            const unsigned long long text = __ballot(cls == 0), modal = __ballot(cls > 0 && cls < SORT_CLASSES - 1);
+            mixed += ((unsigned)text != 0 && (unsigned)modal != 0) + ((text >> 32) != 0 && (modal >> 32) != 0);
+            classes(cls, [&](int c, unsigned long long same) {
+                if (lane == 0) {
+                    atomicAdd(&s_total[c], __popcll(same));
+                    if (chunk < first) atomicAdd(&s_before[c], __popcll(same));
+                }
+            });
+        }
+    }
+    if (lane == 0) atomicAdd(&s_mixed, mixed);
+    const int mine = first + tid;
+    const int64_t f = mine < S ? row[mine] : 0;
+    const int cls = mine < S ? sort_class(f) : -1;
+    int earlier = 0;  // rows of my class in front of me in the wave
+    classes(cls, [&](int c, unsigned long long same) {
+        if (lane == 0) s_wave[wave][c] = __popcll(same);
+        if (cls == c) earlier = __popcll(same & ((1ull << lane) - 1ull));
+    });
+    __syncthreads();
+    if (tid < SORT_CLASSES) {
+        int base = 0;
+        for (int c = 0; c < tid; ++c) base += s_total[c];
+        s_base[tid] = base + s_before[tid];
+        int run = 0;
+        for (int w = 0; w < SORT_CHUNK / 64; ++w) {
+            const int n = s_wave[w][tid];
+            s_wave[w][tid] = run;
+            run += n;
+        }
+    }
+    __syncthreads();
+    const bool move = s_mixed * SORT_MIXED >= (S + 31) / 32;
+    if (blockIdx.x == 0 && tid == 0) rows_moved[b] = move ? 1 : 0;
+    if (mine < S) {
+        const int64_t at = (int64_t)b * rows_sb + (move ? s_base[cls] + s_wave[wave][cls] + earlier : mine);
+        rows[at] = mine;
+        rows_bits[at] = f;
+    } else if (mine < S_rounded) {
+        rows[(int64_t)b * rows_sb + mine] = S;
+        rows_bits[(int64_t)b * rows_sb + mine] = 0;
+    }
+}
+
+int launch_sorted_plan(const int64_t* bf, int64_t bf_stride_b, int* rows, int64_t* rows_bits, int64_t rows_sb, int* rows_moved, uint8_t* fine,
+                       int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B, int S,
+                       hipStream_t stream) {
+    const int num_m = (S + BLOCK_M - 1) / BLOCK_M, num_n = (S + BLOCK_N - 1) / BLOCK_N;
+    hipLaunchKernelGGL(sort_rows_kernel, dim3((num_m * BLOCK_M + SORT_CHUNK - 1) / SORT_CHUNK, B), dim3(SORT_CHUNK), 0, stream, bf,
+                       bf_stride_b, S, num_m * BLOCK_M, rows, rows_bits, rows_sb, rows_moved, pair_count);
+    const int flag_groups = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
+    const int flag_blocks_x = min(flag_groups, FLAG_MAX_BLOCKS_X);
+    hipLaunchKernelGGL(indexed_plan_kernel<false>, dim3(flag_blocks_x + 1, num_m, B), dim3(FLAG_WAVES * 64), 0, stream,
+                       (const int64_t*)nullptr, (int64_t)0, 0, (const int64_t*)nullptr, (const int64_t*)nullptr, rows_bits, rows_sb,
+                       const_cast<int64_t*>(bf), bf_stride_b, rows, rows_sb, (int*)nullptr, S, S, num_n, fine, fine_sb, fine_ss,
+                       order, order_sb, flag_blocks_x, flag_groups, rows_moved, (int*)nullptr);
     return (int)hipGetLastError();
 }
 

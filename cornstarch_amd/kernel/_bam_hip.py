@@ -15,7 +15,7 @@ BAM_DTYPE_F16 = 0
 BAM_DTYPE_BF16 = 1
 BAM_MAX_SEQLEN = 4194304
 BAM_STATIC_PLAN_BYTES = 8 << 20
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -73,6 +73,12 @@ class Plan(ctypes.Structure):
         ("col_bits", ctypes.c_void_p),
         ("col_bits_stride_b", ctypes.c_int64),
         ("col_bits_stride_s", ctypes.c_int64),
+        ("rows", ctypes.c_void_p),
+        ("rows_bits", ctypes.c_void_p),
+        ("rows_stride_b", ctypes.c_int64),
+        ("rows_moved", ctypes.c_void_p),
+        ("rows_known", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
         ("B", ctypes.c_int32),
         ("Sq", ctypes.c_int32),
         ("Sk", ctypes.c_int32),
@@ -123,6 +129,8 @@ SIGNATURES = {
     "bam_materialize_mask": [_ptr, _i64, _ptr, _int, _int, _ptr],
     "bam_tile_plan": [_ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _plan, _ptr],
     "bam_tile_plan_counted": [_ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _plan, _ptr, _u32, _ptr],
+    "bam_tile_plan_sorted_counted": [_ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _int, _int, _plan, _ptr, _u32, _ptr],
+    "bam_sorted_plan_workspace_bytes": [_int, _int, ctypes.POINTER(_i64)],
     "bam_host_words_alloc": [_ptr, _int],
     "bam_host_words_free": [_ptr],
     "bam_tile_plan_static": [_ptr, _i64, _ptr, _i64, _i64, _int, _int, _plan, _ptr],

@@ -103,6 +103,9 @@ typedef struct bam_bias {
  * into dk (instead of a recomputation that may differ in the last bit).  The count is device data: read it (for
  * instance with an asynchronous copy enqueued right after the plan builder) before sizing the workspace.
  */
+#define BAM_ROWS_UNKNOWN 0
+#define BAM_ROWS_LEFT 1  /* no sequence's rows have been moved */
+#define BAM_ROWS_MOVED 2 /* every sequence's rows have been moved */
 typedef struct bam_plan {
     const uint8_t* fine;
     int64_t fine_stride_b;
@@ -140,6 +143,15 @@ typedef struct bam_plan {
     const uint32_t* col_bits;
     int64_t col_bits_stride_b;
     int64_t col_bits_stride_s;
+    /* Sorted rows (bam_tile_plan_sorted_counted; null otherwise): slice s of fine, order and ds_entry is the query rows
+     * rows[b * rows_stride_b + 32 s ..] instead of 32 s ..; rows_bits are their bitfields.  Entries past the last row: Sq, 0.
+     * Where rows have been moved, bit 30 is set in the entries of order. */
+    const int32_t* rows;
+    const int64_t* rows_bits;
+    int64_t rows_stride_b;
+    const int32_t* rows_moved; /* (B): 0 where a sequence's rows have been left in their natural order (few mixed slices) */
+    int32_t rows_known;        /* BAM_ROWS_*: set by a caller that has read the builder's count word, saves a launch of dK/dV */
+    int32_t reserved;
     int32_t B;
     int32_t Sq;         /* query rows and keys the plan was built for (equal for plain bitfield attention) */
     int32_t Sk;
@@ -181,6 +193,19 @@ int bam_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t
 int bam_tile_plan_counted(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                           int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
                           uint64_t* count_host, uint32_t count_tag, void* stream);
+
+/*
+ * bam_tile_plan_counted with the query rows sorted -- text rows by position, then the modality rows grouped by their bitfield, then
+ * padding -- so that a slice holds rows that see the same keys.  A slice of a sequence with many short segments otherwise holds
+ * text and modality rows and drags the whole past of the former through all 32.  (A sequence with few such slices keeps its order.)  Bitfield attention only; the attention entry
+ * points then read rows one by one.  plan->row_workloads is null (slices are no longer 32 neighbours); flags, strides and the
+ * order of all outputs are as ever.  The count word then also says, in bits 31 and 30, whether the rows of some sequence have
+ * been moved, or left (neither: not known; the count is below 2^30, larger problems are refused).  Gradients of k and v are summed in another order than with bam_tile_plan.
+ */
+int bam_sorted_plan_workspace_bytes(int B, int S, int64_t* bytes); /* 0 bytes: no plan for so many rows */
+int bam_tile_plan_sorted_counted(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
+                                 int64_t flags_stride_m, void* workspace, int64_t workspace_bytes, int B, int S, bam_plan* plan,
+                                 uint64_t* count_host, uint32_t count_tag, void* stream);
 /* Pinned, coherent host memory for those words (zero-filled; hipHostMalloc / hipHostFree, so not while capturing). */
 int bam_host_words_alloc(uint64_t** words, int n);
 int bam_host_words_free(uint64_t* words);
