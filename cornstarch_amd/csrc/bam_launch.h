@@ -110,6 +110,12 @@ inline bool dkdv_far(const AttnParams& p) {
     return far_rows(p.q, p.Sq, p.d) || far_rows(p.dout, p.Sq, p.d) || far_rows(p.k, p.Sk, p.d) || far_rows(p.v, p.Sk, p.d);
 }
 
+// Whether the forward and dQ walk two tiles at a time (measured at launch_fwd_b and launch_dq_f).
+inline bool two_streams(const AttnParams& p) {
+    const int64_t units = (int64_t)p.num_m * p.B * p.Hq;
+    return units <= (p.D > 64 ? 256 : 512) || (p.D <= 32 && units <= 1024 && p.Sk >= 2560);
+}
+
 // Single-token decode step (one query row per batch element and head, no mask); strides in elements.
 struct DecodeParams {
     const void *q, *k, *v;         // q (B, Hq, D): q_sb, q_sh; k / v (B, Sk, Hkv, D): *_sb, *_ss, *_sh

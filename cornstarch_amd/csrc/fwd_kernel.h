@@ -540,14 +540,10 @@ static int launch_fwd_s(const AttnParams& p, hipStream_t stream) {
 // 25.2, 1024 (256 workgroups) 31.8 -> 27.3, 2 x 700 (384) 31.0 -> 30.7, 2048 (512) 57.5 -> 57.2, 3001 (768) 88 -> 103; D 64:
 // 1000 * 24.1 -> 19.2, 2 x 700 24.2 -> 22.0, 2048 43.4 -> 40.9, 3001 62 -> 69.  At D = 32 two such workgroups fit a unit: 2048
 // 37.8 -> 28.2, 3001 52.4 -> 40.7, 4096 (1024) 69 -> 61, but with short lists 8 x 300 (768) 16.0 -> 19.5, 4 x 1024 27.8 -> 30.4.
-static bool fwd_two_streams(const AttnParams& p) {
-    const int64_t units = (int64_t)p.num_m * p.B * p.Hq;
-    return units <= (p.D > 64 ? 256 : 512) || (p.D <= 32 && units <= 1024 && p.Sk >= 2560);
-}
 template <typename T, int D, bool BIAS, bool LONG>
 static int launch_fwd_b(const AttnParams& p, hipStream_t stream) {
     if constexpr (!LONG)
-        if (fwd_two_streams(p)) return launch_fwd_s<T, D, BIAS, false, 2>(p, stream);
+        if (two_streams(p)) return launch_fwd_s<T, D, BIAS, false, 2>(p, stream);
     return launch_fwd_s<T, D, BIAS, LONG, 1>(p, stream);
 }
 template <typename T, int D, bool LONG>

@@ -1,4 +1,4 @@
-"""The forward with few workgroups walks two tiles at a time and merges two partial results per row.  Every sequence of a batch
+"""The forward and dQ with few workgroups walk two tiles at a time and merge two partial results per row.  Every sequence of a batch
 that is large enough to go tile by tile, against the same sequence by itself."""
 
 import pytest
@@ -35,4 +35,28 @@ def test_a_sequence_of_a_large_batch_equals_the_sequence_alone(S, D, biased):
         live = torch.isfinite(lse[b])
         assert torch.equal(live, torch.isfinite(lse1[0])) and (lse1[0] - lse[b])[live].abs().max().item() <= 2.0**-8
         assert torch.isfinite(o1).all() and torch.equal(lse[b][~live], lse1[0][~live])
+    BA.BitfieldUtils.clear_cache()
+
+
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("D", [32, 40, 64])
+@pytest.mark.parametrize("S", [64, 65, 130, 200, 257])
+def test_gradients_of_a_sequence_of_a_large_batch_equal_those_alone(S, D, biased):
+    Hq, Hkv = 8, 2
+    B = 1024 // (Hq * ((S + 127) // 128)) + 1
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v, do = ((torch.randn(B, S, H, D, generator=g, device="cuda")).bfloat16() for H in (Hq, Hkv, Hkv, Hq))
+    bf = random_bitfield(B, S, seed=S, pad=S // 9).cuda()
+    bias = torch.randn(1, Hq, 1, S, generator=g, device="cuda") if biased else None
+
+    def gradients(rows):
+        BA.BitfieldUtils.clear_cache()
+        x = [t[rows].detach().requires_grad_(True) for t in (q, k, v)]
+        return torch.autograd.grad(BA.bitfield_attn_func(*x, bf[rows], bias), x, do[rows])
+
+    batch = gradients(slice(None))
+    for b in (0, B // 2, B - 1):
+        for one, all_ in zip(gradients(slice(b, b + 1)), batch):
+            # o and the lse differ by a rounding of P to bf16 (2^-9 a term), which delta and P carry into the gradients
+            assert torch.isfinite(one).all() and rel_l2(one[0].float(), all_[b].float()) <= 2.0**-7
     BA.BitfieldUtils.clear_cache()
