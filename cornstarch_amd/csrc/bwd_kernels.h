@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const AttnParams p)
 // ---------------------------------------------------------------------------------------
 // dK, dV.  One workgroup = one 128-key tile of one (batch, kv head), 8 waves: wave w owns keys
 // [32 (w & 3), +32) and works on rows [32 (w >> 2), +32) of every 64-row tile of Q / dO that streams
-// through LDS (double buffered), so each SIMD holds two waves whose MFMA and softmax phases
+// through LDS (two or four buffers), so each SIMD holds two waves whose MFMA and softmax phases
 // interleave.  A 64-row tile is a PAIR of 32-row slices taken from the list of slices that have work
 // for this key tile (they need not be neighbours in the sequence), one slice per row stream; a wave
 // whose own 32 x 32 class is "empty" sits the tile out.  K and V of the tile sit in LDS for the whole kernel and are
@@ -90,20 +90,26 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
     constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
     static_assert(!(SORTED && LONG), "no plan for so many rows");
+    // A tile is 16 MFMAs per wave at head dims up to 64, half of what it is above, and there is room for four buffers: two tiles
+    // are copied ahead and the workgroup meets after every second one.  dK/dV alone, us, a meeting per tile -> per two: D 64, 3001
+    // tokens, 32 / 8 heads 190 -> 180, 2 x 700 57.7 -> 54.9, 8 x 4096, 16 heads 555 -> 532; D 32: 3001 148.8 -> 139.8.
+    // (SORTED has row numbers to copy one tile earlier still.)
+    constexpr bool DEEP = D <= 64 && !SORTED && !LONG;
+    constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
     __shared__ u32x4 sK[128 * NCH];
     __shared__ u32x4 sV[128 * NCH];
-    __shared__ u32x4 sQ[2][DKDV_QT * NCH];
-    __shared__ u32x4 sDO[2][DKDV_QT * NCH];
-    __shared__ __attribute__((aligned(16))) float sLse[2][DKDV_QT];      // natural-log lse of the rows
-    __shared__ __attribute__((aligned(16))) float sDelta[2][DKDV_QT];
-    __shared__ __attribute__((aligned(16))) int64_t sQbf[2][DKDV_QT];    // raw bitfields of the rows
+    __shared__ u32x4 sQ[NB][DKDV_QT * NCH];
+    __shared__ u32x4 sDO[NB][DKDV_QT * NCH];
+    __shared__ __attribute__((aligned(16))) float sLse[NB][DKDV_QT];      // natural-log lse of the rows
+    __shared__ __attribute__((aligned(16))) float sDelta[NB][DKDV_QT];
+    __shared__ __attribute__((aligned(16))) int64_t sQbf[NB][DKDV_QT];    // raw bitfields of the rows
     // their positions (ROW_POS).  SORTED: a tile's rows are gathered, so their numbers have to be here a tile earlier
-    __shared__ __attribute__((aligned(16))) int sQpos[SORTED ? 3 : 2][DKDV_QT];
+    __shared__ __attribute__((aligned(16))) int sQpos[SORTED ? 3 : NB][DKDV_QT];
     __shared__ __attribute__((aligned(16))) unsigned sWq[DKDV_THREADS / 64][5][32];  // per-wave rule constants
     // DENSE with packed mask bits: for the two slices of the tile, one word per key of the workgroup's 128 keys
-    __shared__ unsigned sColBits[MODE == MASK_DENSE ? 2 : 1][2][MODE == MASK_DENSE ? 128 : 1];
+    __shared__ unsigned sColBits[MODE == MASK_DENSE ? NB : 1][2][MODE == MASK_DENSE ? 128 : 1];
     __shared__ int sListStore[MAX_SLICE_LIST + 1];  // entry -1: partner of the first entry of an odd count
     int* const sList = sListStore + 1;
     __shared__ int sCount;
@@ -361,10 +367,10 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     // ds_pos: position of the wave's slice in the slice list.
     // returns true when the wave has issued its two dS stores (they may stay in flight over the end of the iteration)
     // pos_cur, pos_nxt: the buffers of the tile's positions and of those that are copied now
-    auto tile_step = [&](int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int pos_cur, int pos_nxt) -> bool {
+    auto tile_step = [&](int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int nxt, int pos_cur, int pos_nxt) -> bool {
         if (cls == 0) {
 #pragma unroll
-            for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, cur ^ 1, pos_nxt);
+            for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, nxt, pos_nxt);
             return false;
         }
         const int ds_e = ds_base + ds_pos;
@@ -406,7 +412,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                     dp = T::mfma(a[j], bb[j], dp);
                 else
                     s = T::mfma(a[j], bb[j], j < 2 ? zero16 : s);
-                if (j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, cur ^ 1, pos_nxt);
+                if (j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, nxt, pos_nxt);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -600,6 +606,16 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             };
             advance();
             int n_lo = __builtin_amdgcn_readfirstlane(entry_lo(r_nxt)), n_hi = __builtin_amdgcn_readfirstlane(entry_hi(r_nxt));
+            // DEEP: two tiles are copied ahead, f_* is the one between the current tile and the one that is copied
+            int f_lo = n_lo, f_hi = n_hi, f_g = g_nxt, f_r = r_nxt;
+            if constexpr (DEEP) {
+                const TileSource second = tile_source(hv_nxt, (n_lo >> 8) * 32, (n_hi >> 8) * 32);
+#pragma unroll
+                for (int j = 0; j < NLOADS; ++j) issue_copy(j, second, 1, 1);
+                advance();
+                n_lo = __builtin_amdgcn_readfirstlane(entry_lo(r_nxt));
+                n_hi = __builtin_amdgcn_readfirstlane(entry_hi(r_nxt));
+            }
             wait_async();
             asm volatile("" : "+v"(klo), "+v"(khi), "+v"(kpos));  // (see arrived())
             __syncthreads();
@@ -611,13 +627,13 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
             load_kv_operands();
             int pos_cur = 0;  // SORTED: it % 3
             for (int it = 0; it < total; ++it) {
-                const int cur = it & 1;
+                const int cur = it & (NB - 1), nxt = DEEP ? (it + 2) & (NB - 1) : cur ^ 1;
                 // pair after next (SORTED: the one behind it): its list entries are requested now and picked up at the end of
                 // the iteration
                 const int r_req = SORTED ? after(after(r_nxt)) : after(r_nxt);
                 const int x_lo = entry_lo(r_req), x_hi = entry_hi(r_req);
                 TileSource next;
-                const int p1 = SORTED ? (pos_cur == 2 ? 0 : pos_cur + 1) : cur ^ 1, p2 = SORTED ? (pos_cur == 0 ? 2 : pos_cur - 1) : cur ^ 1;
+                const int p1 = SORTED ? (pos_cur == 2 ? 0 : pos_cur + 1) : nxt, p2 = SORTED ? (pos_cur == 0 ? 2 : pos_cur - 1) : nxt;
                 if constexpr (SORTED) {
                     next = gathered_source(hv_nxt, sQpos[p1], (n_lo >> 8) * 32, (n_hi >> 8) * 32, (a_lo >> 8) * 32, (a_hi >> 8) * 32);
                 } else {
@@ -626,11 +642,17 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                 const int mine = st ? e_hi : e_lo;
                 fetch_bias_key(hk * G + g_cur);
                 const bool stored = tile_step(cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur, (mine >> 8) * 32, n - 2 - 2 * r_cur + st,
-                                              next, SORTED ? pos_cur : cur, p2);
-                g_cur = g_nxt;
-                r_cur = r_nxt;
-                e_lo = n_lo;
-                e_hi = n_hi;
+                                              next, nxt, SORTED ? pos_cur : cur, p2);
+                g_cur = DEEP ? f_g : g_nxt;
+                r_cur = DEEP ? f_r : r_nxt;
+                e_lo = DEEP ? f_lo : n_lo;
+                e_hi = DEEP ? f_hi : n_hi;
+                if (DEEP) {
+                    f_lo = n_lo;
+                    f_hi = n_hi;
+                    f_g = g_nxt;
+                    f_r = r_nxt;
+                }
                 advance();
                 n_lo = SORTED ? a_lo : __builtin_amdgcn_readfirstlane(x_lo);
                 n_hi = SORTED ? a_hi : __builtin_amdgcn_readfirstlane(x_hi);
@@ -639,6 +661,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
                     a_hi = __builtin_amdgcn_readfirstlane(x_hi);
                     pos_cur = p1;
                 }
+                // DEEP: after every second tile the next two have landed and their buffers are free again
+                if (DEEP && (it & 1) == 0) continue;
                 // the copies of the next tile must have landed; the two dS stores, issued after them, may stay in flight
                 if (SAVE && stored)
                     asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
