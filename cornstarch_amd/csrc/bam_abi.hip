@@ -811,24 +811,45 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
                     a->flags_stride_m, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->bias, a->plan, stream, true);
 }
 
-// How many workgroups share the q heads of a kv head in dK/dV.  One workgroup per (key tile, kv head) walks all of them one
-// after the other, so calls with grouped heads leave most compute units without one until the sequence is long.  As many
-// parts as keep the launch within one workgroup per compute unit (beyond that the parts queue behind each other).  Whole
-// training step, bf16, D 64, one part -> parts: 1 x 1024 tokens, 32 / 8 heads 139 -> 98 us; 1 x 2048, 32 / 4 heads
-// 363 -> 183; 1 x 4000, 16 / 4 heads 401 -> 286; D 128: 1 x 700, 16 / 4 heads 138 -> 105; 1 x 1024, 32 / 8 heads
-// 180 -> 117; 1 x 3000, 16 / 4 heads 456 -> 319.  The price is a launch (4 to 6 us), an allocation and their host work, so at
-// least 32 steps over a pair of slices have to go: 4 x 400 tokens, 6 / 1 heads, D 40 (35 steps) 94 -> 58 to 98 us with the
-// speed of the host; 512 tokens, 16 / 4 heads (24 steps) 83 -> 95, 2 x 283, 6 / 2 heads (10 steps) 86 -> 91.
+// How many workgroups share the q heads of a kv head in dK/dV.  One workgroup per (key tile, kv head) walks all of them one after
+// the other and the launch lasts as long as the first key tile's; dealt to parts, the tiles level out over the 256 compute units.
+// The price is fp32 sums through memory and a launch that adds them.  The estimate, in us: a step over a pair of slices takes
+// `step`, a workgroup kStart steps besides, tiles fall off linearly in length (a causal mask); the launch takes the longest
+// workgroup, or the work per compute unit and kTail of the longest.  Fitted to 42 training steps (D 32, 64, 128; 6 to 32 q heads,
+// 1 to 8 kv heads, 300 to 9000 tokens), of which it takes the fastest number of parts, or one within 5 %; gains of a few
+// per cent are not there (1 x 16384 tokens, 2 parts: dK/dV 4115 -> 4069 and 56 for the sum).  One part -> parts,
+// kernels of a step, us, 32 / 8 heads, D 128: 300 tokens 87 -> 68 (4 parts), 2 x 700 147 -> 120 (4), 2500 380 -> 305 (2), 3001
+// 453 -> 355 (2), 5000 861 -> 790 (2), but 4 x 1537 (416 workgroups) 412 -> 445; 16 / 4 heads, 9000 tokens 1404 -> 1255; D 64:
+// 3001 tokens 322 -> 256, 5000 560 -> 513.  At least 32 steps have to go: below, the host is what a training step waits for (4 x 400
+// tokens, 6 / 1 heads, D 40, 35 steps: 94 -> 58 to 98 us with the speed of the host; 2 x 283, 6 / 2 heads, 10 steps: 86 -> 91).
 static int dkdv_parts(const bam_attn* a) {
-    if (a->head_runs > 1 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32) return 1;
+    if (a->head_runs > 1 || a->B <= 0 || a->Sk <= 0 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32)
+        return 1;
     if (bam::far_rows(a->q.stride_s, a->Sq, a->D) || bam::far_rows(a->dout.stride_s, a->Sq, a->D) ||
         bam::far_rows(a->k.stride_s, a->Sk, a->D) || bam::far_rows(a->v.stride_s, a->Sk, a->D))
         return 1;  // (the instantiation for such rows has no parts)
-    const int G = a->Hq / a->Hkv, pairs = (a->Sq + 63) / 64;
-    const int64_t units = (int64_t)a->B * a->Hkv * ((a->Sk + 127) / 128);
-    for (int parts = G; parts > 1; --parts)
-        if (G % parts == 0 && units * parts <= 256) return (int64_t)(G - G / parts) * pairs >= 32 ? parts : 1;
-    return 1;
+    const int G = a->Hq / a->Hkv;
+    const double tiles = (a->Sk + 127) / 128, pairs = (a->Sq + 63) / 64, step = a->D > 96 ? 1.25 : a->D > 64 ? 1.1 : a->D > 32 ? 0.79 : 0.63;
+    constexpr double kStart = 7.8, kTail = 0.28, kBytesPerUs = 8.7e6, kLaunch = 6;  // (the parts stay in the last-level cache)
+    const double units = a->B * (double)a->Hkv * tiles, rows = (double)a->B * a->Sk * a->Hkv;
+    auto estimate = [&](int parts) {
+        const double longest = pairs * G / parts, share = units * ((pairs + 1) / 2 * G + kStart * parts) / 256 + kTail * longest;
+        const double sum = parts > 1 ? kLaunch + 2 * 2 * 4 * rows * a->D * parts / kBytesPerUs : 0;
+        return step * (longest + kStart > share ? longest + kStart : share) + sum;
+    };
+    const double one = estimate(1);
+    int best = 1;
+    double least = one - (one > 130 ? 0.06 * one : 8);  // the host's launch and allocation have to come out, and the estimate's error
+    for (int parts = 2; parts <= G; ++parts) {
+        if (G % parts || 2 * 4 * rows * a->D * parts > 1e9 || units * parts > 1e6) continue;
+        if ((G - G / parts) * pairs < 32) continue;
+        const double t = estimate(parts);
+        if (t < least) {
+            least = t;
+            best = parts;
+        }
+    }
+    return best;
 }
 static int64_t dkdv_part_floats(const bam_attn* a, int parts) { return (int64_t)a->B * a->Sk * a->Hkv * parts * a->D; }
 
