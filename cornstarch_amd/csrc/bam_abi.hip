@@ -509,8 +509,7 @@ int bam_tile_plan_sorted_counted(const int64_t* bf, int64_t bf_stride_b, int8_t*
     PlanLayout l;
     BAM_TRY(place_plan(who, workspace, workspace_bytes, B, S, S, plan, l, false, true));
     char* w = (char*)workspace;
-    BAM_TRY(launched(bam::launch_tile_flags(bf, bf_stride_b, flags, flags_stride_b, flags_stride_m, B, S, (hipStream_t)stream), who));
-    BAM_TRY(launched(bam::launch_sorted_plan(bf, bf_stride_b, (int*)(w + l.rows_off), (int64_t*)(w + l.rows_bits_off), l.rows_sb,
+    BAM_TRY(launched(bam::launch_sorted_plan(bf, bf_stride_b, flags, flags_stride_b, flags_stride_m, (int*)(w + l.rows_off), (int64_t*)(w + l.rows_bits_off), l.rows_sb,
                                              (int*)(w + l.rows_moved_off), (uint8_t*)(w + l.fine_off), l.fine_sb, l.fine_ss, (int*)(w + l.order_off), l.order_sb,
                                              (int*)(w + l.count_off), B, S, (hipStream_t)stream),
                      who));

@@ -148,11 +148,12 @@ int launch_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int
 // (pair_count: the counter launch_ds_entries adds to, reset here)
 int launch_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                      int64_t flags_stride_m, uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int* order,
-                     int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream);
-// Sorted rows (see AttnParams::rows; S_rounded entries per sequence), and flags-free plan over them: fine and order.
-int launch_sorted_plan(const int64_t* bf, int64_t bf_stride_b, int* rows, int64_t* rows_bits, int64_t rows_sb, int* rows_moved, uint8_t* fine,
-                       int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B, int S,
-                       hipStream_t stream);
+                     int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream, int* rows = nullptr,
+                     int64_t* rows_bits = nullptr, int64_t rows_sb = 0, int* rows_moved = nullptr);
+// The same with sorted rows (see AttnParams::rows; S_rounded entries per sequence).
+int launch_sorted_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m,
+                       int* rows, int64_t* rows_bits, int64_t rows_sb, int* rows_moved, uint8_t* fine, int64_t fine_sb,
+                       int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream);
 int launch_materialize_mask(const int64_t* bf, int64_t bf_stride_b, uint8_t* out, int B, int S,
                             hipStream_t stream);
 int launch_flag_row_workloads(const int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m, int B, int num_m,

@@ -230,10 +230,11 @@ bool bitfield_ready(const Tensor& bf) {
            bf.size(1) > 0 && !bf.is_inference() && plain(bf);
 }
 
-// From here on the plan's rows are sorted (where the segments are many).  Below, the longer plan builder weighs more than what a
-// sequence with a few segments gains: forward + backward of 8192 tokens, 4 segments, 32 / 8 heads, D 128 1687 -> 1714 us (30
-// segments: 1873 -> 1678); 16384 tokens, 4 segments 7335 -> 7363.
-constexpr int64_t kSortedRows = 16384;
+// From here on the plan's rows are sorted (where the segments are many).  A sequence with few segments, whose rows stay, pays the
+// launch that finds that out: 4 us, which may be 2 % of the shortest forward over 16384 tokens (4 heads, D 32) and is at most 0.7 %
+// from here on.  Many segments gain 5 to 28 %: forward + backward of 65536 tokens with 200 segments 62.9 -> 47.7 ms, forward alone
+// of 32768 tokens with 60, 16 / 4 heads, D 64 1920 -> 1730 us.
+constexpr int64_t kSortedRows = 32768;
 
 // flags (and plan, up to 131072 tokens) of an int64 (B, S) mask on the GPU
 Flags bitfield_flags(const Tensor& mask) {

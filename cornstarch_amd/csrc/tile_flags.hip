@@ -182,6 +182,139 @@ __device__ __forceinline__ void slice_keys_chunk_indexed(const Rows& rows, int S
     }
 }
 
+// Sorted rows: text rows by position, then the modality rows grouped by their bitfield, by position inside a group, then
+// padding.  A counting sort over 64 classes; different bitfields may share a class (only the packing of the slices suffers).  A
+// workgroup of 256 threads places 1024 rows of one sequence; it counts the classes of all rows for itself (512 KiB of bitfields out
+// of L2 for 65536 rows, eight loads in flight per thread) instead of waiting for the others, beside the workgroups that compute
+// the flags, which take longer (17000 rows: 20.3 us with and 19.6 without; 28.8 when it took 64 rows of one bitfield one by one).
+// Rows are only moved where at least one slice in SORT_MIXED holds text and modality rows: dK/dV gathers moved rows one by one,
+// which costs it 3 %.  Training step, 32 / 8 heads, D 128, natural -> sorted: 65536 tokens, 200 segments (20 % of the slices
+// mixed) 64.3 -> 48.2 ms; 8192 tokens, 30 segments (23 %) 1.87 -> 1.68 ms, 4 segments (3 %) 1.717 -> 1.722 ms; 16384 tokens, 4
+// segments (1.6 %) 7.36 -> 7.46 ms.
+constexpr int SORT_CHUNK = 1024, SORT_CLASSES = 64, SORT_MIXED = 32;
+struct SortedRows {
+    int* rows;           // null: not asked for
+    int64_t* rows_bits;
+    int64_t rows_sb;
+    int* rows_moved;
+};
+__device__ __forceinline__ int sort_class(int64_t f) {
+    const uint64_t bits = (uint64_t)f & ((1ull << 62) - 1ull);
+    if (bits & 1) return 0;
+    if (bits == 0) return SORT_CLASSES - 1;
+    if ((bits & (bits - 1)) == 0) return 1 + (__ffsll((long long)bits) - 1) % (SORT_CLASSES - 2);
+    return 1 + (int)((bits * 0x9E3779B97F4A7C15ull) >> 40) % (SORT_CLASSES - 2);
+}
+// f(class, lanes that hold it) for every class among the wave's lanes (cls < 0: none)
+template <typename F>
+__device__ __forceinline__ void each_class(int cls, F f) {
+    unsigned long long left = __ballot(cls >= 0);
+    while (left != 0) {  // wave-uniform
+        const int c = __builtin_amdgcn_readlane(cls, __builtin_ctzll(left));
+        const unsigned long long same = __ballot(cls == c);
+        f(c, same);
+        left &= ~same;
+    }
+}
+__device__ void sort_rows_part(const int64_t* __restrict__ row, int S, int S_rounded, int part, int b, const SortedRows& out) {
+    constexpr int THREADS = FLAG_WAVES * 64, GROUPS = SORT_CHUNK / 64;
+    __shared__ int s_mixed, s_total[SORT_CLASSES], s_before[SORT_CLASSES], s_base[SORT_CLASSES];
+    __shared__ int s_group[GROUPS][SORT_CLASSES];  // rows of a class in each run of 64 rows, then in front of it
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int first = part * SORT_CHUNK;
+    if (tid == 0) s_mixed = 0;
+    if (tid < SORT_CLASSES) s_total[tid] = s_before[tid] = 0;
+    for (int i = tid; i < GROUPS * SORT_CLASSES; i += THREADS) s_group[0][i] = 0;
+    __syncthreads();
+    int mixed = 0;  // slices (in natural order) that hold text and modality rows, among those this wave has looked at
+    // 64 rows of one bitfield (most of them are) only add to the counts of the run they belong to
+    int64_t run_bits = 0;
+    int run_total = 0, run_before = 0;
+    auto end_run = [&]() {
+        if (run_total > 0 && lane == 0) {
+            const int c = sort_class(run_bits);
+            atomicAdd(&s_total[c], run_total);
+            if (run_before > 0) atomicAdd(&s_before[c], run_before);
+        }
+        run_total = run_before = 0;
+    };
+    constexpr int AHEAD = 8;
+    for (int i0 = 0; i0 < S; i0 += AHEAD * THREADS) {
+        int64_t f[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int i = i0 + u * THREADS + tid;
+            f[u] = i < S ? row[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int run = i0 + u * THREADS, i = run + tid;
+            const int64_t f0 = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)f[u]) |
+                               (int64_t)__builtin_amdgcn_readfirstlane((int)(f[u] >> 32)) << 32;
+            if (run + wave * 64 + 64 <= S && __all(f[u] == f0)) {
+                if (f0 != run_bits) {
+                    end_run();
+                    run_bits = f0;
+                }
+                run_total += 64;
+                run_before += run < first ? 64 : 0;
+                continue;
+            }
+            const int cls = i < S ? sort_class(f[u]) : -1;
+            const unsigned long long text = __ballot(cls == 0), modal = __ballot(cls > 0 && cls < SORT_CLASSES - 1);
+            mixed += ((unsigned)text != 0 && (unsigned)modal != 0) + ((text >> 32) != 0 && (modal >> 32) != 0);
+            each_class(cls, [&](int c, unsigned long long same) {
+                if (lane == 0) {
+                    atomicAdd(&s_total[c], __popcll(same));
+                    if (run < first) atomicAdd(&s_before[c], __popcll(same));
+                }
+            });
+        }
+    }
+    end_run();
+    if (lane == 0) atomicAdd(&s_mixed, mixed);
+    int64_t f[GROUPS / FLAG_WAVES];
+    int cls[GROUPS / FLAG_WAVES], earlier[GROUPS / FLAG_WAVES];
+#pragma unroll
+    for (int u = 0; u < GROUPS / FLAG_WAVES; ++u) {
+        const int mine = first + u * THREADS + tid;
+        f[u] = mine < S ? row[mine] : 0;
+        cls[u] = mine < S ? sort_class(f[u]) : -1;
+        earlier[u] = 0;  // rows of my class in front of me in the run of 64
+        each_class(cls[u], [&](int c, unsigned long long same) {
+            if (lane == 0) s_group[u * FLAG_WAVES + wave][c] = __popcll(same);
+            if (cls[u] == c) earlier[u] = __popcll(same & ((1ull << lane) - 1ull));
+        });
+    }
+    __syncthreads();
+    if (tid < SORT_CLASSES) {
+        int base = 0;
+        for (int c = 0; c < tid; ++c) base += s_total[c];
+        s_base[tid] = base + s_before[tid];
+        int before = 0;
+        for (int g = 0; g < GROUPS; ++g) {
+            const int n = s_group[g][tid];
+            s_group[g][tid] = before;
+            before += n;
+        }
+    }
+    __syncthreads();
+    const bool move = s_mixed * SORT_MIXED >= (S + 31) / 32;
+    if (part == 0 && tid == 0) out.rows_moved[b] = move ? 1 : 0;
+#pragma unroll
+    for (int u = 0; u < GROUPS / FLAG_WAVES; ++u) {
+        const int mine = first + u * THREADS + tid;
+        if (mine < S) {
+            const int64_t at = (int64_t)b * out.rows_sb + (move ? s_base[cls[u]] + s_group[u * FLAG_WAVES + wave][cls[u]] + earlier[u] : mine);
+            out.rows[at] = mine;
+            out.rows_bits[at] = f[u];
+        } else if (mine < S_rounded) {
+            out.rows[(int64_t)b * out.rows_sb + mine] = S;
+            out.rows_bits[(int64_t)b * out.rows_sb + mine] = 0;
+        }
+    }
+}
+
 // FINE: also write the class of every 32-row x 32-column tile (the four row slices of each flag tile) to
 // fine[b][4 m + w][n]; same 0 / 1 / 2 meaning, "full" again over the in-range cells only.
 template <bool FINE>
@@ -193,10 +326,17 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void tile_flags_kernel(const int64
                                                                     uint8_t* __restrict__ fine, int64_t fine_sb,
                                                                     int64_t fine_ss, int* __restrict__ order,
                                                                     int64_t order_sb, int flag_blocks_x,
-                                                                    int flag_groups, int* __restrict__ pair_count) {
+                                                                    int flag_groups, int* __restrict__ pair_count,
+                                                                    SortedRows sorted) {
     // (the pair counter of the numbering kernel that follows in the stream starts from zero)
     if (FINE && pair_count != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0)
         *pair_count = 0;
+    if (FINE && (int)blockIdx.x > flag_blocks_x) {  // the workgroups that sort the rows
+        const int S_rounded = (int)gridDim.y * BLOCK_M;
+        if ((int)blockIdx.y * SORT_CHUNK < S_rounded)
+            sort_rows_part(bf + (int64_t)blockIdx.z * bf_stride_b, S, S_rounded, blockIdx.y, blockIdx.z, sorted);
+        return;
+    }
     if (FINE && (int)blockIdx.x >= flag_blocks_x) {  // the workgroups that sort the slices (see slice_order_part)
         const int part = blockIdx.y;
         if (part * RANKED_PER_GROUP < 4 * (int)gridDim.y)
@@ -457,6 +597,7 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
     int64_t fine_ss, int* __restrict__ order, int64_t order_sb, int flag_blocks_x, int flag_groups, const int* __restrict__ rows_moved, int* __restrict__ pair_count) {
     typedef typename std::conditional<GATHER, IndexedRows, GatheredRows>::type Rows;
     const int b = blockIdx.z;
+    if (rows_moved != nullptr && rows_moved[b] == 0) return;  // the plan in natural order stays
     Rows q_rows, k_rows;
     if constexpr (GATHER) {
         q_rows = IndexedRows{bf + (int64_t)b * bf_sb, idx_q, L};
@@ -472,7 +613,7 @@ __global__ __launch_bounds__(FLAG_WAVES * 64) void indexed_plan_kernel(
         if (part * RANKED_PER_GROUP < slots)
             slice_order_ranked([&](int base, unsigned long long* sk) { slice_keys_chunk_indexed(q_rows, Sq, ns, base, sk); }, ns,
                                slots, part, order + (int64_t)b * order_sb,
-                               rows_moved != nullptr && rows_moved[b] != 0 ? ORDER_MOVED : 0);
+                               rows_moved != nullptr ? ORDER_MOVED : 0);
         return;
     }
     __shared__ int64_t q_bits[BLOCK_M];
@@ -1110,129 +1251,37 @@ int launch_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int
     dim3 grid(flag_blocks_x, num_m, B);
     hipLaunchKernelGGL(tile_flags_kernel<false>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_stride_b, flags,
                        flags_stride_b, flags_stride_m, S, num_n, (uint8_t*)nullptr, (int64_t)0, (int64_t)0, (int*)nullptr,
-                       (int64_t)0, flag_blocks_x, flag_groups, (int*)nullptr);
+                       (int64_t)0, flag_blocks_x, flag_groups, (int*)nullptr, SortedRows{});
     return (int)hipGetLastError();
 }
 
 int launch_tile_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                      int64_t flags_stride_m, uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int* order,
-                     int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream) {
+                     int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream, int* rows, int64_t* rows_bits,
+                     int64_t rows_sb, int* rows_moved) {
     const int num_m = (S + BLOCK_M - 1) / BLOCK_M, num_n = (S + BLOCK_N - 1) / BLOCK_N;
     const int flag_groups = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
     const int flag_blocks_x = min(flag_groups, FLAG_MAX_BLOCKS_X);
     // one more column of workgroups: (flag_blocks_x, part, b) ranks 64 slices; 4 num_m slots need
-    // ceil(4 num_m / 64) <= num_m parts
-    dim3 grid(flag_blocks_x + 1, num_m, B);
+    // ceil(4 num_m / 64) <= num_m parts.  With sorted rows another one sorts, 1024 rows each
+    dim3 grid(flag_blocks_x + (rows != nullptr ? 2 : 1), num_m, B);
     hipLaunchKernelGGL(tile_flags_kernel<true>, grid, dim3(FLAG_WAVES * 64), 0, stream, bf, bf_stride_b, flags,
                        flags_stride_b, flags_stride_m, S, num_n, fine, fine_sb, fine_ss, order, order_sb, flag_blocks_x,
-                       flag_groups, pair_count);
+                       flag_groups, pair_count, SortedRows{rows, rows_bits, rows_sb, rows_moved});
     return (int)hipGetLastError();
 }
 
-// Sorts the rows of every sequence (whose slices are mixed enough) for launch_sorted_plan: text rows by position, then the modality rows grouped by their
-// bitfield, by position inside a group, then padding.  A counting sort over 64 classes; different bitfields may share a class (only
-// the packing of the slices suffers).  A workgroup places 1024 rows; it counts the classes of all rows for itself (512 KiB of
-// bitfields out of L2 for 65536 rows, eight loads in flight per thread) instead of waiting for the others.
-// Rows are only moved where at least one slice in SORT_MIXED holds text and modality rows: dK/dV gathers moved rows one by one,
-// which costs it 3 %.  Training step, 32 / 8 heads, D 128, natural -> sorted: 65536 tokens, 200 segments (20 % of the slices
-// mixed) 64.3 -> 48.2 ms; 8192 tokens, 30 segments (23 %) 1.87 -> 1.68 ms, 4 segments (3 %) 1.717 -> 1.722 ms; 16384 tokens, 4
-// segments (1.6 %) 7.36 -> 7.46 ms.
-constexpr int SORT_CHUNK = 1024, SORT_CLASSES = 64, SORT_MIXED = 32;
-__device__ __forceinline__ int sort_class(int64_t f) {
-    const uint64_t bits = (uint64_t)f & ((1ull << 62) - 1ull);
-    if (bits & 1) return 0;
-    if (bits == 0) return SORT_CLASSES - 1;
-    if ((bits & (bits - 1)) == 0) return 1 + (__ffsll((long long)bits) - 1) % (SORT_CLASSES - 2);
-    return 1 + (int)((bits * 0x9E3779B97F4A7C15ull) >> 40) % (SORT_CLASSES - 2);
-}
-__global__ __launch_bounds__(SORT_CHUNK) void sort_rows_kernel(const int64_t* __restrict__ bf, int64_t bf_sb, int S, int S_rounded,
-                                                              int* __restrict__ rows, int64_t* __restrict__ rows_bits,
-                                                              int64_t rows_sb, int* __restrict__ rows_moved,
-                                                              int* __restrict__ pair_count) {
-    __shared__ int s_mixed;
-    __shared__ int s_total[SORT_CLASSES], s_before[SORT_CLASSES], s_base[SORT_CLASSES];
-    __shared__ int s_wave[SORT_CHUNK / 64][SORT_CLASSES];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.y;
-    const int first = blockIdx.x * SORT_CHUNK;
-    if (pair_count != nullptr && blockIdx.x == 0 && b == 0 && tid == 0) *pair_count = 0;
-    const int64_t* row = bf + (int64_t)b * bf_sb;
-    if (tid < SORT_CLASSES) s_total[tid] = s_before[tid] = 0;
-    if (tid == 0) s_mixed = 0;
-    s_wave[wave][lane] = 0;
-    __syncthreads();
-    int mixed = 0;  // slices (in natural order) that hold text and modality rows, among those this wave has looked at
-    // every class of the wave's 64 rows at once: add(class, count, this lane's number among the earlier ones)
-    auto classes = [&](int cls, auto add) {
-        unsigned long long left = __ballot(cls >= 0);
-        while (left != 0) {  // wave-uniform
-            const int c = __builtin_amdgcn_readlane(cls, __builtin_ctzll(left));
-            const unsigned long long same = __ballot(cls == c);
-            add(c, same);
-            left &= ~same;
-        }
-    };
-    constexpr int AHEAD = 8;
-    for (int i0 = 0; i0 < S; i0 += AHEAD * SORT_CHUNK) {
-        int64_t f[AHEAD];
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            const int i = i0 + u * SORT_CHUNK + tid;
-            f[u] = i < S ? row[i] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            const int chunk = i0 + u * SORT_CHUNK, i = chunk + tid;
-            const int cls = i < S ? sort_class(f[u]) : -1;
-            const unsigned long long text = __ballot(cls == 0), modal = __ballot(cls > 0 && cls < SORT_CLASSES - 1);
-            mixed += ((unsigned)text != 0 && (unsigned)modal != 0) + ((text >> 32) != 0 && (modal >> 32) != 0);
-            classes(cls, [&](int c, unsigned long long same) {
-                if (lane == 0) {
-                    atomicAdd(&s_total[c], __popcll(same));
-                    if (chunk < first) atomicAdd(&s_before[c], __popcll(same));
-                }
-            });
-        }
-    }
-    if (lane == 0) atomicAdd(&s_mixed, mixed);
-    const int mine = first + tid;
-    const int64_t f = mine < S ? row[mine] : 0;
-    const int cls = mine < S ? sort_class(f) : -1;
-    int earlier = 0;  // rows of my class in front of me in the wave
-    classes(cls, [&](int c, unsigned long long same) {
-        if (lane == 0) s_wave[wave][c] = __popcll(same);
-        if (cls == c) earlier = __popcll(same & ((1ull << lane) - 1ull));
-    });
-    __syncthreads();
-    if (tid < SORT_CLASSES) {
-        int base = 0;
-        for (int c = 0; c < tid; ++c) base += s_total[c];
-        s_base[tid] = base + s_before[tid];
-        int run = 0;
-        for (int w = 0; w < SORT_CHUNK / 64; ++w) {
-            const int n = s_wave[w][tid];
-            s_wave[w][tid] = run;
-            run += n;
-        }
-    }
-    __syncthreads();
-    const bool move = s_mixed * SORT_MIXED >= (S + 31) / 32;
-    if (blockIdx.x == 0 && tid == 0) rows_moved[b] = move ? 1 : 0;
-    if (mine < S) {
-        const int64_t at = (int64_t)b * rows_sb + (move ? s_base[cls] + s_wave[wave][cls] + earlier : mine);
-        rows[at] = mine;
-        rows_bits[at] = f;
-    } else if (mine < S_rounded) {
-        rows[(int64_t)b * rows_sb + mine] = S;
-        rows_bits[(int64_t)b * rows_sb + mine] = 0;
-    }
-}
-
-int launch_sorted_plan(const int64_t* bf, int64_t bf_stride_b, int* rows, int64_t* rows_bits, int64_t rows_sb, int* rows_moved, uint8_t* fine,
-                       int64_t fine_sb, int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B, int S,
-                       hipStream_t stream) {
+// Flags and plan in natural order and the sorted rows in one launch; a second one replaces the plan of the sequences whose rows have
+// been moved (the workgroups of the others end at once).  Builder in us, natural order -> here: 17000 tokens, where nothing moves, 28 -> 33
+// (a forward over 24637 tokens, 16 heads, D 80: 1.02 times as long with a sort and a whole second plan in front); 65536 tokens,
+// moved, 230 -> 420.
+int launch_sorted_plan(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b, int64_t flags_stride_m,
+                       int* rows, int64_t* rows_bits, int64_t rows_sb, int* rows_moved, uint8_t* fine, int64_t fine_sb,
+                       int64_t fine_ss, int* order, int64_t order_sb, int* pair_count, int B, int S, hipStream_t stream) {
+    const int rc = launch_tile_plan(bf, bf_stride_b, flags, flags_stride_b, flags_stride_m, fine, fine_sb, fine_ss, order, order_sb,
+                                    pair_count, B, S, stream, rows, rows_bits, rows_sb, rows_moved);
+    if (rc != 0) return rc;
     const int num_m = (S + BLOCK_M - 1) / BLOCK_M, num_n = (S + BLOCK_N - 1) / BLOCK_N;
-    hipLaunchKernelGGL(sort_rows_kernel, dim3((num_m * BLOCK_M + SORT_CHUNK - 1) / SORT_CHUNK, B), dim3(SORT_CHUNK), 0, stream, bf,
-                       bf_stride_b, S, num_m * BLOCK_M, rows, rows_bits, rows_sb, rows_moved, pair_count);
     const int flag_groups = (num_n + FLAG_COLS_PER_BLOCK - 1) / FLAG_COLS_PER_BLOCK;
     const int flag_blocks_x = min(flag_groups, FLAG_MAX_BLOCKS_X);
     hipLaunchKernelGGL(indexed_plan_kernel<false>, dim3(flag_blocks_x + 1, num_m, B), dim3(FLAG_WAVES * 64), 0, stream,

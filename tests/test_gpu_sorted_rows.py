@@ -1,4 +1,4 @@
-"""Plans with sorted rows (``bam_tile_plan_sorted_counted``; the public functions take them from 16384 tokens on): their contents
+"""Plans with sorted rows (``bam_tile_plan_sorted_counted``; the public functions take them from 32768 tokens on): their contents
 against the definition, and attention with them against attention with a plan in natural order."""
 
 import ctypes
@@ -142,9 +142,11 @@ def test_attention_does_not_depend_on_the_order_of_the_rows(S, D, handover, bias
         assert torch.isfinite(a).all() and rel_l2(a.float(), b.float()) <= 2.0**-8, name
 
 
-@pytest.mark.parametrize("S,D", [(16384, 64), (16500, 128)])
-def test_the_public_function_takes_it_from_16384_tokens_on(S, D):
+@pytest.mark.parametrize("S,D", [(32768, 64), (32900, 128)])
+def test_the_public_function_takes_it_from_32768_tokens_on(S, D):
     Hq, Hkv = 2, 1
+    below = random_bitfield(1, 32767, seed=1).to(dev())
+    assert not BA.BitfieldUtils.plan_for(BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(below), below).struct.rows
     g = torch.Generator(device=dev()).manual_seed(S)
     q, k, v, do = (torch.randn(1, S, H, D, generator=g, device=dev()).bfloat16() for H in (Hq, Hkv, Hkv, Hq))
     bf = random_bitfield(1, S, seed=1).to(dev())
