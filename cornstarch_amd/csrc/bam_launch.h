@@ -110,10 +110,17 @@ inline bool dkdv_far(const AttnParams& p) {
     return far_rows(p.q, p.Sq, p.d) || far_rows(p.dout, p.Sq, p.d) || far_rows(p.k, p.Sk, p.d) || far_rows(p.v, p.Sk, p.d);
 }
 
-// Whether the forward and dQ walk two tiles at a time (measured at launch_fwd_b and launch_dq_f).
+// Whether the forward and dQ walk two tiles at a time (measured at launch_fwd_b and launch_dq_f).  One workgroup with one stream
+// needs about 1.4 us a tile (D 128) whether it shares its compute unit or not, so that up to some 800 workgroups the longest list
+// decides, not the sum; two streams take 1.85 us for two tiles, but a unit then runs its workgroups one after the other and shows
+// each one's first loads and stores, which short lists do not win back.
 inline bool two_streams(const AttnParams& p) {
     const int64_t units = (int64_t)p.num_m * p.B * p.Hq;
-    return units <= (p.D > 64 ? 256 : 512) || (p.D <= 32 && units <= 1024 && p.Sk >= 2560);
+    int64_t most = p.D > 64 && p.Sk < 2000 ? 384 : 512;
+    if (p.D <= 32 && p.Sk >= 2560) most = p.bias != nullptr ? 768 : 1024;
+    if (p.D > 32 && p.mask_mode != MASK_INDEXED && p.mask_mode != MASK_DENSE && p.bias == nullptr)
+        most = p.Sk >= (p.D > 64 ? 8192 : 4608) ? 768 : p.Sk >= 3072 ? 640 : most;
+    return units <= most;
 }
 
 // Single-token decode step (one query row per batch element and head, no mask); strides in elements.

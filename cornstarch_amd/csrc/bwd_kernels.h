@@ -1235,8 +1235,9 @@ static int launch_dq_s(const AttnParams& p, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 // Two streams where the forward takes them.  dQ alone, us, one stream -> two: D 64, 1000 tokens, 8 heads 27.1 -> 22.7, 1024, 32 heads
-// 29.4 -> 25.1, 2 x 700 28.4 -> 27.2, 2048 (512 workgroups) 50.9 -> 49.8, 3001 (768) 77 -> 87; with a bias 2 x 2048, 16 heads 64.1 ->
-// 59.2; D 32: 2048 46.4 -> 35.9, 3001 64.1 -> 52.9, 4096 (1024) 84.3 -> 77.0, 8 x 300 (768) 18.8 -> 24.3.
+// 29.4 -> 25.1, 2 x 700 28.4 -> 27.2, 2048 (512 workgroups) 50.9 -> 49.8, 3001 (768) 77 -> 87, 4096 (640) 91.6 -> 81.1, 5000 (640)
+// 108 -> 90, 24000 (752) 497 -> 428; with a bias 2 x 2048, 16 heads 64.1 -> 59.2; D 32: 2048 46.4 -> 35.9, 3001 64.1 -> 52.9, 4096
+// (1024) 84.3 -> 77.0, 8 x 300 (768) 18.8 -> 24.3.
 template <typename T, int D, int BIAS, bool LONG>
 static int launch_dq_f(const AttnParams& p, hipStream_t stream) {
     if constexpr (!LONG && D <= 64)  // (above, dQ is computed from the stored dS but for rare calls)

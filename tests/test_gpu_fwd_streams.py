@@ -60,3 +60,23 @@ def test_gradients_of_a_sequence_of_a_large_batch_equal_those_alone(S, D, biased
             # o and the lse differ by a rounding of P to bf16 (2^-9 a term), which delta and P carry into the gradients
             assert torch.isfinite(one).all() and rel_l2(one[0].float(), all_[b].float()) <= 2.0**-7
     BA.BitfieldUtils.clear_cache()
+
+
+# either side of the lines up to which two tiles are walked at a time: (few sequences: two, more of them: one)
+@pytest.mark.parametrize("D,S,few,many", [(32, 2570, 3, 7), (64, 3100, 3, 4), (64, 5000, 2, 3), (96, 2005, 4, 5), (128, 1990, 3, 4), (128, 3100, 3, 4), (128, 8200, 1, 2)])
+def test_long_lists_on_either_side_of_the_line(D, S, few, many):
+    Hq, Hkv = 8, 2
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v, do = ((torch.randn(many, S, H, D, generator=g, device="cuda")).bfloat16() for H in (Hq, Hkv, Hkv, Hq))
+    bf = random_bitfield(many, S, seed=S, pad=S // 9).cuda()
+
+    def run(n):
+        BA.BitfieldUtils.clear_cache()
+        x = [t[:n].detach().requires_grad_(True) for t in (q, k, v)]
+        o = BA.bitfield_attn_func(*x, bf[:n].contiguous())
+        return o.detach(), *torch.autograd.grad(o, x, do[:n])
+
+    for bound, one, two in zip((2.0**-8, 2.0**-7, 2.0**-7, 2.0**-7), run(many), run(few)):  # (as above)
+        for b in range(few):
+            assert torch.isfinite(two[b]).all() and rel_l2(two[b].float(), one[b].float()) <= bound
+    BA.BitfieldUtils.clear_cache()
