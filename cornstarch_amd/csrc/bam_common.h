@@ -336,6 +336,15 @@ __device__ __forceinline__ void xcd_group_map(int bid, int num_units, int G, int
     }
 }
 
+// Workgroups come with falling amounts of work, two to a compute unit.  Where they all start at once (257 to 512 of them) the
+// second one of a unit should be short where the first is long: those from the 257th on are taken in reverse order, eight (one
+// per XCD) at a time.
+__device__ __forceinline__ int mirror_second(int bid, int blocks) {
+    constexpr int UNITS = 256;
+    const int full = blocks & ~7;
+    return blocks <= UNITS || blocks > 2 * UNITS || bid < UNITS || bid >= full ? bid : UNITS + full - 8 - (bid & ~7) + (bid & 7);
+}
+
 // Which (batch x row-group index, kv head, member of the kv group) a workgroup of the forward / dQ kernels takes.
 // Within an XCD the hardware deals consecutive workgroups to the four shader engines in turn and starts them strictly
 // in order, so four consecutive workgroups of an XCD should carry the same amount of work or the engines with the

@@ -80,3 +80,25 @@ def test_long_lists_on_either_side_of_the_line(D, S, few, many):
         for b in range(few):
             assert torch.isfinite(two[b]).all() and rel_l2(two[b].float(), one[b].float()) <= bound
     BA.BitfieldUtils.clear_cache()
+
+
+# dQ from the stored dS with 257 to 512 workgroups: long and short ones share a compute unit; with 258 and 270 of them the last ones
+# are not whole runs of eight
+@pytest.mark.parametrize("B,Hq,Hkv,S", [(3, 6, 3, 1900), (1, 6, 6, 43 * 128), (2, 16, 4, 2047), (8, 8, 8, 515)])
+def test_dq_of_workgroups_taken_in_another_order(B, Hq, Hkv, S):
+    D = 128
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v, do = ((torch.randn(B, S, H, D, generator=g, device="cuda")).bfloat16() for H in (Hq, Hkv, Hkv, Hq))
+    bf = random_bitfield(B, S, seed=S, pad=S // 9).cuda()
+
+    def dq(heads, kv):  # one kv head at a time: 43 to 64 workgroups, in the order of their lengths
+        BA.BitfieldUtils.clear_cache()
+        x = [t.detach().requires_grad_(True) for t in (q[:, :, heads], k[:, :, kv], v[:, :, kv])]
+        return torch.autograd.grad(BA.bitfield_attn_func(*x, bf), x[0], do[:, :, heads])[0]
+
+    whole, G = dq(slice(None), slice(None)), Hq // Hkv
+    for h in range(Hkv):
+        part = dq(slice(h * G, (h + 1) * G), slice(h, h + 1))
+        # (another number of workgroups decides about the forward's streams: a rounding of P to bf16, as above)
+        assert torch.isfinite(whole).all() and rel_l2(whole[:, :, h * G : (h + 1) * G].float(), part.float()) <= 2.0**-7
+    BA.BitfieldUtils.clear_cache()
