@@ -116,8 +116,9 @@ inline bool dkdv_far(const AttnParams& p) {
 // each one's first loads and stores, which short lists do not win back.
 inline bool two_streams(const AttnParams& p) {
     const int64_t units = (int64_t)p.num_m * p.B * p.Hq;
-    int64_t most = p.D > 64 && p.Sk < 2000 ? 384 : 512;
-    if (p.D <= 32 && p.Sk >= 2560) most = p.bias != nullptr ? 768 : 1024;
+    if (p.Sk <= (p.D > 32 ? 128 : 64)) return false;  // a tile or two: nothing to share
+    int64_t most = p.Sk < 768 ? 256 : p.Sk < 1152 ? 384 : p.Sk < 1600 ? 480 : 512;
+    if (p.D <= 32) most = p.Sk < 192 ? 256 : p.Sk < 384 ? 448 : p.Sk < 2560 ? 512 : p.bias != nullptr ? 768 : 1024;
     if (p.D > 32 && p.mask_mode != MASK_INDEXED && p.mask_mode != MASK_DENSE && p.bias == nullptr)
         most = p.Sk >= (p.D > 64 ? 8192 : 4608) ? 768 : p.Sk >= 3072 ? 640 : most;
     return units <= most;

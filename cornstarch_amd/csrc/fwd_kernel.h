@@ -537,13 +537,16 @@ static int launch_fwd_s(const AttnParams& p, hipStream_t stream) {
 // Two streams halve the chain of tiles a workgroup walks and double the waves of a compute unit that has one workgroup; the price
 // is a workgroup that fills the unit (D = 64 and above), so that nothing runs beside its first loads and its stores.  Forward
 // kernel alone, bf16, us, one stream -> two (workgroups in brackets):
-//   D 128:  1000 tokens (384) 36.2 -> 34.5, (512) 37.7 -> 42.5;  1500 (384) 45.9 -> 36.6, (480) 47.8 -> 47.5;  2000 (384) 53.5 ->
+//   D 128:  60 tokens (64) 8.3 -> 9.9;  120 (288) 14.5 -> 21.9;  250 (256) 17.4 -> 16.3, (384) 19.7 -> 25.6;  640 (240) 24.0 ->
+//           21.0, (320) 26.2 -> 28.3;  1000 (384) 36.2 -> 34.5, (512) 37.7 -> 42.5;  1500 (384) 45.9 -> 36.6, (480) 47.8 -> 47.5;  2000 (384) 53.5 ->
 //           42.8, (512) 55.1 -> 54.7, (640) 58.2 -> 64.4;  3200 (500) 78.5 -> 69.0, (600) 81.6 -> 76.2, (775) 88.4 -> 104.1;  5000
 //           (400) 109 -> 83, (640) 121 -> 102, (760) 129 -> 135;  12000 (564) 268 -> 201;  24000 (752) 588 -> 510, D 80, 32000 (1000)
 //           771 -> 828
-//   D 64:   1000 (640) 32.2 -> 40.3;  2600 (630) 56.5 -> 51.8, (756) 58.5 -> 62.9;  4096 (640) 78.1 -> 66.2, (768) 80.7 -> 80.4;
+//   D 64:   60 (256) 7.6 -> 8.7;  250 (256) 14.0 -> 12.4, (384) 15.3 -> 19.4;  640 (320) 21.8 -> 22.3, (480) 23.0 -> 26.8;  900
+//           (384) 26.9 -> 25.6, (512) 28.7 -> 30.6;  1500 (480) 37.1 -> 33.1;  1000 (640) 32.2 -> 40.3;  2600 (630) 56.5 -> 51.8, (756) 58.5 -> 62.9;  4096 (640) 78.1 -> 66.2, (768) 80.7 -> 80.4;
 //           6500 (765) 117 -> 110;  24000 (752) 421 -> 336;  8000 (1008) 156 -> 173
-//   D 32 (two such workgroups fit a unit):  2048 (512) 37.8 -> 28.2, 3001 (768) 52.4 -> 40.7, 4096 (1024) 69 -> 61, but with short
+//   D 32 (two such workgroups fit a unit):  60 (64) 6.9 -> 7.5;  120 (288) 9.9 -> 10.7;  250 (384) 13.3 -> 12.1, (512) 13.8 ->
+//           14.1;  500 (512) 18.1 -> 16.8;  2048 (512) 37.8 -> 28.2, 3001 (768) 52.4 -> 40.7, 4096 (1024) 69 -> 61, but with short
 //           lists 8 x 300 (768) 16.0 -> 19.5, 4 x 1024 (1024) 27.8 -> 30.4;  with a bias 4096 (640) 82 -> 77, (1024) 85 -> 107
 //   above 512 workgroups, D 128:  bool masks 4096 (640) 98 -> 104, 8192 (768) 203 -> 217;  index tensors 8192 (640) 222 -> 229;
 //           bias 4096 (640) 116 -> 121
