@@ -38,10 +38,8 @@ __device__ __forceinline__ void dma_b128_stream(const void* sbase, unsigned voff
                  : "memory");
 }
 // The 16-byte copy through a buffer descriptor over [base, base + DMA_RANGE): a lane whose offset lies beyond reads nothing
-// and the hardware writes zeros to its LDS slot.  The descriptor's last two words stay in registers over the loop; K tiles
-// copied this way instead of by dma_b128, whole step: 1 x 8192 tokens, D 128 no change (1903 / 1904 us), 8 x 4096, D 64
-// 1142 / 1147, decode of 8 x 8192 keys 48.7 / 48.7.  The forward at D 32 (2 x 2048 tokens, 16 heads) takes 30.5 us with dma_b128,
-// 31.7 with K alone copied this way and 31.5 with K and V; 1 x 8192 tokens 130 / 134 / 131.
+// and the hardware writes zeros to its LDS slot.  For the K tiles of the decode step (8 x 8192 keys: 48.7 us either way); the other
+// kernels copy through RowView.
 constexpr unsigned DMA_RANGE = 0x80000000u, DMA_ZERO = 0xC0000000u;  // (room below for 31 rows of 2^24 bytes: decode steps back)
 template <int SITE = 0>
 __device__ __forceinline__ void dma_b128_ranged(const void* sbase, unsigned voff, unsigned lds_base) {
