@@ -887,6 +887,9 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
                        a->dv.ptr, m, a->flags, st, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->accumulate, true, true,
                        a->bias, nullptr, true));
     all.o = {a->o.ptr, a->o.stride_b, a->o.stride_s, a->o.stride_h};
+    if (reinterpret_cast<uintptr_t>(a->lse_scaled) & 3u)
+        return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: lse_scaled is not 4-byte aligned");
+    all.lse_scaled = a->bias == nullptr && all.D <= 64 ? a->lse_scaled : nullptr;
     // head dims up to 64: the dQ kernel runs first and computes delta on the way; above, dK/dV needs it first
     const bool dq_first = all.D <= 64;
     if (!dq_first) BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
@@ -923,6 +926,7 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         skip(p.dv, hk, gsz);
         p.lse += (int64_t)r * hq * p.Sq_rounded;
         p.delta += (int64_t)r * hq * p.Sq_rounded;
+        if (p.lse_scaled != nullptr) p.lse_scaled += (int64_t)r * hq * p.Sq_rounded;
         p.Hq = hq;
         p.Hkv = hk;
         if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));

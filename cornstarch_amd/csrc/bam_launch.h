@@ -36,6 +36,7 @@ struct AttnParams {
     int kv_parts;
     float* lse;                // (B, Hq, Sq_rounded)
     float* delta;              // (B, Hq, Sq_rounded)
+    float* lse_scaled;         // head dims up to 64: lse * log2(e), from the dQ kernel to dK/dV; null = dK/dV scales lse itself
     // Bitfields of the query rows (B, Sq) and of the keys (B, Sk), and their global positions.  Plain
     // attention: both point at the one bitfield tensor and the positions are null (position = row /
     // column number).  Index-tensor attention (context-parallel shards): gathered copies and positions.

@@ -6,7 +6,7 @@ namespace bam {
 
 template <typename T, int D>
 static int launch_dkdv_save_t(const AttnParams& p, hipStream_t stream) {
-    return p.bias != nullptr ? launch_dkdv_save_b<T, D, true>(p, stream) : launch_dkdv_save_b<T, D, false>(p, stream);
+    return p.bias != nullptr ? launch_dkdv_b<T, D, true, false, true>(p, stream) : launch_dkdv_b<T, D, false, false, true>(p, stream);
 }
 
 int launch_bwd_dkdv_save(const AttnParams& p, int dtype, hipStream_t stream) {

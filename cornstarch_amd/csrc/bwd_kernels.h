@@ -85,7 +85,11 @@ constexpr int DKDV_THREADS = 512;
 // no pass loop at all (a loop around the main loop costs registers and a few per cent).
 // SAVE: every wave also stores its 32 x 32 block of -dS / scale (the packed operand of the dK product) to p.ds_ws, where
 // the dQ kernel of bwd_dq_saved.h picks it up instead of recomputing S and dP.  Record and block layout: AttnParams.
-template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false>
+// SCALED (head dims up to 64, where the dQ kernel runs first): the rows' lse * log2(e) comes from there (p.lse_scaled), the same
+// numbers with one of some seven vector instructions per MFMA less.  dK/dV alone, us: 8 x 4096 tokens, 16 heads, D 64 582 -> 560,
+// 3001, 32 / 8 heads 103 -> 100, D 32, 4096 118 -> 111.  (Above D 64 the delta pre-pass would have to write it: 8192 tokens, 32 / 8
+// heads, D 128 dK/dV 957 -> 943 but the pre-pass 22.9 -> 27.2, 25.6 with the rows of a head side by side; 4 x 1537 no gain.)
+template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false, bool SCALED = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
     constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
@@ -254,7 +258,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         hv.q.init((const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)h * p.q.sh), 2 * p.q.ss, Sq, 2 * p.d);
         hv.g.init((const char*)p.dout.ptr + 2 * ((int64_t)b * p.dout.sb + (int64_t)h * p.dout.sh), 2 * p.dout.ss, Sq, 2 * p.d);
         if (small < 2)
-            hv.small.init((small == 0 ? p.lse : p.delta) + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded, 4, Sq, 4);
+            hv.small.init((small == 0 ? (SCALED ? p.lse_scaled : p.lse) : p.delta) + (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded, 4, Sq, 4);
         else if (DENSE)  // (one row per slice)
             hv.small.init(p.col_bits + (int64_t)b * p.col_bits_sb + nt * 128 + (small - 2) * 64, p.col_bits_ss * 4, (Sq + 31) >> 5, 256);
         else
@@ -439,7 +443,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
         for (int grp = 0; grp < 4; ++grp) {
             const f32x4 l4 = *(const f32x4*)&sLse[cur][qr + 8 * grp + 4 * hi];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) s[4 * grp + x] = __builtin_amdgcn_exp2f(fmaf(s[4 * grp + x], c2, l4[x] * -LOG2E));
+            for (int x = 0; x < 4; ++x) s[4 * grp + x] = __builtin_amdgcn_exp2f(fmaf(s[4 * grp + x], c2, SCALED ? -l4[x] : l4[x] * -LOG2E));
         }
         if (DENSE) {
             if (cls == 1 && col_bits_on) {
@@ -840,7 +844,11 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
 #pragma unroll
             for (int kk = 0; kk < (D <= 64 ? KK : 1); ++kk) part[kk] = chunk_dot<T>(oreg[kk], greg[kk]);
             dlt = half_swap_sum(KK == 4 ? (part[0] + part[2]) + (part[1] + part[KK - 1]) : part[0] + part[1]);
-            if (stream == 0 && qvalid && hi == 0) p.delta[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] = dlt;
+            if (stream == 0 && qvalid && hi == 0) {
+                const int64_t at = (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow;
+                p.delta[at] = dlt;
+                if (p.lse_scaled != nullptr) p.lse_scaled[at] = lse_row * LOG2E;
+            }
         }
         qb = make_query_bits(qf, qpos);
         lse2 = (!qvalid || lse_row == -INFINITY) ? INFINITY : lse_row * LOG2E;
@@ -1191,37 +1199,28 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
 // such workgroups: 16 us, their LDS keeps them from running beside each other).
 inline bool rows_may_be_moved(const AttnParams& p) { return p.rows != nullptr && p.rows_known != BAM_ROWS_LEFT; }
 inline bool rows_may_be_left(const AttnParams& p) { return p.rows == nullptr || p.rows_known != BAM_ROWS_MOVED; }
-template <typename T, int D, bool BIAS, bool LONG>
-static int launch_dkdv_b(const AttnParams& p, hipStream_t stream) {
+template <typename T, int D, bool BIAS, bool LONG, bool SAVE, bool SCALED>
+static int launch_dkdv_m(const AttnParams& p, hipStream_t stream) {
     const int blocks = p.num_kt * p.B * p.Hkv;  // one workgroup per 128-key tile
     if (p.mask_mode == MASK_INDEXED)
-        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, LONG, SAVE, SCALED>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     else if (p.mask_mode == MASK_DENSE)
-        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_DENSE, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_DENSE, BIAS, LONG, SAVE, SCALED>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     else {
         if constexpr (!LONG) {  // (beyond, there are no sorted rows)
             if (rows_may_be_moved(p))
-                hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_SORTED, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+                hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_SORTED, BIAS, LONG, SAVE, SCALED>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
         }
         if (LONG || rows_may_be_left(p))
-            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, LONG>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
+            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, LONG, SAVE, SCALED>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     }
     return (int)hipGetLastError();
 }
-template <typename T, int D, bool BIAS>
-static int launch_dkdv_save_b(const AttnParams& p, hipStream_t stream) {
-    const int blocks = p.num_kt * p.B * p.Hkv;
-    if (p.mask_mode == MASK_INDEXED)
-        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-    else if (p.mask_mode == MASK_DENSE)
-        hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_DENSE, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-    else {
-        if (rows_may_be_moved(p))
-            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_SORTED, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-        if (rows_may_be_left(p))
-            hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, false, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-    }
-    return (int)hipGetLastError();
+template <typename T, int D, bool BIAS, bool LONG, bool SAVE = false>
+static int launch_dkdv_b(const AttnParams& p, hipStream_t stream) {
+    if constexpr (!BIAS && !LONG && D <= 64)
+        if (p.lse_scaled != nullptr) return launch_dkdv_m<T, D, BIAS, LONG, SAVE, true>(p, stream);
+    return launch_dkdv_m<T, D, BIAS, LONG, SAVE, false>(p, stream);
 }
 template <typename T, int D, int BIAS, bool LONG, int STREAMS>
 static int launch_dq_s(const AttnParams& p, hipStream_t stream) {

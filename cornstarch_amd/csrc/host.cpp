@@ -406,7 +406,8 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
                   const Tensor& lse, const Tensor& dq, const Tensor& dk, const Tensor& dv, bool accumulate) {
     const c10::DeviceGuard guard(q.device());
     const at::NoGradGuard no_grad;
-    Tensor delta = at::empty_like(lse);
+    const bool scaled = q.size(3) <= 64 && c.bias == nullptr;
+    Tensor delta = at::empty({(scaled ? 2 : 1) * lse.numel()}, lse.options());  // and the scaled lse
     bam_plan desc = {};  // (its own copy: what is known of the rows may still change)
     if (plan) {
         plan.core->look();
@@ -422,6 +423,7 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     a.dv = tensor4(dv);
     a.lse = lse.data_ptr<float>();
     a.delta = delta.data_ptr<float>();
+    if (scaled) a.lse_scaled = a.delta + lse.numel();
     a.accumulate = accumulate ? 1 : 0;
     Tensor ws;
     if (plan && desc.rows != nullptr && a.D <= 64) {  // (one launch of dK/dV instead of two; it is there by the time the forward starts)

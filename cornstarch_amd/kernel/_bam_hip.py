@@ -114,6 +114,7 @@ class Attn(ctypes.Structure):
         ("scale", ctypes.c_float),
         ("parts_workspace", ctypes.c_void_p),
         ("parts_bytes", ctypes.c_int64),
+        ("lse_scaled", ctypes.c_void_p),
     ]
 
 
