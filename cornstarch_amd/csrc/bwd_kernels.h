@@ -86,8 +86,8 @@ constexpr int DKDV_THREADS = 512;
 // SAVE: every wave also stores its 32 x 32 block of -dS / scale (the packed operand of the dK product) to p.ds_ws, where
 // the dQ kernel of bwd_dq_saved.h picks it up instead of recomputing S and dP.  Record and block layout: AttnParams.
 // SCALED (head dims up to 64, where the dQ kernel runs first): the rows' lse * log2(e) comes from there (p.lse_scaled), the same
-// numbers with one of some seven vector instructions per MFMA less.  dK/dV alone, us: 8 x 4096 tokens, 16 heads, D 64 582 -> 560,
-// 3001, 32 / 8 heads 103 -> 100, D 32, 4096 118 -> 111.  (Above D 64 the delta pre-pass would have to write it: 8192 tokens, 32 / 8
+// numbers with one of some seven vector instructions per MFMA less.  dK/dV alone, us: 8 x 4096 tokens, 16 heads, D 64 581 -> 571
+// (0.6 % of the step), 3001, 32 / 8 heads 103.4 -> 101.5, D 32, 4096 118 -> 112.  (Above D 64 the delta pre-pass would have to write it: 8192 tokens, 32 / 8
 // heads, D 128 dK/dV 957 -> 943 but the pre-pass 22.9 -> 27.2, 25.6 with the rows of a head side by side; 4 x 1537 no gain.)
 template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false, bool SCALED = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
