@@ -186,6 +186,72 @@ Plan plan_of(const py::object& o) {
     return Plan{o.cast<std::shared_ptr<PlanCore>>(), hold(o)};
 }
 
+void hip_check(hipError_t e, const char* what) {
+    if (e == hipSuccess) return;
+    (void)hipGetLastError();
+    throw BamFailure(std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// What one call computed and a later one may find again (flags, plan, gathered index arrays), and the stream that computes it.  A
+// later call on that stream just uses it.  On another one it first waits for an event behind the launches, and the caching allocator
+// learns that this stream uses the memory too.  An event costs the stream it is recorded on 4.7 us, so it is recorded when the first
+// such call asks; a stream that torch does not own may be gone by then, or share its handle with another, and gets it at once.
+class Prepared {
+public:
+    // after the launches
+    Prepared(Stream stream, std::vector<Tensor> results, std::shared_ptr<PlanCore> plan)
+        : stream_(stream), results_(std::move(results)), plan_(std::move(plan)) {
+        if (plan_) results_.push_back(plan_->workspace);
+        if (external()) record();
+    }
+    Prepared(const Prepared&) = delete;
+    ~Prepared() {
+        if (event_ != nullptr) (void)hipEventDestroy(event_);
+    }
+    // Call before the results are used on the current stream.  False: they cannot be, the caller has to compute its own.
+    bool use() {
+        const Stream now = current_stream(stream_.device());
+        if (now == stream_ && !external()) return true;
+        const std::lock_guard<std::mutex> lock(mutex_);
+        if (!done_) {
+            const c10::DeviceGuard guard(stream_.device());
+            const c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+            if (event_ == nullptr) {
+                hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+                if (stream_.stream() != nullptr) hip_check(hipStreamIsCapturing(stream_.stream(), &status), "state of a stream");
+                if (status != hipStreamCaptureStatusNone) return false;  // (the event would become part of that graph)
+                record();
+            }
+            if (now.stream() != nullptr && capturing()) {  // (replays run on any stream: the results are there before the capture goes on)
+                hip_check(hipEventSynchronize(event_), "wait for a plan");
+                done_ = true;
+            } else if (hipEventQuery(event_) == hipSuccess) {
+                done_ = true;
+            } else {
+                (void)hipGetLastError();
+                hip_check(hipStreamWaitEvent(now.stream(), event_, 0), "wait for a plan");
+            }
+        }
+        for (const Tensor& t : results_) t.record_stream(c10::Stream::unpack3(now.id(), now.device_index(), c10::DeviceType::CUDA));
+        return true;
+    }
+
+private:
+    // (the id of a stream of torch's own is not its handle, except for the default stream, whose handle is null)
+    bool external() const { return stream_.stream() != nullptr && stream_.id() == reinterpret_cast<int64_t>(stream_.stream()); }
+    void record() {
+        const c10::DeviceGuard guard(stream_.device());
+        hip_check(hipEventCreateWithFlags(&event_, hipEventDisableTiming), "event behind a plan");
+        hip_check(hipEventRecord(event_, stream_.stream()), "event behind a plan");
+    }
+    const Stream stream_;
+    std::vector<Tensor> results_;
+    const std::shared_ptr<PlanCore> plan_;
+    std::mutex mutex_;
+    hipEvent_t event_ = nullptr;
+    bool done_ = false;
+};
+
 // ------------------------------------------------------------------ caches (one entry each; guarded by the GIL)
 // An entry belongs to the very memory it was computed from: it keeps that tensor alive and compares address, shape,
 // strides, device and version counter.
@@ -193,7 +259,10 @@ struct Cached {
     Tensor owner, flags;
     uint32_t version = 0;
     Plan plan;
-    bool hit(const Tensor& t) const {
+    std::shared_ptr<Prepared> prepared;
+    // whether this is the entry of `t`; flags and plan are then ready for the current stream
+    bool hit(const Tensor& t) const { return matches(t) && (!prepared || prepared->use()); }
+    bool matches(const Tensor& t) const {
         return !t.is_inference() && owner.defined() && flags.defined() && owner.data_ptr() == t.data_ptr() && owner.sizes() == t.sizes() &&
                owner_strides == t.strides() && version == t._version() && owner.device() == t.device();
     }
@@ -201,13 +270,14 @@ struct Cached {
 };
 Cached g_bitfield, g_mask;
 
-void store(Cached& slot, const Tensor& owner, const Tensor& flags, Plan plan) {
+void store(Cached& slot, const Tensor& owner, const Tensor& flags, Plan plan, const Stream& stream) {
     if (owner.is_inference()) return;  // no version counter: nothing would tell that it has been written to
     Cached fresh;
     fresh.owner = owner;
     fresh.owner_strides = owner.strides().vec();
     fresh.flags = flags;
     fresh.version = owner._version();
+    fresh.prepared = std::make_shared<Prepared>(stream, std::vector<Tensor>{flags}, plan.core);
     fresh.plan = std::move(plan);
     std::swap(slot, fresh);  // the old entry goes after the new one is in place: its end may run Python code, which may call here
 }
@@ -266,7 +336,7 @@ Flags bitfield_flags(const Tensor& mask) {
                              (int)B, (int)S, stream.stream()),
               "bam_tile_flags");
     }
-    store(g_bitfield, mask, flags, plan);
+    store(g_bitfield, mask, flags, plan, stream);
     return {flags, plan};
 }
 
@@ -310,7 +380,7 @@ Flags mask_flags(const Tensor& mask) {
                                   stream.stream()),
               "bam_mask_tile_flags");
     }
-    store(g_mask, mask, flags, plan);
+    store(g_mask, mask, flags, plan, stream);
     return {flags, plan};
 }
 
@@ -684,7 +754,7 @@ py::object backward(Tensor dout, const Tensor& q, const Tensor& k, const Tensor&
 }
 
 // Index-tensor attention: gathers bitfields and positions of rows and keys, fills the bam_index_view at `view` and builds
-// the plan.  -> (tensors to keep alive, plan or None)
+// the plan.  -> (the arrays as a Prepared, plan or None)
 py::tuple index_view(const Tensor& bf, const Tensor& idx_q, const Tensor& idx_k, int64_t view) {
     const c10::DeviceGuard guard(bf.device());
     const Stream stream = current_stream(bf.device());
@@ -714,7 +784,7 @@ py::tuple index_view(const Tensor& bf, const Tensor& idx_q, const Tensor& idx_k,
                                    qb + B * Sq, Sk, qp + Sq, (int)B, stream.stream()),
               "bam_gather_bitfields");
     }
-    return py::make_tuple(py::make_tuple(bits, pos), plan.py_object());
+    return py::make_tuple(std::make_shared<Prepared>(stream, std::vector<Tensor>{bits, pos}, plan.core), plan.py_object());
 }
 
 // Counters of the decode step's merge, zero between calls, one set per stream: the calls of a stream run in order, those
@@ -784,6 +854,7 @@ PYBIND11_MODULE(_bam_host, m) {
         .def_readonly("flags_version", &PlanCore::flags_version)
         .def_property_readonly("struct_address", [](const PlanCore& c) { return (int64_t)&c.plan; })
         .def("ds_pairs", &PlanCore::wait_pairs, py::call_guard<py::gil_scoped_release>());
+    py::class_<Prepared, std::shared_ptr<Prepared>>(m, "Prepared").def("use", &Prepared::use);
     // once, by the Python layer: its subclass of PlanCore and the exception its callers expect
     m.def("setup", [](py::object plan_type, py::object error_type) {
         g_plan_type = plan_type.release().ptr();
@@ -816,6 +887,7 @@ PYBIND11_MODULE(_bam_host, m) {
     });
     m.def("cached_bitfield_flags", []() -> py::object {
         const Tensor flags = g_bitfield.flags;
+        if (g_bitfield.prepared) g_bitfield.prepared->use();
         return flags.defined() ? py::cast(flags) : py::none();
     });
     m.def("cached_bitfield_plan", []() { return g_bitfield.plan.py_object(); });

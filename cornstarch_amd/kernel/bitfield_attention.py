@@ -394,8 +394,8 @@ class _IndexView:
         self.struct = _bam_hip.IndexView()
         # gathered bitfields and positions (named in the struct), and the plan of the shard: classes of its 32 x 32 tiles,
         # slice order
-        arrays, self.plan = _host.index_view(bf, *idx, ctypes.addressof(self.struct))
-        self._keep = (arrays, idx)
+        self._prepared, self.plan = _host.index_view(bf, *idx, ctypes.addressof(self.struct))
+        self._keep = idx
 
         self.address = ctypes.addressof(self.struct)
 
@@ -414,7 +414,7 @@ class _IndexView:
             raise ValueError("offsets_q and offsets_k must be given together")
         key = tuple(_host.tensor_key(t) for t in (bitfield_mask, offsets_q, offsets_k))
         with _CACHE_LOCK:
-            if cls._last is not None and cls._last[0] == key:
+            if cls._last is not None and cls._last[0] == key and cls._last[1]._prepared.use():
                 return cls._last[1]
             view = cls(bitfield_mask, offsets_q, offsets_k)
             cls._last = (key, view, (bitfield_mask, offsets_q, offsets_k))
