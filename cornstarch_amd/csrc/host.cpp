@@ -196,7 +196,10 @@ void hip_check(hipError_t e, const char* what) {
 // later call on that stream just uses it.  On another one it first waits for an event behind the launches, and the caching allocator
 // learns that this stream uses the memory too.  An event costs the stream it is recorded on 4.7 us, so it is recorded when the first
 // such call asks; a stream that torch does not own may be gone by then, or share its handle with another, and gets it at once.
-class Prepared {
+// A call under capture makes the graph an owner: its replays read the results after the caches have moved on.
+class Prepared : public std::enable_shared_from_this<Prepared> {
+    typedef std::shared_ptr<Prepared> Held;
+
 public:
     // after the launches
     Prepared(Stream stream, std::vector<Tensor> results, std::shared_ptr<PlanCore> plan)
@@ -211,9 +214,10 @@ public:
     // Call before the results are used on the current stream.  False: they cannot be, the caller has to compute its own.
     bool use() {
         const Stream now = current_stream(stream_.device());
-        if (now == stream_ && !external()) return true;
+        const bool captured = now.stream() != nullptr && capturing(), elsewhere = now != stream_ || external();
+        if (!captured && !elsewhere) return true;
         const std::lock_guard<std::mutex> lock(mutex_);
-        if (!done_) {
+        if (elsewhere && !done_) {
             const c10::DeviceGuard guard(stream_.device());
             const c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
             if (event_ == nullptr) {
@@ -222,7 +226,7 @@ public:
                 if (status != hipStreamCaptureStatusNone) return false;  // (the event would become part of that graph)
                 record();
             }
-            if (now.stream() != nullptr && capturing()) {  // (replays run on any stream: the results are there before the capture goes on)
+            if (captured) {  // (replays run on any stream: the results are there before the capture goes on)
                 hip_check(hipEventSynchronize(event_), "wait for a plan");
                 done_ = true;
             } else if (hipEventQuery(event_) == hipSuccess) {
@@ -232,9 +236,23 @@ public:
                 hip_check(hipStreamWaitEvent(now.stream(), event_, 0), "wait for a plan");
             }
         }
-        for (const Tensor& t : results_) t.record_stream(c10::Stream::unpack3(now.id(), now.device_index(), c10::DeviceType::CUDA));
+        if (captured)
+            give_to_graph(now);
+        else
+            for (const Tensor& t : results_) t.record_stream(c10::Stream::unpack3(now.id(), now.device_index(), c10::DeviceType::CUDA));
         return true;
     }
+    // What graphs that are gone owned.  (The runtime lets go of it where the last graph is destroyed, under its own locks: there
+    // the reference only changes hands.)
+    static void collect() {
+        std::vector<Held*> gone;
+        {
+            const std::lock_guard<std::mutex> lock(dropped_mutex());
+            gone.swap(dropped());
+        }
+        for (Held* h : gone) delete h;
+    }
+    static int64_t held_by_graphs() { return held_.load(); }
 
 private:
     // (the id of a stream of torch's own is not its handle, except for the default stream, whose handle is null)
@@ -244,12 +262,46 @@ private:
         hip_check(hipEventCreateWithFlags(&event_, hipEventDisableTiming), "event behind a plan");
         hip_check(hipEventRecord(event_, stream_.stream()), "event behind a plan");
     }
+    static std::mutex& dropped_mutex() {
+        static std::mutex* m = new std::mutex;  // never destroyed: a graph may outlive static destruction
+        return *m;
+    }
+    static std::vector<Held*>& dropped() {
+        static auto* v = new std::vector<Held*>;
+        return *v;
+    }
+    static void drop(void* held) {
+        const std::lock_guard<std::mutex> lock(dropped_mutex());
+        dropped().push_back(static_cast<Held*>(held));
+        --held_;
+    }
+    // The graph that `stream` is being captured into, and what is instantiated from it, own a reference through a user object.
+    void give_to_graph(const Stream& stream) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        hipGraph_t graph = nullptr;
+        hip_check(hipStreamGetCaptureInfo_v2(stream.stream(), &status, &id, &graph, nullptr, nullptr), "graph of a capture");
+        if (graph == graph_ && id == capture_) return;
+        auto held = std::make_unique<Held>(shared_from_this());
+        hipUserObject_t owner = nullptr;
+        hip_check(hipUserObjectCreate(&owner, held.get(), &Prepared::drop, 1, hipUserObjectNoDestructorSync), "owner of a plan");
+        held.release();
+        ++held_;
+        const hipError_t e = hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove);
+        if (e != hipSuccess) (void)hipUserObjectRelease(owner, 1);
+        hip_check(e, "owner of a plan");
+        graph_ = graph;
+        capture_ = id;
+    }
+    static inline std::atomic<int64_t> held_{0};
     const Stream stream_;
     std::vector<Tensor> results_;
     const std::shared_ptr<PlanCore> plan_;
     std::mutex mutex_;
     hipEvent_t event_ = nullptr;
     bool done_ = false;
+    hipGraph_t graph_ = nullptr;  // the last one that became an owner, and its capture
+    unsigned long long capture_ = 0;
 };
 
 // ------------------------------------------------------------------ caches (one entry each; guarded by the GIL)
@@ -271,6 +323,7 @@ struct Cached {
 Cached g_bitfield, g_mask;
 
 void store(Cached& slot, const Tensor& owner, const Tensor& flags, Plan plan, const Stream& stream) {
+    Prepared::collect();
     if (owner.is_inference()) return;  // no version counter: nothing would tell that it has been written to
     Cached fresh;
     fresh.owner = owner;
@@ -908,7 +961,12 @@ PYBIND11_MODULE(_bam_host, m) {
         std::swap(g_mask, gone);
     });
     m.def("decode_counter_sets", []() { return g_counters.size(); });
+    m.def("held_by_graphs", []() {
+        Prepared::collect();
+        return Prepared::held_by_graphs();
+    });
     m.def("release_memory", []() {
+        Prepared::collect();
         count_words().release();
         g_counters.clear();
     });

@@ -1,5 +1,7 @@
-"""Cached flags, plans and gathered index arrays used on another stream than the one that computes them.  The first stream is kept
+"""Cached flags, plans and gathered index arrays used on another stream than the one that computes them, and by graphs.  The first stream is kept
 busy (`_sleep`), so that the launches that fill them are still queued when the second stream's call is made."""
+
+import time
 
 import pytest
 import torch
@@ -145,3 +147,67 @@ def test_a_capture_finds_finished_plans_only(inputs, call, streams):
             assert torch.equal(a, b)
             b.zero_()
         torch.cuda.synchronize()
+
+
+def _until(done):
+    """The runtime may let go of a destroyed graph from a thread of its own."""
+    for _ in range(500):
+        if done():
+            return
+        time.sleep(0.01)
+    assert done()
+
+
+@pytest.mark.parametrize("call", CALLS, ids=lambda f: f.__name__)
+def test_a_graph_owns_the_plans_it_reads(inputs, call):
+    """The caches hold one entry each: what a graph was captured with stays its own, and goes when the graph goes."""
+    from cornstarch_amd.kernel._bam_hip import host
+
+    want = call(*inputs)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    before = host.held_by_graphs()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(*inputs)
+        got = call(*inputs)  # a second layer
+    assert host.held_by_graphs() == before + 1
+    kept = _mask.of, _indexed.flags, _indexed.rows
+    for other in (S, S // 2):  # other masks take the entries, their memory and that of the old ones
+        q, k, v, do = (t[:, :other].contiguous() for t in inputs[:4])
+        bf = torch.flip(inputs[4], (1,))[:, :other].contiguous()
+        _mask.of = BA.materialize_bitfield_mask(bf)
+        _indexed.rows = torch.arange(other, device="cuda")
+        _indexed.flags = BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(bf).clone()
+        call(q, k, v, do, bf)
+        junk = [torch.full((n,), 255, dtype=torch.uint8, device="cuda") for n in (1 << 10, 1 << 12, 1 << 14, 1 << 16, 1 << 18) for _ in range(16)]
+        torch.cuda.synchronize()
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(want, got):
+            assert torch.equal(a, b)
+        del junk
+    _mask.of, _indexed.flags, _indexed.rows = kept
+    del graph
+    _until(lambda: host.held_by_graphs() == before)
+
+
+def test_an_entry_made_anew_is_owned_by_the_next_graph(inputs):
+    from cornstarch_amd.kernel._bam_hip import host
+
+    want = _flags_and_plan(*inputs)
+    before, graphs = host.held_by_graphs(), []
+    for _ in range(3):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            got = _flags_and_plan(*inputs)
+    assert host.held_by_graphs() == before + 3
+    _forget()
+    del graphs[:2]
+    _until(lambda: host.held_by_graphs() == before + 1)
+    graphs[0].replay()
+    torch.cuda.synchronize()
+    for a, b in zip(want, got):
+        assert torch.equal(a, b)
