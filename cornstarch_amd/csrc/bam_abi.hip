@@ -330,7 +330,7 @@ extern "C" {
 
 const char* bam_last_error(void) { return g_error; }
 
-int bam_abi_version(void) { return 13; }
+int bam_abi_version(void) { return 14; }
 
 int bam_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                    int64_t flags_stride_m, int B, int S, void* stream) {
@@ -368,7 +368,7 @@ PlanLayout plan_layout(int B, int Sq, int Sk) {
     l.tile_order_off = l.tile_count_off + up(B * ((Sk + 127) / 128) * 4, 256);
     l.group_count_off = l.tile_order_off + up(B * ((Sk + 127) / 128) * 4, 256);
     l.group_order_off = l.group_count_off + up(B * num_m * 4, 256);
-    l.row_workloads_off = l.group_order_off + up(B * num_m * 4, 256);
+    l.row_workloads_off = l.group_order_off + up((B * num_m + 1) * 4, 256);
     l.bytes = l.row_workloads_off + up(num_m * 8, 256);
     // the packed mask of bam_mask_tile_plan: rows padded to 128, keys to 128, 32-key blocks to an even number
     l.row_sn = num_m * 128;

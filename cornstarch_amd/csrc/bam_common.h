@@ -345,6 +345,22 @@ __device__ __forceinline__ int mirror_second(int bid, int blocks) {
     return blocks <= UNITS || blocks > 2 * UNITS || bid < UNITS || bid >= full ? bid : UNITS + full - 8 - (bid & ~7) + (bid & 7);
 }
 
+// How many q heads make the key tile lists of a plan (groups of them, `sum` tiles in all, the longest of `longest` tiles) so level
+// that a forward or dQ workgroup of two streams walks two of them side by side instead of splitting one.  Of lists that are equally
+// long two side by side take the time that both would take one after the other, and a compute unit that does the latter shows first
+// loads and stores twice.  With n = groups x heads workgroups, lengths that fall linearly and the longest first, a compute unit walks
+// max(longest / 2, longest - 2 (longest - mean) 256 / n) pairs of tiles; the streams take a list each where that saves less than the
+// 5 pairs (some 9 us at D 128, 6 at D 64) that the second workgroup's start and end cost.  Forward alone, us, one stream / two on a
+// list / a list each: nothing hidden, D 128, 4096 tokens (512 workgroups) 150 / 147 / 138, 2048 (384) 66 / 75 / 64, 1024 (320) 37 /
+// 46 / 37; D 96, 2 x 2003 (512) 64 / 71 / 63; D 64, 3 x 1024 (384) 25 / 32 / 26, 4096 (512) 87 / 95 / 87; causal, D 128, 4096 tokens
+// 90 / 80 / 111.
+__device__ __forceinline__ int level_heads(int groups, long long sum, int longest) {
+    if (longest > 1024) return 0x7FFFFFFF;  // (a stream's half of the list array)
+    if (longest <= 10) return 0;
+    const long long per_head = 5ll * groups * groups;
+    return (int)min((((long long)longest * groups - sum) * 512 + per_head - 1) / per_head, 0x7FFFFFFFll);
+}
+
 // Which (batch x row-group index, kv head, member of the kv group) a workgroup of the forward / dQ kernels takes.
 // Within an XCD the hardware deals consecutive workgroups to the four shader engines in turn and starts them strictly
 // in order, so four consecutive workgroups of an XCD should carry the same amount of work or the engines with the

@@ -87,7 +87,7 @@ struct AttnParams {
     const int* tile_order;
     // Optional (plan): the groups of four slices of all sequences (code b * num_m + group) by falling number of
     // 64-key tiles their workgroup visits; the forward and dQ kernels take their workgroups in this order (null:
-    // group by group, the sequences of the batch side by side).
+    // group by group, the sequences of the batch side by side).  Behind the codes: level_heads of the numbers.
     const int* group_order;
     // MASK_DENSE with a plan: the mask packed to bits, once per orientation (null = read the mask bytes).
     // row_bits (B, row_bits_sn-strided 32-key blocks, rows): bit c of word (n, r) = mask[r][32 n + c];
@@ -111,17 +111,18 @@ inline bool dkdv_far(const AttnParams& p) {
     return far_rows(p.q, p.Sq, p.d) || far_rows(p.dout, p.Sq, p.d) || far_rows(p.k, p.Sk, p.d) || far_rows(p.v, p.Sk, p.d);
 }
 
-// Whether the forward and dQ walk two tiles at a time (measured at launch_fwd_b and launch_dq_f).  One workgroup with one stream
-// needs about 1.4 us a tile (D 128) whether it shares its compute unit or not, so that up to some 800 workgroups the longest list
+// Whether the forward and dQ run with two streams of waves (measured at launch_fwd_b and launch_dq_f).  One workgroup with one
+// stream needs about 1.4 us a tile (D 128) whether it shares its compute unit or not, so that with few workgroups the longest list
 // decides, not the sum; two streams take 1.85 us for two tiles, but a unit then runs its workgroups one after the other and shows
-// each one's first loads and stores, which short lists do not win back.
+// each one's first loads and stores, which short lists do not win back, nor do lists that are all equally long: from 257 workgroups
+// on the kernel looks at the plan (streams_side_by_side) and does without it where there is none.  Above 512 it depends on the
+// mask, which the host does not know: there one stream.
 inline bool two_streams(const AttnParams& p) {
     const int64_t units = (int64_t)p.num_m * p.B * p.Hq;
     if (p.Sk <= (p.D > 32 ? 128 : 64)) return false;  // a tile or two: nothing to share
     int64_t most = p.Sk < 768 ? 256 : p.Sk < 1152 ? 384 : p.Sk < 1600 ? 480 : 512;
     if (p.D <= 32) most = p.Sk < 192 ? 256 : p.Sk < 384 ? 448 : p.Sk < 2560 ? 512 : p.bias != nullptr ? 768 : 1024;
-    if (p.D > 32 && p.mask_mode != MASK_INDEXED && p.mask_mode != MASK_DENSE && p.bias == nullptr)
-        most = p.Sk >= (p.D > 64 ? 8192 : 4608) ? 768 : p.Sk >= 3072 ? 640 : most;
+    if (p.D > 32 && p.group_order == nullptr && most > 256) most = 256;
     return units <= most;
 }
 
@@ -187,8 +188,8 @@ int launch_mask_tile_plan(const uint8_t* mask, int8_t* flags, int64_t flags_stri
 // *count must be zero when the kernel starts (the plan kernels reset it).  tile_count (B, ceil(Sk/128)) scratch and
 // tile_order (B * ceil(Sk/128)): the key tiles by falling number of pairs, written by a second small launch; both may
 // be null, and no order is written beyond MAX_RANKED tiles.  The same for the groups of four slices in the plan's slice
-// order (order, order_sb): group_count (B * num_m) scratch, group_order (B * num_m) = the groups by falling number of
-// 64-key tiles they visit.  row_workloads (num_m int64, or null): per 128-row block, the number of its 128 x 32 tiles
+// order (order, order_sb): group_count (B * num_m) scratch, group_order (B * num_m + 1) = the groups by falling number of
+// 64-key tiles they visit, then level_heads of these numbers.  row_workloads (num_m int64, or null): per 128-row block, the number of its 128 x 32 tiles
 // with an allowed pair, summed over the batch.  count_host (pinned host memory, or null): receives count_tag << 32 | count,
 // and with rows_moved (sorted rows, or null) in bits 31 and 30 whether rows of some sequence have been moved, or left.
 int launch_ds_entries(const uint8_t* fine, int64_t fine_sb, int64_t fine_ss, int B, int Sq, int Sk, int* entry,

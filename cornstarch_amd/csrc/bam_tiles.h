@@ -259,15 +259,24 @@ __device__ __forceinline__ int row_of_slot(const AttnParams& p, const WaveSlices
     return ws.moved && valid ? p.rows[(int64_t)b * p.rows_sb + slot] : slot;
 }
 
+// A word of the plan at a wave-uniform address, by a scalar load (whatever stands in front of it).
+__device__ __forceinline__ int plan_word(const int* at) {
+    return *(const __attribute__((address_space(4))) int*)(unsigned long long)at;
+}
+
 __device__ __forceinline__ WaveSlices pick_wave_slices(const AttnParams& p, int b, int grp) {
     WaveSlices w;
     w.moved = false;
     if (p.fine != nullptr) {
         const int* ord = p.order + (int64_t)b * p.order_sb + 4 * grp;
-        w.moved = order_moved(ord[0]);  // (a group has a first slice)
+        int code[4];  // (one load: left in the loop below, the compiler waits for each before it asks for the next)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) code[x] = plan_word(ord + x);
+        asm volatile("" ::"s"(code[0]), "s"(code[1]), "s"(code[2]), "s"(code[3]));
+        w.moved = order_moved(code[0]);  // (a group has a first slice)
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-            w.slice[x] = order_slice(ord[x]);
+            w.slice[x] = order_slice(code[x]);
             w.cls_row[x] = w.slice[x] >= 0
                                ? (const int8_t*)p.fine + (int64_t)b * p.fine_sb + (int64_t)w.slice[x] * p.fine_ss
                                : nullptr;
@@ -284,6 +293,14 @@ __device__ __forceinline__ WaveSlices pick_wave_slices(const AttnParams& p, int 
     return w;
 }
 
+// Two streams, more workgroups than compute units: whether the streams take a unit each (level_heads).
+__device__ __forceinline__ bool streams_side_by_side(const AttnParams& p) {
+    const int groups = p.num_m * p.B;
+    return p.group_order != nullptr && groups * p.Hq > 256 && p.Hq >= plan_word(p.group_order + groups);
+}
+// (units 8 apart are on the same XCD and, in head_unit_map, heads that read the same rows)
+__device__ __forceinline__ int side_unit(int block, int stream) { return 16 * (block >> 3) + (block & 7) + 8 * stream; }
+
 // List, in ascending order, the 64-key tiles the four slices of a workgroup have to visit, among the (at most
 // MAX_LIST) tiles starting at tile kt_begin; longer sequences are walked in several passes.
 // entry = (tile << 8) | c0 | c1 << 2 | c2 << 4 | c3 << 6 ; c_w is the class of the tile for wave w's slice:
@@ -293,12 +310,14 @@ __device__ __forceinline__ WaveSlices pick_wave_slices(const AttnParams& p, int 
 // Executed by wave 0; the caller synchronizes before reading.
 // STREAMS = 2: the even and the odd tiles make a list each (the second at list + MAX_LIST / 2, its length in count_out[1]).  Which
 // list a tile is in does not depend on what else is listed, so a row's result does not depend on its neighbours or the plan.
+// (split false: one list all the same.)
 template <int STREAMS = 1>
 __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int num_n, int S, int lane, int kt_begin,
-                                                    int* list, int* count_out) {
+                                                    int* list, int* count_out, bool split = STREAMS > 1) {
     const int nkt = min((S + 63) >> 6, kt_begin + MAX_LIST);
     int count[STREAMS] = {};
-    const int mine = STREAMS > 1 ? lane & 1 : 0;  // (kt_begin is even)
+    const int mine = STREAMS > 1 && split ? lane & 1 : 0;  // (kt_begin is even)
+    const unsigned long long even = split ? 0x5555555555555555ull : ~0ull;
     for (int base = kt_begin; base < nkt; base += 64) {
         const int kt = base + lane;
         int packed = 0;
@@ -315,16 +334,16 @@ __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int nu
             }
         }
         unsigned long long bal = __ballot(packed != 0), own = bal;
-        if (STREAMS > 1) own &= mine ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull;
+        if (STREAMS > 1) own &= mine ? ~even : even;
         const int at = (mine ? MAX_LIST / 2 + count[STREAMS - 1] : count[0]) + __popcll(own & ((1ull << lane) - 1ull));
         if (packed) list[at] = (kt << 8) | packed;
 #pragma unroll
         for (int x = 0; x < STREAMS; ++x)
-            count[x] += __popcll(STREAMS == 1 ? bal : bal & (x ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull));
+            count[x] += __popcll(STREAMS == 1 ? bal : bal & (x ? ~even : even));
     }
 #pragma unroll
     for (int x = 0; x < STREAMS; ++x)
-        if (lane == 0) count_out[x] = count[x];
+        if (lane == 0 && (x == 0 || split)) count_out[x] = count[x];
     wait_lds();
 }
 

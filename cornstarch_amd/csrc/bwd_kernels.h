@@ -782,16 +782,27 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
 
     int ub, hk, g;
     head_unit_map(blockIdx.x, p.num_m * p.B, p.Hkv, G, ub, hk, g);
+    int code = p.group_order != nullptr ? plan_word(p.group_order + ub) : 0;
+    bool side = false, idle = false;  // the streams take a unit each; ... and there is none left for this one
+    if constexpr (STREAMS > 1 && D > 32) {
+        side = streams_side_by_side(p);
+        if (__builtin_expect(side, 0)) {
+            const int units = p.num_m * p.B * p.Hq, unit = side_unit(blockIdx.x, stream);
+            if (side_unit(blockIdx.x, 0) >= units) return;
+            idle = unit >= units;
+            head_unit_map(idle ? 0 : unit, p.num_m * p.B, p.Hkv, G, ub, hk, g);
+            code = plan_word(p.group_order + ub);
+        }
+    }
     int b = ub % p.B, grp = ub / p.B;
     if (p.group_order != nullptr) {  // with a plan: the groups of all sequences by falling length of their tile lists
-        const int code = p.group_order[ub];
         b = code / p.num_m;
         grp = code - b * p.num_m;
     }
     const int h = hk * G + g;
     const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
 
-    const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
+    const int slice = idle ? -1 : __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
     const int slot = (slice < 0 ? 0 : slice) * 32 + l32;
     const bool qvalid = slice >= 0 && slot < Sq;
     const int qrow = row_of_slot(p, ws, b, slot, qvalid);
@@ -830,7 +841,8 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
     }
     const int qpos = (IDX && qvalid) ? p.posq[qrow] : qrow;
     // (the row loads above are in flight while wave 0 reads the class rows and the first tile is on its way)
-    if (wave == 0 && stream == 0) build_key_tile_list<STREAMS>(ws, p.num_n, Sk, lane, 0, sList, sCount);  // first pass (usually the only one)
+    if (wave == 0 && (stream == 0 || side))  // first pass (usually the only one)
+        build_key_tile_list<STREAMS>(ws, p.num_n, idle ? 0 : Sk, lane, 0, sList + stream * (MAX_LIST / 2), sCount + stream, !side);
     QueryBits qb = {};
     float lse2 = INFINITY;
     // With o given, this launch also is the delta pre-pass: it runs in front of the dK/dV kernel, has the rows of dO in
@@ -844,7 +856,7 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
 #pragma unroll
             for (int kk = 0; kk < (D <= 64 ? KK : 1); ++kk) part[kk] = chunk_dot<T>(oreg[kk], greg[kk]);
             dlt = half_swap_sum(KK == 4 ? (part[0] + part[2]) + (part[1] + part[KK - 1]) : part[0] + part[1]);
-            if (stream == 0 && qvalid && hi == 0) {
+            if ((stream == 0 || side) && qvalid && hi == 0) {
                 const int64_t at = (int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow;
                 p.delta[at] = dlt;
                 if (p.lse_scaled != nullptr) p.lse_scaled[at] = lse_row * LOG2E;
@@ -1147,7 +1159,8 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
     // Two streams: each hands over the columns that the other one finishes, through the tile arrays, which nobody reads any more.
     constexpr int DB0 = STREAMS > 1 ? (DB + 1) / 2 : DB;
     f32x4* const park = (f32x4*)sK_all + wave * (DB * 4 * 64);
-    if constexpr (STREAMS > 1) {
+    const bool merged = STREAMS > 1 && !side;
+    if (merged) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
             if ((db < DB0) == (stream == 1)) {
@@ -1171,14 +1184,14 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
         char* dqp = (char*)p.dq.ptr + 2 * ((int64_t)b * p.dq.sb + (int64_t)qrow * p.dq.ss + (int64_t)h * p.dq.sh);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
+            if (merged && (db < DB0) != (stream == 0)) continue;
             store_block16<T>(dqp + 64 * db, p.d - 32 * db, hi, [&](int i) { return dq[db][i] * p.scale; });
         }
     } else if (qvalid) {
         float* dqp = (float*)p.dq.ptr + ((int64_t)b * p.dq.sb + (int64_t)qrow * p.dq.ss + (int64_t)h * p.dq.sh);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
+            if (merged && (db < DB0) != (stream == 0)) continue;
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
                 if (32 * db + 8 * grp >= p.d) break;
@@ -1234,8 +1247,7 @@ static int launch_dq_s(const AttnParams& p, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 // Two streams where the forward takes them.  dQ alone, us, one stream -> two: D 64, 1000 tokens, 8 heads 27.1 -> 22.7, 1024, 32 heads
-// 29.4 -> 25.1, 2 x 700 28.4 -> 27.2, 2048 (512 workgroups) 50.9 -> 49.8, 3001 (768) 77 -> 87, 4096 (640) 91.6 -> 81.1, 5000 (640)
-// 108 -> 90, 24000 (752) 497 -> 428; with a bias 2 x 2048, 16 heads 64.1 -> 59.2; D 32: 2048 46.4 -> 35.9, 3001 64.1 -> 52.9, 4096
+// 29.4 -> 25.1, 2 x 700 28.4 -> 27.2, 2048 (512 workgroups) 50.9 -> 49.8, 3001 (768) 77 -> 87; with a bias 2 x 2048, 16 heads 64.1 -> 59.2; D 32: 2048 46.4 -> 35.9, 3001 64.1 -> 52.9, 4096
 // (1024) 84.3 -> 77.0, 8 x 300 (768) 18.8 -> 24.3.
 template <typename T, int D, int BIAS, bool LONG>
 static int launch_dq_f(const AttnParams& p, hipStream_t stream) {

@@ -69,9 +69,20 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
 
     int ub, hk, g;
     head_unit_map(blockIdx.x, p.num_m * p.B, p.Hkv, G, ub, hk, g);
+    int code = p.group_order != nullptr ? plan_word(p.group_order + ub) : 0;
+    bool side = false, idle = false;  // the streams take a unit each; ... and there is none left for this one
+    if constexpr (STREAMS > 1 && D > 32) {
+        side = streams_side_by_side(p);
+        if (__builtin_expect(side, 0)) {
+            const int units = p.num_m * p.B * p.Hq, unit = side_unit(blockIdx.x, stream);
+            if (side_unit(blockIdx.x, 0) >= units) return;
+            idle = unit >= units;
+            head_unit_map(idle ? 0 : unit, p.num_m * p.B, p.Hkv, G, ub, hk, g);
+            code = plan_word(p.group_order + ub);
+        }
+    }
     int b = ub % p.B, grp = ub / p.B;
     if (p.group_order != nullptr) {  // with a plan: the groups of all sequences by falling length of their tile lists
-        const int code = p.group_order[ub];
         b = code / p.num_m;
         grp = code - b * p.num_m;
     }
@@ -79,7 +90,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
 
     // ---- per-lane query state -------------------------------------------------------
-    const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
+    const int slice = idle ? -1 : __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
     const int slot = (slice < 0 ? 0 : slice) * 32 + l32;
     const bool qvalid = slice >= 0 && slot < Sq;
     const int qrow = row_of_slot(p, ws, b, slot, qvalid);
@@ -97,7 +108,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     int qpos = (IDX && qvalid) ? p.posq[qrow] : qrow;
     QueryBits qb = {};  // of qf and qpos, once they have arrived
     // (the row loads above are in flight while the class rows are read and the first tile is on its way)
-    if (wave == 0 && stream == 0) build_key_tile_list<STREAMS>(ws, p.num_n, Sk, lane, 0, sList, sCount);  // first pass (usually the only one)
+    if (wave == 0 && (stream == 0 || side))  // first pass (usually the only one)
+        build_key_tile_list<STREAMS>(ws, p.num_n, idle ? 0 : Sk, lane, 0, sList + stream * (MAX_LIST / 2), sCount + stream, !side);
 
     f32x16 o[DB];
 #pragma unroll
@@ -475,7 +487,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     constexpr int DB0 = STREAMS > 1 ? (DB + 1) / 2 : DB;  // stream 0 finishes the column blocks below DB0, stream 1 the others
     f32x4* const park = (f32x4*)sK_all + wave * (DB * 4 * 64);
     float* const park_ml = (float*)sV_all;
-    if constexpr (STREAMS > 1) {
+    const bool merged = STREAMS > 1 && !side;
+    if (merged) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
             if ((db < DB0) == (stream == 1)) {
@@ -495,20 +508,20 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         m_i = m;
     }
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-    if (stream == 0 && hi == 0 && slice >= 0)
+    if ((stream == 0 || side) && hi == 0 && slice >= 0)
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] =
             ltot > 0.f ? (m_i * c2 + __builtin_amdgcn_logf(ltot)) * LN2 : -INFINITY;
     // A wave without a slice (plan: slot 4 grp + wave of the order lies past the last slice) owns the 32 padding rows
     // of that slot, so that every row of the rounded lse is written whether or not a plan is given.
-    if (stream == 0 && hi == 0 && slice < 0 && 32 * (4 * grp + wave) + 31 < p.Sq_rounded)
+    if ((stream == 0 || side) && !idle && hi == 0 && slice < 0 && 32 * (4 * grp + wave) + 31 < p.Sq_rounded)
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + 32 * (4 * grp + wave) + l32] = -INFINITY;
     if (qvalid) {
         char* op = (char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
+            if (merged && (db < DB0) != (stream == 0)) continue;
             f32x16 x = o[db];
-            if constexpr (STREAMS > 1) {
+            if (merged) {
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
                     const f32x4 other = park[(4 * db + grp) * 64 + lane];
@@ -536,22 +549,20 @@ static int launch_fwd_s(const AttnParams& p, hipStream_t stream) {
 }
 // Two streams halve the chain of tiles a workgroup walks and double the waves of a compute unit that has one workgroup; the price
 // is a workgroup that fills the unit (D = 64 and above), so that nothing runs beside its first loads and its stores.  Forward
-// kernel alone, bf16, us, one stream -> two (workgroups in brackets):
+// kernel alone, bf16, us, one stream -> two (workgroups in brackets; lists of a causal mask with a few segments):
 //   D 128:  60 tokens (64) 8.3 -> 9.9;  120 (288) 14.5 -> 21.9;  250 (256) 17.4 -> 16.3, (384) 19.7 -> 25.6;  640 (240) 24.0 ->
 //           21.0, (320) 26.2 -> 28.3;  1000 (384) 36.2 -> 34.5, (512) 37.7 -> 42.5;  1500 (384) 45.9 -> 36.6, (480) 47.8 -> 47.5;  2000 (384) 53.5 ->
-//           42.8, (512) 55.1 -> 54.7, (640) 58.2 -> 64.4;  3200 (500) 78.5 -> 69.0, (600) 81.6 -> 76.2, (775) 88.4 -> 104.1;  5000
-//           (400) 109 -> 83, (640) 121 -> 102, (760) 129 -> 135;  12000 (564) 268 -> 201;  24000 (752) 588 -> 510, D 80, 32000 (1000)
-//           771 -> 828
+//           42.8, (512) 55.1 -> 54.7
 //   D 64:   60 (256) 7.6 -> 8.7;  250 (256) 14.0 -> 12.4, (384) 15.3 -> 19.4;  640 (320) 21.8 -> 22.3, (480) 23.0 -> 26.8;  900
-//           (384) 26.9 -> 25.6, (512) 28.7 -> 30.6;  1500 (480) 37.1 -> 33.1;  1000 (640) 32.2 -> 40.3;  2600 (630) 56.5 -> 51.8, (756) 58.5 -> 62.9;  4096 (640) 78.1 -> 66.2, (768) 80.7 -> 80.4;
-//           6500 (765) 117 -> 110;  24000 (752) 421 -> 336;  8000 (1008) 156 -> 173
+//           (384) 26.9 -> 25.6, (512) 28.7 -> 30.6;  1500 (480) 37.1 -> 33.1;  1000 (640) 32.2 -> 40.3
 //   D 32 (two such workgroups fit a unit):  60 (64) 6.9 -> 7.5;  120 (288) 9.9 -> 10.7;  250 (384) 13.3 -> 12.1, (512) 13.8 ->
 //           14.1;  500 (512) 18.1 -> 16.8;  2048 (512) 37.8 -> 28.2, 3001 (768) 52.4 -> 40.7, 4096 (1024) 69 -> 61, but with short
-//           lists 8 x 300 (768) 16.0 -> 19.5, 4 x 1024 (1024) 27.8 -> 30.4;  with a bias 4096 (640) 82 -> 77, (1024) 85 -> 107
-//   above 512 workgroups, D 128:  bool masks 4096 (640) 98 -> 104, 8192 (768) 203 -> 217;  index tensors 8192 (640) 222 -> 229;
-//           bias 4096 (640) 116 -> 121
-// Masks that hide nothing, with twice the work in lists of the same length, lose (the host does not see that): 4096 (512) D 128
-// 134 -> 141, D 64 95 -> 104.
+//           lists 8 x 300 (768) 16.0 -> 19.5, 4 x 1024 (1024) 27.8 -> 30.4;  with a bias 4096 (640) 82 -> 77, (1024) 85 -> 107;
+//           nothing hidden: 2048 (512) 34.4 -> 32.3, 3001 (768) 69.1 -> 66.9, 4096 (1024) 118 -> 112
+// Above 512 workgroups and D 32 the mask decides: text only / 4 / 10 segments / nothing hidden, D 128, 5000 tokens (640) 119 -> 128 /
+// 118 -> 108 / 128 -> 99 / 234 -> 241;  3200 (600) 79 -> 89 / 82 -> 80 / 92 -> 71 / 158 -> 165;  8192 (768) 220 -> 240 / 205 -> 205 /
+// 198 -> 151 / 409 -> 415;  D 64, 6500 (765) 109 -> 124 / 120 -> 111 / 136 -> 94 / 204 -> 219.  The host launches before anybody
+// has seen the lists, and the plainest mask is the one that loses: one stream.
 template <typename T, int D, bool BIAS, bool LONG>
 static int launch_fwd_b(const AttnParams& p, hipStream_t stream) {
     if constexpr (!LONG)

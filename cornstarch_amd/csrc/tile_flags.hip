@@ -1049,6 +1049,7 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__
                                                          unsigned long long* __restrict__ count_host,
                                                          unsigned long long count_tag, const int* __restrict__ rows_moved, int B) {
     __shared__ __attribute__((aligned(16))) int s_cnt[DS_MAX_ORDERED_TILES];
+    __shared__ int s_sum[4];
     const int tid = threadIdx.x;
     if (count_host != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && tid < 64) {
         unsigned moved = 0;  // with sorted rows: whether some sequence's rows have been moved (bit 31), or left (bit 30)
@@ -1070,7 +1071,16 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__
     }
     if ((int)blockIdx.x * 64 >= n_tiles) return;  // (workgroup-uniform)
     const int padded = (n_tiles + 15) & ~15;
-    for (int i = tid; i < padded; i += 256) s_cnt[i] = i < n_tiles ? tile_count[i] : -1;  // padding ranks behind everything
+    int mine = 0;
+    for (int i = tid; i < padded; i += 256) {
+        s_cnt[i] = i < n_tiles ? tile_count[i] : -1;  // padding ranks behind everything
+        mine += i < n_tiles ? s_cnt[i] : 0;
+    }
+    if (blockIdx.y == 1) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off);
+        if ((tid & 63) == 0) s_sum[tid >> 6] = mine;
+    }
     __syncthreads();
     const int i = blockIdx.x * 64 + (tid >> 2), sub = tid & 3;
     const int c = i < n_tiles ? s_cnt[i] : 0;
@@ -1086,7 +1096,10 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const int* __restrict__
     }
     rank += __shfl_xor(rank, 1);
     rank += __shfl_xor(rank, 2);
-    if (sub == 0 && i < n_tiles) tile_order[rank] = i;
+    if (sub == 0 && i < n_tiles) {
+        tile_order[rank] = i;
+        if (blockIdx.y == 1 && rank == 0) tile_order[n_tiles] = level_heads(n_tiles, (long long)s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3], c);
+    }
 }
 
 // Both launches in one, for plans of up to SMALL_PLAN_WORDS (slice, 128-key tile) pairs (at 16384 the two are as fast): every workgroup computes the
@@ -1196,6 +1209,19 @@ __global__ __launch_bounds__(SMALL_PLAN_THREADS) void small_plan_kernel(
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1) rank += __shfl_xor(rank, off);
         if (g < n_groups && sub == 0) group_order[rank] = g;
+        if (gb == 0 && wave == 0) {
+            int sum = 0, longest = 0;
+            for (int j = lane; j < n_groups; j += 64) {
+                sum += s_cnt[j];
+                longest = max(longest, s_cnt[j]);
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                sum += __shfl_xor(sum, off);
+                longest = max(longest, __shfl_xor(longest, off));
+            }
+            if (lane == 0) group_order[n_groups] = level_heads(n_groups, sum, longest);
+        }
         return;
     }
     // ---- 16 row blocks, one per wave: their non-empty 128 x 32 tiles over the whole batch

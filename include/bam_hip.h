@@ -125,7 +125,8 @@ typedef struct bam_plan {
     const int32_t* group_order; /* device, B * ceil(Sq/128) ints, or null (more than 8192 groups): the groups of four
                                    slices of `order` (code b * ceil(Sq/128) + group) by falling number of 64-key tiles
                                    they visit, the order in which the forward and dQ kernels take their workgroups, so
-                                   that the longest start first whatever the sequences of a batch look like */
+                                   that the longest start first whatever the sequences of a batch look like; one more int
+                                   behind them: from how many q heads on the kernels take the lists for level */
     const int64_t* row_workloads; /* device, ceil(Sq/128) int64: per 128-row block, the number of its 128 x 32 tiles in
                                      which some pair is allowed, summed over the batch -- sum(flags > 0) over batch and
                                      key columns, the workloads the reference's makespan-minimizing sequence split sorts
