@@ -2,6 +2,7 @@
 // The declarations (with the reference call sites they replace) are in include/bam_hip.h.
 #include "../../include/bam_hip.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
@@ -330,7 +331,7 @@ extern "C" {
 
 const char* bam_last_error(void) { return g_error; }
 
-int bam_abi_version(void) { return 14; }
+int bam_abi_version(void) { return 15; }
 
 int bam_tile_flags(const int64_t* bf, int64_t bf_stride_b, int8_t* flags, int64_t flags_stride_b,
                    int64_t flags_stride_m, int B, int S, void* stream) {
@@ -813,14 +814,20 @@ int bam_attn_fwd(const bam_attn* a, void* stream) {
 // How many workgroups share the q heads of a kv head in dK/dV.  One workgroup per (key tile, kv head) walks all of them one after
 // the other and the launch lasts as long as the first key tile's; dealt to parts, the tiles level out over the 256 compute units.
 // The price is fp32 sums through memory and a launch that adds them.  The estimate, in us: a step over a pair of slices takes
-// `step`, a workgroup kStart steps besides, tiles fall off linearly in length (a causal mask); the launch takes the longest
-// workgroup, or the work per compute unit and kTail of the longest.  Fitted to 42 training steps (D 32, 64, 128; 6 to 32 q heads,
-// 1 to 8 kv heads, 300 to 9000 tokens), of which it takes the fastest number of parts, or one within 5 %; gains of a few
-// per cent are not there (1 x 16384 tokens, 2 parts: dK/dV 4115 -> 4069 and 56 for the sum).  One part -> parts,
-// kernels of a step, us, 32 / 8 heads, D 128: 300 tokens 87 -> 68 (4 parts), 2 x 700 147 -> 120 (4), 2500 380 -> 305 (2), 3001
-// 453 -> 355 (2), 5000 861 -> 790 (2), but 4 x 1537 (416 workgroups) 412 -> 445; 16 / 4 heads, 9000 tokens 1404 -> 1255; D 64:
-// 3001 tokens 322 -> 256, 5000 560 -> 513.  At least 32 steps have to go: below, the host is what a training step waits for (4 x 400
-// tokens, 6 / 1 heads, D 40, 35 steps: 94 -> 58 to 98 us with the speed of the host; 2 x 283, 6 / 2 heads, 10 steps: 86 -> 91).
+// `step`, a workgroup kStart steps besides, tiles fall off linearly in length (as a causal mask's do, or less where the plan's pairs
+// are known to be more, or there is no mask); the launch takes the longest workgroup, or the work per compute unit and kTail of the
+// longest, or (level lists: what the causal fit has in kTail) what a compute unit takes that gets k + 1 of the 256 k + 1 longest.
+// Fitted to 42 training steps with segments (D 32, 64, 128; 6 to 32 q heads, 1 to 8 kv heads, 300 to 9000 tokens), of which it takes
+// the fastest number of parts, or one within 5 %; gains of a few per cent are not there (1 x 16384 tokens, 2 parts: dK/dV 4115 ->
+// 4069 and 56 for the sum).  One part -> parts, kernels of a step, us, 32 / 8 heads, D 128: 2 x 700 147 -> 120 (4), 2500 380 -> 305
+// (2), 3001 453 -> 355 (2), 5000 861 -> 790 (2), but 4 x 1537 (416 workgroups) 412 -> 445; 16 / 4 heads, 9000 tokens 1404 -> 1255;
+// D 64: 3001 tokens 322 -> 256, 5000 560 -> 513.  At least 32 steps have to go: below, the host is what a training step waits for
+// (4 x 400 tokens, 6 / 1 heads, D 40, 35 steps: 94 -> 58 to 98 us with the speed of the host; 2 x 283, 6 / 2 heads, 10 steps: 86 ->
+// 91; 300 tokens, 32 / 8 heads, 15 steps: kernels 87 -> 68, not taken).
+// Nothing hidden, backward, us, 32 / 8 heads, D 128, parts of the causal estimate -> of the known lists: 2500 tokens 434 (2) -> 405
+// (1), 3001 526 (2) -> 496 (1), 2 x 1537 311 (2) -> 287 (1), 5000 1336 (2) -> 1282 (4); no mask: 2500 479 (2) -> 424 (1).
+// Up to D 64 the host does not wait for the pairs, so a mask that hides nothing gets the causal estimate's parts: D 64, 3001 tokens
+// one part 314, two 330, 4096 501 / 506, but 5000 983 / 821.
 static int dkdv_parts(const bam_attn* a) {
     if (a->head_runs > 1 || a->B <= 0 || a->Sk <= 0 || a->Hkv <= 0 || a->Hq <= a->Hkv || a->Hq % a->Hkv || a->Sq > bam::MAX_SLICE_LIST * 32)
         return 1;
@@ -831,10 +838,14 @@ static int dkdv_parts(const bam_attn* a) {
     const double tiles = (a->Sk + 127) / 128, pairs = (a->Sq + 63) / 64, step = a->D > 96 ? 1.25 : a->D > 64 ? 1.1 : a->D > 32 ? 0.79 : 0.63;
     constexpr double kStart = 7.8, kTail = 0.28, kBytesPerUs = 8.7e6, kLaunch = 6;  // (the parts stay in the last-level cache)
     const double units = a->B * (double)a->Hkv * tiles, rows = (double)a->B * a->Sk * a->Hkv;
+    double mean = a->mode == BAM_MASK_DENSE && a->mask == nullptr ? pairs : (pairs + 1) / 2;
+    if (a->pairs > 0) mean = std::min(pairs, std::max(mean, a->pairs / (2.0 * a->B * tiles)));
     auto estimate = [&](int parts) {
-        const double longest = pairs * G / parts, share = units * ((pairs + 1) / 2 * G + kStart * parts) / 256 + kTail * longest;
-        const double sum = parts > 1 ? kLaunch + 2 * 2 * 4 * rows * a->D * parts / kBytesPerUs : 0;
-        return step * (longest + kStart > share ? longest + kStart : share) + sum;
+        const double longest = pairs * G / parts, share = units * (mean * G + kStart * parts) / 256 + kTail * longest;
+        double time = longest + kStart > share ? longest + kStart : share;
+        for (int k = 1; mean > (pairs + 1) / 2 && k <= 8 && 256 * k < units * parts; ++k)
+            time = std::max(time, (k + 1) * (longest - 2 * (longest - mean * G / parts) * 256 * k / (units * parts) + kStart));
+        return step * time + (parts > 1 ? kLaunch + 2 * 2 * 4 * rows * a->D * parts / kBytesPerUs : 0);
     };
     const double one = estimate(1);
     int best = 1;

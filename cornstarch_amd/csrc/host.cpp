@@ -558,7 +558,7 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     if (plan && a.D > 64 && a.Sk <= 131072) {
         optional<py::gil_scoped_release> release;
         if (PyGILState_Check()) release.emplace();
-        plan.core->wait_pairs();
+        a.pairs = plan.core->wait_pairs();
         release.reset();
         desc.rows_known = plan.core->rows_known.load();
         py::gil_scoped_acquire gil;

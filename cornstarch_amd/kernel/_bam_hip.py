@@ -15,7 +15,7 @@ BAM_DTYPE_F16 = 0
 BAM_DTYPE_BF16 = 1
 BAM_MAX_SEQLEN = 4194304
 BAM_STATIC_PLAN_BYTES = 8 << 20
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -115,6 +115,7 @@ class Attn(ctypes.Structure):
         ("parts_workspace", ctypes.c_void_p),
         ("parts_bytes", ctypes.c_int64),
         ("lse_scaled", ctypes.c_void_p),
+        ("pairs", _i64),
     ]
 
 

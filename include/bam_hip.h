@@ -507,6 +507,7 @@ typedef struct bam_attn {
     void* parts_workspace; /* bam_attn_bwd: may be null; bam_attn_bwd_parts bytes, 16-byte aligned */
     int64_t parts_bytes;
     float* lse_scaled; /* bam_attn_bwd: scratch of the size of lse for lse * log2(e), used up to head dim 64; may be null */
+    int64_t pairs;     /* bam_attn_bwd(_parts): *plan.ds_count if the host knows it (the same in both calls), otherwise 0 */
 } bam_attn;
 int bam_attn_fwd(const bam_attn* args, void* stream);
 int bam_attn_bwd(const bam_attn* args, void* stream);

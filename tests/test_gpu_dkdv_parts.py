@@ -11,11 +11,11 @@ from tests.helpers import random_bitfield
 pytestmark = pytest.mark.gpu
 
 
-# units = B * Hkv * ceil(S / 128); parts: the largest divisor of Hq / Hkv with units * parts <= 256
+# (how many parts each of them gets: test_dkdv_parts.py)
 @pytest.mark.parametrize("B,S,Hq,Hkv,D", [
     (1, 129, 16, 1, 32), (1, 700, 32, 8, 40), (1, 2100, 6, 3, 56), (4, 400, 6, 1, 64),
-    (3, 1000, 24, 4, 64),  # 96 units: 2 parts of 3 heads
-    (1, 4100, 12, 3, 8),   # 99 units: 2 parts of 2
+    (3, 1000, 24, 4, 64),  # 3 parts of 2 heads
+    (1, 4100, 12, 3, 8),   # 4 parts of 1
     (1, 700, 32, 8, 128), (2, 900, 16, 4, 96), (1, 2003, 12, 4, 112),  # with the hand-over of dS
     (2, 283, 6, 2, 64), (4, 1537, 8, 4, 32),  # one part: too little to share, enough workgroups
 ])
