@@ -549,12 +549,6 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     if (scaled) a.lse_scaled = a.delta + lse.numel();
     a.accumulate = accumulate ? 1 : 0;
     Tensor ws;
-    if (plan && desc.rows != nullptr && a.D <= 64) {  // (one launch of dK/dV instead of two; it is there by the time the forward starts)
-        optional<py::gil_scoped_release> release;
-        if (PyGILState_Check()) release.emplace();
-        plan.core->wait_pairs();
-        desc.rows_known = plan.core->rows_known.load();
-    }
     if (plan && a.D > 64 && a.Sk <= 131072) {
         optional<py::gil_scoped_release> release;
         if (PyGILState_Check()) release.emplace();

@@ -211,3 +211,29 @@ def test_an_entry_made_anew_is_owned_by_the_next_graph(inputs):
     torch.cuda.synchronize()
     for a, b in zip(want, got):
         assert torch.equal(a, b)
+
+
+def test_a_backward_up_to_head_dim_64_does_not_wait_for_the_gpu():
+    """Sorted rows (32768 tokens on) are launched as they come: the host does not need to know whether they were moved."""
+    n, h, d = 32768, 1, 64
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = [torch.randn(1, n, h, d, generator=g, device="cuda").bfloat16().requires_grad_(True) for _ in range(3)]
+    do = torch.randn(1, n, h, d, generator=g, device="cuda").bfloat16()
+    bf = random_bitfield(1, n, seed=4).cuda()
+
+    def step():
+        _forget()
+        return torch.autograd.grad(BA.bitfield_attn_func(*x, bf), x, do)
+
+    want = step()
+    torch.cuda.synchronize()
+    held = torch.cuda.Event()
+    torch.cuda._sleep(20 * BUSY)
+    held.record()
+    got = step()
+    waited = held.query()
+    torch.cuda.synchronize()
+    assert not waited
+    for a, b in zip(want, got):
+        assert torch.equal(a, b)
+    _forget()
