@@ -41,6 +41,9 @@ __device__ __forceinline__ void dma_b128_stream(const void* sbase, unsigned voff
 // and the hardware writes zeros to its LDS slot.  For the K tiles of the decode step (8 x 8192 keys: 48.7 us either way); the other
 // kernels copy through RowView.
 constexpr unsigned DMA_RANGE = 0x80000000u, DMA_ZERO = 0xC0000000u;  // (room below for 31 rows of 2^24 bytes: decode steps back)
+// The same for RowView, whose descriptors end below 2^31 and whose copies add a scalar offset below 2^31: beyond any of them, and
+// the sum stays below 2^32.
+constexpr unsigned ROW_ZERO = 0x80000000u;
 template <int SITE = 0>
 __device__ __forceinline__ void dma_b128_ranged(const void* sbase, unsigned voff, unsigned lds_base) {
     const unsigned long long base = reinterpret_cast<unsigned long long>(sbase);  // (48 bits: no stride in the second word)
@@ -148,15 +151,15 @@ struct TileStage {
     unsigned goff[CPT];
     int wave_first;  // first chunk slot this wave fills with instruction 0
 
-    // chunks: how many 16-byte chunks a row has in global memory (d / 8)
-    __device__ __forceinline__ void setup(int64_t row_stride_bytes, int chunks, int tid) {
+    // chunks: how many 16-byte chunks a row has in global memory (d / 8); zero: the offset that reads zeros
+    __device__ __forceinline__ void setup(int64_t row_stride_bytes, int chunks, int tid, unsigned zero = ROW_ZERO) {
         wave_first = __builtin_amdgcn_readfirstlane(tid & ~63);
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int id = tid + THREADS * i;
             const int row = id / NCH, pc = id % NCH;
             const int c = pc ^ swz<D>(row);
-            goff[i] = ZERO_PAD && c >= chunks ? DMA_ZERO : (unsigned)(row * row_stride_bytes + (c < chunks ? c : 0) * 16);
+            goff[i] = ZERO_PAD && c >= chunks ? zero : (unsigned)(row * row_stride_bytes + (c < chunks ? c : 0) * 16);
         }
     }
     // tile_base: first row of the tile in global memory, tile_lds: lds_addr() of the LDS tile

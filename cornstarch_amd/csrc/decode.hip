@@ -125,7 +125,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 1 ? 2 : 1) void decode_kernel(
     TileStage<D, DEC_KT, 64, true> stK;
     TileStage<D, DEC_KT, 64> stV;
     constexpr int CPT = TileStage<D, DEC_KT, 64>::CPT;
-    stK.setup(2 * p.k_ss, chunks, lane);
+    stK.setup(2 * p.k_ss, chunks, lane, DMA_ZERO);
     stV.setup(2 * p.v_ss, chunks, lane);
 
     // ---- Q: rows = heads, zero rows past the last head, zero columns past the head dim ----

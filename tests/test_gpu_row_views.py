@@ -68,6 +68,25 @@ def test_rows_two_gigabytes_apart(far, D):
         assert torch.isfinite(b).all() and rel_l2(b.float(), a.float()) <= 2e-3
 
 
+@pytest.mark.parametrize("D", [8, 40, 64, 72, 120])
+@pytest.mark.parametrize("far", [0, 1, 2, 3], ids=["q", "k", "v", "do"])
+def test_rows_between_one_and_two_gigabytes_apart(far, D):
+    # head dims between the compiled ones: the columns past them are zeros wherever in the tensor a tile starts
+    B, S, Hq, Hkv = 1, 121, 4, 2
+    plain = _inputs(B, S, Hq, Hkv, D, torch.bfloat16, far + D)
+    stride = (1 << 23) - 8  # 120 rows of it are 2.01e9 bytes
+    spread = list(plain)
+    t = plain[far]
+    store = torch.full(((S - 1) * stride + t.shape[2] * D,), float("inf"), dtype=t.dtype, device="cuda")
+    spread[far] = store.as_strided(t.shape, (stride, stride, D, 1))
+    spread[far].copy_(t)
+    bf = random_bitfield(B, S, seed=7).cuda()
+    attend = lambda q, k, v: BA.bitfield_attn_func(q, k, v, bf)  # noqa: E731
+    for a, b in zip(_step(*plain, attend), _step(*spread, attend)):
+        assert torch.isfinite(b).all() and torch.equal(a, b)
+    BA.BitfieldUtils.clear_cache()
+
+
 @pytest.mark.parametrize("D", [40, 128])
 @pytest.mark.parametrize("S", [70, 96])
 def test_rows_that_overlap(S, D):
