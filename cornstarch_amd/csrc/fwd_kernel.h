@@ -487,8 +487,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     constexpr int DB0 = STREAMS > 1 ? (DB + 1) / 2 : DB;  // stream 0 finishes the column blocks below DB0, stream 1 the others
     f32x4* const park = (f32x4*)sK_all + wave * (DB * 4 * 64);
     float* const park_ml = (float*)sV_all;
-    const bool merged = STREAMS > 1 && !side;
-    if (merged) {
+    if (STREAMS > 1 && !side) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
             if ((db < DB0) == (stream == 1)) {
@@ -517,11 +516,16 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + 32 * (4 * grp + wave) + l32] = -INFINITY;
     if (qvalid) {
         char* op = (char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
+        if (__builtin_expect(side, 0)) {  // (a loop of its own: the other one reads the partner's blocks together)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) store_block16<T>(op + 64 * db, p.d - 32 * db, hi, [&](int i) { return o[db][i] * inv; });
+            return;
+        }
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            if (merged && (db < DB0) != (stream == 0)) continue;
+            if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
             f32x16 x = o[db];
-            if (merged) {
+            if constexpr (STREAMS > 1) {
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
                     const f32x4 other = park[(4 * db + grp) * 64 + lane];
