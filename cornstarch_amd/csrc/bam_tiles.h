@@ -267,19 +267,24 @@ __device__ __forceinline__ int plan_word(const int* at) {
     return *(const __attribute__((address_space(4))) int*)(unsigned long long)at;
 }
 
+// ONE_LOAD: the four codes in one load; left alone, the compiler waits for each before it asks for the next (0.5 us of a launch).
+// Not with a bias, whose kernels spill scalars: dQ at D 32 over a bias matrix got 2 % slower.
+template <bool ONE_LOAD = true>
 __device__ __forceinline__ WaveSlices pick_wave_slices(const AttnParams& p, int b, int grp) {
     WaveSlices w;
     w.moved = false;
     if (p.fine != nullptr) {
         const int* ord = p.order + (int64_t)b * p.order_sb + 4 * grp;
-        int code[4];  // (one load: left in the loop below, the compiler waits for each before it asks for the next)
+        int code[4];
+        if constexpr (ONE_LOAD) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) code[x] = plan_word(ord + x);
-        asm volatile("" ::"s"(code[0]), "s"(code[1]), "s"(code[2]), "s"(code[3]));
-        w.moved = order_moved(code[0]);  // (a group has a first slice)
+            for (int x = 0; x < 4; ++x) code[x] = plan_word(ord + x);
+            asm volatile("" ::"s"(code[0]), "s"(code[1]), "s"(code[2]), "s"(code[3]));
+        }
+        w.moved = order_moved(ONE_LOAD ? code[0] : ord[0]);  // (a group has a first slice)
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-            w.slice[x] = order_slice(code[x]);
+            w.slice[x] = order_slice(ONE_LOAD ? code[x] : ord[x]);
             w.cls_row[x] = w.slice[x] >= 0
                                ? (const int8_t*)p.fine + (int64_t)b * p.fine_sb + (int64_t)w.slice[x] * p.fine_ss
                                : nullptr;

@@ -782,9 +782,11 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
 
     int ub, hk, g;
     head_unit_map(blockIdx.x, p.num_m * p.B, p.Hkv, G, ub, hk, g);
-    int code = p.group_order != nullptr ? plan_word(p.group_order + ub) : 0;
+    constexpr bool MAY_SIDE = STREAMS > 1 && D > 32;
+    int code = 0;
     bool side = false, idle = false;  // the streams take a unit each; ... and there is none left for this one
-    if constexpr (STREAMS > 1 && D > 32) {
+    if constexpr (MAY_SIDE) {
+        if (p.group_order != nullptr) code = plan_word(p.group_order + ub);
         side = streams_side_by_side(p);
         if (__builtin_expect(side, 0)) {
             const int units = p.num_m * p.B * p.Hq, unit = side_unit(blockIdx.x, stream);
@@ -796,11 +798,12 @@ __global__ __launch_bounds__(DQ_THREADS * STREAMS, D > 64 || BIAS_FORM == BIAS_T
     }
     int b = ub % p.B, grp = ub / p.B;
     if (p.group_order != nullptr) {  // with a plan: the groups of all sequences by falling length of their tile lists
+        if constexpr (!MAY_SIDE) code = p.group_order[ub];
         b = code / p.num_m;
         grp = code - b * p.num_m;
     }
     const int h = hk * G + g;
-    const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
+    const WaveSlices ws = pick_wave_slices<!BIAS>(p, b, grp);  // group 0 is the heaviest
 
     const int slice = idle ? -1 : __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
     const int slot = (slice < 0 ? 0 : slice) * 32 + l32;

@@ -69,9 +69,11 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
 
     int ub, hk, g;
     head_unit_map(blockIdx.x, p.num_m * p.B, p.Hkv, G, ub, hk, g);
-    int code = p.group_order != nullptr ? plan_word(p.group_order + ub) : 0;
+    constexpr bool MAY_SIDE = STREAMS > 1 && D > 32;
+    int code = 0;
     bool side = false, idle = false;  // the streams take a unit each; ... and there is none left for this one
-    if constexpr (STREAMS > 1 && D > 32) {
+    if constexpr (MAY_SIDE) {
+        if (p.group_order != nullptr) code = plan_word(p.group_order + ub);
         side = streams_side_by_side(p);
         if (__builtin_expect(side, 0)) {
             const int units = p.num_m * p.B * p.Hq, unit = side_unit(blockIdx.x, stream);
@@ -83,11 +85,12 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     }
     int b = ub % p.B, grp = ub / p.B;
     if (p.group_order != nullptr) {  // with a plan: the groups of all sequences by falling length of their tile lists
+        if constexpr (!MAY_SIDE) code = p.group_order[ub];
         b = code / p.num_m;
         grp = code - b * p.num_m;
     }
     const int h = hk * G + g;
-    const WaveSlices ws = pick_wave_slices(p, b, grp);  // group 0 is the heaviest
+    const WaveSlices ws = pick_wave_slices<!BIAS>(p, b, grp);  // group 0 is the heaviest
 
     // ---- per-lane query state -------------------------------------------------------
     const int slice = idle ? -1 : __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
@@ -487,7 +490,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     constexpr int DB0 = STREAMS > 1 ? (DB + 1) / 2 : DB;  // stream 0 finishes the column blocks below DB0, stream 1 the others
     f32x4* const park = (f32x4*)sK_all + wave * (DB * 4 * 64);
     float* const park_ml = (float*)sV_all;
-    if (STREAMS > 1 && !side) {
+    auto meet = [&]() {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
             if ((db < DB0) == (stream == 1)) {
@@ -505,7 +508,9 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         theirs = __builtin_amdgcn_exp2f((m_other - muse) * c2);
         ltot = stream == 0 ? fmaf(ltot, mine, l_other * theirs) : fmaf(l_other, theirs, ltot * mine);
         m_i = m;
-    }
+    };
+    if constexpr (STREAMS > 1)
+        if (!side) meet();
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
     if ((stream == 0 || side) && hi == 0 && slice >= 0)
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + qrow] =
@@ -516,11 +521,12 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         p.lse[(int64_t)b * p.lse_sb + (int64_t)h * p.Sq_rounded + 32 * (4 * grp + wave) + l32] = -INFINITY;
     if (qvalid) {
         char* op = (char*)p.o.ptr + 2 * ((int64_t)b * p.o.sb + (int64_t)qrow * p.o.ss + (int64_t)h * p.o.sh);
-        if (__builtin_expect(side, 0)) {  // (a loop of its own: the other one reads the partner's blocks together)
+        if constexpr (MAY_SIDE)
+            if (__builtin_expect(side, 0)) {  // (a loop of its own: the other one reads the partner's blocks together)
 #pragma unroll
-            for (int db = 0; db < DB; ++db) store_block16<T>(op + 64 * db, p.d - 32 * db, hi, [&](int i) { return o[db][i] * inv; });
-            return;
-        }
+                for (int db = 0; db < DB; ++db) store_block16<T>(op + 64 * db, p.d - 32 * db, hi, [&](int i) { return o[db][i] * inv; });
+                return;
+            }
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             if (STREAMS > 1 && (db < DB0) != (stream == 0)) continue;
