@@ -106,8 +106,8 @@ struct RowView {
 // WAIT: wait states in front of the copy, less one.  A scalar register that a vector instruction has written (the reload of a
 // spilled one) must not be read by a memory instruction within five wait states, and the compiler does not look into an asm
 // statement.  Instantiations whose scalar registers spill in the loop pass 4 (COPY_WAIT); the others need the one state after
-// the write of M0: waiting five everywhere costs 1 to 2.5 % of every kernel (forward + backward of 1 x 8192 tokens, 32 / 8
-// heads, D 128: 1769 -> 1791 us).  tests/test_copy_hazard.py looks at every copy of the built library.
+// the write of M0: waiting five everywhere costs 1.2 % (forward + backward of 1 x 8192 tokens, 32 / 8 heads, D 128: 1769 ->
+// 1791 us).  tests/test_copy_hazard.py looks at every copy of the built library.
 template <int WAIT>
 __device__ __forceinline__ void copy_b128(const TileSrc& src, unsigned voff, unsigned lds_base) {
     asm volatile("s_nop %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(src.desc), "s"(src.off),
@@ -317,8 +317,8 @@ __device__ __forceinline__ int side_unit(int block, int stream) { return 16 * (b
 // the end of the sequence (those columns must still be masked out of the softmax).
 // Executed by wave 0; the caller synchronizes before reading.
 // STREAMS = 2: the even and the odd tiles make a list each (the second at list + MAX_LIST / 2, its length in count_out[1]).  Which
-// list a tile is in does not depend on what else is listed, so a row's result does not depend on its neighbours or the plan.
-// (split false: one list all the same.)
+// list a tile is in does not depend on what else is listed, so the tiles of a slice are added up in the same order whatever group or
+// plan it is in.  (split false: one list all the same.)
 template <int STREAMS = 1>
 __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int num_n, int S, int lane, int kt_begin,
                                                     int* list, int* count_out, bool split = STREAMS > 1) {

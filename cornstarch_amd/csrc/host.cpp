@@ -356,7 +356,8 @@ bool bitfield_ready(const Tensor& bf) {
 // From here on the plan's rows are sorted (where the segments are many).  A sequence with few segments, whose rows stay, pays the
 // launch that finds that out: 4 us, which may be 2 % of the shortest forward over 16384 tokens (4 heads, D 32) and is at most 0.7 %
 // from here on.  Many segments gain 5 to 28 %: forward + backward of 65536 tokens with 200 segments 62.9 -> 47.7 ms, forward alone
-// of 32768 tokens with 60, 16 / 4 heads, D 64 1920 -> 1730 us.
+// of 32768 tokens with 60, 16 / 4 heads, D 64 1920 -> 1730 us.  Shorter ones with many segments would gain as well (8192 tokens with
+// 30: 1873 -> 1678) and do without, as nobody knows how many there are before that launch.
 constexpr int64_t kSortedRows = 32768;
 
 // flags (and plan, up to 131072 tokens) of an int64 (B, S) mask on the GPU
