@@ -325,6 +325,7 @@ Cached g_bitfield, g_mask;
 void store(Cached& slot, const Tensor& owner, const Tensor& flags, Plan plan, const Stream& stream) {
     Prepared::collect();
     if (owner.is_inference()) return;  // no version counter: nothing would tell that it has been written to
+    if (stream.stream() != nullptr && capturing()) return;  // (flags without a plan: replays compute them, in the graph's memory)
     Cached fresh;
     fresh.owner = owner;
     fresh.owner_strides = owner.strides().vec();

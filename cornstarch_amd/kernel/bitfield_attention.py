@@ -417,7 +417,8 @@ class _IndexView:
             if cls._last is not None and cls._last[0] == key and cls._last[1]._prepared.use():
                 return cls._last[1]
             view = cls(bitfield_mask, offsets_q, offsets_k)
-            cls._last = (key, view, (bitfield_mask, offsets_q, offsets_k))
+            if not torch.cuda.is_current_stream_capturing():  # (without a plan: replays gather, into the graph's memory)
+                cls._last = (key, view, (bitfield_mask, offsets_q, offsets_k))
             return view
 
     @classmethod

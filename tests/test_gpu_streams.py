@@ -237,3 +237,39 @@ def test_a_backward_up_to_head_dim_64_does_not_wait_for_the_gpu():
     for a, b in zip(want, got):
         assert torch.equal(a, b)
     _forget()
+
+
+@pytest.mark.parametrize("indexed", [False, True])
+def test_what_a_capture_computes_stays_out_of_the_caches(indexed):
+    """Beyond 131072 rows there is no plan, so flags and index views can be made in a capture: in the graph's memory, by its replays."""
+    n = 131200
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn(1, rows, 1, 32, generator=g, device="cuda").bfloat16() for rows in (n, 256, 256))
+    bf = torch.full((1, n), 2, dtype=torch.int64, device="cuda")
+    bf[:, ::40000] = (1 << 62) | 3
+    rows = torch.arange(n, device="cuda")
+
+    def call():
+        if not indexed:
+            return BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(bf)
+        view = BA._IndexView.get(bf, rows, rows[:256])
+        assert view.plan is None
+        flags = torch.full((1, -(-n // 128), 8), 1, dtype=torch.int8, device="cuda")
+        return BA._bitfield_attn_forward(q, k, v, bf, flags, rows, rows[:256])[0]
+
+    want = call().clone()
+    torch.cuda.synchronize()
+    _forget()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = call()
+    eager = call()  # nothing has been replayed yet
+    torch.cuda.synchronize()
+    assert torch.equal(eager, want)
+    for _ in range(3):
+        got.zero_()
+        _forget()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    _forget()
