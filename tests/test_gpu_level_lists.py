@@ -38,6 +38,34 @@ def test_level_lists_equal_one_stream(S, H, few, many, D, kind):
     _MaskPlan.forget()
 
 
+# index tensors, both forms of a bias, grouped heads, nearly level lists (one text row in 300): forward and dQ
+@pytest.mark.parametrize("kind", ["indexed", "bias row", "bias matrix", "grouped", "nearly"])
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("S,H,few,many", [(1601, 21, 1, 2), (1300, 12, 3, 6)])
+def test_other_forms_of_level_lists_equal_one_stream(S, H, few, many, D, kind):
+    Hkv = H // 3 if kind == "grouped" else H
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v, do = (torch.randn(many, S, h, D, generator=g, device="cuda").bfloat16() for h in (H, Hkv, Hkv, H))
+    bias = torch.randn(1, H, S if kind == "bias matrix" else 1, S, generator=g, device="cuda") if "bias" in kind else None
+    rows = torch.arange(S, device="cuda") if kind == "indexed" else None
+
+    def run(n):
+        bf = torch.full((n, S), 2, dtype=torch.int64, device="cuda")
+        if kind == "nearly":
+            bf[:, 150::300] = (1 << 62) | 2
+        x = [t[:n].contiguous() for t in (q, k, v, do)]
+        BA.BitfieldUtils.clear_cache()
+        flags = BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(bf)
+        o, lse, scale = BA._bitfield_attn_forward(*x[:3], bf, flags, rows, rows, bias=bias)
+        grads = [torch.zeros(t.shape, device="cuda") for t in x[:3]]
+        BA._bitfield_attn_backward(x[3], *x[:3], o, bf, flags, lse, *grads, rows, rows, bias=bias, softmax_scale=scale)
+        return o, lse, grads[0]
+
+    for a, b in zip(run(many), run(few)):
+        assert not torch.isnan(b).any() and torch.equal(a[:few], b)
+    BA.BitfieldUtils.clear_cache()
+
+
 # both forms of the plan builder's last launches
 @pytest.mark.parametrize("B,S", [(1, 1), (1, 65), (3, 515), (2, 1300), (5, 2000), (1, 9000), (70, 130)])
 def test_the_plan_knows_how_level_its_lists_are(B, S):
