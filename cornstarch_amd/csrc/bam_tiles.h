@@ -309,6 +309,24 @@ __device__ __forceinline__ bool streams_side_by_side(const AttnParams& p) {
 // (units 8 apart are on the same XCD and, in head_unit_map, heads that read the same rows)
 __device__ __forceinline__ int side_unit(int block, int stream) { return 16 * (block >> 3) + (block & 7) + 8 * stream; }
 
+// The class bytes of 64-key tile kt (< nkt, or one that does not matter) for the four slices.  Without branches: the eight loads
+// are on their way together, where each waited for the one before as long as slices that are not there were skipped.
+struct TileClasses {
+    int f[4][2];
+};
+__device__ __forceinline__ TileClasses load_tile_classes(const WaveSlices& ws, int num_n, int nkt, int kt) {
+    TileClasses c;
+    const int at = 2 * max(min(kt, nkt - 1), 0), second = min(at + 1, num_n - 1);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        const int8_t* row = ws.cls_row[x] != nullptr ? ws.cls_row[x] : ws.cls_row[0];  // (a group has a first slice)
+        c.f[x][0] = row[at];
+        c.f[x][1] = row[second];
+    }
+    return c;
+}
+__device__ __forceinline__ int key_tiles(int S, int kt_begin) { return min((S + 63) >> 6, kt_begin + MAX_LIST); }
+
 // List, in ascending order, the 64-key tiles the four slices of a workgroup have to visit, among the (at most
 // MAX_LIST) tiles starting at tile kt_begin; longer sequences are walked in several passes.
 // entry = (tile << 8) | c0 | c1 << 2 | c2 << 4 | c3 << 6 ; c_w is the class of the tile for wave w's slice:
@@ -316,31 +334,32 @@ __device__ __forceinline__ int side_unit(int block, int stream) { return 16 * (b
 // A tile is "full" for a slice only when both of its 32-column classes say so AND it has no column past
 // the end of the sequence (those columns must still be masked out of the softmax).
 // Executed by wave 0; the caller synchronizes before reading.
+// first: load_tile_classes of this lane's first tile.  The classes of the next 64 tiles are asked for before those at hand are
+// looked at.
 // STREAMS = 2: the even and the odd tiles make a list each (the second at list + MAX_LIST / 2, its length in count_out[1]).  Which
 // list a tile is in does not depend on what else is listed, so the tiles of a slice are added up in the same order whatever group or
 // plan it is in.  (split false: one list all the same.)
 template <int STREAMS = 1>
-__device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int num_n, int S, int lane, int kt_begin,
+__device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int num_n, int S, int lane, int kt_begin, const TileClasses& first,
                                                     int* list, int* count_out, bool split = STREAMS > 1) {
-    const int nkt = min((S + 63) >> 6, kt_begin + MAX_LIST);
+    const int nkt = key_tiles(S, kt_begin);
     int count[STREAMS] = {};
     const int mine = STREAMS > 1 && split ? lane & 1 : 0;  // (kt_begin is even)
     const unsigned long long even = split ? 0x5555555555555555ull : ~0ull;
+    TileClasses cur = first;
     for (int base = kt_begin; base < nkt; base += 64) {
+        const TileClasses next = load_tile_classes(ws, num_n, nkt, base + 64 + lane);
         const int kt = base + lane;
+        const bool second = 2 * kt + 1 < num_n, inside = (kt + 1) * 64 <= S;
         int packed = 0;
-        if (kt < nkt) {
-            const bool second = 2 * kt + 1 < num_n, inside = (kt + 1) * 64 <= S;
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                if (ws.cls_row[x] == nullptr) continue;  // wave-uniform
-                const int f0 = ws.cls_row[x][2 * kt];
-                const int f1 = second ? ws.cls_row[x][2 * kt + 1] : 0;
-                int cls = 0;
-                if (f0 > 0 || f1 > 0) cls = (f0 == 2 && f1 == 2 && inside) ? 2 : 1;
-                packed |= cls << (2 * x);
-            }
+        for (int x = 0; x < 4; ++x) {
+            const int f0 = cur.f[x][0], f1 = second ? cur.f[x][1] : 0;
+            int cls = 0;
+            if (f0 > 0 || f1 > 0) cls = (f0 == 2 && f1 == 2 && inside) ? 2 : 1;
+            packed |= ws.cls_row[x] != nullptr ? cls << (2 * x) : 0;
         }
+        if (kt >= nkt) packed = 0;
         unsigned long long bal = __ballot(packed != 0), own = bal;
         if (STREAMS > 1) own &= mine ? ~even : even;
         const int at = (mine ? MAX_LIST / 2 + count[STREAMS - 1] : count[0]) + __popcll(own & ((1ull << lane) - 1ull));
@@ -348,6 +367,7 @@ __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int nu
 #pragma unroll
         for (int x = 0; x < STREAMS; ++x)
             count[x] += __popcll(STREAMS == 1 ? bal : bal & (x ? ~even : even));
+        cur = next;
     }
 #pragma unroll
     for (int x = 0; x < STREAMS; ++x)
@@ -355,25 +375,37 @@ __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int nu
     wait_lds();
 }
 
+// The four class bytes (key columns 4 nt ..) of slice s (< s_end, or one that does not matter), low byte first.
+__device__ __forceinline__ unsigned load_slice_classes(const AttnParams& p, int b, int nt, int s, int s_end) {
+    s = max(min(s, s_end - 1), 0);
+    if (p.fine != nullptr)  // (rows of the plan's classes are padded to 16 bytes)
+        return *(const unsigned*)(p.fine + (int64_t)b * p.fine_sb + (int64_t)s * p.fine_ss + 4 * nt);
+    const int8_t* f = p.flags + (int64_t)b * p.flags_sb + (int64_t)(s >> 2) * p.flags_sm;
+    unsigned c = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) c |= (unsigned)(f[min(4 * nt + w, p.num_n - 1)] & 3) << (8 * w);
+    return c;
+}
+
 // List, in ascending order, the 32-row slices among [s_begin, s_end) (at most MAX_SLICE_LIST of them; longer
 // sequences are walked in several passes) that have work for a 128-key tile (4 class columns).
 // entry = (slice << 8) | c0 | c1 << 2 | c2 << 4 | c3 << 6, c_w = class of (slice, key column 4 nt + w).
 // With a plan the classes are those of the 32 x 32 tiles; without one a slice inherits the flags of its
 // 128-row block.
-__device__ __forceinline__ void build_slice_list(const AttnParams& p, int b, int nt, int lane, int s_begin, int s_end,
+// first: load_slice_classes of this lane's first slice.
+__device__ __forceinline__ void build_slice_list(const AttnParams& p, int b, int nt, int lane, int s_begin, int s_end, unsigned first,
                                                  int* list, int* count_out) {
     const int ns = s_end;
     int count = 0;
+    unsigned cur = first;
     for (int base = s_begin; base < ns; base += 64) {
+        const unsigned next = load_slice_classes(p, b, nt, base + 64 + lane, ns);
         const int s = base + lane;
         int packed = 0;
         if (s < ns) {
-            const int8_t* f = p.fine != nullptr
-                                  ? (const int8_t*)p.fine + (int64_t)b * p.fine_sb + (int64_t)s * p.fine_ss + 4 * nt
-                                  : p.flags + (int64_t)b * p.flags_sb + (int64_t)(s >> 2) * p.flags_sm + 4 * nt;
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                int fw = (4 * nt + w < p.num_n) ? f[w] & 3 : 0;
+                int fw = (4 * nt + w < p.num_n) ? (int)(cur >> (8 * w)) & 3 : 0;
                 if ((s + 1) * 32 > p.Sq) fw = min(fw, 1);  // rows past the end have to be masked out
                 packed |= fw << (2 * w);
             }
@@ -381,6 +413,7 @@ __device__ __forceinline__ void build_slice_list(const AttnParams& p, int b, int
         const unsigned long long bal = __ballot(packed != 0);
         if (packed) list[count + __popcll(bal & ((1ull << lane) - 1ull))] = (s << 8) | packed;
         count += __popcll(bal);
+        cur = next;
     }
     // list[-1] (the caller leaves room for it) repeats the first entry with all classes cleared: a consumer that
     // takes the entries in pairs from the end finds a harmless partner for the first entry of an odd count there.

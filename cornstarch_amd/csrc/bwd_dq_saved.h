@@ -24,27 +24,27 @@ constexpr int DQS_THREADS = 256;
 
 // List, in ascending order, the 64-key tiles the four slices of a workgroup have to visit (at most MAX_LIST).
 // entry = (tile << 16) | sum_w (c0_w | c1_w << 2) << (4 w), c0 / c1 = class of the tile's two 32-key halves for wave
-// w's slice.  Executed by wave 0; the caller synchronizes before reading.
-__device__ __forceinline__ void build_key_half_list(const WaveSlices& ws, int num_n, int S, int lane, int* list,
+// w's slice.  first: load_tile_classes of this lane's first tile.  Executed by wave 0; the caller synchronizes before reading.
+__device__ __forceinline__ void build_key_half_list(const WaveSlices& ws, int num_n, int S, int lane, const TileClasses& first, int* list,
                                                     int* count_out) {
-    const int nkt = (S + 63) >> 6;
+    const int nkt = key_tiles(S, 0);
     int count = 0;
+    TileClasses cur = first;
     for (int base = 0; base < nkt; base += 64) {
+        const TileClasses next = load_tile_classes(ws, num_n, nkt, base + 64 + lane);
         const int kt = base + lane;
+        const bool second = 2 * kt + 1 < num_n;
         int packed = 0;
-        if (kt < nkt) {
-            const bool second = 2 * kt + 1 < num_n;
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                if (ws.cls_row[x] == nullptr) continue;  // wave-uniform
-                const int f0 = ws.cls_row[x][2 * kt] & 3;
-                const int f1 = second ? (ws.cls_row[x][2 * kt + 1] & 3) : 0;
-                packed |= (f0 | (f1 << 2)) << (4 * x);
-            }
+        for (int x = 0; x < 4; ++x) {
+            const int f0 = cur.f[x][0] & 3, f1 = second ? cur.f[x][1] & 3 : 0;
+            packed |= ws.cls_row[x] != nullptr ? (f0 | (f1 << 2)) << (4 * x) : 0;
         }
+        if (kt >= nkt) packed = 0;
         const unsigned long long bal = __ballot(packed != 0);
         if (packed) list[count + __popcll(bal & ((1ull << lane) - 1ull))] = (kt << 16) | packed;
         count += __popcll(bal);
+        cur = next;
     }
     if (lane == 0) *count_out = count;
     wait_lds();
@@ -96,13 +96,29 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
     const int h = hk * G + g;
     const WaveSlices ws = pick_wave_slices(p, b, grp);  // the plan's order (the launcher requires a plan)
 
-    if (wave == 0) build_key_half_list(ws, p.num_n, Sk, lane, sList, &sCount);
+    TileClasses first_classes = {};
+    if (wave == 0) first_classes = load_tile_classes(ws, p.num_n, key_tiles(Sk, 0), lane);
 
     const int slice = __builtin_amdgcn_readfirstlane(wave == 0 ? ws.slice[0] : wave == 1 ? ws.slice[1] : wave == 2 ? ws.slice[2] : ws.slice[3]);
     // column n of a dS block holds query row 8 * ((n & 15) >> 2) + 4 * (n >> 4) + (n & 3) of the slice
     const int slot = (slice < 0 ? 0 : slice) * 32 + 8 * ((l32 & 15) >> 2) + 4 * (l32 >> 4) + (l32 & 3);
     const bool qvalid = slice >= 0 && slot < Sq;
     const int qrow = row_of_slot(p, ws, b, slot, qvalid);
+    // Record numbers of the slice's pairs, 64 key tiles at a time: lane j holds the one of 128-key tile 64 ent_chunk + j.  The first
+    // 64 are asked for together with the classes, before anybody knows which of them are needed.
+    // The loaded value is handed on through an instruction of its own, so that the compiler's wait for the load sits
+    // right here (once per 128 tiles) and not in front of every later use: a wait for this load is a wait for every
+    // tile copy in flight.
+    const int* entry_row = p.ds_entry + (int64_t)b * p.ds_entry_sb + (int64_t)(slice < 0 ? 0 : slice) * p.num_kt;
+    int ent_vec = 0, ent_chunk = 0;
+    auto load_entries = [&](int chunk) {
+        const int e = entry_row[min(64 * chunk + lane, p.num_kt - 1)];
+        ent_chunk = chunk;
+        return e;
+    };
+    auto keep_entries = [&](int e) { asm volatile("v_mov_b32 %0, %1" : "=v"(ent_vec) : "v"(e)); };
+    const int first_entries = load_entries(0);
+    if (wave == 0) build_key_half_list(ws, p.num_n, Sk, lane, first_classes, sList, &sCount);
 
     f32x16 dq[DB];
 #pragma unroll
@@ -120,18 +136,11 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
     constexpr unsigned TILE_BYTES = DQS_KT * NCH * 16;
     // records of this q head; record e (a slice x 128-key tile pair) is 8 KiB = four 2 KiB blocks
     const char* ds_head = (const char*)p.ds_ws + (((int64_t)h * p.ds_capacity) << 13);
-    const int* entry_row = p.ds_entry + (int64_t)b * p.ds_entry_sb + (int64_t)(slice < 0 ? 0 : slice) * p.num_kt;
-
-    // record numbers of the coming list entries, 64 at a time: lane j holds the one of list entry base + j.
-    // The loaded value is handed on through an instruction of its own, so that the compiler's wait for the load sits
-    // right here (once per 64 tiles) and not in front of every later use: a wait for this load is a wait for every
-    // tile copy in flight.
-    int ent_vec = 0;
-    auto load_entries = [&](int base, int n) {
-        const int j = base + lane;
-        int e = 0;
-        if (j < n && slice >= 0) e = entry_row[sList[j] >> 17];  // 64-key tile kt -> 128-key tile kt / 2
-        asm volatile("v_mov_b32 %0, %1" : "=v"(ent_vec) : "v"(e));
+    // record number of the pair of list entry `entry` (64-key tile kt -> 128-key tile kt / 2; the entries come in ascending order)
+    auto entry_number = [&](int entry) {
+        const int tile = entry >> 17;
+        if ((tile >> 6) != ent_chunk) keep_entries(load_entries(tile >> 6));
+        return __builtin_amdgcn_readlane(ent_vec, tile & 63);
     };
 
     // copy of the K tile of list entry `entry` into buffer buf (shared by the four waves)
@@ -196,12 +205,12 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
     __syncthreads();
     const int n = sCount;
     if (n > 0) {
-        load_entries(0, n);
+        keep_entries(first_entries);
         int entry = __builtin_amdgcn_readfirstlane(sList[0]);
         int next = __builtin_amdgcn_readfirstlane(sList[n > 1 ? 1 : 0]);
         issue_k(entry, 0);
-        issue_ds(entry, __builtin_amdgcn_readlane(ent_vec, 0), 0);
-        if (n > 1) issue_ds(next, __builtin_amdgcn_readlane(ent_vec, 1), 1);
+        issue_ds(entry, entry_number(entry), 0);
+        if (n > 1) issue_ds(next, entry_number(next), 1);
         wait_async();
         __syncthreads();
         for (int it = 0; it < n; ++it) {
@@ -212,9 +221,8 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
             const int i2 = it + 2;
             int entry2 = -1, e2 = 0;
             if (i2 < n) {
-                if ((i2 & 63) == 0) load_entries(i2, n);
                 entry2 = __builtin_amdgcn_readfirstlane(sList[i2]);
-                e2 = __builtin_amdgcn_readlane(ent_vec, i2 & 63);
+                e2 = entry_number(entry2);
             }
             const int issued = tile_step(cur, entry, entry2, e2);
             entry = next;

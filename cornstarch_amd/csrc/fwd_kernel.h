@@ -97,6 +97,11 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     const int slot = (slice < 0 ? 0 : slice) * 32 + l32;
     const bool qvalid = slice >= 0 && slot < Sq;
     const int qrow = row_of_slot(p, ws, b, slot, qvalid);
+    // (the class bytes are asked for ahead of the rows: loads arrive in order)
+    const bool lists = wave == 0 && (stream == 0 || side);
+    const int list_keys = idle ? 0 : Sk;
+    TileClasses first_classes = {};
+    if (lists) first_classes = load_tile_classes(ws, p.num_n, key_tiles(list_keys, 0), lane);
     u32x4 qreg[KK];
     {
         const char* qp = (const char*)p.q.ptr + 2 * ((int64_t)b * p.q.sb + (int64_t)qrow * p.q.ss + (int64_t)h * p.q.sh);
@@ -111,8 +116,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     int qpos = (IDX && qvalid) ? p.posq[qrow] : qrow;
     QueryBits qb = {};  // of qf and qpos, once they have arrived
     // (the row loads above are in flight while the class rows are read and the first tile is on its way)
-    if (wave == 0 && (stream == 0 || side))  // first pass (usually the only one)
-        build_key_tile_list<STREAMS>(ws, p.num_n, idle ? 0 : Sk, lane, 0, sList + stream * (MAX_LIST / 2), sCount + stream, !side);
+    if (lists)  // first pass (usually the only one)
+        build_key_tile_list<STREAMS>(ws, p.num_n, list_keys, lane, 0, first_classes, sList + stream * (MAX_LIST / 2), sCount + stream, !side);
 
     f32x16 o[DB];
 #pragma unroll
@@ -480,7 +485,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         kt_begin += MAX_LIST;
         if (kt_begin >= nkt_total) break;
         __syncthreads();  // everybody has read the list of the pass that just ended
-        if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, kt_begin, sList, sCount);
+        if (wave == 0) build_key_tile_list(ws, p.num_n, Sk, lane, kt_begin, load_tile_classes(ws, p.num_n, key_tiles(Sk, kt_begin), kt_begin + lane), sList, sCount);
     }
 
     // ---- epilogue: normalize, write O (q dtype) and LSE (natural log) -------------------
