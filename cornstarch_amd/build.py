@@ -19,7 +19,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libbam_hip.so")
 HOST_PATH = os.path.join(PKG_DIR, "_bam_host.so")
 # the longest compilations first: they are spread over the workers
-SOURCES = ["bwd_long.hip", "bwd_dkdv.hip", "bwd_dkdv_save.hip", "bwd_dq_saved.hip", "bwd_dq.hip", "fwd_long.hip", "fwd.hip", "tile_flags.hip", "decode.hip", "bam_abi.hip"]
+SOURCES = ["bwd_long.hip", "bwd_dkdv.hip", "bwd_dkdv_save.hip", "bwd_dq_saved.hip", "bwd_dq.hip", "bwd_both.hip", "fwd_long.hip", "fwd.hip", "tile_flags.hip", "decode.hip", "bam_abi.hip"]
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}",

@@ -905,8 +905,9 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
     const bool dq_first = all.D <= 64;
     if (!dq_first) BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
     const int parts = a->parts_workspace != nullptr ? dkdv_parts(a) : 1;
-    auto dkdv = [&](const bam::AttnParams& p) -> int {
-        if (parts == 1) return launched(launch_dkdv(p, a->dtype, stream), "bam_attn_bwd (dk/dv)");
+    // launch_kv: what launches dK/dV, given its parameters; the parts are added up behind it
+    auto with_parts = [&](const bam::AttnParams& p, auto launch_kv) -> int {
+        if (parts == 1) return launched(launch_kv(p), "bam_attn_bwd (dk/dv)");
         const int64_t floats = dkdv_part_floats(a, parts);
         if (a->parts_bytes < 2 * 4 * floats || (reinterpret_cast<uintptr_t>(a->parts_workspace) & 15u))
             return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: parts workspace of %lld bytes, %lld needed, 16-byte aligned",
@@ -919,8 +920,11 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         part.grad_typed = 2;
         part.kv_parts = parts;
         part.Hkv = p.Hkv * parts;
-        BAM_TRY(launched(launch_dkdv(part, a->dtype, stream), "bam_attn_bwd (dk/dv)"));
+        BAM_TRY(launched(launch_kv(part), "bam_attn_bwd (dk/dv)"));
         return launched(bam::launch_sum_parts(p, ws, ws + floats, parts, a->dtype, (hipStream_t)stream), "bam_attn_bwd (sum)");
+    };
+    auto dkdv = [&](const bam::AttnParams& p) -> int {
+        return with_parts(p, [&](const bam::AttnParams& kv) { return launch_dkdv(kv, a->dtype, stream); });
     };
     // The heads in runs of whole kv heads, every run through the same dS workspace: the launches of a stream run in
     // order, so a run's dQ kernel has read the workspace before the next run's dK/dV kernel writes it.
@@ -941,6 +945,13 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         p.Hq = hq;
         p.Hkv = hk;
         if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
+        if (dq_first && runs == 1 && bam::both_in_one_launch(p)) {
+            BAM_TRY(launched(bam::launch_bwd_preprocess(p, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
+            bam::AttnParams q = p;
+            q.o.ptr = nullptr;  // (delta is there)
+            BAM_TRY(with_parts(p, [&](const bam::AttnParams& kv) { return bam::launch_bwd_both(kv, q, a->dtype, (hipStream_t)stream); }));
+            continue;
+        }
         if (dq_first) {
             BAM_TRY(launched(launch_dq(p, a->dtype, stream), "bam_attn_bwd (dq)"));
             BAM_TRY(dkdv(p));

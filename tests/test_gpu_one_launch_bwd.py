@@ -1,0 +1,57 @@
+"""dK/dV and dQ of small problems in one launch (head dims 33 to 64), against the oracle: either side of the sizes where it starts and
+ends, two streams on a list and side by side, one workgroup of dK/dV, parts, a bias, a bool mask, index tensors, accumulated gradients."""
+
+import pytest
+import torch
+
+from cornstarch_amd.kernel import bitfield_attention as BA
+from cornstarch_amd.kernel.attention import flash_attn_func
+from oracle import bam_oracle as O
+from tests.helpers import random_bitfield
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D", [
+    (1, 128, 2, 1, 64), (1, 129, 2, 1, 64),        # from three key tiles on
+    (1, 700, 42, 42, 64), (1, 700, 43, 43, 64),    # 252 and 258 workgroups of dQ: up to 256 with so few keys
+    (2, 1030, 21, 3, 40), (1, 1500, 40, 8, 48),    # 378, 480: the plan decides how the streams share the lists; parts
+    (1, 1601, 4, 4, 56),
+])
+@pytest.mark.parametrize("form", ["plain", "bias", "mask", "index", "level"])
+def test_gradients_against_the_oracle(B, S, Hq, Hkv, D, form):
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(S + D)
+    q, do = ((torch.randn(B, S, Hq, D, generator=g) * 0.5).bfloat16() for _ in range(2))
+    k, v = ((torch.randn(B, S, Hkv, D, generator=g) * 0.5).bfloat16() for _ in range(2))
+    bf = random_bitfield(B, S, seed=S, pad=S // 13)
+    if form == "level":  # nothing hidden
+        bf = torch.full_like(bf, 2)
+    bias = torch.randn(1, Hq, 1, S, generator=g) if form == "bias" else None
+    want = O.attention_backward(q, k, v, bf, do, bias=bias) if form == "bias" else O.attention_backward(q, k, v, bf, do)
+    qd, kd, vd, dod, bfd = (t.to(dev) for t in (q, k, v, do, bf))
+    BA.BitfieldUtils.clear_cache()
+    if form == "index":  # the rows and keys in another order, gradients accumulated
+        flags = BA.BitfieldUtils.materialize_compressed_mask_from_bitfield_mask(bfd)
+        order = torch.arange(S).roll(-128 * (S // 256))
+        if S % 128:  # (flags of whole blocks can be reordered)
+            order = torch.arange(S)
+        idx = order.to(dev)
+        blocks = order[::128] // 128
+        flags = flags[:, blocks.to(dev)][:, :, (order[::32] // 32).to(dev)].contiguous()
+        qs, ks, vs, dos = (t[:, idx].contiguous() for t in (qd, kd, vd, dod))
+        o, lse, scale = BA._bitfield_attn_forward(qs, ks, vs, bfd, flags, idx, idx)
+        grads = [torch.ones(t.shape, dtype=torch.float32, device=dev) for t in (qs, ks, vs)]
+        BA._bitfield_attn_backward(dos, qs, ks, vs, o, bfd, flags, lse, *grads, idx, idx, softmax_scale=scale)
+        got = [torch.empty_like(t).index_copy_(1, idx, t - 1.0) for t in grads]
+    else:
+        leaves = [t.requires_grad_(True) for t in (qd, kd, vd)]
+        if form == "mask":
+            o = flash_attn_func(*leaves, mask=BA.materialize_bitfield_mask(bfd).to(torch.bool).contiguous())
+        else:
+            o = BA.bitfield_attn_func(*leaves, bfd, None if bias is None else bias.to(dev))
+        got = torch.autograd.grad(o, leaves, dod)
+    # probabilities and dS are rounded to bf16 before they are multiplied: 2^-9 a term, a few times that in the norm
+    for name, x, y in zip(("dq", "dk", "dv"), got, want):
+        rel = ((x.float().cpu() - y).norm() / y.norm()).item()
+        assert rel <= 1e-2, f"{name}: {rel}"
