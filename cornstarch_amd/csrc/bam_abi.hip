@@ -870,8 +870,8 @@ int bam_attn_bwd_parts(const bam_attn* a, int64_t* bytes) {
     return BAM_OK;
 }
 
-int bam_attn_bwd(const bam_attn* a, void* stream) {
-    if (a == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: null pointer");
+// The parameters of a backward, all heads at once, with the plan and the workspace of `a` (plan: where they are put together).
+static int attn_bwd_params(const bam_attn* a, bam_plan& plan, bam::AttnParams& all) {
     MaskSource m;
     BAM_TRY(attn_source(a, m));
     BAM_TRY(check_problem(a->B, m.Sq, m.Sk, a->Hq, a->Hkv, a->D, a->dtype, true));
@@ -881,7 +881,6 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
     if (a->Hkv % runs) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: %d runs do not divide %d kv heads", runs, a->Hkv);
     if (runs > 1 && a->bias != nullptr)  // a bias is indexed by absolute head
         return fail(BAM_ERR_UNSUPPORTED, "bam_attn_bwd: heads are not taken in runs with a bias");
-    bam_plan plan;
     if (a->plan != nullptr) {
         plan = *a->plan;
         plan.ds_workspace = a->ds_workspace;
@@ -892,8 +891,6 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
                             a->dout.stride_h, a->dq.stride_b,   a->dq.stride_s,   a->dq.stride_h, a->dk.stride_b, a->dk.stride_s,
                             a->dk.stride_h,   a->dv.stride_b,   a->dv.stride_s,   a->dv.stride_h, a->flags_stride_b,
                             a->flags_stride_m};
-    const int hq = a->Hq / runs, hk = a->Hkv / runs, gsz = a->accumulate ? 4 : 2;
-    bam::AttnParams all = {};
     BAM_TRY(bwd_params(all, "bam_attn_bwd", a->q.ptr, a->k.ptr, a->v.ptr, a->dout.ptr, a->lse, a->delta, a->dq.ptr, a->dk.ptr,
                        a->dv.ptr, m, a->flags, st, a->B, a->Hq, a->Hkv, a->D, a->scale, a->dtype, a->accumulate, true, true,
                        a->bias, nullptr, true));
@@ -901,10 +898,35 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
     if (reinterpret_cast<uintptr_t>(a->lse_scaled) & 3u)
         return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: lse_scaled is not 4-byte aligned");
     all.lse_scaled = a->bias == nullptr && all.D <= 64 ? a->lse_scaled : nullptr;
+    // (a run's workspace is checked with the run's heads)
+    if (a->plan != nullptr && runs == 1) BAM_TRY(fill_plan(all, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
+    return BAM_OK;
+}
+static bool attn_bwd_one_launch(const bam_attn* a, const bam::AttnParams& all, int parts) {
+    return a->head_runs <= 1 && bam::both_in_one_launch(all, (int64_t)all.num_kt * all.B * all.Hkv * parts, a->pairs);
+}
+
+int bam_attn_bwd_takes_ds(const bam_attn* a, int* takes) {
+    if (a == nullptr || takes == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd_takes_ds: null pointer");
+    bam_plan plan;
+    bam::AttnParams all = {};
+    BAM_TRY(attn_bwd_params(a, plan, all));
+    all.ds_ws = nullptr;
+    *takes = a->plan != nullptr && all.D > 64 && all.Sk <= 131072 && !attn_bwd_one_launch(a, all, dkdv_parts(a)) ? 1 : 0;
+    return BAM_OK;
+}
+
+int bam_attn_bwd(const bam_attn* a, void* stream) {
+    if (a == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd: null pointer");
+    bam_plan plan;
+    bam::AttnParams all = {};
+    BAM_TRY(attn_bwd_params(a, plan, all));
+    const int runs = a->head_runs > 1 ? a->head_runs : 1, hq = a->Hq / runs, hk = a->Hkv / runs, gsz = a->accumulate ? 4 : 2;
     // head dims up to 64: the dQ kernel runs first and computes delta on the way; above, dK/dV needs it first
     const bool dq_first = all.D <= 64;
     if (!dq_first) BAM_TRY(launched(bam::launch_bwd_preprocess(all, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
     const int parts = a->parts_workspace != nullptr ? dkdv_parts(a) : 1;
+    const bool one_launch = attn_bwd_one_launch(a, all, parts);
     // launch_kv: what launches dK/dV, given its parameters; the parts are added up behind it
     auto with_parts = [&](const bam::AttnParams& p, auto launch_kv) -> int {
         if (parts == 1) return launched(launch_kv(p), "bam_attn_bwd (dk/dv)");
@@ -944,9 +966,9 @@ int bam_attn_bwd(const bam_attn* a, void* stream) {
         if (p.lse_scaled != nullptr) p.lse_scaled += (int64_t)r * hq * p.Sq_rounded;
         p.Hq = hq;
         p.Hkv = hk;
-        if (a->plan != nullptr) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, m.Sq, m.Sk));
-        if (dq_first && runs == 1 && bam::both_in_one_launch(p)) {
-            BAM_TRY(launched(bam::launch_bwd_preprocess(p, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
+        if (a->plan != nullptr && runs > 1) BAM_TRY(fill_plan(p, "bam_attn_bwd", &plan, a->B, p.Sq, p.Sk));
+        if (one_launch) {
+            if (dq_first) BAM_TRY(launched(bam::launch_bwd_preprocess(p, a->dtype, (hipStream_t)stream), "bam_attn_bwd (delta)"));
             bam::AttnParams q = p;
             q.o.ptr = nullptr;  // (delta is there)
             BAM_TRY(with_parts(p, [&](const bam::AttnParams& kv) { return bam::launch_bwd_both(kv, q, a->dtype, (hipStream_t)stream); }));

@@ -201,8 +201,8 @@ int launch_bwd_preprocess(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dkdv(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dq(const AttnParams& p, int dtype, hipStream_t stream);
 // Whether dK/dV and dQ go into one launch, behind the delta pre-pass; and that launch (kv: dK/dV's parameters,
-// those of the parts where there are any).
-bool both_in_one_launch(const AttnParams& p);
+// those of the parts where there are any).  dkdv_blocks: the workgroups of dK/dV; pairs: the plan's count if it is known, else 0.
+bool both_in_one_launch(const AttnParams& p, int64_t dkdv_blocks, int64_t pairs);
 int launch_bwd_both(const AttnParams& kv, const AttnParams& p, int dtype, hipStream_t stream);
 // dk, dv of p from the parts that a dK/dV launch with kv_parts left at `parts_dk` and `parts_dv` (contiguous).
 int launch_sum_parts(const AttnParams& p, const float* parts_dk, const float* parts_dv, int parts, int dtype, hipStream_t stream);

@@ -682,7 +682,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_both_kernel(const AttnPar
         DqShared<D, MODE, BIAS_FORM, 2> dq;
     } sh;
     if ((int)blockIdx.x < dkdv_blocks)
-        dkdv_work<T, D, MODE, BIAS, false, false, !BIAS>(kv, blockIdx.x, sh.dkdv);
+        dkdv_work<T, D, MODE, BIAS, false, false, !BIAS && D <= 64>(kv, blockIdx.x, sh.dkdv);
     else
         dq_work<T, D, MODE, BIAS_FORM, false, 2>(p, blockIdx.x - dkdv_blocks, sh.dq);
 }

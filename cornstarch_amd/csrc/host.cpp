@@ -551,12 +551,18 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     if (scaled) a.lse_scaled = a.delta + lse.numel();
     a.accumulate = accumulate ? 1 : 0;
     Tensor ws;
-    if (plan && a.D > 64 && a.Sk <= 131072) {
+    // Small problems take no dS workspace and do not wait for the plan's count; where the count decides, it is waited for and asked again.
+    int takes_ds = 0;
+    check(bam_attn_bwd_takes_ds(&a, &takes_ds), "bam_attn_bwd_takes_ds");
+    if (takes_ds) {
         optional<py::gil_scoped_release> release;
         if (PyGILState_Check()) release.emplace();
         a.pairs = plan.core->wait_pairs();
         release.reset();
         desc.rows_known = plan.core->rows_known.load();
+        check(bam_attn_bwd_takes_ds(&a, &takes_ds), "bam_attn_bwd_takes_ds");
+    }
+    if (takes_ds) {
         py::gil_scoped_acquire gil;
         py::tuple got = plan.py_object().attr("backward_workspace")(a.B, a.Hq, a.Hkv, a.D, a.Sk, c.bias == nullptr);
         a.head_runs = got[0].cast<int>();

@@ -158,6 +158,7 @@ SIGNATURES = {
     "bam_attn_fwd": [_attn, _ptr],
     "bam_attn_bwd": [_attn, _ptr],
     "bam_attn_bwd_parts": [_attn, _ptr],
+    "bam_attn_bwd_takes_ds": [_attn, _ptr],
     "bam_decode_counted": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr, _i64, _ptr],
     "bam_decode": [_ptr] * 4 + [_i64] * 10 + [_int] * 5 + [_f32, _int, _int, _f32, _ptr, _i64, _ptr],
 }

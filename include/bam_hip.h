@@ -514,6 +514,10 @@ int bam_attn_bwd(const bam_attn* args, void* stream);
 /* Bytes of scratch with which bam_attn_bwd deals the q heads of a kv head to several workgroups of its dK/dV launch and sums
  * their parts (0: this call would not).  Looks at the sizes and head_runs only. */
 int bam_attn_bwd_parts(const bam_attn* args, int64_t* bytes);
+/* Whether bam_attn_bwd should be given a dS workspace (1) or not (0: head dims up to 64, more than 131072 keys, no plan, or a problem
+ * of 768 keys and more that is small enough for dK/dV and dQ to share one launch, which is faster).  The answer may turn to 0 once
+ * `pairs` is known. */
+int bam_attn_bwd_takes_ds(const bam_attn* args, int* takes);
 
 #ifdef __cplusplus
 }

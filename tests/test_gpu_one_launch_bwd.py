@@ -1,5 +1,6 @@
-"""dK/dV and dQ of small problems in one launch (head dims 33 to 64), against the oracle: either side of the sizes where it starts and
-ends, two streams on a list and side by side, one workgroup of dK/dV, parts, a bias, a bool mask, index tensors, accumulated gradients."""
+"""dK/dV and dQ of small problems in one launch (head dims above 32), against the oracle: either side of the sizes where it starts and
+ends, two streams on a list and side by side, one workgroup of dK/dV, parts, a bias, a bool mask, index tensors, accumulated gradients;
+and which of them take a dS workspace."""
 
 import pytest
 import torch
@@ -7,7 +8,8 @@ import torch
 from cornstarch_amd.kernel import bitfield_attention as BA
 from cornstarch_amd.kernel.attention import flash_attn_func
 from oracle import bam_oracle as O
-from tests.helpers import random_bitfield
+from tests.helpers import random_bitfield, rel_l2
+from tests.test_gpu_ds_handover import inputs, run_backward
 
 pytestmark = pytest.mark.gpu
 
@@ -17,6 +19,9 @@ pytestmark = pytest.mark.gpu
     (1, 700, 42, 42, 64), (1, 700, 43, 43, 64),    # 252 and 258 workgroups of dQ: up to 256 with so few keys
     (2, 1030, 21, 3, 40), (1, 1500, 40, 8, 48),    # 378, 480: the plan decides how the streams share the lists; parts
     (1, 1601, 4, 4, 56),
+    (1, 767, 4, 4, 96), (1, 768, 4, 2, 72),        # above head dim 64: from 768 keys on
+    (1, 1030, 16, 2, 128), (1, 1500, 11, 11, 80),  # parts; 264 workgroups: the count decides (level lists: two launches)
+    (1, 2049, 15, 15, 128), (1, 1030, 29, 29, 128),  # 510 and 522 workgroups
 ])
 @pytest.mark.parametrize("form", ["plain", "bias", "mask", "index", "level"])
 def test_gradients_against_the_oracle(B, S, Hq, Hkv, D, form):
@@ -55,3 +60,21 @@ def test_gradients_against_the_oracle(B, S, Hq, Hkv, D, form):
     for name, x, y in zip(("dq", "dk", "dv"), got, want):
         rel = ((x.float().cpu() - y).norm() / y.norm()).item()
         assert rel <= 1e-2, f"{name}: {rel}"
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,level,takes", [
+    (1100, 32, 32, False, True), (1500, 20, 20, True, True),    # 576 workgroups; 480, nothing hidden
+    (1500, 20, 20, False, False), (2048, 8, 8, True, False),    # 480, of which the count says that they are uneven; 256
+])
+def test_which_sizes_hand_ds_over(S, Hq, Hkv, level, takes, monkeypatch):
+    dev = torch.device("cuda:0")
+    bf = torch.full((1, S), 2) if level else random_bitfield(1, S, seed=S, pad=3)
+    q, k, v, do = (t.to(dev) for t in inputs(1, S, Hq, Hkv, 128, torch.bfloat16, seed=S))
+    allocated, real = [], BA._TilePlan._allocate
+    monkeypatch.setattr(BA._TilePlan, "_allocate", staticmethod(lambda nbytes, device: allocated.append(nbytes) or real(nbytes, device)))
+    with_ds = run_backward(q, k, v, do, bf.to(dev), True, monkeypatch)
+    assert len(allocated) == takes
+    recomputed = run_backward(q, k, v, do, bf.to(dev), False, monkeypatch)
+    assert torch.equal(with_ds[1], recomputed[1]) and torch.equal(with_ds[2], recomputed[2])
+    assert rel_l2(with_ds[0].float(), recomputed[0].float()) <= 2e-3  # the same rounded dS values, summed in another order
+    BA.BitfieldUtils.clear_cache()
