@@ -11,6 +11,18 @@ __device__ __forceinline__ unsigned lds_addr(const void* p) {
     return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)p;
 }
 
+// LDS reads at a byte address: 16 bytes, and the two halves of a transposed operand (see lds_read_transposed)
+template <typename V>
+__device__ __forceinline__ V lds_read16(unsigned at) {
+    return *(const __attribute__((address_space(3))) V*)at;
+}
+__device__ __forceinline__ u32x4 lds_read_transposed_at(unsigned a, unsigned b) {
+    typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
+    const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)a));
+    const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)b));
+    return u32x4{x[0], x[1], y[0], y[1]};
+}
+
 // One direct global -> LDS copy instruction.  Lane l fetches `bytes` (16 or 4) from
 // sbase + voff and the hardware writes them to LDS byte address lds_base + l * bytes;
 // sbase and lds_base must be wave-uniform.  The LDS base travels in M0: it is handed to the asm

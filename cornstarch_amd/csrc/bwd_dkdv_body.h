@@ -1,6 +1,7 @@
 // The work of dK/dV workgroup `block`, for the parameters p and with the LDS arrays that the function around this text declares:
-// bwd_dkdv_kernel and dkdv_work (bwd_kernels.h).  As one function that both call it costs a launch of nothing but dK/dV 0.8 to 1 % above
-// head dim 64 (8192 tokens, 32 / 8 heads, D 128: step 1727 -> 1741 us): the compiler spreads its registers another way.
+// bwd_dkdv_kernel, dkdv_work and (NARROW: four waves) bwd_dkdv_narrow_kernel (bwd_kernels.h).  As one function that they call it costs a
+// launch of nothing but dK/dV 0.8 to 1 % above head dim 64 (8192 tokens, 32 / 8 heads, D 128: step 1727 -> 1741 us): the compiler
+// spreads its registers another way.
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wave & 3, st = wave >> 2;
     const int hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
@@ -35,7 +36,7 @@
 
     const int ns_total = (Sq + 31) >> 5;
     // ---- K, V of the tile -> LDS (once) ---------------------------------------------------
-    {
+    if constexpr (!NARROW) {
         TileStage<D, 128, DKDV_THREADS> stK, stV;
         stK.setup(2 * p.k.ss, p.d / 8, tid);
         stV.setup(2 * p.v.ss, p.d / 8, tid);
@@ -78,7 +79,7 @@
     // columns past it become zero in K and V: the Q and dO tiles hold other numbers there.
     auto negate_v_tile = [&]() {
 #pragma unroll
-        for (int i = 0; i < (128 * NCH) / DKDV_THREADS; ++i) {
+        for (int i = 0; i < (NARROW ? 0 : (128 * NCH) / DKDV_THREADS); ++i) {
             const int id = tid + DKDV_THREADS * i;
             u32x4 x = sV[id];
 #pragma unroll
@@ -96,8 +97,24 @@
     constexpr bool KV_REGS = D <= 64;
     u32x4 kfrag[KV_REGS ? KK : 1], vfrag[KV_REGS ? KK : 1];
     bool kv_loaded = false;
+    if constexpr (NARROW) {  // from memory, zeros past the head dim
+        static_assert(KV_REGS && !DENSE && !SORTED && !SAVE && !LONG, "the forms it is compiled for");
+        const char* kp = (const char*)p.k.ptr + 2 * ((int64_t)b * p.k.sb + (int64_t)key * p.k.ss + (int64_t)kv_head * p.k.sh);
+        const char* vp = (const char*)p.v.ptr + 2 * ((int64_t)b * p.v.sb + (int64_t)key * p.v.ss + (int64_t)kv_head * p.v.sh);
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) {
+            const int c = 16 * kk + 8 * hi;
+            u32x4 x = {0u, 0u, 0u, 0u}, y = {0u, 0u, 0u, 0u};
+            if (kvalid && c < p.d) {
+                x = *(const u32x4*)(kp + 2 * c);
+                y = *(const u32x4*)(vp + 2 * c);
+            }
+            kfrag[kk] = x;
+            vfrag[kk] = y;
+        }
+    }
     auto load_kv_operands = [&]() {  // after the V tile has been negated and a barrier has published it
-        if (KV_REGS && !kv_loaded) {
+        if (KV_REGS && !NARROW && !kv_loaded) {
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
                 kfrag[kk] = lds_read_chunk<D>(sK, 32 * kg + l32, 2 * kk + hi);
@@ -107,11 +124,11 @@
         }
     };
 
-    typedef SliceStage<D, DKDV_THREADS> Stage;
+    typedef SliceStage<D, NARROW ? DKDV_NARROW_THREADS : DKDV_THREADS> Stage;
     constexpr int CPT = Stage::CPT;
     // copy instructions per wave and tile: Q, dO, one of the small rows and (IDX) the row positions
     constexpr int NLOADS = 2 * CPT + 1 + (IDX ? 1 : 0);
-    static_assert(NLOADS <= 2 * KK, "one copy per MFMA of the S / dP phase");
+    static_assert(NLOADS <= 2 * KK * (NARROW ? 2 : 1), "one copy per MFMA of the S / dP phase");
     Stage stQ, stDO;
     stQ.setup(SORTED ? 0 : 2 * p.q.ss, p.d / 8, tid);
     stDO.setup(SORTED ? 0 : 2 * p.dout.ss, p.d / 8, tid);
@@ -231,10 +248,19 @@
             copy_b32<WAIT>(t.pos, t.pos_voff, lds_addr(sQpos) + pos_buf * (DKDV_QT * 4u));
     };
 
+    // NARROW: where this lane reads in tile 0 and in its rows, as byte addresses; what a k-slice, a block of columns, a half of the
+    // tile and the other array add are constants, XORed or in the instruction (see chunk_slot: the swizzle takes bits 1 to 3 of the row)
+    constexpr unsigned ROW_BYTES = NCH * 16, DO_AT = NB * TILE_BYTES, DELTA_AT = NB * DKDV_QT * 4;
+    unsigned chunk_lane = 0, transposed_lane = 0;
+    if constexpr (NARROW) {
+        const int i = lane & 15, r = 4 * hi + (i >> 2);
+        chunk_lane = ldsQ + 16u * (unsigned)chunk_slot<D>(l32, hi);
+        transposed_lane = ldsQ + 16u * (unsigned)chunk_slot<D>(r, 2 * half16 + ((i & 3) >> 1)) + 8u * (i & 1);
+    }
+
     // One 64-row tile held in buffer cur against this wave's 32 keys; the wave's 32 rows sit at sequence
     // rows myrow0.. and its class for them is cls.  The copies of the next tile into the other buffer
     // are issued one per MFMA of the S / dP phase, or back to back when this wave has nothing to compute.
-    const int qr = 32 * st;  // this wave's rows inside the 64-row tile
     // The wave's flag class is extracted with a per-lane copy of the key group number on purpose: a branch
     // condition the compiler can prove wave-uniform makes it restructure the loop around that branch, and the
     // result needs far more registers than a wave has.
@@ -258,13 +284,19 @@
     // ds_pos: position of the wave's slice in the slice list.
     // returns true when the wave has issued its two dS stores (they may stay in flight over the end of the iteration)
     // pos_cur, pos_nxt: the buffers of the tile's positions and of those that are copied now
-    auto tile_step = [&](int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int nxt, int pos_cur, int pos_nxt) -> bool {
+    // qr: this wave's rows inside the 64-row tile.  NARROW: the caller issues the copies; what derives from the lane is derived anew for
+    // every block (`own`), it would take the registers of the K and V operands otherwise
+    auto tile_step = [&](const int qr, int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int nxt, int pos_cur,
+                         int pos_nxt) __attribute__((always_inline)) -> bool {
         if (cls == 0) {
 #pragma unroll
-            for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, nxt, pos_nxt);
+            for (int j = 0; j < (NARROW ? 0 : NLOADS); ++j) issue_copy(j, next, nxt, pos_nxt);
             return false;
         }
         const int ds_e = ds_base + ds_pos;
+        int own = lane;
+        if (NARROW) asm volatile("" : "+v"(own));
+        const int lane = own, hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
         const u32x4* tQ = sQ[cur];
         const u32x4* tG = sDO[cur];
         // ---- S = Q K^T and dP = dO V^T : 32 queries x 32 keys, two accumulator chains; both operands of
@@ -273,7 +305,33 @@
         // zero: the chain then delivers delta - dO V^T = -(dP - delta) with no subtraction left for the VALU.
         // The sign is carried through dS into dK and taken back by the epilogue.
         f32x16 s, dp;
-        {
+        const unsigned tile_at = (unsigned)(cur * TILE_BYTES + qr * ROW_BYTES);
+        const unsigned row_at = 16u * hi + (lds_addr(sLse) + (unsigned)(cur * (DKDV_QT * 4) + qr * 4));
+        if constexpr (NARROW) {
+            constexpr int NOP = 2 * KK, AHEAD = 3;
+            const unsigned at = chunk_lane + tile_at;
+            u32x4 a[NOP];
+            auto operand = [&](int j) { return lds_read16<u32x4>((at ^ (unsigned)(32 * (j >> 1))) + ((j & 1) ? DO_AT : 0u)); };
+            a[0] = operand(0);
+#pragma unroll
+            for (int grp = 0; grp < 4; ++grp) {
+                const f32x4 d4 = lds_read16<f32x4>(row_at + DELTA_AT + 32u * grp);
+#pragma unroll
+                for (int x = 0; x < 4; ++x) dp[4 * grp + x] = d4[x];
+            }
+#pragma unroll
+            for (int j = 1; j < AHEAD; ++j) a[j] = operand(j);
+#pragma unroll
+            for (int j = 0; j < NOP; ++j) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (j + AHEAD < NOP) a[j + AHEAD] = operand(j + AHEAD);
+                if (j & 1)
+                    dp = T::mfma(a[j], vfrag[KV_REGS ? j >> 1 : 0], dp);
+                else
+                    s = T::mfma(a[j], kfrag[KV_REGS ? j >> 1 : 0], j < 2 ? zero16 : s);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        } else {
             constexpr int NOP = 2 * KK, AHEAD = 3;  // MFMA j: S (j even) or dP (j odd), k-slice j / 2
             constexpr int FIRST = SORTED ? (NOP - NLOADS < 4 ? NOP - NLOADS : 4) : 0;  // the copies start behind MFMA FIRST - 1
             u32x4 a[NOP], bb[NOP];
@@ -328,7 +386,7 @@
         }
 #pragma unroll
         for (int grp = 0; grp < 4; ++grp) {
-            const f32x4 l4 = *(const f32x4*)&sLse[cur][qr + 8 * grp + 4 * hi];
+            const f32x4 l4 = NARROW ? lds_read16<f32x4>(row_at + 32u * grp) : *(const f32x4*)&sLse[cur][qr + 8 * grp + 4 * hi];
 #pragma unroll
             for (int x = 0; x < 4; ++x) s[4 * grp + x] = __builtin_amdgcn_exp2f(fmaf(s[4 * grp + x], c2, SCALED ? -l4[x] : l4[x] * -LOG2E));
         }
@@ -382,6 +440,22 @@
                         sWq[wave][4][l32] = (unsigned)qb.lim;
                     }
                 }
+                if constexpr (NARROW) {  // (row by row: 20 registers less)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
+                        QueryBits qb;
+                        qb.a_lo = sWq[wave][0][r];
+                        qb.a_hi = sWq[wave][1][r];
+                        qb.x_lo = sWq[wave][2][r];
+                        qb.x_hi = sWq[wave][3][r];
+                        qb.lim = (int)sWq[wave][4][r];
+                        qb.text = (unsigned)qb.lim < 0x7FFFFFFFu;
+                        s[i] = allow_pair(qb, klo, khi, kpos) ? s[i] : 0.f;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                } else
 #pragma unroll
                 for (int grp = 0; grp < 4; ++grp) {
                     const int roff = 8 * grp + 4 * hi;
@@ -413,7 +487,26 @@
             dsb[t] = pack8<T>(dp, 8 * t);
         }
         // ---- dV^T += dO^T P ; dK^T += Q^T dS -------------------------------------------------
-        {
+        if constexpr (NARROW) {
+            const unsigned at = transposed_lane + tile_at;
+            u32x4 tg[2][DB], tq[2][DB];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    const unsigned x = (at ^ (64u * db)) + 16u * t * ROW_BYTES, y = (at ^ (64u * db + 16u)) + (16u * t + 8u) * ROW_BYTES;
+                    tg[t][db] = lds_read_transposed_at(x + DO_AT, y + DO_AT);
+                    tq[t][db] = lds_read_transposed_at(x, y);
+                }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    dv[db] = T::mfma(tg[t][db], pb[t], dv[db]);
+                    dk[db] = T::mfma(tq[t][db], dsb[t], dk[db]);
+                }
+            sched_pipeline_mfma_lds<4 * DB, 4, 2>();
+        } else {
             u32x4 tg[2][DB], tq[2][DB];
 #pragma unroll
             for (int t = 0; t < 2; ++t)
@@ -451,7 +544,7 @@
     // of its own; dK and dV live in registers and simply carry over.
     for (int s_end = ns_total;;) {
         lds_barrier();
-        const int n = sCount;
+        const int n = NARROW ? __builtin_amdgcn_readfirstlane(sCount) : sCount;
         // Main loop: the listed slices are taken in pairs from the END of the list (the workgroups of one kv head
         // that are resident together then read the same Q / dO rows at about the same time, and all but the first
         // of them find them in L2); pair r = entries n - 2 - 2 r (row stream 0) and n - 1 - 2 r (row stream 1).
@@ -510,7 +603,17 @@
             wait_async();
             asm volatile("" : "+v"(klo), "+v"(khi), "+v"(kpos));  // (see arrived())
             __syncthreads();
-            if (!v_negated) {  // K, V and the first tile have landed
+            if constexpr (NARROW) {
+                if (!v_negated) {
+                    arrived(kfrag);
+                    arrived(vfrag);
+#pragma unroll
+                    for (int kk = 0; kk < (KV_REGS ? KK : 1); ++kk)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) vfrag[kk][e] ^= 0x80008000u;
+                    v_negated = true;
+                }
+            } else if (!v_negated) {  // K, V and the first tile have landed
                 negate_v_tile();
                 v_negated = true;
                 __syncthreads();
@@ -522,7 +625,7 @@
                 // pair after next (SORTED: the one behind it): its list entries are requested now and picked up at the end of
                 // the iteration
                 const int r_req = SORTED ? after(after(r_nxt)) : after(r_nxt);
-                const int x_lo = entry_lo(r_req), x_hi = entry_hi(r_req);
+                int x_lo = entry_lo(r_req), x_hi = entry_hi(r_req);
                 TileSource next;
                 const int p1 = SORTED ? (pos_cur == 2 ? 0 : pos_cur + 1) : nxt, p2 = SORTED ? (pos_cur == 0 ? 2 : pos_cur - 1) : nxt;
                 if constexpr (SORTED) {
@@ -532,7 +635,18 @@
                 }
                 const int mine = st ? e_hi : e_lo;
                 fetch_bias_key(hk * G + g_cur);
-                const bool stored = tile_step(cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur, (mine >> 8) * 32, n - 2 - 2 * r_cur + st,
+                if constexpr (NARROW) {  // both slices, one after the other
+#pragma unroll
+                    for (int j = 0; j < NLOADS; ++j) issue_copy(j, next, nxt, nxt);
+                    x_lo = __builtin_amdgcn_readfirstlane(x_lo);
+                    x_hi = __builtin_amdgcn_readfirstlane(x_hi);
+#pragma unroll (D > 32 ? 1 : 2)
+                    for (int half = 0; half < 2; ++half) {
+                        const int e = half ? e_hi : e_lo;
+                        tile_step(32 * half, cur, (e >> (2 * kg_lane)) & 3, hk * G + g_cur, (e >> 8) * 32, 0, next, nxt, cur, nxt);
+                    }
+                }
+                const bool stored = !NARROW && tile_step(32 * st, cur, (mine >> (2 * kg_lane)) & 3, hk * G + g_cur, (mine >> 8) * 32, n - 2 - 2 * r_cur + st,
                                               next, nxt, SORTED ? pos_cur : cur, p2);
                 g_cur = DEEP ? f_g : g_nxt;
                 r_cur = DEEP ? f_r : r_nxt;
@@ -594,6 +708,11 @@
             f32x16 x = acc[db];
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
+                if constexpr (NARROW) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) x[4 * grp + i] *= factor;
+                    continue;
+                }
                 const f32x4 other = park[((half * DB + db) * 4 + grp) * 64 + lane];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) x[4 * grp + i] = (x[4 * grp + i] + other[i]) * factor;
@@ -611,6 +730,12 @@
             }
         }
     };
+    if constexpr (NARROW) {
+        if (!kvalid) return;
+        finish(dk, 0, -p.scale, p.dk);
+        finish(dv, 1, 1.f, p.dv);
+        return;
+    }
     if (st == 0)
         hand_over(dv, 1);
     else

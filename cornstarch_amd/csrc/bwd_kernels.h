@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const AttnParams p)
 // buffers one after the other (workgroup barrier in between), so the result stays
 // deterministic and atomic free.
 constexpr int DKDV_QT = 64;
-constexpr int DKDV_THREADS = 512;
+constexpr int DKDV_THREADS = 512, DKDV_NARROW_THREADS = 256;
 
 // MODE (MASK_*): MASK_INDEXED = explicit global positions p.posq / p.posk and gathered bitfield arrays;
 // MASK_DENSE = a materialized bool mask read from global memory in partial tiles.
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
     constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
     static_assert(!(SORTED && LONG), "no plan for so many rows");
-    constexpr bool DEEP = DKDV_DEEP<D, MODE, LONG>;
+    constexpr bool NARROW = false, DEEP = DKDV_DEEP<D, MODE, LONG>;
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
@@ -149,12 +149,50 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 #include "bwd_dkdv_body.h"
 }
 
+// The same work for head dims up to 64 by four waves, one for each 32 keys, that take both slices of a pair one after the other: three
+// workgroups fit a unit, so a third wave per SIMD fills the gaps of MFMAs, arithmetic and LDS reads (each 450 to 550 cycles of a 32 x 32
+// block's 1050 at head dim 64 with two), and a workgroup's start and end pass behind the others' work.  168 registers: every wave
+// holds its K and V operands, and nothing lies in LDS but Q, dO and the small rows; the LDS addresses of a block are one per access
+// form and XORs of constants (75 vector instructions a block beside the MFMAs; 93 in the kernel above, and 144 if the compiler
+// derives them anew); the rule constants of a block are read one row at a time.  (Spilled K and V operands, read back between
+// the tile copies, wait for those: step 1.26 -> 1.42 ms at 8 x 4096.)  No partial sums to add at the end.
+// Step, us, eight waves -> four: D 64: 8 x 4096, 16 heads 1312 -> 1236, 8 x 2048 397 -> 373, 32 x 512, 32 heads 461 ->
+// 414, 8 x 4096, 32 / 8 heads 2415 -> 2339, 16384, 16 heads, nothing hidden 5192 -> 5195; D 32: 8 x 2048, 16 heads 290 -> 249, 16 x 512, 32
+// heads 170 -> 141, 2 x 8192, 16 heads 831 -> 767.
+template <typename T, int D, int MODE, bool BIAS, bool SCALED>
+__global__ __launch_bounds__(DKDV_NARROW_THREADS, 3) void bwd_dkdv_narrow_kernel(const AttnParams p) {
+    constexpr bool IDX = MODE == MASK_INDEXED, DENSE = false, SORTED = false, ROW_POS = IDX, LONG = false, SAVE = false;
+    constexpr bool NARROW = true, DEEP = false;
+    constexpr int NB = 2;
+    constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
+    constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
+    __shared__ __attribute__((aligned(256))) u32x4 sTiles[2 * NB][DKDV_QT * NCH];
+    u32x4 (*const sQ)[DKDV_QT * NCH] = sTiles;
+    u32x4 (*const sDO)[DKDV_QT * NCH] = sTiles + NB;
+    u32x4* const sK = sTiles[0];  // (not in LDS: named by code that is not compiled for this kernel)
+    u32x4* const sV = sTiles[0];
+    __shared__ __attribute__((aligned(16))) float sRowNumbers[2 * NB][DKDV_QT];
+    float (*const sLse)[DKDV_QT] = sRowNumbers;
+    float (*const sDelta)[DKDV_QT] = sRowNumbers + NB;
+    __shared__ __attribute__((aligned(16))) int64_t sQbf[NB][DKDV_QT];
+    __shared__ __attribute__((aligned(16))) int sQpos[NB][DKDV_QT];
+    __shared__ __attribute__((aligned(16))) unsigned sWq[4][5][32];
+    __shared__ unsigned sColBits[1][2][1];
+    __shared__ int sListStore[MAX_SLICE_LIST + 1];
+    int* const sList = sListStore + 1;
+    __shared__ int sCount;
+
+    const int block = blockIdx.x;
+#include "bwd_dkdv_body.h"
+}
+
 // The work of workgroup `block` of a dK/dV launch, in LDS of the caller's.
 template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE, bool SCALED>
 __device__ __forceinline__ void dkdv_work(const AttnParams& p, const int block, DkdvShared<D, MODE, LONG>& sh) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
     constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
     static_assert(!(SORTED && LONG), "no plan for so many rows");
+    constexpr bool NARROW = false;
     constexpr bool DEEP = DKDV_DEEP<D, MODE, LONG>;
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
@@ -696,6 +734,20 @@ inline bool rows_may_be_left(const AttnParams& p) { return p.rows == nullptr || 
 template <typename T, int D, bool BIAS, bool LONG, bool SAVE, bool SCALED>
 static int launch_dkdv_m(const AttnParams& p, hipStream_t stream) {
     const int blocks = p.num_kt * p.B * p.Hkv;  // one workgroup per 128-key tile
+    // Four waves (bwd_dkdv_narrow_kernel) where there are more than four workgroups a unit.  Few leave the units a wave or two per SIMD: step,
+    // us, D 32, 512 workgroups (2 x 2048, 16 heads) 107 -> 110, 576 (4 x 3000, 6 heads) 156 -> 160; D 64, 512 (8192, 32 / 8 heads) 1045 -> 1196.
+    // (From 768 on they win: 8 x 700, 16 heads, D 32 93 -> 87, D 64 3 x 2048 185 -> 179.  But a tile's partial sums then come in another
+    // order, and the sequences of a call of ordinary size are to have the bits that they have in one of half or twice the size.)
+    // A bias takes registers that head dim 64 does not have: 8192, 16 heads 648 -> 672 (D 32: 8 x 2048 330 -> 282).
+    if constexpr (D <= 64 && !LONG && !SAVE && !(BIAS && D > 32)) {
+        if (p.rows == nullptr && blocks > 1024 && p.mask_mode != MASK_DENSE) {
+            if (p.mask_mode == MASK_INDEXED)
+                hipLaunchKernelGGL((bwd_dkdv_narrow_kernel<T, D, MASK_INDEXED, BIAS, SCALED>), dim3(blocks), dim3(DKDV_NARROW_THREADS), 0, stream, p);
+            else
+                hipLaunchKernelGGL((bwd_dkdv_narrow_kernel<T, D, MASK_BITFIELD, BIAS, SCALED>), dim3(blocks), dim3(DKDV_NARROW_THREADS), 0, stream, p);
+            return (int)hipGetLastError();
+        }
+    }
     if (p.mask_mode == MASK_INDEXED)
         hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, LONG, SAVE, SCALED>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
     else if (p.mask_mode == MASK_DENSE)
