@@ -248,15 +248,17 @@
             copy_b32<WAIT>(t.pos, t.pos_voff, lds_addr(sQpos) + pos_buf * (DKDV_QT * 4u));
     };
 
-    // NARROW: where this lane reads in tile 0 and in its rows, as byte addresses; what a k-slice, a block of columns, a half of the
-    // tile and the other array add are constants, XORed or in the instruction (see chunk_slot: the swizzle takes bits 1 to 3 of the row)
+    // Where this lane reads in tile 0, as byte addresses.  What a k-slice, a block of columns, a half of the tile and the other array add
+    // are constants, XORed (the swizzle of chunk_slot takes bits 0 to 3 of the row; the tiles start at multiples of 256) or in the
+    // instruction.  From chunk_slot access by access, a block of 32 x 32 took 133 vector instructions beside its MFMAs at head dim
+    // 128, 99 now, and 256 registers, 234 now.  Step, us, D 128: 8192 tokens, 32 / 8 heads 1720 -> 1696, 65536 47.5 -> 46.7 ms, 4 x 1537
+    // 364.5 -> 359, a bool mask, 2 x 4096, 16 heads 502 -> 494; 2 x 2003, 16 heads, D 96 169.2 -> 167.2.
     constexpr unsigned ROW_BYTES = NCH * 16, DO_AT = NB * TILE_BYTES, DELTA_AT = NB * DKDV_QT * 4;
-    unsigned chunk_lane = 0, transposed_lane = 0;
-    if constexpr (NARROW) {
-        const int i = lane & 15, r = 4 * hi + (i >> 2);
-        chunk_lane = ldsQ + 16u * (unsigned)chunk_slot<D>(l32, hi);
-        transposed_lane = ldsQ + 16u * (unsigned)chunk_slot<D>(r, 2 * half16 + ((i & 3) >> 1)) + 8u * (i & 1);
-    }
+    const int lane16 = lane & 15;
+    const unsigned chunk_lane = ldsQ + 16u * (unsigned)chunk_slot<D>(l32, hi);
+    const unsigned transposed_lane =
+        ldsQ + 16u * (unsigned)chunk_slot<D>(4 * hi + (lane16 >> 2), 2 * half16 + ((lane16 & 3) >> 1)) + 8u * (lane16 & 1);
+    const unsigned kv_lane = NARROW ? 0u : lds_addr(sK) + 16u * (unsigned)chunk_slot<D>(32 * kg + l32, hi);
 
     // One 64-row tile held in buffer cur against this wave's 32 keys; the wave's 32 rows sit at sequence
     // rows myrow0.. and its class for them is cls.  The copies of the next tile into the other buffer
@@ -297,8 +299,6 @@
         int own = lane;
         if (NARROW) asm volatile("" : "+v"(own));
         const int lane = own, hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
-        const u32x4* tQ = sQ[cur];
-        const u32x4* tG = sDO[cur];
         // ---- S = Q K^T and dP = dO V^T : 32 queries x 32 keys, two accumulator chains; both operands of
         // every MFMA come from LDS and are requested AHEAD MFMAs in front of their use
         // The V tile in LDS is NEGATED (see negate_v_tile), and the dP accumulator starts from delta instead of
@@ -307,12 +307,21 @@
         f32x16 s, dp;
         const unsigned tile_at = (unsigned)(cur * TILE_BYTES + qr * ROW_BYTES);
         const unsigned row_at = 16u * hi + (lds_addr(sLse) + (unsigned)(cur * (DKDV_QT * 4) + qr * 4));
-        if constexpr (NARROW) {
-            constexpr int NOP = 2 * KK, AHEAD = 3;
+        {
+            constexpr int NOP = 2 * KK, AHEAD = D > 64 ? 2 : 3;  // MFMA j: S (j even) or dP (j odd), k-slice j / 2.  (3 at D 128: 1731 -> 1727)
+            constexpr int FIRST = SORTED ? (NOP - NLOADS < 4 ? NOP - NLOADS : 4) : 0;  // the copies start behind MFMA FIRST - 1
+            constexpr unsigned V_AT = 128 * ROW_BYTES;
             const unsigned at = chunk_lane + tile_at;
-            u32x4 a[NOP];
+            u32x4 a[NOP], bb[NOP];
             auto operand = [&](int j) { return lds_read16<u32x4>((at ^ (unsigned)(32 * (j >> 1))) + ((j & 1) ? DO_AT : 0u)); };
+            auto kv = [&](int j) {
+                if constexpr (KV_REGS)
+                    return (j & 1) ? vfrag[j >> 1] : kfrag[j >> 1];
+                else
+                    return lds_read16<u32x4>((kv_lane ^ (unsigned)(32 * (j >> 1))) + ((j & 1) ? V_AT : 0u));
+            };
             a[0] = operand(0);
+            bb[0] = kv(0);
 #pragma unroll
             for (int grp = 0; grp < 4; ++grp) {
                 const f32x4 d4 = lds_read16<f32x4>(row_at + DELTA_AT + 32u * grp);
@@ -320,48 +329,22 @@
                 for (int x = 0; x < 4; ++x) dp[4 * grp + x] = d4[x];
             }
 #pragma unroll
-            for (int j = 1; j < AHEAD; ++j) a[j] = operand(j);
-#pragma unroll
-            for (int j = 0; j < NOP; ++j) {
-                __builtin_amdgcn_sched_barrier(0);
-                if (j + AHEAD < NOP) a[j + AHEAD] = operand(j + AHEAD);
-                if (j & 1)
-                    dp = T::mfma(a[j], vfrag[KV_REGS ? j >> 1 : 0], dp);
-                else
-                    s = T::mfma(a[j], kfrag[KV_REGS ? j >> 1 : 0], j < 2 ? zero16 : s);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        } else {
-            constexpr int NOP = 2 * KK, AHEAD = 3;  // MFMA j: S (j even) or dP (j odd), k-slice j / 2
-            constexpr int FIRST = SORTED ? (NOP - NLOADS < 4 ? NOP - NLOADS : 4) : 0;  // the copies start behind MFMA FIRST - 1
-            u32x4 a[NOP], bb[NOP];
-            a[0] = lds_read_chunk<D>(tQ, qr + l32, hi);  // the operands of the first MFMA go first
-            bb[0] = KV_REGS ? kfrag[0] : lds_read_chunk<D>(sK, 32 * kg + l32, hi);
-#pragma unroll
-            for (int grp = 0; grp < 4; ++grp) {
-                const f32x4 d4 = *(const f32x4*)&sDelta[cur][qr + 8 * grp + 4 * hi];
-#pragma unroll
-                for (int x = 0; x < 4; ++x) dp[4 * grp + x] = d4[x];
-            }
-#pragma unroll
             for (int j = 1; j < AHEAD; ++j) {
-                a[j] = lds_read_chunk<D>((j & 1) ? tG : tQ, qr + l32, 2 * (j >> 1) + hi);
-                bb[j] = KV_REGS ? ((j & 1) ? vfrag[j >> 1] : kfrag[j >> 1])
-                                : lds_read_chunk<D>((j & 1) ? sV : sK, 32 * kg + l32, 2 * (j >> 1) + hi);
+                a[j] = operand(j);
+                bb[j] = kv(j);
             }
 #pragma unroll
             for (int j = 0; j < NOP; ++j) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (j + AHEAD < NOP) {
-                    a[j + AHEAD] = lds_read_chunk<D>(((j + AHEAD) & 1) ? tG : tQ, qr + l32, 2 * ((j + AHEAD) >> 1) + hi);
-                    bb[j + AHEAD] = KV_REGS ? (((j + AHEAD) & 1) ? vfrag[(j + AHEAD) >> 1] : kfrag[(j + AHEAD) >> 1])
-                                            : lds_read_chunk<D>(((j + AHEAD) & 1) ? sV : sK, 32 * kg + l32, 2 * ((j + AHEAD) >> 1) + hi);
+                    a[j + AHEAD] = operand(j + AHEAD);
+                    bb[j + AHEAD] = kv(j + AHEAD);
                 }
                 if (j & 1)
                     dp = T::mfma(a[j], bb[j], dp);
                 else
                     s = T::mfma(a[j], bb[j], j < 2 ? zero16 : s);
-                if (j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, nxt, pos_nxt);
+                if (!NARROW && j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, nxt, pos_nxt);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -386,7 +369,7 @@
         }
 #pragma unroll
         for (int grp = 0; grp < 4; ++grp) {
-            const f32x4 l4 = NARROW ? lds_read16<f32x4>(row_at + 32u * grp) : *(const f32x4*)&sLse[cur][qr + 8 * grp + 4 * hi];
+            const f32x4 l4 = lds_read16<f32x4>(row_at + 32u * grp);
 #pragma unroll
             for (int x = 0; x < 4; ++x) s[4 * grp + x] = __builtin_amdgcn_exp2f(fmaf(s[4 * grp + x], c2, SCALED ? -l4[x] : l4[x] * -LOG2E));
         }
@@ -487,7 +470,7 @@
             dsb[t] = pack8<T>(dp, 8 * t);
         }
         // ---- dV^T += dO^T P ; dK^T += Q^T dS -------------------------------------------------
-        if constexpr (NARROW) {
+        {
             const unsigned at = transposed_lane + tile_at;
             u32x4 tg[2][DB], tq[2][DB];
 #pragma unroll
@@ -497,23 +480,6 @@
                     const unsigned x = (at ^ (64u * db)) + 16u * t * ROW_BYTES, y = (at ^ (64u * db + 16u)) + (16u * t + 8u) * ROW_BYTES;
                     tg[t][db] = lds_read_transposed_at(x + DO_AT, y + DO_AT);
                     tq[t][db] = lds_read_transposed_at(x, y);
-                }
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int db = 0; db < DB; ++db) {
-                    dv[db] = T::mfma(tg[t][db], pb[t], dv[db]);
-                    dk[db] = T::mfma(tq[t][db], dsb[t], dk[db]);
-                }
-            sched_pipeline_mfma_lds<4 * DB, 4, 2>();
-        } else {
-            u32x4 tg[2][DB], tq[2][DB];
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int db = 0; db < DB; ++db) {
-                    tg[t][db] = lds_read_transposed<D>(tG, lane, qr + 16 * t + 4 * hi, 32 * db + 16 * half16);
-                    tq[t][db] = lds_read_transposed<D>(tQ, lane, qr + 16 * t + 4 * hi, 32 * db + 16 * half16);
                 }
 #pragma unroll
             for (int t = 0; t < 2; ++t)

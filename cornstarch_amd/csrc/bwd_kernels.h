@@ -104,7 +104,7 @@ template <int D, int MODE, bool LONG>
 struct DkdvShared {
     static constexpr int NB = DKDV_DEEP<D, MODE, LONG> ? 4 : 2;  // tile buffers
     static constexpr int NCH = LDS_COLS<D> / 8;
-    u32x4 k[128 * NCH];
+    __attribute__((aligned(256))) u32x4 k[128 * NCH];
     u32x4 v[128 * NCH];
     u32x4 q[NB][DKDV_QT * NCH];
     u32x4 dout[NB][DKDV_QT * NCH];
@@ -129,12 +129,14 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
-    __shared__ u32x4 sK[128 * NCH];
-    __shared__ u32x4 sV[128 * NCH];
-    __shared__ u32x4 sQ[NB][DKDV_QT * NCH];
-    __shared__ u32x4 sDO[NB][DKDV_QT * NCH];
-    __shared__ __attribute__((aligned(16))) float sLse[NB][DKDV_QT];      // natural-log lse of the rows
-    __shared__ __attribute__((aligned(16))) float sDelta[NB][DKDV_QT];
+    __shared__ __attribute__((aligned(256))) u32x4 sTiles[(2 * 128 + 2 * NB * DKDV_QT) * NCH];
+    u32x4* const sK = sTiles;
+    u32x4* const sV = sTiles + 128 * NCH;
+    u32x4 (*const sQ)[DKDV_QT * NCH] = (u32x4 (*)[DKDV_QT * NCH])(sTiles + 256 * NCH);
+    u32x4 (*const sDO)[DKDV_QT * NCH] = sQ + NB;
+    __shared__ __attribute__((aligned(16))) float sRowNumbers[2 * NB][DKDV_QT];
+    float (*const sLse)[DKDV_QT] = sRowNumbers;  // natural-log lse of the rows
+    float (*const sDelta)[DKDV_QT] = sRowNumbers + NB;
     __shared__ __attribute__((aligned(16))) int64_t sQbf[NB][DKDV_QT];    // raw bitfields of the rows
     // their positions (ROW_POS).  SORTED: a tile's rows are gathered, so their numbers have to be here a tile earlier
     __shared__ __attribute__((aligned(16))) int sQpos[SORTED ? 3 : NB][DKDV_QT];
@@ -152,9 +154,8 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 // The same work for head dims up to 64 by four waves, one for each 32 keys, that take both slices of a pair one after the other: three
 // workgroups fit a unit, so a third wave per SIMD fills the gaps of MFMAs, arithmetic and LDS reads (each 450 to 550 cycles of a 32 x 32
 // block's 1050 at head dim 64 with two), and a workgroup's start and end pass behind the others' work.  168 registers: every wave
-// holds its K and V operands, and nothing lies in LDS but Q, dO and the small rows; the LDS addresses of a block are one per access
-// form and XORs of constants (75 vector instructions a block beside the MFMAs; 93 in the kernel above, and 144 if the compiler
-// derives them anew); the rule constants of a block are read one row at a time.  (Spilled K and V operands, read back between
+// holds its K and V operands, and nothing lies in LDS but Q, dO and the small rows; what derives from the lane is derived anew for
+// every block (75 vector instructions a block beside the MFMAs); the rule constants of a block are read one row at a time.  (Spilled K and V operands, read back between
 // the tile copies, wait for those: step 1.26 -> 1.42 ms at 8 x 4096.)  No partial sums to add at the end.
 // Step, us, eight waves -> four: D 64: 8 x 4096, 16 heads 1312 -> 1236, 8 x 2048 397 -> 373, 32 x 512, 32 heads 461 ->
 // 414, 8 x 4096, 32 / 8 heads 2415 -> 2339, 16384, 16 heads, nothing hidden 5192 -> 5195; D 32: 8 x 2048, 16 heads 290 -> 249, 16 x 512, 32
