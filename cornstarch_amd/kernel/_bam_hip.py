@@ -15,7 +15,7 @@ BAM_DTYPE_F16 = 0
 BAM_DTYPE_BF16 = 1
 BAM_MAX_SEQLEN = 4194304
 BAM_STATIC_PLAN_BYTES = 8 << 20
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -181,10 +181,13 @@ def load() -> ctypes.CDLL:
             "(run `python -m cornstarch_amd.build`); there is no fallback path"
         )
     lib = ctypes.CDLL(LIB_PATH)
-    lib.bam_last_error.restype = ctypes.c_char_p
-    lib.bam_last_error.argtypes = []
     lib.bam_abi_version.restype = _int
     lib.bam_abi_version.argtypes = []
+    # (first: a library of another number may lack functions that are looked up below)
+    if lib.bam_abi_version() != ABI_VERSION:
+        raise BamError(f"libbam_hip.so has ABI {lib.bam_abi_version()}, this binding expects {ABI_VERSION}")
+    lib.bam_last_error.restype = ctypes.c_char_p
+    lib.bam_last_error.argtypes = []
     lib.bam_plan_workspace_bytes.restype = _i64
     lib.bam_plan_workspace_bytes.argtypes = [_int, _int]
     lib.bam_plan_workspace_bytes_rect.restype = _i64
@@ -199,8 +202,6 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = _int
-    if lib.bam_abi_version() != ABI_VERSION:
-        raise BamError(f"libbam_hip.so has ABI {lib.bam_abi_version()}, this binding expects {ABI_VERSION}")
     _lib = lib
     return lib
 
@@ -216,6 +217,7 @@ def _load_host():
     """The native host layer (csrc/host.cpp), which calls the library above."""
     import torch  # noqa: F401  (its libraries first: the host layer is linked against them)
 
+    load()  # (a library of another number is refused as such, not by the symbol that the host layer misses)
     try:
         from cornstarch_amd import _bam_host
     except ImportError as e:

@@ -161,7 +161,7 @@ typedef struct bam_plan {
 
 const char* bam_last_error(void);
 
-/* ABI version of this library (bumped on any signature change). */
+/* ABI version of this library (bumped when a function is added or a signature changes). */
 int bam_abi_version(void);
 
 /*

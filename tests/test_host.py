@@ -6,6 +6,7 @@ the baseline document describes."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -53,6 +54,19 @@ def test_library_exports_every_declared_symbol():
     # a mask plan also holds the mask packed to bits, once per orientation: a quarter of the mask's bytes
     extra = lib2.bam_mask_plan_workspace_bytes(1, 8192, 8192) - lib2.bam_plan_workspace_bytes_rect(1, 8192, 8192)
     assert extra == 2 * 8192 * 8192 // 8 and lib2.bam_mask_plan_workspace_bytes(1, 131073, 64) == 0
+
+
+def test_a_library_of_another_abi_version_is_refused_by_its_number(tmp_path, monkeypatch):
+    """Also where it lacks functions that the binding needs; and the number moves when one is added."""
+    assert (_bam_hip.ABI_VERSION, len(_declared_symbols())) == (16, 41)
+    (tmp_path / "old.c").write_text(f"int bam_abi_version(void) {{ return {_bam_hip.ABI_VERSION - 1}; }}")
+    old = str(tmp_path / "old.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", old, str(tmp_path / "old.c")], check=True)
+    monkeypatch.setattr(_bam_hip, "LIB_PATH", old)
+    monkeypatch.setattr(_bam_hip, "_lib", None)
+    for load in (_bam_hip.load, _bam_hip._load_host):
+        with pytest.raises(_bam_hip.BamError, match=f"has ABI {_bam_hip.ABI_VERSION - 1}, this binding expects"):
+            load()
 
 
 def test_abi_rejects_bad_arguments_without_touching_the_gpu():
