@@ -551,14 +551,17 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
     if (scaled) a.lse_scaled = a.delta + lse.numel();
     a.accumulate = accumulate ? 1 : 0;
     Tensor ws;
-    // Small problems take no dS workspace and do not wait for the plan's count; where the count decides, it is waited for and asked again.
+    // Small problems take no dS workspace and are launched without waiting for the plan's count; where the count decides, it is waited
+    // for and asked again.
     int takes_ds = 0;
     check(bam_attn_bwd_takes_ds(&a, &takes_ds), "bam_attn_bwd_takes_ds");
-    if (takes_ds) {
+    auto wait_pairs = [&]() {
         optional<py::gil_scoped_release> release;
         if (PyGILState_Check()) release.emplace();
-        a.pairs = plan.core->wait_pairs();
-        release.reset();
+        return plan.core->wait_pairs();
+    };
+    if (takes_ds) {
+        a.pairs = wait_pairs();
         desc.rows_known = plan.core->rows_known.load();
         check(bam_attn_bwd_takes_ds(&a, &takes_ds), "bam_attn_bwd_takes_ds");
     }
@@ -582,6 +585,9 @@ void run_backward(Call c, const Plan& plan, const Tensor& dout, const Tensor& q,
         }
     }
     check(bam_attn_bwd(&a, current_stream(q.device()).stream()), "bam_attn_bwd");
+    // The count of a small problem is waited for behind its launches, which the GPU works on meanwhile: a plan whose launch failed is
+    // refused by the backward here as well, and not by whatever synchronizes next.
+    if (plan && a.D > 64 && a.Sk <= 131072) wait_pairs();
 }
 
 // ------------------------------------------------------------------ autograd

@@ -323,3 +323,29 @@ def test_a_plan_of_another_problem_is_refused():
     assert BA.BitfieldUtils.plan_for(flags, bf) is plan
     BA.BitfieldUtils.clear_cache()
     assert BA.BitfieldUtils.plan_for(flags, bf) is None
+
+
+@pytest.mark.parametrize("S,Hq", [(1024, 8), (1500, 20), (1100, 32)])  # one launch by the sizes, by the count; a dS workspace
+def test_a_plan_whose_count_never_arrives_is_refused(S, Hq):
+    """The word that the count is stored to is cleared on the host, as if the last launch of the plan builder had failed: every
+    backward that takes such a plan for a hand-over of dS, or may take it for one, raises once the stream has run dry."""
+    bf = random_bitfield(1, S, seed=S, pad=3).to(dev())
+    flags, _, _, plan = build_plan(bf)
+    q, k, v, do = (torch.randn(1, S, Hq, 128, device=dev(), dtype=torch.bfloat16) for _ in range(4))
+    o, lse, scale = BA._bitfield_attn_forward(q, k, v, bf, flags)
+    torch.cuda.synchronize()
+    # (the word's address and tag follow the bam_plan inside the plan object; the tag is in the word's upper half)
+    behind = ctypes.addressof(plan.struct) + ctypes.sizeof(_bam_hip.Plan)
+    tag = ctypes.c_uint32.from_address(behind + 8).value
+    word = ctypes.c_uint64.from_address(ctypes.c_uint64.from_address(behind).value)
+    stored = word.value
+    assert stored >> 32 == tag
+    try:
+        word.value = 0
+        with pytest.raises(_bam_hip.BamError, match="pair count of a plan never arrived"):
+            BA._bitfield_attn_backward_overwrite(do, q, k, v, o, bf, flags, lse, scale)
+    finally:
+        word.value = stored
+    got = BA._bitfield_attn_backward_overwrite(do, q, k, v, o, bf, flags, lse, scale)
+    assert plan.ds_pairs() == stored & 0xFFFFFFFF and all(torch.isfinite(g).all() for g in got)
+    BA.BitfieldUtils.clear_cache()
