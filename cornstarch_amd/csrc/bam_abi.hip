@@ -166,6 +166,9 @@ int fill_plan(bam::AttnParams& p, const char* who, const bam_plan* plan, int B, 
     p.fine = plan->fine;
     p.fine_sb = plan->fine_stride_b;
     p.fine_ss = plan->fine_stride_s;
+    // (a caller may lay the classes out by itself: rows of ceil(Sk / 32) bytes, at any address)
+    p.fine_words = plan->fine_stride_s >= 4 * (((int64_t)Sk + 127) / 128) &&
+                   ((reinterpret_cast<uintptr_t>(plan->fine) | (uintptr_t)plan->fine_stride_b | (uintptr_t)plan->fine_stride_s) & 3u) == 0;
     p.order = plan->order;
     p.order_sb = plan->order_stride_b;
     p.tile_order = plan->ds_tile_order;  // may be null

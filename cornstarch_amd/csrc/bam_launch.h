@@ -62,6 +62,7 @@ struct AttnParams {
     // neighbours need about the same keys, heaviest first, (B, 4 * num_m) ints, -1 = no slice.
     const uint8_t* fine;
     int64_t fine_sb, fine_ss;
+    int fine_words;            // the bytes of four neighbouring tiles, 4 n .., are one aligned, in-range word (the builders' plans)
     const int* order;
     int64_t order_sb;
     // Optional (plan of bitfield attention): the query rows sorted so that every slice holds rows that see the same keys.

@@ -390,9 +390,9 @@ __device__ __forceinline__ void build_key_tile_list(const WaveSlices& ws, int nu
 // The four class bytes (key columns 4 nt ..) of slice s (< s_end, or one that does not matter), low byte first.
 __device__ __forceinline__ unsigned load_slice_classes(const AttnParams& p, int b, int nt, int s, int s_end) {
     s = max(min(s, s_end - 1), 0);
-    if (p.fine != nullptr)  // (rows of the plan's classes are padded to 16 bytes)
-        return *(const unsigned*)(p.fine + (int64_t)b * p.fine_sb + (int64_t)s * p.fine_ss + 4 * nt);
-    const int8_t* f = p.flags + (int64_t)b * p.flags_sb + (int64_t)(s >> 2) * p.flags_sm;
+    const int8_t* f = p.fine != nullptr ? (const int8_t*)p.fine + (int64_t)b * p.fine_sb + (int64_t)s * p.fine_ss
+                                        : p.flags + (int64_t)b * p.flags_sb + (int64_t)(s >> 2) * p.flags_sm;
+    if (p.fine_words) return *(const unsigned*)(f + 4 * nt);
     unsigned c = 0;
 #pragma unroll
     for (int w = 0; w < 4; ++w) c |= (unsigned)(f[min(4 * nt + w, p.num_n - 1)] & 3) << (8 * w);

@@ -349,3 +349,35 @@ def test_a_plan_whose_count_never_arrives_is_refused(S, Hq):
     got = BA._bitfield_attn_backward_overwrite(do, q, k, v, o, bf, flags, lse, scale)
     assert plan.ds_pairs() == stored & 0xFFFFFFFF and all(torch.isfinite(g).all() for g in got)
     BA.BitfieldUtils.clear_cache()
+
+
+@pytest.mark.parametrize("B,S,H,D", [(1, 100, 2, 128), (2, 283, 4, 64), (1, 700, 4, 128), (36, 129, 32, 64)])  # the last: four-wave dK/dV
+@pytest.mark.parametrize("offset", [0, 1])
+def test_classes_laid_out_by_the_caller(B, S, H, D, offset):
+    """Rows of ceil(S/32) class bytes without padding, at any address: dK/dV must not read them as words.  Bytes around them say
+    "full", the results are those of the builder's rows of 16-byte multiples."""
+    bf = random_bitfield(B, S, seed=S, pad=3).to(dev())
+    flags, fine, _, plan = build_plan(bf)
+    slots, num_n = 4 * flags.shape[1], fine.shape[2]
+    assert fine.shape[1] == slots
+    room = torch.full((fine.numel() + 64,), 2, dtype=torch.uint8, device=dev())
+    room[16 + offset : 16 + offset + fine.numel()] = fine.reshape(-1)
+    own = _bam_hip.Plan.from_buffer_copy(plan.struct)
+    own.fine, own.fine_stride_b, own.fine_stride_s = room.data_ptr() + 16 + offset, slots * num_n, num_n
+
+    class Own:
+        def byref(self):
+            return ctypes.byref(own)
+
+    q, k, v, do = (torch.randn(B, S, H, D, device=dev(), dtype=torch.bfloat16) for _ in range(4))
+    o, lse, scale = BA._bitfield_attn_forward(q, k, v, bf, flags)
+    delta = torch.empty_like(lse)
+    BA._launch_bwd_preprocess(o, do, delta)
+    got = []
+    for p in (plan, Own()):
+        got.append((torch.empty_like(k), torch.empty_like(v)))
+        BA._launch_bwd_dkdv(q, k, v, do, lse, delta, *got[-1], bf, flags, scale, accumulate=False, plan=p)
+    torch.cuda.synchronize()
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+    BA.BitfieldUtils.clear_cache()
