@@ -76,9 +76,9 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const AttnParams p)
 // With S = Q K^T computed as queries x keys, a lane of the C fragment owns ONE key and 16
 // query rows, so P and dS feed dV^T = dO^T P and dK^T = Q^T dS as B operands from registers;
 // Q^T and dO^T come from the transposing LDS read of the same row-major tiles.
-// The two waves that share a key group hold partial sums; they add them to the caller's
-// buffers one after the other (workgroup barrier in between), so the result stays
-// deterministic and atomic free.
+// The two waves that share a key group hold partial sums; at the end one hands its dV over through LDS, the other its dK, and each
+// adds up and stores what it has received: deterministic and atomic free.  (Four-wave form: a wave takes both rows of slices, and
+// holds the whole sums.)
 constexpr int DKDV_QT = 64;
 constexpr int DKDV_THREADS = 512, DKDV_NARROW_THREADS = 256;
 
@@ -100,9 +100,10 @@ constexpr int DKDV_THREADS = 512, DKDV_NARROW_THREADS = 256;
 template <int D, int MODE, bool LONG>
 constexpr bool DKDV_DEEP = D <= 64 && MODE != MASK_SORTED && !LONG;
 
-template <int D, int MODE, bool LONG>
+// LDS of dkdv_work.  (The kernels declare the same arrays one by one.)
+template <int D, int MODE>
 struct DkdvShared {
-    static constexpr int NB = DKDV_DEEP<D, MODE, LONG> ? 4 : 2;  // tile buffers
+    static constexpr int NB = DKDV_DEEP<D, MODE, false> ? 4 : 2;  // tile buffers
     static constexpr int NCH = LDS_COLS<D> / 8;
     __attribute__((aligned(256))) u32x4 k[128 * NCH];
     u32x4 v[128 * NCH];
@@ -111,8 +112,7 @@ struct DkdvShared {
     __attribute__((aligned(16))) float lse[NB][DKDV_QT];    // natural-log lse of the rows
     __attribute__((aligned(16))) float delta[NB][DKDV_QT];
     __attribute__((aligned(16))) int64_t qbf[NB][DKDV_QT];  // raw bitfields of the rows
-    // their positions (indexed and sorted rows).  Sorted: a tile's rows are gathered, so their numbers have to be here a tile earlier
-    __attribute__((aligned(16))) int qpos[MODE == MASK_SORTED ? 3 : NB][DKDV_QT];
+    __attribute__((aligned(16))) int qpos[NB][DKDV_QT];     // their positions (MASK_INDEXED)
     __attribute__((aligned(16))) unsigned wq[DKDV_THREADS / 64][5][32];  // per-wave rule constants
     // MASK_DENSE with packed mask bits: for the two slices of the tile, one word per key of the workgroup's 128 keys
     unsigned col_bits[MODE == MASK_DENSE ? NB : 1][2][MODE == MASK_DENSE ? 128 : 1];
@@ -187,17 +187,20 @@ __global__ __launch_bounds__(DKDV_NARROW_THREADS, 3) void bwd_dkdv_narrow_kernel
 #include "bwd_dkdv_body.h"
 }
 
-// The work of workgroup `block` of a dK/dV launch, in LDS of the caller's.
-template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE, bool SCALED>
-__device__ __forceinline__ void dkdv_work(const AttnParams& p, const int block, DkdvShared<D, MODE, LONG>& sh) {
-    constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
-    constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
-    static_assert(!(SORTED && LONG), "no plan for so many rows");
-    constexpr bool NARROW = false;
+// The work of workgroup `block` of a dK/dV launch, in LDS of the caller's: rows in natural order, one pass, no dS kept.
+template <typename T, int D, int MODE, bool BIAS, bool SCALED>
+__device__ __forceinline__ void dkdv_work(const AttnParams& p, const int block, DkdvShared<D, MODE>& sh) {
+    constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, ROW_POS = IDX;
+    constexpr bool NARROW = false, SORTED = false, LONG = false, SAVE = false;
     constexpr bool DEEP = DKDV_DEEP<D, MODE, LONG>;
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
+    typedef DkdvShared<D, MODE> Shared;
+    static_assert(alignof(Shared) % 256 == 0 && offsetof(Shared, k) % 256 == 0 && offsetof(Shared, q) % 256 == 0 &&
+                      offsetof(Shared, v) - offsetof(Shared, k) == sizeof(Shared::k) && offsetof(Shared, dout) - offsetof(Shared, q) == sizeof(Shared::q) &&
+                      offsetof(Shared, delta) - offsetof(Shared, lse) == sizeof(Shared::lse),
+                  "the second array of each pair is read at a constant behind the first, and addresses below 256 are XORed");
     auto &sK = sh.k, &sV = sh.v;
     auto &sQ = sh.q, &sDO = sh.dout;
     auto &sLse = sh.lse, &sDelta = sh.delta;
@@ -725,11 +728,11 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_both_kernel(const AttnPar
     static_assert(DKDV_THREADS == 2 * DQ_THREADS, "dQ with two streams");
     constexpr bool BIAS = BIAS_FORM != BIAS_NONE;
     __shared__ union {
-        DkdvShared<D, MODE, false> dkdv;
+        DkdvShared<D, MODE> dkdv;
         DqShared<D, MODE, BIAS_FORM, 2> dq;
     } sh;
     if ((int)blockIdx.x < dkdv_blocks)
-        dkdv_work<T, D, MODE, BIAS, false, false, !BIAS && D <= 64>(kv, blockIdx.x, sh.dkdv);
+        dkdv_work<T, D, MODE, BIAS, !BIAS && D <= 64>(kv, blockIdx.x, sh.dkdv);
     else
         dq_work<T, D, MODE, BIAS_FORM, false, 2>(p, blockIdx.x - dkdv_blocks, sh.dq);
 }
