@@ -912,8 +912,7 @@ static bool attn_bwd_one_launch(const bam_attn* a, const bam::AttnParams& all, i
 int bam_attn_bwd_takes_ds(const bam_attn* a, int* takes) {
     if (a == nullptr || takes == nullptr) return fail(BAM_ERR_INVALID_ARGUMENT, "bam_attn_bwd_takes_ds: null pointer");
     *takes = a->plan != nullptr && a->D > 64 && a->Sk <= 131072 ? 1 : 0;
-    // (what both_in_one_launch says without a closer look: the host asks twice a backward)
-    if (*takes == 0 || a->Sk < 768 || (int64_t)((a->Sq + 127) / 128) * a->B * a->Hq > 512) return BAM_OK;
+    if (*takes == 0 || !bam::one_launch_sizes(a->Sq, a->Sk, a->B, a->Hq)) return BAM_OK;
     bam_plan plan;
     bam::AttnParams all = {};
     BAM_TRY(attn_bwd_params(a, plan, all));

@@ -204,6 +204,8 @@ int launch_bwd_dq(const AttnParams& p, int dtype, hipStream_t stream);
 // Whether dK/dV and dQ go into one launch, behind the delta pre-pass; and that launch (kv: dK/dV's parameters,
 // those of the parts where there are any).  dkdv_blocks: the workgroups of dK/dV; pairs: the plan's count if it is known, else 0.
 bool both_in_one_launch(const AttnParams& p, int64_t dkdv_blocks, int64_t pairs);
+// The sizes at which that is looked at above head dim 64 at all, for a host that asks before every backward.
+inline bool one_launch_sizes(int Sq, int Sk, int B, int Hq) { return Sk >= 768 && (int64_t)((Sq + 127) / 128) * B * Hq <= 512; }
 int launch_bwd_both(const AttnParams& kv, const AttnParams& p, int dtype, hipStream_t stream);
 // dk, dv of p from the parts that a dK/dV launch with kv_parts left at `parts_dk` and `parts_dv` (contiguous).
 int launch_sum_parts(const AttnParams& p, const float* parts_dk, const float* parts_dv, int parts, int dtype, hipStream_t stream);

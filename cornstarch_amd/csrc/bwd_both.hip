@@ -33,15 +33,16 @@ static int launch_both_t(const AttnParams& kv, const AttnParams& p, hipStream_t 
 // heads 86.4 -> 70.7; D 80, 1024, 16 heads 101.5 -> 81.7.  Up to two rounds (512) where the count, waited for, leaves the lists
 // uneven: 4096, 8 heads, pairs of 0.52 of the tiles 240.2 -> 203.3, 0.54 235.7 -> 230.1, 0.73 268.4 -> 272.2; 3000, 10 / 2 heads 0.51
 // 197.8 -> 167.6, 8 heads 0.65 189.5 -> 177.8; 8192, 4 heads, D 80 366.5 -> 314.6; 4096, 6 / 1 heads (parts) 233.7 -> 183.7; 2048, 16
-// heads, nothing hidden 180.2 -> 188.9.  Beyond: 2048, 24 heads 166.9 -> 170.7, 20 heads 157.0 -> 153.9.  Below 768 keys it would be
-// as good (4 x 283, 16 / 4 heads 100.7 -> 79.0, the host's wait), but those are the calls whose callers are known to bound or refuse
-// the workspace, and to compare bits with and without runs of heads: they are asked as before.
+// heads, nothing hidden 180.2 -> 188.9.  Beyond: 2048, 24 heads 166.9 -> 170.7, 20 heads 157.0 -> 153.9.  The line at 768
+// keys is not one of speed: below it one launch would be as good (4 x 283, 16 / 4 heads 100.7 -> 79.0, the host's wait ahead of the
+// launches).  The tests of the hand-over (a limit or a failing allocation of its workspace, the same bits in runs of heads) hold calls
+// of up to 640 keys to asking for a workspace.
 bool both_in_one_launch(const AttnParams& p, int64_t dkdv_blocks, int64_t pairs) {
     if (p.D < 64 || !two_streams(p) || p.rows != nullptr) return false;
     if (p.D > 64) {
         const int64_t blocks = (int64_t)p.num_m * p.B * p.Hq + dkdv_blocks;
         const bool few_pairs = pairs > 0 && 3 * pairs <= 2 * (int64_t)p.B * p.num_kt * ((p.Sq + 31) / 32);
-        if (p.ds_ws != nullptr || p.Sk < 768 || blocks > (few_pairs ? 512 : 256)) return false;
+        if (p.ds_ws != nullptr || !one_launch_sizes(p.Sq, p.Sk, p.B, p.Hq) || blocks > (few_pairs ? 512 : 256)) return false;
     }
     if (p.Sq > MAX_SLICE_LIST * 32 || p.Sk > MAX_LIST * DQ_KT || dkdv_far(p)) return false;  // (walked in passes)
     return p.bias == nullptr ? p.D > 64 || p.lse_scaled != nullptr : p.bias_sm == 0 && p.bias_vec;
