@@ -24,6 +24,7 @@ def parts(B, S, Hq, Hkv, D, mode=0, pairs=0):
 @pytest.mark.parametrize("shape,want", [
     ((1, 129, 16, 1, 32), 16), ((1, 700, 32, 8, 40), 4), ((1, 2100, 6, 3, 56), 2), ((4, 400, 6, 1, 64), 6), ((3, 1000, 24, 4, 64), 3),
     ((1, 4100, 12, 3, 8), 4), ((1, 700, 32, 8, 128), 4), ((2, 900, 16, 4, 96), 4), ((1, 2003, 12, 4, 112), 3),
+    ((2, 700, 16, 4, 96), 4), ((1, 1000, 72, 8, 80), 9),
     ((2, 283, 6, 2, 64), 1), ((4, 1537, 8, 4, 32), 1),
     ((1, 512, 8, 1, 64), 8),
     ((1, 300, 32, 8, 128), 1),   # 15 steps saved: 32 are asked for

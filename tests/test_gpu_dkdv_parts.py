@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     (1, 129, 16, 1, 32), (1, 700, 32, 8, 40), (1, 2100, 6, 3, 56), (4, 400, 6, 1, 64),
     (3, 1000, 24, 4, 64),  # 3 parts of 2 heads
     (1, 4100, 12, 3, 8),   # 4 parts of 1
-    (1, 700, 32, 8, 128), (2, 900, 16, 4, 96), (1, 2003, 12, 4, 112),  # with the hand-over of dS
+    (1, 700, 32, 8, 128), (2, 700, 16, 4, 96), (1, 1000, 72, 8, 80),  # with the hand-over of dS
+    (2, 900, 16, 4, 96), (1, 2003, 12, 4, 112),  # in one launch with dQ
     (2, 283, 6, 2, 64), (4, 1537, 8, 4, 32),  # one part: too little to share, enough workgroups
 ])
 @pytest.mark.parametrize("bias", [False, True])

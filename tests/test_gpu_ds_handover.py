@@ -16,6 +16,7 @@ from tests.helpers import random_bitfield, rel_l2
 pytestmark = pytest.mark.gpu
 
 GRAD_REL_L2 = 5e-2
+ALLOCATE = BA._TilePlan._allocate
 
 
 def dev():
@@ -73,9 +74,13 @@ def test_pair_numbering_against_the_fine_classes(S):
     BA.BitfieldUtils.clear_cache()
 
 
-def run_backward(q, k, v, do, bf, handover, monkeypatch, accumulate=False):
+def run_backward(q, k, v, do, bf, handover, monkeypatch, accumulate=False, hands_over=None):
+    """handover: whether the limit lets dS be handed over; hands_over: whether the sizes do (None: they do if they may)."""
     monkeypatch.setattr(BA, "_ds_workspace_limit", (lambda device: 1 << 40) if handover else (lambda device: 0))
     flags, plan = build(bf)
+    allocated = []
+    monkeypatch.setattr(BA._TilePlan, "_allocate",
+                        staticmethod(lambda nbytes, device: allocated.append(nbytes) or ALLOCATE(nbytes, device)))
     o, lse, scale = BA._bitfield_attn_forward(q, k, v, bf, flags)
     if accumulate:
         grads = [torch.zeros_like(t, dtype=torch.float32) for t in (q, k, v)]
@@ -84,21 +89,27 @@ def run_backward(q, k, v, do, bf, handover, monkeypatch, accumulate=False):
         grads = BA._bitfield_attn_backward_overwrite(do, q, k, v, o, bf, flags, lse, scale)
     torch.cuda.synchronize()
     assert plan.struct.ds_workspace is None  # detached after the launches
+    assert len(allocated) == (handover if hands_over is None else hands_over)
+    monkeypatch.setattr(BA._TilePlan, "_allocate", staticmethod(ALLOCATE))
     return [g.clone() for g in grads]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("B,S,Hq,Hkv", [(2, 57, 2, 1), (1, 283, 4, 4), (2, 517, 4, 2), (1, 1000, 8, 2), (1, 2048, 4, 1)])
+@pytest.mark.parametrize("B,S,Hq,Hkv,hands_over", [
+    (2, 57, 2, 1, True), (1, 283, 4, 4, True), (2, 517, 4, 2, True),
+    (1, 1000, 8, 2, False), (1, 2048, 4, 1, False),   # in one launch whatever the limit: only the oracle tells
+    (1, 1000, 64, 16, True), (1, 2048, 28, 7, True),  # 640 and more than 560 workgroups, with parts
+])
 @pytest.mark.parametrize("accumulate", [False, True], ids=["typed", "fp32"])
-def test_handover_equals_recomputation(dtype, B, S, Hq, Hkv, accumulate, monkeypatch):
+def test_handover_equals_recomputation(dtype, B, S, Hq, Hkv, hands_over, accumulate, monkeypatch):
     d = dev()
     bf = random_bitfield(B, S, seed=S, pad=3).to(d)
     q, k, v, do = (t.to(d) for t in inputs(B, S, Hq, Hkv, 128, dtype, seed=S))
-    with_ds = run_backward(q, k, v, do, bf, True, monkeypatch, accumulate)
+    with_ds = run_backward(q, k, v, do, bf, True, monkeypatch, accumulate, hands_over)
     recomputed = run_backward(q, k, v, do, bf, False, monkeypatch, accumulate)
     assert torch.equal(with_ds[1], recomputed[1]) and torch.equal(with_ds[2], recomputed[2])  # dk, dv: same kernel
     assert rel_l2(with_ds[0].float(), recomputed[0].float()) <= 2e-3
-    again = run_backward(q, k, v, do, bf, True, monkeypatch, accumulate)
+    again = run_backward(q, k, v, do, bf, True, monkeypatch, accumulate, hands_over)
     assert all(torch.equal(a, b) for a, b in zip(with_ds, again))                            # no atomics: reruns agree
     for got, want in zip(with_ds, O.attention_backward(q, k, v, bf, do)):
         assert torch.isfinite(got).all() and rel_l2(got.float(), want) <= GRAD_REL_L2
