@@ -175,3 +175,32 @@ def test_a_plan_is_not_built_by_a_capture():
         torch.cuda.synchronize()
         assert torch.equal(out, want)
     BA.BitfieldUtils.clear_cache()
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(700, 8, 2, 64), (1024, 8, 8, 128), (1030, 8, 2, 96), (2048, 16, 16, 128)])
+def test_the_one_launch_backward_in_a_capture(S, Hq, Hkv, D):
+    """dK/dV and dQ in one launch (with parts; by the sizes, by the count), with a plan that was built before the capture."""
+    q, k, v, do = (t.to(dev()).requires_grad_(n < 3) for n, t in enumerate(make_inputs(1, S, Hq, Hkv, D, torch.bfloat16, seed=S)))
+    bf = random_bitfield(1, S, seed=S, pad=5).to(dev())
+
+    def step():
+        o = BA.bitfield_attn_func(q, k, v, bf)
+        return o.detach(), *torch.autograd.grad(o, (q, k, v), do)
+
+    BA.BitfieldUtils.clear_cache()
+    step()  # builds the plan, loads the code objects
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for seed in range(3):
+        with torch.no_grad():
+            for dst, src in zip((q, k, v, do), make_inputs(1, S, Hq, Hkv, D, torch.bfloat16, seed=seed)):
+                dst.copy_(src)
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, a, b in zip(("o", "dq", "dk", "dv"), out, step()):
+            assert torch.equal(a, b), name
+    BA.BitfieldUtils.clear_cache()
