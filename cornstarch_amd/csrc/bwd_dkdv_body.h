@@ -277,7 +277,7 @@
     float bias_key = 0.f;
     int bias_head = -1;
     auto fetch_bias_key = [&](int h) {
-        if (BIAS && p.bias_sm == 0 && h != bias_head) {
+        if (BIAS && (KEY_BIAS || p.bias_sm == 0) && h != bias_head) {
             bias_head = h;
             bias_key = kvalid ? load_bias1<T>(p.bias, (int64_t)b * p.bias_sb + (int64_t)h * p.bias_sh + key, p.bias_f32 != 0) : 0.f;
             asm volatile("" : "+v"(bias_key));  // arrives here, not at its first use between the tile copies
@@ -351,7 +351,7 @@
         // ---- P = exp(scale s - lse) on allowed pairs, -dS/scale = P (delta - dP)   (the factor `-scale` of dS
         // is applied once to dK in the epilogue).  C fragment: register i <-> query row
         // 8*(i/4) + 4*hi + i%4 of this wave's 32 rows.
-        if (BIAS && p.bias_sm == 0) {
+        if (BIAS && (KEY_BIAS || p.bias_sm == 0)) {
             // the per-key ("vector") form: one value per key and head, fetched when the head changes
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[i] = fmaf(s[i], p.scale, bias_key);

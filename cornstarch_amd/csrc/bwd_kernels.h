@@ -125,7 +125,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
     constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
     static_assert(!(SORTED && LONG), "no plan for so many rows");
-    constexpr bool NARROW = false, DEEP = DKDV_DEEP<D, MODE, LONG>;
+    constexpr bool NARROW = false, KEY_BIAS = false, DEEP = DKDV_DEEP<D, MODE, LONG>;
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 template <typename T, int D, int MODE, bool BIAS, bool SCALED>
 __global__ __launch_bounds__(DKDV_NARROW_THREADS, 3) void bwd_dkdv_narrow_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = false, SORTED = false, ROW_POS = IDX, LONG = false, SAVE = false;
-    constexpr bool NARROW = true, DEEP = false;
+    constexpr bool NARROW = true, KEY_BIAS = false, DEEP = false;
     constexpr int NB = 2;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
@@ -192,6 +192,7 @@ template <typename T, int D, int MODE, bool BIAS, bool SCALED>
 __device__ __forceinline__ void dkdv_work(const AttnParams& p, const int block, DkdvShared<D, MODE>& sh) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, ROW_POS = IDX;
     constexpr bool NARROW = false, SORTED = false, LONG = false, SAVE = false;
+    constexpr bool KEY_BIAS = BIAS;  // (both_in_one_launch refuses a bias with rows of its own)
     constexpr bool DEEP = DKDV_DEEP<D, MODE, LONG>;
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
