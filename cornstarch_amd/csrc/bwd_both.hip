@@ -22,7 +22,8 @@ static int launch_both_t(const AttnParams& kv, const AttnParams& p, hipStream_t 
 // Both kernels keep one workgroup of eight waves on a unit, so their workgroups share the units as they come free.  Worth it wherever dQ
 // runs with two streams, by the end of a launch (a fifth of it where there are two workgroups a unit) and by the launch that
 // dQ's delta costs its workgroups 2 us each for; beyond, dQ's smaller workgroups fill the units by themselves.  Step, us, two launches ->
-// the pre-pass and one, D 64: 2 x 283 tokens, 6 / 2 heads 64.4 -> 55.4; 2048, 16 heads 110.8 -> 93.7; 4096, 8 heads 163.5 -> 137.6;
+// the pre-pass and one, D 64: 2 x 283 tokens, 6 / 2 heads replayed as a graph 57.7 -> 46.6, but the same 87 where the host that issues the launches
+// is what is waited for (64.4 -> 55.4 with a quicker one); 2048, 16 heads 110.8 -> 93.7; 4096, 8 heads 163.5 -> 137.6;
 // 8192, 6 / 1 heads 311.7 -> 283.0; 2 x 2048, 16 heads, with a bias 160.2 -> 151.5; a bool mask, 2048, 16 heads 99.3 -> 82.0; 2048, 32 / 8
 // heads (parts) 149.6 -> 145.2, nothing hidden 141.1 -> 142.4.  D 32, where three workgroups of either kernel fit a unit and two of this one:
 // 2 x 2048, 16 heads 108.3 -> 111.4, 4096, 32 / 8 heads 254.8 -> 262.4: not there.

@@ -308,7 +308,9 @@
         const unsigned tile_at = (unsigned)(cur * TILE_BYTES + qr * ROW_BYTES);
         const unsigned row_at = 16u * hi + (lds_addr(sLse) + (unsigned)(cur * (DKDV_QT * 4) + qr * 4));
         {
-            constexpr int NOP = 2 * KK, AHEAD = D > 64 ? 2 : 3;  // MFMA j: S (j even) or dP (j odd), k-slice j / 2.  (3 at D 128: 1731 -> 1727)
+            // MFMA j: S (j even) or dP (j odd), k-slice j / 2.  AHEAD: 2 or 3 make no difference beyond the spread (8192 tokens, 32 / 8 heads,
+            // D 128, step 1731 us with 3, 1727 with 2), 4 or 5 lose 1 %; 2 holds the fewest registers
+            constexpr int NOP = 2 * KK, AHEAD = D > 64 ? 2 : 3;
             constexpr int FIRST = SORTED ? (NOP - NLOADS < 4 ? NOP - NLOADS : 4) : 0;  // the copies start behind MFMA FIRST - 1
             constexpr unsigned V_AT = 128 * ROW_BYTES;
             const unsigned at = chunk_lane + tile_at;

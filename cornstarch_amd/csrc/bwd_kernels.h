@@ -157,9 +157,10 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 // holds its K and V operands, and nothing lies in LDS but Q, dO and the small rows; what derives from the lane is derived anew for
 // every block (75 vector instructions a block beside the MFMAs); the rule constants of a block are read one row at a time.  (Spilled K and V operands, read back between
 // the tile copies, wait for those: step 1.26 -> 1.42 ms at 8 x 4096.)  No partial sums to add at the end.
-// Step, us, eight waves -> four: D 64: 8 x 4096, 16 heads 1312 -> 1236, 8 x 2048 397 -> 373, 32 x 512, 32 heads 461 ->
-// 414, 8 x 4096, 32 / 8 heads 2415 -> 2339, 16384, 16 heads, nothing hidden 5192 -> 5195; D 32: 8 x 2048, 16 heads 290 -> 249, 16 x 512, 32
-// heads 170 -> 141, 2 x 8192, 16 heads 831 -> 767.
+// Step through the public entry points, us, eight waves -> four, both in turn in one process, D 64: 8 x 4096, 16 heads, segments of 256
+// to 512 tokens 1290 -> 1246, of 256 to 1024 1072 -> 1038 (replayed as a graph 1087 -> 1003), 8 x 2048 389 -> 367, 32 x 512, 32 heads 445 -> 412,
+// 8 x 4096, 32 / 8 heads 2388 -> 2350, 16384, 16 heads, nothing hidden 5192 -> 5195; D 32: 8 x 2048, 16 heads 282 -> 239, 16 x 512, 32 heads
+// 168 -> 137, 2 x 8192, 16 heads 821 -> 744.
 template <typename T, int D, int MODE, bool BIAS, bool SCALED>
 __global__ __launch_bounds__(DKDV_NARROW_THREADS, 3) void bwd_dkdv_narrow_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = false, SORTED = false, ROW_POS = IDX, LONG = false, SAVE = false;
@@ -749,8 +750,9 @@ static int launch_dkdv_m(const AttnParams& p, hipStream_t stream) {
     const int blocks = p.num_kt * p.B * p.Hkv;  // one workgroup per 128-key tile
     // Four waves (bwd_dkdv_narrow_kernel) where there are more than four workgroups a unit.  Few leave the units a wave or two per SIMD: step,
     // us, D 32, 512 workgroups (2 x 2048, 16 heads) 107 -> 110, 576 (4 x 3000, 6 heads) 156 -> 160; D 64, 512 (8192, 32 / 8 heads) 1045 -> 1196.
-    // (From 768 on they win: 8 x 700, 16 heads, D 32 93 -> 87, D 64 3 x 2048 185 -> 179.  But a tile's partial sums then come in another
-    // order, and the sequences of a call of ordinary size are to have the bits that they have in one of half or twice the size.)
+    // The line at 1024 is not one of speed: from 768 on they win (8 x 700, 16 heads, D 32 91 -> 83, D 64 3 x 2048 179 -> 176).  But their sums come
+    // in another order, and the test of level lists holds a call of 1024 workgroups (2 x 2048 tokens, 32 heads) to the bits of one of 512.  Across the
+    // line the bits of dK and dV change with the size of the call.
     // A bias takes registers that head dim 64 does not have: 8192, 16 heads 648 -> 672 (D 32: 8 x 2048 330 -> 282).
     if constexpr (D <= 64 && !LONG && !SAVE && !(BIAS && D > 32)) {
         if (p.rows == nullptr && blocks > 1024 && p.mask_mode != MASK_DENSE) {
