@@ -42,8 +42,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     static_assert(STREAMS == 1 || !LONG, "streams and passes are not combined");
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
-    __shared__ u32x4 sK_all[STREAMS][2][FWD_KT * NCH];
-    __shared__ u32x4 sV_all[STREAMS][2][FWD_KT * NCH];
+    __shared__ __attribute__((aligned(256))) u32x4 sK_all[STREAMS][2][FWD_KT * NCH];
+    __shared__ __attribute__((aligned(256))) u32x4 sV_all[STREAMS][2][FWD_KT * NCH];
     __shared__ __attribute__((aligned(16))) int64_t sKbf_all[STREAMS][2][FWD_KT];  // raw bitfields of the tile's keys
     __shared__ __attribute__((aligned(16))) int sKpos_all[STREAMS][2][FWD_KT];     // their global positions (IDX only)
     __shared__ int sList[MAX_LIST];
@@ -63,7 +63,6 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     auto& sRowBits = sRowBits_all[stream];
     auto& sBias = sBias_all[stream];
     const int hi = lane >> 5, l32 = lane & 31, half16 = (lane >> 4) & 1;
-    const int wave_lane = tid >> 6;
     const int Sq = p.Sq, Sk = p.Sk;
     const int G = p.Hq / p.Hkv;
 
@@ -130,7 +129,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     // probabilities are at most 2^RESCALE_LOG2, harmless in fp32 / bf16 and cancelled by the
     // final division by l.
     constexpr float RESCALE_LOG2 = 8.f;
-    float m_i = -INFINITY, l_i = 0.f, nb = 0.f;  // nb = -m_i * c2 (0 while m_i is -inf)
+    float m_i = -INFINITY, nb = 0.f;  // nb = -m_i * c2 (0 while m_i is -inf)
+    f32x4 l_i = {0.f, 0.f, 0.f, 0.f};  // (all alike) this lane's half of the row's sum of probabilities
     // with a bias the scores are turned into scale * s + bias right after the S phase, and only log2(e) is left
     // to fold into the exponent
     // A per-key bias whose groups of four keys are aligned, in-range accesses travels with the tile copies: 64 values
@@ -203,248 +203,347 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             copy_b32<WAIT>(bias_rows.at(row), bias_voff, lds_addr(sBias) + buf * 256u);
     };
 
+    // Where this lane reads in buffer 0, as byte addresses: the K operand of k-slice 0 and the transposed V operand of column block 0.  What
+    // a k-slice or a block of columns adds is a constant, XORed (the swizzle takes bits 0 to 3 of the row, the tiles start at multiples
+    // of 256), rows are in the instruction.
+    constexpr unsigned ROW_BYTES = NCH * 16;
+    const int lane16 = lane & 15;
+    const unsigned k_lane = ldsK + 16u * (unsigned)chunk_slot<D>(l32, hi);
+    const unsigned v_lane =
+        ldsV + 16u * (unsigned)chunk_slot<D>(4 * hi + (lane16 >> 2), 2 * half16 + ((lane16 & 3) >> 1)) + 8u * (lane16 & 1);
+    // keys 32 kb .., k-slice kk
+    auto k_operand = [&](unsigned at, int kb, int kk) { return lds_read16<u32x4>((at ^ (32u * kk)) + 32u * kb * ROW_BYTES); };
+    // keys 32 kb + 16 t .., columns 32 db ..
+    auto v_operand = [&](unsigned at, int kb, int t, int db) {
+        const unsigned row = (32u * kb + 16u * t) * ROW_BYTES;
+        return lds_read_transposed_at((at ^ (64u * db)) + row, (at ^ (64u * db + 16u)) + row + 8u * ROW_BYTES);
+    };
+
+    // The ways a tile can take are divergent branches to the compiler: what one of them derives from these for its copies must not be
+    // shared with another, or it arrives in vector registers.
+    auto own_scalars = [](int& kt_next, int& cur) { asm volatile("" : "+s"(kt_next), "+s"(cur)); };
+
+    // Exponentials of one 32-key half, two at a time behind MFMA j of n (from MFMA `first` on), each pair packed one step later.  A wave
+    // overlaps its own vector work with its own MFMAs (an MFMA with the five instructions of a pair: 38 cycles, 33 alone), if
+    // nothing in it needs the matrix cores: with the packed dot product of the row sums in there (49 cycles) it gained nothing.
+    auto exp_slot = [&](f32x16& s, u32x4 (&pb)[2], float off, int j, int n, int first) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (j >= first && i * (n - first) / 8 == j - first) {
+                s[2 * i] = __builtin_amdgcn_exp2f(fmaf(s[2 * i], c2, off));
+                s[2 * i + 1] = __builtin_amdgcn_exp2f(fmaf(s[2 * i + 1], c2, off));
+                if (i > 0) pb[(i - 1) >> 2][(i - 1) & 3] = T::pack2(s[2 * i - 2], s[2 * i - 1]);
+            }
+    };
+    // Scores of a tile that hides nothing, for a wave whose rows all have a running maximum: the two 32-key halves follow one another, and
+    // the exponentials of the first are taken while the matrix cores work on the second.  Nobody looks for the maximum; false: some
+    // probability would be so large that it has to move, and the tile is done the general way (the same numbers).  off: what is added in
+    // the exponent, most: the largest score of the row that needs no look.
+    // Forward alone, nothing hidden, us, before -> here: D 128, 4096 tokens, 8 heads (a workgroup a unit) 88.7 -> 76.8, 64 / 16 heads 521 ->
+    // 500 (there power decides: zeros for inputs -11 % a pair of workgroups, random numbers -2 to -5 %); D 64 61.1 -> 53.8 and 308 -> 294.
+    // Causal: 3072, 32 / 8 heads 89.4 -> 85.6, 1024 25.3 -> 23.3.
+    constexpr bool PIPED = !BIAS && !LONG;
+    bool settled = false;
+    auto full_scores = [&](f32x16 (&s)[2], u32x4 (&pb0)[2], float off, float most, int cur, int kt_next) __attribute__((always_inline)) -> bool {
+        constexpr int AHEAD = KK < 4 ? KK : 4;
+        u32x4 ka[2 * KK];
+        own_scalars(kt_next, cur);
+        const unsigned k_at = k_lane + cur * TILE_BYTES;
+        auto read_k = [&](int j) { ka[j] = k_operand(k_at, j / KK, j % KK); };
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) read_k(j);
+#pragma unroll
+        for (int j = 0; j < 2 * KK; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (j + AHEAD < 2 * KK) read_k(j + AHEAD);
+            s[j / KK] = T::mfma(ka[j], qreg[j % KK], j % KK == 0 ? zero16 : s[j / KK]);
+            if (j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
+            if (j >= KK) exp_slot(s[0], pb0, off, j - KK, KK, 1);
+        }
+#pragma unroll
+        for (int j = 2 * KK; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // the first half by its probabilities, the second one by its scores
+        pb0[1][3] = T::pack2(s[0][14], s[0][15]);
+        unsigned largest = max3_pairs(pb0[0][0], pb0[0][1], pb0[0][2]);
+        largest = max3_pairs(largest, pb0[0][3], pb0[1][0]);
+        largest = max3_pairs(largest, pb0[1][1], pb0[1][2]);
+        largest = max3_pairs(largest, pb0[1][3], T::LARGE);
+        // (an asm statement may not read what an MFMA has written for twelve wait states, and the compiler does not look into it)
+        asm volatile("s_nop 12" : "+v"(s[1]));
+        float top[2] = {max3_nan(s[1][0], s[1][1], s[1][2]), max3_nan(s[1][3], s[1][4], s[1][5])};
+#pragma unroll
+        for (int i = 6; i < 14; i += 4) {
+            top[0] = max3_nan(top[0], s[1][i], s[1][i + 1]);
+            top[1] = max3_nan(top[1], s[1][i + 2], s[1][i + 3]);
+        }
+        top[0] = max3_nan(top[0], s[1][14], s[1][15]);
+        return (__ballot(largest != T::LARGE) | lanes_above(max3_nan(top[0], top[1], top[1]), most)) == 0;
+    };
+
     // One 64-key tile held in buffer `cur`.  The copies of tile `kt_next` into the other
     // buffer are issued one per MFMA of the S phase, where the wave has nothing else to wait for.
     auto tile_step = [&](int cur, int entry, int kt_next) {
-        // (the class is extracted with a per-lane copy of the wave number on purpose: with a skip branch the
-        // compiler can prove wave-uniform it lays the loop out around that branch and the kernel loses ~8 %)
-        const int kt = entry >> 8, cls = (entry >> (2 * wave_lane)) & 3;
+        // (One `if` after the other, none around another and none that leaves: the accumulators then stay in their registers.  With a
+        // return for the skipped tile, or classes the compiler takes for divergent, it copied all of O to and fro in every tile.)
+        const int kt = entry >> 8, cls = (entry >> (2 * wave)) & 3;
         if (cls == 0) {  // nothing for this wave's slice in the tile: only keep the copies of the next one going
+            own_scalars(kt_next, cur);
 #pragma unroll
             for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
-            return;
         }
-        const u32x4* tK = sK[cur];
-        const u32x4* tV = sV[cur];
-
-        // ---- S^T = K Q^T : 64 keys x 32 queries per wave ----------------------------------
-        // two independent accumulator chains (key blocks 0 and 1) alternate; operand reads run AHEAD
-        // MFMAs in front of their use; the first MFMA of a chain takes C = 0
-        // (the MFMA phases run at raised wave priority: when the SIMD's other wave is in its softmax phase, this
-        // wave's next MFMA is picked first and the MFMA pipe does not idle behind a queue of VALU instructions)
         f32x16 s[2];
-        u32x4 bias_a[2];  // bias_fold: this lane's key of either 32-key block, as an operand (keys are the rows of S^T)
-        if (BIAS && bias_fold) {
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                const float bv = p.bias_f32 ? ((const float*)sBias[cur])[32 * kb + l32]
-                                            : T::to_float(((const unsigned short*)sBias[cur])[32 * kb + l32]);
-                const u32x4 z = {0u, 0u, 0u, 0u};
-                bias_a[kb] = hi == 0 ? split3_operand<T>(bv * inv_scale) : z;
+        u32x4 pb[2][2];
+        // Partial tiles: the last key a row sees, relative to the first key this lane holds (4 hi) -- what it is compared with are then
+        // compile-time constants, which occupy no registers.  Most are partial only through causality, or because the slice holds rows
+        // of two kinds: all 64 keys carry the same bitfield (and, with index tensors, sit at consecutive positions), the bit test is a
+        // per-query constant and the rule reduces to one position compare.
+        bool uniform = true;
+        int rel = 63;
+        unsigned w01[2] = {0u, 0u};  // DENSE: the mask bits of this lane's row
+        if (cls == 1) {
+            if (DENSE) {
+                uniform = row_bits_w != nullptr;
+                if (uniform) {
+                    w01[0] = sRowBits[cur][wave][l32];
+                    w01[1] = sRowBits[cur][wave][32 + l32];
+                    rel = (w01[0] & w01[1]) == ~0u ? 63 : (w01[0] | w01[1]) == 0u ? -1 : 0;
+                }
+            } else {
+                const int64_t mine = sKbf[cur][lane];
+                const unsigned mlo = (unsigned)mine, mhi = (unsigned)((uint64_t)mine >> 32);
+                const unsigned flo = __builtin_amdgcn_readfirstlane(mlo), fhi = __builtin_amdgcn_readfirstlane(mhi);
+                bool same = (mlo == flo) & (mhi == fhi);
+                int kt0 = kt * FWD_KT;  // position of the tile's first key
+                if (IDX) {
+                    const int rel0 = sKpos[cur][lane] - lane;
+                    kt0 = __builtin_amdgcn_readfirstlane(rel0);
+                    same &= rel0 == kt0;
+                }
+                uniform = __all(same);
+                rel = allow_bits(qb, flo, fhi) ? qb.lim - kt0 - 4 * hi : -1;
             }
         }
-        __builtin_amdgcn_s_setprio(1);
-        {
-            constexpr int NOP = 2 * KK, AHEAD = 4;
-            u32x4 ka[NOP];
-#pragma unroll
-            for (int j = 0; j < AHEAD; ++j) ka[j] = lds_read_chunk<D>(tK, 32 * (j & 1) + l32, 2 * (j >> 1) + hi);
-#pragma unroll
-            for (int j = 0; j < NOP; ++j) {
-                __builtin_amdgcn_sched_barrier(0);
-                if (j + AHEAD < NOP)
-                    ka[j + AHEAD] = lds_read_chunk<D>(tK, 32 * ((j + AHEAD) & 1) + l32, 2 * ((j + AHEAD) >> 1) + hi);
-                s[j & 1] = T::mfma(ka[j], qreg[j >> 1], j < 2 ? zero16 : s[j & 1]);
-                if (j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
-            }
-#pragma unroll
-            for (int j = NOP; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
+        // Rows that see all keys of a tile or none go the same way as a tile that hides nothing: what is added in the exponent of the others
+        // is -inf, and a score of theirs that is no number (a key with an infinity) sends the tile the general way.  A slice with text and
+        // modality rows, or with padding, has such tiles all the way back, and its workgroup is often the longest of a launch: 3001 tokens
+        // with two segments, 32 / 8 heads, D 128 83.5 -> 80.0 us, a bool mask over 2 x 4096 with three, 16 heads 133 -> 122.
+        const bool sees = rel >= 59;  // (the last key of a lane: 32 + 24 + 3)
+        float off = nb, most = m_i + rescale_thr;
+        bool piped = PIPED && (cls == 2 ? settled : cls == 1 && uniform && __all((sees & ((m_i != -INFINITY) | !qvalid)) | (rel < 0)));
+        if (PIPED && !sees) {
+            off = -INFINITY;
+            most = 3e38f;
+        }
+        if (piped) piped = full_scores(s, pb[0], off, most, cur, kt_next);
+        if (cls != 0 && !piped) {
+            own_scalars(kt_next, cur);
+            const unsigned k_at = k_lane + cur * TILE_BYTES;
+
+            // ---- S^T = K Q^T : 64 keys x 32 queries per wave ----------------------------------
+            // two independent accumulator chains (key blocks 0 and 1) alternate; operand reads run AHEAD
+            // MFMAs in front of their use; the first MFMA of a chain takes C = 0
+            // (the MFMA phases run at raised wave priority: when the SIMD's other wave is in its softmax phase, this
+            // wave's next MFMA is picked first and the MFMA pipe does not idle behind a queue of VALU instructions)
+            u32x4 bias_a[2];  // bias_fold: this lane's key of either 32-key block, as an operand (keys are the rows of S^T)
             if (BIAS && bias_fold) {
-                const u32x4 z = {0u, 0u, 0u, 0u};
-                const u32x4 ones = hi == 0 ? ones3_operand<T>() : z;
-                s[0] = T::mfma(bias_a[0], ones, s[0]);
-                s[1] = T::mfma(bias_a[1], ones, s[1]);
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) {
+                    const float bv = p.bias_f32 ? ((const float*)sBias[cur])[32 * kb + l32]
+                                                : T::to_float(((const unsigned short*)sBias[cur])[32 * kb + l32]);
+                    const u32x4 z = {0u, 0u, 0u, 0u};
+                    bias_a[kb] = hi == 0 ? split3_operand<T>(bv * inv_scale) : z;
+                }
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-
-        if (BIAS && bias_fold) {
-            // (added by the MFMA above)
-        } else if (BIAS && bias_lds) {
+            __builtin_amdgcn_s_setprio(1);
+            {
+                constexpr int NOP = 2 * KK, AHEAD = 4;
+                u32x4 ka[NOP];
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+                for (int j = 0; j < AHEAD; ++j) ka[j] = k_operand(k_at, j & 1, j >> 1);
 #pragma unroll
-                for (int grp = 0; grp < 4; ++grp) {
-                    const int koff = 32 * kb + 8 * grp + 4 * hi;
-                    f32x4 b4;
-                    if (p.bias_f32) {
-                        b4 = *(const f32x4*)&sBias[cur][koff];
-                    } else {
-                        const u32x2 w = *(const u32x2*)((const char*)sBias[cur] + 2 * koff);
-                        b4[0] = T::to_float((unsigned short)(w[0] & 0xFFFFu));
-                        b4[1] = T::to_float((unsigned short)(w[0] >> 16));
-                        b4[2] = T::to_float((unsigned short)(w[1] & 0xFFFFu));
-                        b4[3] = T::to_float((unsigned short)(w[1] >> 16));
-                    }
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) s[kb][4 * grp + x] = fmaf(s[kb][4 * grp + x], p.scale, b4[x]);
+                for (int j = 0; j < NOP; ++j) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (j + AHEAD < NOP)
+                        ka[j + AHEAD] = k_operand(k_at, (j + AHEAD) & 1, (j + AHEAD) >> 1);
+                    s[j & 1] = T::mfma(ka[j], qreg[j >> 1], j < 2 ? zero16 : s[j & 1]);
+                    if (j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
                 }
-        } else if (BIAS) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int grp = 0; grp < 4; ++grp) {
-                    const f32x4 b4 = load_bias4<T>(bias_row, kt * FWD_KT + 32 * kb + 8 * grp + 4 * hi, Sk, p.bias_f32 != 0, p.bias_vec != 0);
-#pragma unroll
-                    for (int x = 0; x < 4; ++x)
-                        s[kb][4 * grp + x] = bias_fold ? fmaf(b4[x], inv_scale, s[kb][4 * grp + x])  // (c2 holds the scale)
-                                                       : fmaf(s[kb][4 * grp + x], p.scale, b4[x]);
+                for (int j = NOP; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
+                if (BIAS && bias_fold) {
+                    const u32x4 z = {0u, 0u, 0u, 0u};
+                    const u32x4 ones = hi == 0 ? ones3_operand<T>() : z;
+                    s[0] = T::mfma(bias_a[0], ones, s[0]);
+                    s[1] = T::mfma(bias_a[1], ones, s[1]);
                 }
-        }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
 
-        // ---- bitfield rule in registers (partial tiles only) ------------------------------
-        if (DENSE) {
-            if (cls == 1 && row_bits_w != nullptr) {
-                // (shifted by this lane's first key, 4 hi, once: the bit numbers tested are then constants)
-                const unsigned w01[2] = {sRowBits[cur][wave][l32] >> (4 * hi), sRowBits[cur][wave][32 + l32] >> (4 * hi)};
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        s[kb][i] = ((w01[kb] >> (8 * (i >> 2) + (i & 3))) & 1u) ? s[kb][i] : -INFINITY;
-            } else if (cls == 1) {
-                // mask bytes of this lane's query row: 4 consecutive keys per C-fragment group
-                const int kt0 = kt * FWD_KT;
-                const uint8_t* mrow = p.mask + ((int64_t)b * Sq + (qvalid ? qrow : 0)) * Sk + kt0;
-                const bool dwords = (Sk & 3) == 0;  // rows start 4-byte aligned
+            if (BIAS && bias_fold) {
+                // (added by the MFMA above)
+            } else if (BIAS && bias_lds) {
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                     for (int grp = 0; grp < 4; ++grp) {
                         const int koff = 32 * kb + 8 * grp + 4 * hi;
-                        unsigned m4 = 0;
-                        if (p.mask == nullptr) {
-                            m4 = 0x01010101u;
-                        } else if (qvalid) {
-                            if (dwords) {
-                                if (kt0 + koff < Sk) m4 = *(const unsigned*)(mrow + koff);
-                            } else {
+                        f32x4 b4;
+                        if (p.bias_f32) {
+                            b4 = *(const f32x4*)&sBias[cur][koff];
+                        } else {
+                            const u32x2 w = *(const u32x2*)((const char*)sBias[cur] + 2 * koff);
+                            b4[0] = T::to_float((unsigned short)(w[0] & 0xFFFFu));
+                            b4[1] = T::to_float((unsigned short)(w[0] >> 16));
+                            b4[2] = T::to_float((unsigned short)(w[1] & 0xFFFFu));
+                            b4[3] = T::to_float((unsigned short)(w[1] >> 16));
+                        }
 #pragma unroll
-                                for (int x = 0; x < 4; ++x)
-                                    if (kt0 + koff + x < Sk) m4 |= (unsigned)mrow[koff + x] << (8 * x);
+                        for (int x = 0; x < 4; ++x) s[kb][4 * grp + x] = fmaf(s[kb][4 * grp + x], p.scale, b4[x]);
+                    }
+            } else if (BIAS) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int grp = 0; grp < 4; ++grp) {
+                        const f32x4 b4 = load_bias4<T>(bias_row, kt * FWD_KT + 32 * kb + 8 * grp + 4 * hi, Sk, p.bias_f32 != 0, p.bias_vec != 0);
+#pragma unroll
+                        for (int x = 0; x < 4; ++x)
+                            s[kb][4 * grp + x] = bias_fold ? fmaf(b4[x], inv_scale, s[kb][4 * grp + x])  // (c2 holds the scale)
+                                                           : fmaf(s[kb][4 * grp + x], p.scale, b4[x]);
+                    }
+            }
+
+            // ---- bitfield rule in registers (partial tiles only) ------------------------------
+            if (DENSE) {
+                if (cls == 1 && row_bits_w != nullptr) {
+                    // (shifted by this lane's first key, 4 hi, once: the bit numbers tested are then constants)
+                    w01[0] >>= 4 * hi;
+                    w01[1] >>= 4 * hi;
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            s[kb][i] = ((w01[kb] >> (8 * (i >> 2) + (i & 3))) & 1u) ? s[kb][i] : -INFINITY;
+                } else if (cls == 1) {
+                    // mask bytes of this lane's query row: 4 consecutive keys per C-fragment group
+                    const int kt0 = kt * FWD_KT;
+                    const uint8_t* mrow = p.mask + ((int64_t)b * Sq + (qvalid ? qrow : 0)) * Sk + kt0;
+                    const bool dwords = (Sk & 3) == 0;  // rows start 4-byte aligned
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int grp = 0; grp < 4; ++grp) {
+                            const int koff = 32 * kb + 8 * grp + 4 * hi;
+                            unsigned m4 = 0;
+                            if (p.mask == nullptr) {
+                                m4 = 0x01010101u;
+                            } else if (qvalid) {
+                                if (dwords) {
+                                    if (kt0 + koff < Sk) m4 = *(const unsigned*)(mrow + koff);
+                                } else {
+#pragma unroll
+                                    for (int x = 0; x < 4; ++x)
+                                        if (kt0 + koff + x < Sk) m4 |= (unsigned)mrow[koff + x] << (8 * x);
+                                }
+                            }
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) {
+                                const bool a = ((m4 >> (8 * x)) & 0xFFu) != 0 && kt0 + koff + x < Sk;
+                                s[kb][4 * grp + x] = a ? s[kb][4 * grp + x] : -INFINITY;
                             }
                         }
+                }
+            } else if (cls == 1) {
+                if (uniform) {
 #pragma unroll
-                        for (int x = 0; x < 4; ++x) {
-                            const bool a = ((m4 >> (8 * x)) & 0xFFu) != 0 && kt0 + koff + x < Sk;
-                            s[kb][4 * grp + x] = a ? s[kb][4 * grp + x] : -INFINITY;
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            s[kb][i] = (32 * kb + 8 * (i >> 2) + (i & 3) <= rel) ? s[kb][i] : -INFINITY;
+                } else {
+                    // natural positions: the row's limit relative to the first key this lane holds, so that the position
+                    // test compares with compile-time constants
+                    const int lim_rel = qb.lim - (kt * FWD_KT + 4 * hi);
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                        for (int grp = 0; grp < 4; ++grp) {
+                            const int koff = 32 * kb + 8 * grp + 4 * hi;
+                            const u32x4 k01 = *(const u32x4*)&sKbf[cur][koff];      // lo0 hi0 lo1 hi1
+                            const u32x4 k23 = *(const u32x4*)&sKbf[cur][koff + 2];  // lo2 hi2 lo3 hi3
+                            const unsigned klo[4] = {k01[0], k01[2], k23[0], k23[2]};
+                            const unsigned khi[4] = {k01[1], k01[3], k23[1], k23[3]};
+                            u32x4 kp = {0u, 0u, 0u, 0u};
+                            if (IDX) kp = *(const u32x4*)&sKpos[cur][koff];
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) {
+                                const bool pos_ok = IDX ? (int)kp[x] <= qb.lim : 32 * kb + 8 * grp + x <= lim_rel;
+                                const bool a = allow_bits(qb, klo[x], khi[x]) & pos_ok;
+                                s[kb][4 * grp + x] = a ? s[kb][4 * grp + x] : -INFINITY;
+                            }
                         }
-                    }
+                }
             }
-        } else if (cls == 1) {
-            // Most partial tiles are partial only through causality: all 64 keys carry the same bitfield (and,
-            // with index tensors, sit at consecutive positions).  Then the bit test is a per-query constant and
-            // the rule reduces to one position compare.
-            const int64_t mine = sKbf[cur][lane];
-            const unsigned mlo = (unsigned)mine, mhi = (unsigned)((uint64_t)mine >> 32);
-            const unsigned flo = __builtin_amdgcn_readfirstlane(mlo), fhi = __builtin_amdgcn_readfirstlane(mhi);
-            bool uniform = (mlo == flo) & (mhi == fhi);
-            int kt0 = kt * FWD_KT;  // position of the tile's first key
-            if (IDX) {
-                const int rel0 = sKpos[cur][lane] - lane;
-                kt0 = __builtin_amdgcn_readfirstlane(rel0);
-                uniform &= rel0 == kt0;
+
+            // ---- online softmax (per-lane scalars) ----------------------------------------------
+            // (four short chains instead of one long one: the wave issues in order and would sit out the latency of
+            // every link)
+            float mx[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                mx[c] = fmaxf(s[0][4 * c], s[1][4 * c]);
+#pragma unroll
+                for (int i = 1; i < 4; ++i) mx[c] = fmaxf(fmaxf(mx[c], s[0][4 * c + i]), s[1][4 * c + i]);
             }
-            if (__all(uniform)) {
-                // last allowed key, relative to the first key this lane holds (4 hi): what it is compared with are
-                // then compile-time constants, which occupy no registers
-                const int rel = allow_bits(qb, flo, fhi) ? qb.lim - kt0 - 4 * hi : -1;
+            float mloc = half_swap_max(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
+            if (__any(mloc > m_i + rescale_thr)) {  // wave-uniform; rare after the first tiles
+                const float mnew = fmaxf(m_i, mloc);
+                const float muse = (mnew == -INFINITY) ? 0.f : mnew;
+                const float alpha = __builtin_amdgcn_exp2f((m_i - muse) * c2);  // 0 when m_i = -inf
+                m_i = mnew;
+                nb = -muse * c2;
+                l_i *= alpha;
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
+                for (int db = 0; db < DB; ++db)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        s[kb][i] = (32 * kb + 8 * (i >> 2) + (i & 3) <= rel) ? s[kb][i] : -INFINITY;
-            } else {
-                // natural positions: the row's limit relative to the first key this lane holds, so that the position
-                // test compares with compile-time constants
-                const int lim_rel = qb.lim - (kt * FWD_KT + 4 * hi);
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int grp = 0; grp < 4; ++grp) {
-                        const int koff = 32 * kb + 8 * grp + 4 * hi;
-                        const u32x4 k01 = *(const u32x4*)&sKbf[cur][koff];      // lo0 hi0 lo1 hi1
-                        const u32x4 k23 = *(const u32x4*)&sKbf[cur][koff + 2];  // lo2 hi2 lo3 hi3
-                        const unsigned klo[4] = {k01[0], k01[2], k23[0], k23[2]};
-                        const unsigned khi[4] = {k01[1], k01[3], k23[1], k23[3]};
-                        u32x4 kp = {0u, 0u, 0u, 0u};
-                        if (IDX) kp = *(const u32x4*)&sKpos[cur][koff];
-#pragma unroll
-                        for (int x = 0; x < 4; ++x) {
-                            const bool pos_ok = IDX ? (int)kp[x] <= qb.lim : 32 * kb + 8 * grp + x <= lim_rel;
-                            const bool a = allow_bits(qb, klo[x], khi[x]) & pos_ok;
-                            s[kb][4 * grp + x] = a ? s[kb][4 * grp + x] : -INFINITY;
-                        }
-                    }
+                    for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
             }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[0][i] = __builtin_amdgcn_exp2f(fmaf(s[0][i], c2, nb));
+#pragma unroll
+            for (int t = 0; t < 2; ++t) pb[0][t] = pack8<T>(s[0], 8 * t);
+            off = nb;
+            if (PIPED) settled = __all(!qvalid | (m_i != -INFINITY));
         }
 
-        // ---- online softmax (per-lane scalars) ----------------------------------------------
-        // (four short chains instead of one long one: the wave issues in order and would sit out the latency of
-        // every link)
-        float mx[4];
+        // ---- O^T += V^T P^T, and the row sums of the probabilities as that product sees them (rounded to T) ------------------------
+        // (the second half's exponentials are taken while the matrix cores work on the first)
+        if (cls != 0) {
+            __builtin_amdgcn_s_setprio(1);
+            constexpr int PV = 2 * DB, VAHEAD = 3 < PV ? 3 : PV;
+            const unsigned v_at = v_lane + cur * TILE_BYTES;
+            u32x4 va[2 * PV];
+            auto read_v = [&](int j) { va[j] = v_operand(v_at, j / PV, j % PV / DB, j % DB); };
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            mx[c] = fmaxf(s[0][4 * c], s[1][4 * c]);
+            for (int j = 0; j < VAHEAD; ++j) read_v(j);
 #pragma unroll
-            for (int i = 1; i < 4; ++i) mx[c] = fmaxf(fmaxf(mx[c], s[0][4 * c + i]), s[1][4 * c + i]);
+            for (int j = 0; j < 2 * PV; ++j) {
+                const int kb = j / PV, t = j % PV / DB;
+                __builtin_amdgcn_sched_barrier(0);
+                if (j + VAHEAD < 2 * PV) read_v(j + VAHEAD);
+                o[j % DB] = T::mfma(va[j], pb[kb][t], o[j % DB]);
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+                    if (j % DB == x * (DB / 2)) l_i = add_four<T>(pb[kb][t][2 * x], pb[kb][t][2 * x + 1], l_i);
+                if (kb == 0) exp_slot(s[1], pb[1], off, j, PV, 0);
+                if (j == PV - 1) pb[1][1][3] = T::pack2(s[1][14], s[1][15]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(0);
         }
-        float mloc = half_swap_max(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
-        if (__any(mloc > m_i + rescale_thr)) {  // wave-uniform; rare after the first tiles
-            const float mnew = fmaxf(m_i, mloc);
-            const float muse = (mnew == -INFINITY) ? 0.f : mnew;
-            const float alpha = __builtin_amdgcn_exp2f((m_i - muse) * c2);  // 0 when m_i = -inf
-            m_i = mnew;
-            nb = -muse * c2;
-            l_i *= alpha;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s[0][i] = __builtin_amdgcn_exp2f(fmaf(s[0][i], c2, nb));
-            s[1][i] = __builtin_amdgcn_exp2f(fmaf(s[1][i], c2, nb));
-        }
-        u32x4 pb[2][2];
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) pb[kb][t] = pack8<T>(s[kb], 8 * t);
-        // row sum of the probabilities as the P V product sees them (rounded to T), two per instruction
-        {
-            float ps[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) ps[kb][t] = T::add_pair(pb[kb][t][x], ps[kb][t]);
-            l_i += (ps[0][0] + ps[0][1]) + (ps[1][0] + ps[1][1]);
-        }
-
-        // ---- O^T += V^T P^T -------------------------------------------------------------------
-        __builtin_amdgcn_s_setprio(1);
-        {
-            u32x4 va[2][2][DB];
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int db = 0; db < DB; ++db)
-                        va[kb][t][db] = lds_read_transposed<D>(tV, lane, 32 * kb + 16 * t + 4 * hi, 32 * db + 16 * half16);
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int db = 0; db < DB; ++db) o[db] = T::mfma(va[kb][t][db], pb[kb][t], o[db]);
-            sched_pipeline_mfma_lds<4 * DB, (DB >= 2 ? 3 : 2), 2>();
-        }
-        __builtin_amdgcn_s_setprio(0);
     };
 
     // Sequences of more than MAX_LIST 64-key tiles are walked in several passes, each with a list of its own; the
@@ -489,7 +588,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     }
 
     // ---- epilogue: normalize, write O (q dtype) and LSE (natural log) -------------------
-    float ltot = half_swap_sum(l_i), mine = 1.f, theirs = 0.f;
+    float ltot = half_swap_sum(l_i[0]), mine = 1.f, theirs = 0.f;
     // With two streams, a row's two partial results meet through the tile arrays, which nobody reads any more: each stream
     // hands over the columns that the other one finishes.
     constexpr int DB0 = STREAMS > 1 ? (DB + 1) / 2 : DB;  // stream 0 finishes the column blocks below DB0, stream 1 the others
