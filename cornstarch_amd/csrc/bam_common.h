@@ -87,6 +87,11 @@ struct BF16 {
     static __device__ __forceinline__ f32x4 mfma4(const u32x2& a, const u32x2& b, const f32x4& c) {
         return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
     }
+    // acc + the two elements of a packed pair
+    static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), __builtin_bit_cast(bf16x2, ONES), acc, false);
+    }
     static constexpr unsigned ONES = 0x3F803F80u, LARGE = 0x43804380u;  // two values of 1, of 2^8
     static __device__ __forceinline__ unsigned pack2(float x, float y) {
         typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -107,6 +112,10 @@ struct F16 {
     }
     static __device__ __forceinline__ f32x4 mfma4(const u32x2& a, const u32x2& b, const f32x4& c) {
         return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), __builtin_bit_cast(f16x2, ONES), acc, false);
     }
     static constexpr unsigned ONES = 0x3C003C00u, LARGE = 0x5C005C00u;
     static __device__ __forceinline__ unsigned pack2(float x, float y) {

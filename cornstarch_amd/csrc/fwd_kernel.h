@@ -242,7 +242,11 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
     // Forward alone, nothing hidden, us, before -> here: D 128, 4096 tokens, 8 heads (a workgroup a unit) 88.7 -> 76.8, 64 / 16 heads 521 ->
     // 500 (there power decides: zeros for inputs -11 % a pair of workgroups, random numbers -2 to -5 %); D 64 61.1 -> 53.8 and 308 -> 294.
     // Causal: 3072, 32 / 8 heads 89.4 -> 85.6, 1024 25.3 -> 23.3.
-    constexpr bool PIPED = !BIAS && !LONG;
+    // Not at head dim 32, which has a third of the MFMAs for the same vector work and four waves a SIMD to fill gaps: 4096 tokens, nothing
+    // hidden, 8 heads 46.2 -> 50.0 us, 64 heads 204 -> 208.  Nor do its row sums go to the matrix cores or behind P V: 4 x 2048 tokens with three
+    // segments, 16 heads 45.1 us, as 4 x 4 MFMAs 47.5, as dot products behind the last MFMA 49 (text only 41.1, 42, 38.4), in front of the
+    // first, as here, 44.3 (40.3).
+    constexpr bool PIPED = !BIAS && !LONG && D > 32, SUM_MFMA = D > 32;
     bool settled = false;
     auto full_scores = [&](f32x16 (&s)[2], u32x4 (&pb0)[2], float off, float most, int cur, int kt_next) __attribute__((always_inline)) -> bool {
         constexpr int AHEAD = KK < 4 ? KK : 4;
@@ -302,7 +306,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         bool uniform = true;
         int rel = 63;
         unsigned w01[2] = {0u, 0u};  // DENSE: the mask bits of this lane's row
-        if (cls == 1) {
+        auto classify = [&]() __attribute__((always_inline)) {
             if (DENSE) {
                 uniform = row_bits_w != nullptr;
                 if (uniform) {
@@ -324,7 +328,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
                 uniform = __all(same);
                 rel = allow_bits(qb, flo, fhi) ? qb.lim - kt0 - 4 * hi : -1;
             }
-        }
+        };
+        if (PIPED && cls == 1) classify();
         // Rows that see all keys of a tile or none go the same way as a tile that hides nothing: what is added in the exponent of the others
         // is -inf, and a score of theirs that is no number (a key with an infinity) sends the tile the general way.  A slice with text and
         // modality rows, or with padding, has such tiles all the way back, and its workgroup is often the longest of a launch: 3001 tokens
@@ -417,6 +422,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             }
 
             // ---- bitfield rule in registers (partial tiles only) ------------------------------
+            if (!PIPED && cls == 1) classify();  // (not ahead of the scores, where nobody decides by it)
             if (DENSE) {
                 if (cls == 1 && row_bits_w != nullptr) {
                     // (shifted by this lane's first key, 4 hi, once: the bit numbers tested are then constants)
@@ -522,6 +528,18 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         // ---- O^T += V^T P^T, and the row sums of the probabilities as that product sees them (rounded to T) ------------------------
         // (the second half's exponentials are taken while the matrix cores work on the first)
         if (cls != 0) {
+            if (!SUM_MFMA) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[1][i] = __builtin_amdgcn_exp2f(fmaf(s[1][i], c2, off));
+#pragma unroll
+                for (int t = 0; t < 2; ++t) pb[1][t] = pack8<T>(s[1], 8 * t);
+                float sums[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) sums[c] = T::add_pair(pb[c >> 1][c & 1][x], sums[c]);
+                l_i[0] += (sums[0] + sums[1]) + (sums[2] + sums[3]);
+            }
             __builtin_amdgcn_s_setprio(1);
             constexpr int PV = 2 * DB, VAHEAD = 3 < PV ? 3 : PV;
             const unsigned v_at = v_lane + cur * TILE_BYTES;
@@ -537,9 +555,9 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
                 o[j % DB] = T::mfma(va[j], pb[kb][t], o[j % DB]);
 #pragma unroll
                 for (int x = 0; x < 2; ++x)
-                    if (j % DB == x * (DB / 2)) l_i = add_four<T>(pb[kb][t][2 * x], pb[kb][t][2 * x + 1], l_i);
-                if (kb == 0) exp_slot(s[1], pb[1], off, j, PV, 0);
-                if (j == PV - 1) pb[1][1][3] = T::pack2(s[1][14], s[1][15]);
+                    if (SUM_MFMA && j % DB == x * (DB / 2)) l_i = add_four<T>(pb[kb][t][2 * x], pb[kb][t][2 * x + 1], l_i);
+                if (SUM_MFMA && kb == 0) exp_slot(s[1], pb[1], off, j, PV, 0);
+                if (SUM_MFMA && j == PV - 1) pb[1][1][3] = T::pack2(s[1][14], s[1][15]);
             }
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_setprio(0);
