@@ -235,7 +235,7 @@ template <int D, int MODE, int BIAS_FORM, int STREAMS>
 struct DqShared {
     static constexpr int NCH = LDS_COLS<D> / 8;
     static constexpr bool DENSE = MODE == MASK_DENSE, bias_lds = BIAS_FORM == BIAS_TILES;
-    u32x4 k[STREAMS][2][DQ_KT * NCH];
+    __attribute__((aligned(256))) u32x4 k[STREAMS][2][DQ_KT * NCH];
     u32x4 v[STREAMS][2][DQ_KT * NCH];
     __attribute__((aligned(16))) int64_t kbf[STREAMS][2][DQ_KT];  // raw bitfields of the tile's keys
     __attribute__((aligned(16))) int kpos[STREAMS][2][DQ_KT];     // their global positions (MASK_INDEXED only)
@@ -349,10 +349,11 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
         build_key_tile_list<STREAMS>(ws, p.num_n, list_keys, lane, 0, first_classes, sList + stream * (MAX_LIST / 2), sCount + stream, !side);
     QueryBits qb = {};
     float lse2 = INFINITY;
-    // Head dim 32 has the registers (123 of 168) to start the dP chain from -delta, as dK/dV does: 16 of some 73 vector instructions a
-    // block less.  (At 64 they would have to be reloaded, 160 are taken.)  Step, us: 8 x 2048 tokens, 16 heads 249.0 -> 243.3, 2 x 8192 779
-    // -> 760, 1 x 2048 93.6 -> 92.7.
-    constexpr bool DELTA_FIRST = D <= 32;
+    // Up to head dim 64 there are registers (119 of 128 and 165 of 168) to start the dP chain from -delta, as dK/dV does: 16 of some 73
+    // vector instructions a block less.  Step, us, D 32: 8 x 2048 tokens, 16 heads 249.0 -> 243.3, 2 x 8192 779 -> 760, 1 x 2048 93.6 -> 92.7.
+    // D 64, since the LDS addresses are XORed (160 registers before): dQ of 8 x 4096, 16 heads 314 -> 299, with a bias, in one launch with
+    // dK/dV, 2 x 2048 89.7 -> 87.3.
+    constexpr bool DELTA_FIRST = D <= 64;
     f32x16 minus_delta;
     // With o given, this launch also is the delta pre-pass: it runs in front of the dK/dV kernel, has the rows of dO in
     // registers and covers every row once; a launch and a second reading of dO less (2 x 283 tokens: 3.4 us; 8 x 4096
@@ -449,6 +450,15 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
             copy_b32<WAIT>(bias_rows.at(row), bias_voff, lds_addr(sBias) + buf * 256u);
     };
 
+    // Where this lane reads in buffer 0, as byte addresses, as in the forward: the K operand of k-slice 0 (V: V_AT behind it) and the
+    // transposed K operand of column block 0.
+    constexpr unsigned ROW_BYTES = NCH * 16, V_AT = STREAMS * 2 * TILE_BYTES;
+    static_assert(alignof(decltype(sh)) % 256 == 0, "addresses below 256 are XORed");
+    const int lane16 = lane & 15;
+    const unsigned k_lane = ldsK + 16u * (unsigned)chunk_slot<D>(l32, hi);
+    const unsigned kt_lane =
+        ldsK + 16u * (unsigned)chunk_slot<D>(4 * hi + (lane16 >> 2), 2 * half16 + ((lane16 & 3) >> 1)) + 8u * (lane16 & 1);
+
     // One 64-key tile held in buffer `cur`; the copies of tile kt_next into the other buffer
     // are issued one per MFMA of the first S / dP block.
     auto tile_step = [&](int cur, int entry, int kt_next) {
@@ -460,8 +470,7 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
             for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
             return;
         }
-        const u32x4* tK = sK[cur];
-        const u32x4* tV = sV[cur];
+        const unsigned k_at = k_lane + cur * TILE_BYTES, kt_at = kt_lane + cur * TILE_BYTES;
         // partial tile whose 64 keys all carry the same bitfield: the rule is one position compare
         bool uniform_keys = false;
         int rel = 0;
@@ -494,13 +503,15 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
             {
                 constexpr int NOP = 2 * KK, AHEAD = 4;  // operand j: K chunk (j even) or V chunk (j odd) of k-slice j / 2
                 u32x4 a[NOP];
+                auto operand = [&](int j) {
+                    return lds_read16<u32x4>((k_at ^ (32u * (j >> 1))) + 32u * kb * ROW_BYTES + ((j & 1) ? V_AT : 0u));
+                };
 #pragma unroll
-                for (int j = 0; j < AHEAD; ++j) a[j] = lds_read_chunk<D>((j & 1) ? tV : tK, 32 * kb + l32, 2 * (j >> 1) + hi);
+                for (int j = 0; j < AHEAD; ++j) a[j] = operand(j);
 #pragma unroll
                 for (int j = 0; j < NOP; ++j) {
                     __builtin_amdgcn_sched_barrier(0);
-                    if (j + AHEAD < NOP)
-                        a[j + AHEAD] = lds_read_chunk<D>(((j + AHEAD) & 1) ? tV : tK, 32 * kb + l32, 2 * ((j + AHEAD) >> 1) + hi);
+                    if (j + AHEAD < NOP) a[j + AHEAD] = operand(j + AHEAD);
                     if (j & 1)
                         dp = T::mfma(a[j], greg[j >> 1], j < 2 ? (DELTA_FIRST ? minus_delta : zero16) : dp);
                     else
@@ -617,7 +628,8 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int db = 0; db < DB; ++db)
-                        ta[t][db] = lds_read_transposed<D>(tK, lane, 32 * kb + 16 * t + 4 * hi, 32 * db + 16 * half16);
+                        ta[t][db] = lds_read_transposed_at((kt_at ^ (64u * db)) + (32u * kb + 16u * t) * ROW_BYTES,
+                                                           (kt_at ^ (64u * db + 16u)) + (32u * kb + 16u * t + 8u) * ROW_BYTES);
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
