@@ -76,7 +76,8 @@ struct AttnParams {
     // Optional hand-over of dS from the dK/dV kernel to the dQ kernel (needs the plan; null = none).  ds_entry:
     // number of every (slice, 128-key tile) pair that has work, (B, 4 * num_m, num_kt) ints, -1 = none.  ds_ws: one
     // 8 KiB record per (q head, pair), record (h, e) at ((h * ds_capacity + e) * 8 KiB); inside it four 2 KiB blocks,
-    // one per 32-key group; a block holds, for each of its 32 keys, 32 values of -dS / scale in the input dtype.
+    // one per 32-key group; a block holds, for each of its 32 keys, 32 values of -dS / scale in the input dtype, in four chunks
+    // (bwd_dkdv_body.h: ds_first).
     const int* ds_entry;
     int64_t ds_entry_sb;
     const int* ds_tile_base;   // (B, num_kt): number of the first pair of each 128-key tile; the pairs of a tile are

@@ -267,8 +267,11 @@
     // condition the compiler can prove wave-uniform makes it restructure the loop around that branch, and the
     // result needs far more registers than a wave has.
     const int kg_lane = (tid >> 6) & 3;
-    // SAVE: where this lane's 32 bytes sit inside a 2 KiB block (key l32: 64 bytes, rows 4 hi + {0..3, 8..11, ...} first)
-    const unsigned ds_lane_off = (unsigned)(kg * 2048 + l32 * 64 + hi * 32);
+    // SAVE: where this lane's two chunks sit inside a 2 KiB block (key l32, rows 4 hi + {0..3, 8..11}, then those 16 further on, 1 KiB behind and
+    // four keys across): either store of the wave fills 1 KiB in one piece.  With a key's 64 bytes side by side each store filled every
+    // other 16 bytes: dK/dV alone, us, a causal mask, 8192 tokens, 32 / 8 heads, D 128 1149 -> 1137 (without any store 1012: what is left is the
+    // power that the writes take).  The keys change places in fours so that dQ's transposing reads spread over the LDS banks.
+    const unsigned ds_first = (unsigned)(kg * 2048 + hi * 512 + (l32 ^ (8 * hi)) * 16), ds_second = (ds_first ^ 64u) + 1024u;
     // SAVE: the pairs (slice, this key tile) that have work are numbered consecutively from ds_base, by ascending slice,
     // i.e. in the order of the slice list: pair number = ds_base + position in the list
     int ds_base = 0;
@@ -500,9 +503,9 @@
             // kernel, and should not push the Q / dO rows the other workgroups re-read out of L2
             const unsigned rec_no = (unsigned)__builtin_amdgcn_readfirstlane(h_cur * (int)p.ds_capacity + ds_e);
             const char* rec = (const char*)p.ds_ws + ((uint64_t)rec_no << 13);
-            asm volatile("global_store_dwordx4 %0, %1, %3 nt\n\tglobal_store_dwordx4 %0, %2, %3 offset:16 nt"
+            asm volatile("global_store_dwordx4 %0, %2, %4 nt\n\tglobal_store_dwordx4 %1, %3, %4 nt"
                          :
-                         : "v"(ds_lane_off), "v"(dsb[0]), "v"(dsb[1]), "s"(rec)
+                         : "v"(ds_first), "v"(ds_second), "v"(dsb[0]), "v"(dsb[1]), "s"(rec)
                          : "memory");
         }
         return SAVE;

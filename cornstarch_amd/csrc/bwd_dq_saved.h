@@ -50,30 +50,11 @@ __device__ __forceinline__ void build_key_half_list(const WaveSlices& ws, int nu
     wait_lds();
 }
 
-// Transposed MFMA operand out of a dS block: 32 keys x 32 columns of 2 bytes, 64 bytes per key, no swizzle.  The lane
-// gets column colbase16 + (lane & 15) of keys row0 + {0,1,2,3} and row0 + 8 + {0,1,2,3} (row0 includes 4 * hi).
-__device__ __forceinline__ u32x4 ds_block_read_transposed(const char* block, int lane, int row0, int colbase16) {
-    const int i = lane & 15;
-    const int col = colbase16 + 4 * (i & 3);
-    const int r_a = row0 + (i >> 2);
-    typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
-    const char* pa = block + r_a * 64 + col * 2;
-    s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(pa));
-    s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(pa + 8 * 64));
-    u32x2 ua = __builtin_bit_cast(u32x2, a), ub = __builtin_bit_cast(u32x2, b);
-    u32x4 r;
-    r[0] = ua[0];
-    r[1] = ua[1];
-    r[2] = ub[0];
-    r[3] = ub[1];
-    return r;
-}
-
 template <typename T, int D>
 __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const AttnParams p) {
     constexpr int NCH = LDS_COLS<D> / 8, DB = D / 32;
     __shared__ u32x4 sK[2][DQS_KT * NCH];
-    __shared__ u32x4 sDS[DQS_THREADS / 64][2][256];  // per wave and buffer: two 2 KiB blocks (key halves 0 and 1)
+    __shared__ __attribute__((aligned(256))) u32x4 sDS[DQS_THREADS / 64][2][256];  // per wave and buffer: two 2 KiB blocks (key halves 0 and 1)
     __shared__ int sList[MAX_LIST];
     __shared__ int sCount;
 
@@ -165,6 +146,11 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
         return issued;
     };
 
+    // Where this lane reads in the first block of buffer 0: column 16 half16 + (lane & 15) of keys 4 hi + {0,1,2,3}.  16 keys further are 256
+    // bytes, 8 keys a bit of the address.  (The layout: bwd_dkdv_body.h, ds_first.)
+    const int lane16 = lane & 15, upper = (lane16 >> 1) & 1;
+    const unsigned ds_lane = ldsDS + (unsigned)(upper * 1024 + half16 * 512 + ((4 * hi + (lane16 >> 2)) ^ (4 * upper) ^ (8 * half16)) * 16 + (lane16 & 1) * 8);
+
     // One 64-key tile.  The dS operands are read first; the wave's buffer is then free again and takes the blocks of
     // the tile after next (`entry2`, record `e2`; negative entry2 = nothing left), so that two tiles' worth of
     // workspace reads are in flight per wave: the kernel waits for HBM, not for the MFMAs.  Returns the number of
@@ -173,14 +159,17 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
         // (per-lane copy of the wave number: a skip branch the compiler can prove wave-uniform makes it restructure the loop)
         const int c = (entry >> (4 * wave_lane)) & 15;
         const u32x4* tK = sK[cur];
-        const char* tDS = (const char*)sDS[wave][cur];
+        const unsigned ds_at = ds_lane + cur * 4096u;
         u32x4 bop[2][2];
         if (c != 0) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
-                    if ((c >> (2 * kb)) & 3) bop[kb][t] = ds_block_read_transposed(tDS + kb * 2048, lane, 16 * t + 4 * hi, 16 * half16);
+                    if ((c >> (2 * kb)) & 3) {
+                        const unsigned x = ds_at + 2048u * kb + 256u * t;
+                        bop[kb][t] = lds_read_transposed_at(x, x ^ 128u);
+                    }
             wait_lds();  // the copies below overwrite what was just read
         }
         const int issued = entry2 >= 0 ? issue_ds(entry2, e2, cur) : 0;
