@@ -291,6 +291,8 @@
     // pos_cur, pos_nxt: the buffers of the tile's positions and of those that are copied now
     // qr: this wave's rows inside the 64-row tile.  NARROW: the caller issues the copies; what derives from the lane is derived anew for
     // every block (`own`), it would take the registers of the K and V operands otherwise
+    constexpr bool PH1 = D > 64 && !DENSE, PH2 = PH1;
+    constexpr bool KEY_ROW = BIAS && KEY_BIAS, BESIDE = PH1 && (!BIAS || KEY_BIAS), BESIDE2 = PH2;
     auto tile_step = [&](const int qr, int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int nxt, int pos_cur,
                          int pos_nxt) __attribute__((always_inline)) -> bool {
         if (cls == 0) {
@@ -311,33 +313,43 @@
         const unsigned tile_at = (unsigned)(cur * TILE_BYTES + qr * ROW_BYTES);
         const unsigned row_at = 16u * hi + (lds_addr(sLse) + (unsigned)(cur * (DKDV_QT * 4) + qr * 4));
         {
-            // MFMA j: S (j even) or dP (j odd), k-slice j / 2.  AHEAD: 2 or 3 make no difference beyond the spread (8192 tokens, 32 / 8 heads,
-            // D 128, step 1731 us with 3, 1727 with 2), 4 or 5 lose 1 %; 2 holds the fewest registers
             constexpr int NOP = 2 * KK, AHEAD = D > 64 ? 2 : 3;
             constexpr int FIRST = SORTED ? (NOP - NLOADS < 4 ? NOP - NLOADS : 4) : 0;  // the copies start behind MFMA FIRST - 1
             constexpr unsigned V_AT = 128 * ROW_BYTES;
             const unsigned at = chunk_lane + tile_at;
             u32x4 a[NOP], bb[NOP];
-            auto operand = [&](int j) { return lds_read16<u32x4>((at ^ (unsigned)(32 * (j >> 1))) + ((j & 1) ? DO_AT : 0u)); };
+            auto is_dp = [](int j) { return BESIDE ? j >= KK : (j & 1) != 0; };
+            auto slice = [](int j) { return BESIDE ? j % KK : j >> 1; };
+            auto operand = [&](int j) { return lds_read16<u32x4>((at ^ (unsigned)(32 * slice(j))) + (is_dp(j) ? DO_AT : 0u)); };
             auto kv = [&](int j) {
                 if constexpr (KV_REGS)
-                    return (j & 1) ? vfrag[j >> 1] : kfrag[j >> 1];
+                    return is_dp(j) ? vfrag[slice(j)] : kfrag[slice(j)];
                 else
-                    return lds_read16<u32x4>((kv_lane ^ (unsigned)(32 * (j >> 1))) + ((j & 1) ? V_AT : 0u));
+                    return lds_read16<u32x4>((kv_lane ^ (unsigned)(32 * slice(j))) + (is_dp(j) ? V_AT : 0u));
             };
-            a[0] = operand(0);
-            bb[0] = kv(0);
+            auto read_delta = [&]() {
 #pragma unroll
-            for (int grp = 0; grp < 4; ++grp) {
-                const f32x4 d4 = lds_read16<f32x4>(row_at + DELTA_AT + 32u * grp);
+                for (int grp = 0; grp < 4; ++grp) {
+                    const f32x4 d4 = lds_read16<f32x4>(row_at + DELTA_AT + 32u * grp);
 #pragma unroll
-                for (int x = 0; x < 4; ++x) dp[4 * grp + x] = d4[x];
-            }
+                    for (int x = 0; x < 4; ++x) dp[4 * grp + x] = d4[x];
+                }
+            };
+            f32x4 l4[4];
+            auto probability = [&](int i) {
+                if (BESIDE) s[i] = __builtin_amdgcn_exp2f(fmaf(KEY_ROW ? fmaf(s[i], p.scale, bias_key) : s[i], c2, SCALED ? -l4[i >> 2][i & 3] : l4[i >> 2][i & 3] * -LOG2E));
+            };
 #pragma unroll
-            for (int j = 1; j < AHEAD; ++j) {
+            for (int j = 0; j < AHEAD; ++j) {
                 a[j] = operand(j);
                 bb[j] = kv(j);
+                if (!BESIDE && j == 0) read_delta();
             }
+            // beside MFMA m of dP, from the second one on, and behind the last
+            auto probabilities = [&](int m) {
+#pragma unroll
+                for (int i = 16 * (m - 1) / KK; i < 16 * m / KK; ++i) probability(i);
+            };
 #pragma unroll
             for (int j = 0; j < NOP; ++j) {
                 __builtin_amdgcn_sched_barrier(0);
@@ -345,18 +357,29 @@
                     a[j + AHEAD] = operand(j + AHEAD);
                     bb[j + AHEAD] = kv(j + AHEAD);
                 }
-                if (j & 1)
+                if (BESIDE && j == KK - 2) read_delta();
+                if (is_dp(j))
                     dp = T::mfma(a[j], bb[j], dp);
                 else
-                    s = T::mfma(a[j], bb[j], j < 2 ? zero16 : s);
+                    s = T::mfma(a[j], bb[j], slice(j) == 0 ? zero16 : s);
+                if (BESIDE && j >= KK) {
+                    if (j - KK < 4 && KK >= 4) l4[(j - KK) & 3] = lds_read16<f32x4>(row_at + 32u * (j - KK));
+                    if (KK < 4) {
+                        l4[(2 * (j - KK)) & 3] = lds_read16<f32x4>(row_at + 64u * (j - KK));
+                        l4[(2 * (j - KK) + 1) & 3] = lds_read16<f32x4>(row_at + 64u * (j - KK) + 32u);
+                    }
+                    if (j > KK) probabilities(j - KK);
+                }
                 if (!NARROW && j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, nxt, pos_nxt);
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (BESIDE) probabilities(KK);
         }
         // ---- P = exp(scale s - lse) on allowed pairs, -dS/scale = P (delta - dP)   (the factor `-scale` of dS
         // is applied once to dK in the epilogue).  C fragment: register i <-> query row
         // 8*(i/4) + 4*hi + i%4 of this wave's 32 rows.
-        if (BIAS && (KEY_BIAS || p.bias_sm == 0)) {
+        if (BESIDE) {
+        } else if (BIAS && (KEY_BIAS || p.bias_sm == 0)) {
             // the per-key ("vector") form: one value per key and head, fetched when the head changes
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[i] = fmaf(s[i], p.scale, bias_key);
@@ -372,6 +395,7 @@
                 s[i] = fmaf(s[i], p.scale, bv);
             }
         }
+        if (!BESIDE)
 #pragma unroll
         for (int grp = 0; grp < 4; ++grp) {
             const f32x4 l4 = lds_read16<f32x4>(row_at + 32u * grp);
@@ -466,9 +490,49 @@
                 }
             }
         }
+        u32x4 pb[2], dsb[2];
+        if constexpr (BESIDE2)
+        // ---- dV^T += dO^T P ; dK^T += Q^T dS -------------------------------------------------
+        {
+            const unsigned at = transposed_lane + tile_at;
+            // MFMA j: 16 rows (j / 2 DB), dV then dK, block of columns j % DB
+            constexpr int N2 = 4 * DB, AHEAD2 = 2;
+            u32x4 tr[N2];
+            auto operand = [&](int j) {
+                const int t = j / (2 * DB), db = j % DB;
+                const unsigned x = (at ^ (64u * db)) + 16u * t * ROW_BYTES, y = (at ^ (64u * db + 16u)) + (16u * t + 8u) * ROW_BYTES;
+                const unsigned from = (j / DB) & 1 ? 0u : DO_AT;
+                return lds_read_transposed_at(x + from, y + from);
+            };
+#pragma unroll
+            for (int j = 0; j < AHEAD2; ++j) tr[j] = operand(j);
+            pb[0] = pack8<T>(s, 0);
+            // beside the MFMAs: step i = 0..3 of the gradients of 16 rows
+            auto grad = [&](int t, int w) {
+                const int i = 8 * t + 2 * w;
+                dp[i] *= s[i];  // -dS / scale
+                dp[i + 1] *= s[i + 1];
+                dsb[t][w] = T::pack2(dp[i], dp[i + 1]);
+                if (t == 0) pb[1][w] = T::pack2(s[8 + 2 * w], s[9 + 2 * w]);
+            };
+#pragma unroll
+            for (int j = 0; j < N2; ++j) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (j + AHEAD2 < N2) tr[j + AHEAD2] = operand(j + AHEAD2);
+                const int t = j / (2 * DB), db = j % DB;
+                if ((j / DB) & 1)
+                    dk[db] = T::mfma(tr[j], dsb[t], dk[db]);
+                else
+                    dv[db] = T::mfma(tr[j], pb[t], dv[db]);
+                if (j < 2 * DB)
+#pragma unroll
+                    for (int w = 4 * (j % DB) / DB; w < 4 * (j % DB + 1) / DB; ++w) grad(j / DB, w);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        else {
 #pragma unroll
         for (int i = 0; i < 16; ++i) dp[i] = s[i] * dp[i];  // -dS / scale
-        u32x4 pb[2], dsb[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             pb[t] = pack8<T>(s, 8 * t);
@@ -494,6 +558,7 @@
                     dk[db] = T::mfma(tq[t][db], dsb[t], dk[db]);
                 }
             sched_pipeline_mfma_lds<4 * DB, 4, 2>();
+        }
         }
         if (SAVE) {
             // Issued after the MFMAs of the tile (in front of them they cost the kernel 2 % more).  Record number and
