@@ -286,13 +286,19 @@
             asm volatile("" : "+v"(bias_key));  // arrives here, not at its first use between the tile copies
         }
     };
+    // BESIDE: the chain of S ends before that of dP begins, so that the exponentials are taken beside the MFMAs of dP, and the gradients of 16 rows
+    // beside the dV and dK products of the 16 before (a wave overlaps its own vector work with its own MFMAs).  It gives where a unit's eight
+    // waves do not fill each other's gaps all the time: step, us, D 128, both chains side by side -> one after the other: 4 x 1537 tokens, 32 / 8
+    // heads 312.3 -> 309.4, 2048, 8 heads 101.3 -> 100.5, 8192, 32 / 8 1580 -> 1576, 65536 41.99 -> 41.89 ms, D 96 2 x 2003 166.6 -> 166.1 (the products alone
+    // half of it, the chains alone -1.5 %).  Head dim 64 2 x 4096, 16 heads, a bias 375.8 -> 377.1, with four waves 1016 -> 1063 (168 registers are too few);
+    // a bool mask 461.5 -> 461.6, with spills.
+    constexpr bool KEY_ROW = BIAS && KEY_BIAS, BESIDE = D > 64 && !DENSE && (!BIAS || KEY_BIAS);
+
     // ds_pos: position of the wave's slice in the slice list.
     // returns true when the wave has issued its two dS stores (they may stay in flight over the end of the iteration)
     // pos_cur, pos_nxt: the buffers of the tile's positions and of those that are copied now
     // qr: this wave's rows inside the 64-row tile.  NARROW: the caller issues the copies; what derives from the lane is derived anew for
     // every block (`own`), it would take the registers of the K and V operands otherwise
-    constexpr bool PH1 = D > 64 && !DENSE, PH2 = PH1;
-    constexpr bool KEY_ROW = BIAS && KEY_BIAS, BESIDE = PH1 && (!BIAS || KEY_BIAS), BESIDE2 = PH2;
     auto tile_step = [&](const int qr, int cur, int cls, int h_cur, int myrow0, int ds_pos, const TileSource& next, int nxt, int pos_cur,
                          int pos_nxt) __attribute__((always_inline)) -> bool {
         if (cls == 0) {
@@ -335,9 +341,10 @@
                     for (int x = 0; x < 4; ++x) dp[4 * grp + x] = d4[x];
                 }
             };
+            static_assert(!BESIDE || (KK >= 4 && !SCALED), "the rows' lse is asked for by the first four MFMAs of dP");
             f32x4 l4[4];
             auto probability = [&](int i) {
-                if (BESIDE) s[i] = __builtin_amdgcn_exp2f(fmaf(KEY_ROW ? fmaf(s[i], p.scale, bias_key) : s[i], c2, SCALED ? -l4[i >> 2][i & 3] : l4[i >> 2][i & 3] * -LOG2E));
+                s[i] = __builtin_amdgcn_exp2f(fmaf(KEY_ROW ? fmaf(s[i], p.scale, bias_key) : s[i], c2, l4[i >> 2][i & 3] * -LOG2E));
             };
 #pragma unroll
             for (int j = 0; j < AHEAD; ++j) {
@@ -345,7 +352,7 @@
                 bb[j] = kv(j);
                 if (!BESIDE && j == 0) read_delta();
             }
-            // beside MFMA m of dP, from the second one on, and behind the last
+            // beside MFMA m of dP, from the second one on (S is there by then), and behind the last
             auto probabilities = [&](int m) {
 #pragma unroll
                 for (int i = 16 * (m - 1) / KK; i < 16 * m / KK; ++i) probability(i);
@@ -363,11 +370,7 @@
                 else
                     s = T::mfma(a[j], bb[j], slice(j) == 0 ? zero16 : s);
                 if (BESIDE && j >= KK) {
-                    if (j - KK < 4 && KK >= 4) l4[(j - KK) & 3] = lds_read16<f32x4>(row_at + 32u * (j - KK));
-                    if (KK < 4) {
-                        l4[(2 * (j - KK)) & 3] = lds_read16<f32x4>(row_at + 64u * (j - KK));
-                        l4[(2 * (j - KK) + 1) & 3] = lds_read16<f32x4>(row_at + 64u * (j - KK) + 32u);
-                    }
+                    if (j - KK < 4) l4[(j - KK) & 3] = lds_read16<f32x4>(row_at + 32u * (j - KK));
                     if (j > KK) probabilities(j - KK);
                 }
                 if (!NARROW && j >= FIRST && j - FIRST < NLOADS) issue_copy(j - FIRST, next, nxt, pos_nxt);
@@ -379,6 +382,7 @@
         // is applied once to dK in the epilogue).  C fragment: register i <-> query row
         // 8*(i/4) + 4*hi + i%4 of this wave's 32 rows.
         if (BESIDE) {
+            // (taken above)
         } else if (BIAS && (KEY_BIAS || p.bias_sm == 0)) {
             // the per-key ("vector") form: one value per key and head, fetched when the head changes
 #pragma unroll
@@ -395,12 +399,13 @@
                 s[i] = fmaf(s[i], p.scale, bv);
             }
         }
-        if (!BESIDE)
+        if (!BESIDE) {
 #pragma unroll
-        for (int grp = 0; grp < 4; ++grp) {
-            const f32x4 l4 = lds_read16<f32x4>(row_at + 32u * grp);
+            for (int grp = 0; grp < 4; ++grp) {
+                const f32x4 l4 = lds_read16<f32x4>(row_at + 32u * grp);
 #pragma unroll
-            for (int x = 0; x < 4; ++x) s[4 * grp + x] = __builtin_amdgcn_exp2f(fmaf(s[4 * grp + x], c2, SCALED ? -l4[x] : l4[x] * -LOG2E));
+                for (int x = 0; x < 4; ++x) s[4 * grp + x] = __builtin_amdgcn_exp2f(fmaf(s[4 * grp + x], c2, SCALED ? -l4[x] : l4[x] * -LOG2E));
+            }
         }
         if (DENSE) {
             if (cls == 1 && col_bits_on) {
@@ -491,9 +496,8 @@
             }
         }
         u32x4 pb[2], dsb[2];
-        if constexpr (BESIDE2)
         // ---- dV^T += dO^T P ; dK^T += Q^T dS -------------------------------------------------
-        {
+        if constexpr (BESIDE) {
             const unsigned at = transposed_lane + tile_at;
             // MFMA j: 16 rows (j / 2 DB), dV then dK, block of columns j % DB
             constexpr int N2 = 4 * DB, AHEAD2 = 2;
@@ -529,17 +533,14 @@
                     for (int w = 4 * (j % DB) / DB; w < 4 * (j % DB + 1) / DB; ++w) grad(j / DB, w);
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        else {
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dp[i] = s[i] * dp[i];  // -dS / scale
+            for (int i = 0; i < 16; ++i) dp[i] = s[i] * dp[i];  // -dS / scale
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            pb[t] = pack8<T>(s, 8 * t);
-            dsb[t] = pack8<T>(dp, 8 * t);
-        }
-        // ---- dV^T += dO^T P ; dK^T += Q^T dS -------------------------------------------------
-        {
+            for (int t = 0; t < 2; ++t) {
+                pb[t] = pack8<T>(s, 8 * t);
+                dsb[t] = pack8<T>(dp, 8 * t);
+            }
             const unsigned at = transposed_lane + tile_at;
             u32x4 tg[2][DB], tq[2][DB];
 #pragma unroll
@@ -558,7 +559,6 @@
                     dk[db] = T::mfma(tq[t][db], dsb[t], dk[db]);
                 }
             sched_pipeline_mfma_lds<4 * DB, 4, 2>();
-        }
         }
         if (SAVE) {
             // Issued after the MFMAs of the tile (in front of them they cost the kernel 2 % more).  Record number and
