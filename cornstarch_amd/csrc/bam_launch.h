@@ -211,17 +211,6 @@ int launch_bwd_both(const AttnParams& kv, const AttnParams& p, int dtype, hipStr
 // dk, dv of p from the parts that a dK/dV launch with kv_parts left at `parts_dk` and `parts_dv` (contiguous).
 int launch_sum_parts(const AttnParams& p, const float* parts_dk, const float* parts_dv, int parts, int dtype, hipStream_t stream);
 int launch_decode(const DecodeParams& p, const DecodeSplit& s, int dtype, hipStream_t stream);
-// Whether the dS records of a call, and what dK/dV and dQ read and write beside them, stay in the last-level cache (256 MB) from one
-// kernel to the other.  They are then stored and read without the non-temporal hint, with which they go to memory and back.  Step, us,
-// with the hint -> without (MB of records, of q, dout and dq), D 128: 1 x 1500 tokens, 32 / 8 heads (75, 35) 133.3 -> 131.1, 2048 (136, 48) 184.6
-// -> 180.9, 4 x 700 (72, 66) 146.5 -> 143.8, 3001, 16 / 4 (144, 35) 206.1 -> 203.4;  D 96: 2 x 2003, 16 heads (132, 35) 158.8 -> 157.1.  Beyond the
-// line it is 2300, 32 / 8 (171, 54) 234.0 -> 235.5, 4 x 1024 (144, 96) 212.9 -> 208.4, D 96 2 x 2400 (185, 42) 207.2 -> 199.5, but 8 x 700
-// (144, 131) 213.1 -> 221.2, 3 x 1537 (244, 108) 299.8 -> 308.6, D 96 2 x 2800 (253, 49) 253.3 -> 265.9.  A look at it in the loop of dK/dV
-// costs what it gives: an instantiation, not for a bias or sorted rows (of 32768 tokens and more).  The results are the same.
-inline bool ds_stays_near(const AttnParams& p) {
-    constexpr int64_t NEAR_BYTES = 208ll << 20;
-    return p.rows == nullptr && p.bias == nullptr && (int64_t)p.Hq * p.ds_capacity * 8192 + 6ll * p.B * p.Sq * p.Hq * p.d <= NEAR_BYTES;
-}
 // dK/dV that also stores dS (p.ds_ws), and the dQ kernel that consumes it; D = 128, plan required
 int launch_bwd_dkdv_save(const AttnParams& p, int dtype, hipStream_t stream);
 int launch_bwd_dq_saved(const AttnParams& p, int dtype, hipStream_t stream);

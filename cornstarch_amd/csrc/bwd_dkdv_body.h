@@ -565,20 +565,13 @@
             // record address are wave-uniform (kept in scalar registers); the two 16-byte stores are inline asm so that
             // they take the scalar-base form and stay out of the compiler's load / store bookkeeping, like the tile
             // copies (the caller waits with explicit counts); non-temporal: the blocks are read once, by another
-            // kernel, and should not push the Q / dO rows the other workgroups re-read out of L2 (NEAR: few blocks, which
-            // that kernel finds in the last-level cache)
+            // kernel, and should not push the Q / dO rows the other workgroups re-read out of L2
             const unsigned rec_no = (unsigned)__builtin_amdgcn_readfirstlane(h_cur * (int)p.ds_capacity + ds_e);
             const char* rec = (const char*)p.ds_ws + ((uint64_t)rec_no << 13);
-            if constexpr (NEAR)
-                asm volatile("global_store_dwordx4 %0, %2, %4\n\tglobal_store_dwordx4 %1, %3, %4"
-                             :
-                             : "v"(ds_first), "v"(ds_second), "v"(dsb[0]), "v"(dsb[1]), "s"(rec)
-                             : "memory");
-            else
-                asm volatile("global_store_dwordx4 %0, %2, %4 nt\n\tglobal_store_dwordx4 %1, %3, %4 nt"
-                             :
-                             : "v"(ds_first), "v"(ds_second), "v"(dsb[0]), "v"(dsb[1]), "s"(rec)
-                             : "memory");
+            asm volatile("global_store_dwordx4 %0, %2, %4 nt\n\tglobal_store_dwordx4 %1, %3, %4 nt"
+                         :
+                         : "v"(ds_first), "v"(ds_second), "v"(dsb[0]), "v"(dsb[1]), "s"(rec)
+                         : "memory");
         }
         return SAVE;
     };

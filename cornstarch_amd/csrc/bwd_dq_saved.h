@@ -50,7 +50,7 @@ __device__ __forceinline__ void build_key_half_list(const WaveSlices& ws, int nu
     wait_lds();
 }
 
-template <typename T, int D, bool NEAR>
+template <typename T, int D>
 __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const AttnParams p) {
     constexpr int NCH = LDS_COLS<D> / 8, DB = D / 32;
     __shared__ u32x4 sK[2][DQS_KT * NCH];
@@ -129,12 +129,6 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
 #pragma unroll
         for (int j = 0; j < CPT; ++j) stK.template issue<0>(j, k_rows.at((entry >> 16) * DQS_KT), ldsK + buf * TILE_BYTES);
     };
-    auto copy_ds = [](int site, const char* src, unsigned voff, unsigned lds) {
-        if constexpr (NEAR)
-            site == 1 ? dma_b128<1>(src, voff, lds) : dma_b128<2>(src, voff, lds);
-        else
-            site == 1 ? dma_b128_stream<1>(src, voff, lds) : dma_b128_stream<2>(src, voff, lds);
-    };
     // copies of this wave's dS blocks of tile `entry` (record e), the halves that have work, into its buffer buf;
     // returns the number of copy instructions issued (wave-uniform)
     auto issue_ds = [&](int entry, int e, int buf) -> int {
@@ -145,8 +139,8 @@ __global__ __launch_bounds__(DQS_THREADS, 2) void bwd_dq_saved_kernel(const Attn
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
             if ((c >> (2 * kb)) & 3) {
-                copy_ds(1, rec + kb * 2048, (unsigned)(lane * 16), ldsDS + buf * 4096u + kb * 2048u);
-                copy_ds(2, rec + kb * 2048, (unsigned)(lane * 16 + 1024), ldsDS + buf * 4096u + kb * 2048u + 1024u);
+                dma_b128_stream<1>(rec + kb * 2048, (unsigned)(lane * 16), ldsDS + buf * 4096u + kb * 2048u);
+                dma_b128_stream<2>(rec + kb * 2048, (unsigned)(lane * 16 + 1024), ldsDS + buf * 4096u + kb * 2048u + 1024u);
                 issued += 2;
             }
         return issued;

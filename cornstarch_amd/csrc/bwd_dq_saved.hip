@@ -6,10 +6,7 @@ namespace bam {
 template <typename T, int D>
 static int launch_dq_saved_t(const AttnParams& p, hipStream_t stream) {
     const int blocks = p.num_m * p.B * p.Hq;
-    if (ds_stays_near(p))
-        hipLaunchKernelGGL((bwd_dq_saved_kernel<T, D, true>), dim3(blocks), dim3(DQS_THREADS), 0, stream, p);
-    else
-        hipLaunchKernelGGL((bwd_dq_saved_kernel<T, D, false>), dim3(blocks), dim3(DQS_THREADS), 0, stream, p);
+    hipLaunchKernelGGL((bwd_dq_saved_kernel<T, D>), dim3(blocks), dim3(DQS_THREADS), 0, stream, p);
     return (int)hipGetLastError();
 }
 

@@ -88,8 +88,7 @@ constexpr int DKDV_THREADS = 512, DKDV_NARROW_THREADS = 256;
 // LONG: sequences of more than MAX_SLICE_LIST 32-row slices (131072 rows), walked in several passes; the short form has
 // no pass loop at all (a loop around the main loop costs registers and a few per cent).
 // SAVE: every wave also stores its 32 x 32 block of -dS / scale (the packed operand of the dK product) to p.ds_ws, where
-// the dQ kernel of bwd_dq_saved.h picks it up instead of recomputing S and dP.  Record and block layout: AttnParams.  NEAR: without the
-// non-temporal hint (ds_stays_near).
+// the dQ kernel of bwd_dq_saved.h picks it up instead of recomputing S and dP.  Record and block layout: AttnParams.
 // SCALED (head dims up to 64, where the dQ kernel runs first): the rows' lse * log2(e) comes from there (p.lse_scaled), the same
 // numbers with one of some seven vector instructions per MFMA less.  dK/dV alone, us: 8 x 4096 tokens, 16 heads, D 64 581 -> 571
 // (0.6 % of the step), 3001, 32 / 8 heads 103.4 -> 101.5, D 32, 4096 118 -> 112.  (Above D 64 the delta pre-pass would have to write it: 8192 tokens, 32 / 8
@@ -121,7 +120,7 @@ struct DkdvShared {
     int count;
 };
 
-template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false, bool SCALED = false, bool NEAR = false>
+template <typename T, int D, int MODE, bool BIAS, bool LONG, bool SAVE = false, bool SCALED = false>
 __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, SORTED = MODE == MASK_SORTED;
     constexpr bool ROW_POS = IDX || SORTED;  // the rows' positions travel with the tiles
@@ -165,7 +164,7 @@ __global__ __launch_bounds__(DKDV_THREADS, 2) void bwd_dkdv_kernel(const AttnPar
 template <typename T, int D, int MODE, bool BIAS, bool SCALED>
 __global__ __launch_bounds__(DKDV_NARROW_THREADS, 3) void bwd_dkdv_narrow_kernel(const AttnParams p) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = false, SORTED = false, ROW_POS = IDX, LONG = false, SAVE = false;
-    constexpr bool NARROW = true, NEAR = false, KEY_BIAS = false, DEEP = false;
+    constexpr bool NARROW = true, KEY_BIAS = false, DEEP = false;
     constexpr int NB = 2;
     constexpr int NCH = LDS_COLS<D> / 8, KK = D / 16, DB = D / 32;
     constexpr int WAIT = COPY_WAIT<BIAS, LONG>;
@@ -193,7 +192,7 @@ __global__ __launch_bounds__(DKDV_NARROW_THREADS, 3) void bwd_dkdv_narrow_kernel
 template <typename T, int D, int MODE, bool BIAS, bool SCALED>
 __device__ __forceinline__ void dkdv_work(const AttnParams& p, const int block, DkdvShared<D, MODE>& sh) {
     constexpr bool IDX = MODE == MASK_INDEXED, DENSE = MODE == MASK_DENSE, ROW_POS = IDX;
-    constexpr bool NARROW = false, NEAR = false, SORTED = false, LONG = false, SAVE = false;
+    constexpr bool NARROW = false, SORTED = false, LONG = false, SAVE = false;
     constexpr bool KEY_BIAS = BIAS;  // (both_in_one_launch refuses a bias with rows of its own)
     constexpr bool DEEP = DKDV_DEEP<D, MODE, LONG>;
     constexpr int NB = DEEP ? 4 : 2;  // tile buffers
@@ -773,17 +772,6 @@ static int launch_dkdv_m(const AttnParams& p, hipStream_t stream) {
                 hipLaunchKernelGGL((bwd_dkdv_narrow_kernel<T, D, MASK_INDEXED, BIAS, SCALED>), dim3(blocks), dim3(DKDV_NARROW_THREADS), 0, stream, p);
             else
                 hipLaunchKernelGGL((bwd_dkdv_narrow_kernel<T, D, MASK_BITFIELD, BIAS, SCALED>), dim3(blocks), dim3(DKDV_NARROW_THREADS), 0, stream, p);
-            return (int)hipGetLastError();
-        }
-    }
-    if constexpr (SAVE && !BIAS && !LONG) {
-        if (ds_stays_near(p)) {
-            if (p.mask_mode == MASK_INDEXED)
-                hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_INDEXED, BIAS, LONG, SAVE, SCALED, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-            else if (p.mask_mode == MASK_DENSE)
-                hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_DENSE, BIAS, LONG, SAVE, SCALED, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
-            else
-                hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, MASK_BITFIELD, BIAS, LONG, SAVE, SCALED, true>), dim3(blocks), dim3(DKDV_THREADS), 0, stream, p);
             return (int)hipGetLastError();
         }
     }

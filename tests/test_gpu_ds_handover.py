@@ -334,49 +334,3 @@ def test_runs_of_heads_below_the_limit_when_the_workspace_is_large(monkeypatch):
     monkeypatch.setattr(BA, "_DS_RUN_MIN_WORKGROUPS", 8 * key_tiles + 1)  # no run is large enough: not split
     assert plan.ds_head_runs(B, Hq, Hkv, 128, S) == 1
     BA.BitfieldUtils.clear_cache()
-
-
-# Few records are stored and read without the non-temporal hint (ds_stays_near): the same call with its records so far apart that the
-# sizes say otherwise has the same bits.  Sizes: one slice, remainders of slices and key tiles, grouped heads; head dims that are padded,
-# whose launches are Python's.
-@pytest.mark.parametrize("B,S,Hq,Hkv,D,dtype", [(2, 29, 2, 1, 125, torch.float16), (1, 419, 4, 2, 70, torch.bfloat16), (2, 640, 6, 3, 90, torch.float16),
-                                                (1, 701, 8, 2, 101, torch.bfloat16)])
-@pytest.mark.parametrize("form", ["bitfield", "index", "mask"])
-def test_records_near_and_far(form, B, S, Hq, Hkv, D, dtype, monkeypatch):
-    d = dev()
-    bf = random_bitfield(B, S, seed=S, pad=3).to(d)
-    q, k, v, do = (t.to(d) for t in inputs(B, S, Hq, Hkv, D, dtype, seed=S))
-    capacities = []
-
-    def attach(far):
-        def fn(self, nheads, head_dim, seqlen_k):
-            capacity = max(self.ds_pairs(), (300 << 20) // (8192 * nheads) if far else 1)
-            ws = torch.empty(nheads * capacity * 8192, dtype=torch.uint8, device=d)
-            self.struct.ds_workspace, self.struct.ds_capacity = ws.data_ptr(), capacity
-            capacities.append(nheads * capacity * 8192)
-            return ws
-        return fn
-
-    results = []
-    for far in (False, True):
-        monkeypatch.setattr(BA._TilePlan, "attach_ds_workspace", attach(far))
-        flags, _ = build(bf)
-        if form == "mask":
-            mask = BA.materialize_bitfield_mask(bf).to(torch.bool).contiguous()
-            o, lse, scale = A._flash_attn_forward(q, k, v, mask=mask)
-            grads = [torch.empty_like(t) for t in (q, k, v)]
-            A._flash_attn_backward(do, q, k, v, o, lse, *grads, mask=mask, softmax_scale=scale)
-        else:
-            idx = (torch.arange(S, device=d),) * 2 if form == "index" else (None, None)
-            o, lse, scale = BA._bitfield_attn_forward(q, k, v, bf, flags, *idx)
-            grads = [torch.zeros_like(t, dtype=torch.float32) for t in (q, k, v)]
-            BA._bitfield_attn_backward(do, q, k, v, o, bf, flags, lse, *grads, *idx, softmax_scale=scale)
-        results.append(grads)
-    torch.cuda.synchronize()
-    assert len(capacities) == 2 and capacities[0] < 208 << 20 < capacities[1]
-    for a, b in zip(*results):
-        assert torch.equal(a, b)
-    for x, y in zip(results[0], O.attention_backward(*(t.cpu() for t in (q, k, v)), bf.cpu(), do.cpu())):
-        assert rel_l2(x.float().cpu(), y) <= GRAD_REL_L2
-    A._MaskPlan.forget()
-    BA.BitfieldUtils.clear_cache()
