@@ -349,11 +349,15 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
         build_key_tile_list<STREAMS>(ws, p.num_n, list_keys, lane, 0, first_classes, sList + stream * (MAX_LIST / 2), sCount + stream, !side);
     QueryBits qb = {};
     float lse2 = INFINITY;
-    // Up to head dim 64 there are registers (119 of 128 and 165 of 168) to start the dP chain from -delta, as dK/dV does: 16 of some 73
-    // vector instructions a block less.  Step, us, D 32: 8 x 2048 tokens, 16 heads 249.0 -> 243.3, 2 x 8192 779 -> 760, 1 x 2048 93.6 -> 92.7.
+    // Up to head dim 64 there are registers (without a bias 119 to 125 and 165 to 168 of 168) to start the dP chain from -delta, as dK/dV does:
+    // 16 of some 73 vector instructions a block less.  Step, us, D 32: 8 x 2048 tokens, 16 heads 249.0 -> 243.3, 2 x 8192 779 -> 760, 1 x 2048 93.6 -> 92.7.
     // D 64, since the LDS addresses are XORed (160 registers before): dQ of 8 x 4096, 16 heads 314 -> 299, with a bias, in one launch with
     // dK/dV, 2 x 2048 89.7 -> 87.3.
-    constexpr bool DELTA_FIRST = D <= 64;
+    // Not at head dim 64 where a bias is read group by group, or where the keys take several passes without a bias in the tiles (whose form may have
+    // 256 registers): no register is left there.  133120 tokens, 2 heads, one segment, with it and without 6839 -> 6478 us (62 spilled registers, 31), with
+    // such a bias 13368 -> 11298 (97, 40); a bias per row, 4 x 2048, 16 heads 187 -> 177 (3, none).  Masks gain in several passes all the same
+    // (7692 us with it and 101 spilled registers, without 7842 and 25), a bias in the tiles too (7273, without 7463; none spilled).
+    constexpr bool DELTA_FIRST = D <= 32 || (D <= 64 && BIAS_FORM != BIAS_READ && !(LONG && BIAS_FORM == BIAS_NONE && MODE != MASK_DENSE));
     f32x16 minus_delta;
     // With o given, this launch also is the delta pre-pass: it runs in front of the dK/dV kernel, has the rows of dO in
     // registers and covers every row once; a launch and a second reading of dO less (2 x 283 tokens: 3.4 us; 8 x 4096
