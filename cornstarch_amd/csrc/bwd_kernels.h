@@ -353,11 +353,13 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
     // 16 of some 73 vector instructions a block less.  Step, us, D 32: 8 x 2048 tokens, 16 heads 249.0 -> 243.3, 2 x 8192 779 -> 760, 1 x 2048 93.6 -> 92.7.
     // D 64, since the LDS addresses are XORed (160 registers before): dQ of 8 x 4096, 16 heads 314 -> 299, with a bias, in one launch with
     // dK/dV, 2 x 2048 89.7 -> 87.3.
-    // Not at head dim 64 where a bias is read group by group, or where the keys take several passes without a bias in the tiles (whose form may have
-    // 256 registers): no register is left there.  133120 tokens, 2 heads, one segment, with it and without 6839 -> 6478 us (62 spilled registers, 31), with
-    // such a bias 13368 -> 11298 (97, 40); a bias per row, 4 x 2048, 16 heads 187 -> 177 (3, none).  Masks gain in several passes all the same
-    // (7692 us with it and 101 spilled registers, without 7842 and 25), a bias in the tiles too (7273, without 7463; none spilled).
-    constexpr bool DELTA_FIRST = D <= 32 || (D <= 64 && BIAS_FORM != BIAS_READ && !(LONG && BIAS_FORM == BIAS_NONE && MODE != MASK_DENSE));
+    // At head dim 64 the 16 (equal) values are written anew for every block where a bias is read group by group, or where the keys take several passes
+    // without a bias in the tiles (whose form may have 256 registers): no register is left there to hold them.  dQ, us, held -> written
+    // anew: 133120 tokens, 2 heads, one segment 6643 -> 6173 (spilled registers 62 -> 31), with such a bias 13368 -> 11088 (97 -> 45); a bias per row, 4 x 2048,
+    // 16 heads 178 either way (3 -> 0).  Masks gain from them in several passes all the same (7564 held, 7842 without any start values), and so
+    // does a bias in the tiles (7208, 7463).  All forms have the same sums.
+    constexpr bool DELTA_FIRST = D <= 64;
+    constexpr bool DELTA_HELD = D <= 32 || (DELTA_FIRST && BIAS_FORM != BIAS_READ && !(LONG && BIAS_FORM == BIAS_NONE && MODE != MASK_DENSE));
     f32x16 minus_delta;
     // With o given, this launch also is the delta pre-pass: it runs in front of the dK/dV kernel, has the rows of dO in
     // registers and covers every row once; a launch and a second reading of dO less (2 x 283 tokens: 3.4 us; 8 x 4096
@@ -376,7 +378,7 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
                 if (p.lse_scaled != nullptr) p.lse_scaled[at] = lse_row * LOG2E;
             }
         }
-        if (DELTA_FIRST)
+        if (DELTA_HELD)
 #pragma unroll
             for (int i = 0; i < 16; ++i) minus_delta[i] = -dlt;
         qb = make_query_bits(qf, qpos);
@@ -516,8 +518,14 @@ __device__ __forceinline__ void dq_work(const AttnParams& p, const int block, Dq
                 for (int j = 0; j < NOP; ++j) {
                     __builtin_amdgcn_sched_barrier(0);
                     if (j + AHEAD < NOP) a[j + AHEAD] = operand(j + AHEAD);
+                    if (DELTA_FIRST && !DELTA_HELD && j == 1) {
+                        float here = -dlt;
+                        asm volatile("" : "+v"(here));
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) dp[i] = here;
+                    }
                     if (j & 1)
-                        dp = T::mfma(a[j], greg[j >> 1], j < 2 ? (DELTA_FIRST ? minus_delta : zero16) : dp);
+                        dp = T::mfma(a[j], greg[j >> 1], j < 2 ? (DELTA_HELD ? minus_delta : DELTA_FIRST ? dp : zero16) : dp);
                     else
                         s = T::mfma(a[j], qreg[j >> 1], j < 2 ? zero16 : s);
                     if (kb == 0 && j < NLOADS) issue_copy(j, kt_next, cur ^ 1);

@@ -34,7 +34,7 @@ def test_dq_spills_no_more_than_it_has_to(tmp_path):
         path.write_bytes(code)
         found += spilled(subprocess.run([f"{LLVM}/llvm-readelf", "--notes", str(path)], capture_output=True, text=True, check=True).stdout)
     assert len(found) == 2 * 3 * 3 * 3  # types, mask modes, bias forms; one stream, two, several passes
-    # several passes over 64-bit row addresses: 33 as compiled, 101 over masks (which gain more by what takes them), 44 with a bias
+    # several passes over 64-bit row addresses: 33 as compiled, 101 over masks (which gain more by what takes them), 48 with a bias
     # that is read group by group
     for mode, bias, passes, count in found:
         assert count <= (0 if not passes or bias == 2 else 48 if bias else 104 if mode == 2 else 36), (mode, bias, passes)
