@@ -10,7 +10,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
@@ -83,16 +82,6 @@ struct BF16 {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                        __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
-    // sixteen 4x4 blocks: lane = column lane & 3 of block lane / 4, four k-slots
-    static __device__ __forceinline__ f32x4 mfma4(const u32x2& a, const u32x2& b, const f32x4& c) {
-        return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
-    }
-    // acc + the two elements of a packed pair
-    static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
-        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), __builtin_bit_cast(bf16x2, ONES), acc, false);
-    }
-    static constexpr unsigned ONES = 0x3F803F80u, LARGE = 0x43804380u;  // two values of 1, of 2^8
     static __device__ __forceinline__ unsigned pack2(float x, float y) {
         typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
         bf16x2 v;
@@ -103,6 +92,11 @@ struct BF16 {
     static __device__ __forceinline__ float to_float(unsigned short raw) {
         return __builtin_bit_cast(float, ((unsigned)raw) << 16);
     }
+    // acc + the two elements of a packed pair
+    static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), __builtin_bit_cast(bf16x2, 0x3F803F80u), acc, false);
+    }
 };
 
 struct F16 {
@@ -110,14 +104,6 @@ struct F16 {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                       __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
     }
-    static __device__ __forceinline__ f32x4 mfma4(const u32x2& a, const u32x2& b, const f32x4& c) {
-        return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
-        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), __builtin_bit_cast(f16x2, ONES), acc, false);
-    }
-    static constexpr unsigned ONES = 0x3C003C00u, LARGE = 0x5C005C00u;
     static __device__ __forceinline__ unsigned pack2(float x, float y) {
         typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
         f16x2 v;
@@ -127,6 +113,10 @@ struct F16 {
     }
     static __device__ __forceinline__ float to_float(unsigned short raw) {
         return (float)__builtin_bit_cast(_Float16, raw);
+    }
+    static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), __builtin_bit_cast(f16x2, 0x3C003C00u), acc, false);
     }
 };
 
@@ -139,35 +129,6 @@ __device__ __forceinline__ u32x4 pack8(const f32x16& c, int base) {
     r[2] = T::pack2(c[base + 4], c[base + 5]);
     r[3] = T::pack2(c[base + 6], c[base + 7]);
     return r;
-}
-
-// Largest of three, for pairs of non-negative 16-bit floats of either type: their bits are ordered alike, and what is a NaN as fp16
-// (from 2^121 on as bf16) or an infinity stays above everything else.
-__device__ __forceinline__ unsigned max3_pairs(unsigned a, unsigned b, unsigned c) {
-    unsigned r;
-    asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
-// Largest of three floats, NaN if one of them is, and the lanes where x is more than `most` or a NaN (the translation units are compiled
-// as if there were none).
-__device__ __forceinline__ float max3_nan(float a, float b, float c) {
-    float r;
-    asm("v_maximum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ unsigned long long lanes_above(float x, float most) {
-    unsigned long long lanes;
-    asm("v_cmp_nle_f32 %0, %1, %2" : "=s"(lanes) : "v"(x), "v"(most));
-    return lanes;
-}
-
-// acc + four values of the lane's own (a pair of words of an operand), in every element of acc, on the matrix cores: ones times them as
-// sixteen products of 4 x 4 blocks, in which a lane's values meet nobody else's.  8 cycles; the packed dot product takes two
-// instructions, and neither runs beside an MFMA (13 cycles each then, 5 alone).
-template <typename T>
-__device__ __forceinline__ f32x4 add_four(unsigned w0, unsigned w1, const f32x4& acc) {
-    return T::mfma4(u32x2{T::ONES, T::ONES}, u32x2{w0, w1}, acc);
 }
 
 // Four consecutive elements key .. key + 3 of one row of an attention bias, as floats.  `row` points at the

@@ -202,7 +202,8 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             copy_b32<WAIT>(bias_rows.at(row), bias_voff, lds_addr(sBias) + buf * 256u);
     };
 
-    // Where this lane reads in buffer 0, as byte addresses: the K operand of k-slice 0 and the transposed V operand of column block 0.  What
+    // Where this lane reads in buffer 0, as byte addresses (forward alone, 24 problems of 512 to 8192 tokens, head dims 64 to 128, 1.01x of indices
+    // computed per read: 512 to 1024 tokens 1.02x, 8192 1.005x): the K operand of k-slice 0 and the transposed V operand of column block 0.  What
     // a k-slice or a block of columns adds is a constant, XORed (the swizzle takes bits 0 to 3 of the row, the tiles start at multiples
     // of 256), rows are in the instruction.
     constexpr unsigned ROW_BYTES = NCH * 16;
@@ -218,131 +219,19 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
         return lds_read_transposed_at((at ^ (64u * db)) + row, (at ^ (64u * db + 16u)) + row + 8u * ROW_BYTES);
     };
 
-    // The ways a tile can take are divergent branches to the compiler: what one of them derives from these for its copies must not be
-    // shared with another, or it arrives in vector registers.
-    auto own_scalars = [](int& kt_next, int& cur) { asm volatile("" : "+s"(kt_next), "+s"(cur)); };
-
-    // Exponentials of one 32-key half, two at a time behind MFMA j of n (from MFMA `first` on), each pair packed one step later.  A wave
-    // overlaps its own vector work with its own MFMAs (an MFMA with the five instructions of a pair: 38 cycles, 33 alone), if
-    // nothing in it needs the matrix cores: with the packed dot product of the row sums in there (49 cycles) it gained nothing.
-    auto exp_slot = [&](f32x16& s, u32x4 (&pb)[2], float off, int j, int n, int first) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (j >= first && i * (n - first) / 8 == j - first) {
-                s[2 * i] = __builtin_amdgcn_exp2f(fmaf(s[2 * i], c2, off));
-                s[2 * i + 1] = __builtin_amdgcn_exp2f(fmaf(s[2 * i + 1], c2, off));
-                if (i > 0) pb[(i - 1) >> 2][(i - 1) & 3] = T::pack2(s[2 * i - 2], s[2 * i - 1]);
-            }
-    };
-    // Scores of a tile that hides nothing, for a wave whose rows all have a running maximum: the two 32-key halves follow one another, and
-    // the exponentials of the first are taken while the matrix cores work on the second.  Nobody looks for the maximum; false: some
-    // probability would be so large that it has to move, and the tile is done the general way (the same numbers).  off: what is added in
-    // the exponent, most: the largest score of the row that needs no look.
-    // Forward alone, nothing hidden, us, before -> here: D 128, 4096 tokens, 8 heads (a workgroup a unit) 88.7 -> 76.8, 64 / 16 heads 521 ->
-    // 500 (there power decides: zeros for inputs -11 % a pair of workgroups, random numbers -2 to -5 %); D 64 61.1 -> 53.8 and 308 -> 294.
-    // Causal: 3072, 32 / 8 heads 89.4 -> 85.6, 1024 25.3 -> 23.3.
-    // Not at head dim 32, which has a third of the MFMAs for the same vector work and four waves a SIMD to fill gaps: 4096 tokens, nothing
-    // hidden, 8 heads 46.2 -> 50.0 us, 64 heads 204 -> 208.  Nor do its row sums go to the matrix cores or behind P V: 4 x 2048 tokens with three
-    // segments, 16 heads 45.1 us, as 4 x 4 MFMAs 47.5, as dot products behind the last MFMA 49 (text only 41.1, 42, 38.4), in front of the
-    // first, as here, 44.3 (40.3).
-    constexpr bool PIPED = !BIAS && !LONG && D > 32, SUM_MFMA = D > 32;
-    bool settled = false;
-    auto full_scores = [&](f32x16 (&s)[2], u32x4 (&pb0)[2], float off, float most, int cur, int kt_next) __attribute__((always_inline)) -> bool {
-        constexpr int AHEAD = KK < 4 ? KK : 4;
-        u32x4 ka[2 * KK];
-        own_scalars(kt_next, cur);
-        const unsigned k_at = k_lane + cur * TILE_BYTES;
-        auto read_k = [&](int j) { ka[j] = k_operand(k_at, j / KK, j % KK); };
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int j = 0; j < AHEAD; ++j) read_k(j);
-#pragma unroll
-        for (int j = 0; j < 2 * KK; ++j) {
-            __builtin_amdgcn_sched_barrier(0);
-            if (j + AHEAD < 2 * KK) read_k(j + AHEAD);
-            s[j / KK] = T::mfma(ka[j], qreg[j % KK], j % KK == 0 ? zero16 : s[j / KK]);
-            if (j < NLOADS) issue_copy(j, kt_next, cur ^ 1);
-            if (j >= KK) exp_slot(s[0], pb0, off, j - KK, KK, 1);
-        }
-#pragma unroll
-        for (int j = 2 * KK; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-        // the first half by its probabilities, the second one by its scores
-        pb0[1][3] = T::pack2(s[0][14], s[0][15]);
-        unsigned largest = max3_pairs(pb0[0][0], pb0[0][1], pb0[0][2]);
-        largest = max3_pairs(largest, pb0[0][3], pb0[1][0]);
-        largest = max3_pairs(largest, pb0[1][1], pb0[1][2]);
-        largest = max3_pairs(largest, pb0[1][3], T::LARGE);
-        // (an asm statement may not read what an MFMA has written for twelve wait states, and the compiler does not look into it)
-        asm volatile("s_nop 12" : "+v"(s[1]));
-        float top[2] = {max3_nan(s[1][0], s[1][1], s[1][2]), max3_nan(s[1][3], s[1][4], s[1][5])};
-#pragma unroll
-        for (int i = 6; i < 14; i += 4) {
-            top[0] = max3_nan(top[0], s[1][i], s[1][i + 1]);
-            top[1] = max3_nan(top[1], s[1][i + 2], s[1][i + 3]);
-        }
-        top[0] = max3_nan(top[0], s[1][14], s[1][15]);
-        return (__ballot(largest != T::LARGE) | lanes_above(max3_nan(top[0], top[1], top[1]), most)) == 0;
-    };
-
     // One 64-key tile held in buffer `cur`.  The copies of tile `kt_next` into the other
     // buffer are issued one per MFMA of the S phase, where the wave has nothing else to wait for.
     auto tile_step = [&](int cur, int entry, int kt_next) {
-        // (One `if` after the other, none around another and none that leaves: the accumulators then stay in their registers.  With a
-        // return for the skipped tile, or classes the compiler takes for divergent, it copied all of O to and fro in every tile.)
+        // (One `if` after the other that the compiler does not take for `else`, and none that leaves: the accumulators then stay in their
+        // registers.  With a return for the skipped tile, or classes it takes for divergent, it copied all of O to and fro in every tile.)
         const int kt = entry >> 8, cls = (entry >> (2 * wave)) & 3;
         if (cls == 0) {  // nothing for this wave's slice in the tile: only keep the copies of the next one going
-            own_scalars(kt_next, cur);
 #pragma unroll
             for (int j = 0; j < NLOADS; ++j) issue_copy(j, kt_next, cur ^ 1);
         }
-        f32x16 s[2];
-        u32x4 pb[2][2];
-        // Partial tiles: the last key a row sees, relative to the first key this lane holds (4 hi) -- what it is compared with are then
-        // compile-time constants, which occupy no registers.  Most are partial only through causality, or because the slice holds rows
-        // of two kinds: all 64 keys carry the same bitfield (and, with index tensors, sit at consecutive positions), the bit test is a
-        // per-query constant and the rule reduces to one position compare.
-        bool uniform = true;
-        int rel = 63;
-        unsigned w01[2] = {0u, 0u};  // DENSE: the mask bits of this lane's row
-        auto classify = [&]() __attribute__((always_inline)) {
-            if (DENSE) {
-                uniform = row_bits_w != nullptr;
-                if (uniform) {
-                    w01[0] = sRowBits[cur][wave][l32];
-                    w01[1] = sRowBits[cur][wave][32 + l32];
-                    rel = (w01[0] & w01[1]) == ~0u ? 63 : (w01[0] | w01[1]) == 0u ? -1 : 0;
-                }
-            } else {
-                const int64_t mine = sKbf[cur][lane];
-                const unsigned mlo = (unsigned)mine, mhi = (unsigned)((uint64_t)mine >> 32);
-                const unsigned flo = __builtin_amdgcn_readfirstlane(mlo), fhi = __builtin_amdgcn_readfirstlane(mhi);
-                bool same = (mlo == flo) & (mhi == fhi);
-                int kt0 = kt * FWD_KT;  // position of the tile's first key
-                if (IDX) {
-                    const int rel0 = sKpos[cur][lane] - lane;
-                    kt0 = __builtin_amdgcn_readfirstlane(rel0);
-                    same &= rel0 == kt0;
-                }
-                uniform = __all(same);
-                rel = allow_bits(qb, flo, fhi) ? qb.lim - kt0 - 4 * hi : -1;
-            }
-        };
-        if (PIPED && cls == 1) classify();
-        // Rows that see all keys of a tile or none go the same way as a tile that hides nothing: what is added in the exponent of the others
-        // is -inf, and a score of theirs that is no number (a key with an infinity) sends the tile the general way.  A slice with text and
-        // modality rows, or with padding, has such tiles all the way back, and its workgroup is often the longest of a launch: 3001 tokens
-        // with two segments, 32 / 8 heads, D 128 83.5 -> 80.0 us, a bool mask over 2 x 4096 with three, 16 heads 133 -> 122.
-        const bool sees = rel >= 59;  // (the last key of a lane: 32 + 24 + 3)
-        float off = nb, most = m_i + rescale_thr;
-        bool piped = PIPED && (cls == 2 ? settled : cls == 1 && uniform && __all((sees & ((m_i != -INFINITY) | !qvalid)) | (rel < 0)));
-        if (PIPED && !sees) {
-            off = -INFINITY;
-            most = 3e38f;
-        }
-        if (piped) piped = full_scores(s, pb[0], off, most, cur, kt_next);
-        if (cls != 0 && !piped) {
-            own_scalars(kt_next, cur);
+        int work = cls;
+        asm volatile("" : "+s"(work));
+        if (work != 0) {
             const unsigned k_at = k_lane + cur * TILE_BYTES;
 
             // ---- S^T = K Q^T : 64 keys x 32 queries per wave ----------------------------------
@@ -350,6 +239,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             // MFMAs in front of their use; the first MFMA of a chain takes C = 0
             // (the MFMA phases run at raised wave priority: when the SIMD's other wave is in its softmax phase, this
             // wave's next MFMA is picked first and the MFMA pipe does not idle behind a queue of VALU instructions)
+            f32x16 s[2];
             u32x4 bias_a[2];  // bias_fold: this lane's key of either 32-key block, as an operand (keys are the rows of S^T)
             if (BIAS && bias_fold) {
 #pragma unroll
@@ -421,12 +311,10 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             }
 
             // ---- bitfield rule in registers (partial tiles only) ------------------------------
-            if (!PIPED && cls == 1) classify();  // (not ahead of the scores, where nobody decides by it)
             if (DENSE) {
                 if (cls == 1 && row_bits_w != nullptr) {
                     // (shifted by this lane's first key, 4 hi, once: the bit numbers tested are then constants)
-                    w01[0] >>= 4 * hi;
-                    w01[1] >>= 4 * hi;
+                    const unsigned w01[2] = {sRowBits[cur][wave][l32] >> (4 * hi), sRowBits[cur][wave][32 + l32] >> (4 * hi)};
 #pragma unroll
                     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -462,7 +350,23 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
                         }
                 }
             } else if (cls == 1) {
-                if (uniform) {
+                // Most partial tiles are partial only through causality: all 64 keys carry the same bitfield (and,
+                // with index tensors, sit at consecutive positions).  Then the bit test is a per-query constant and
+                // the rule reduces to one position compare.
+                const int64_t mine = sKbf[cur][lane];
+                const unsigned mlo = (unsigned)mine, mhi = (unsigned)((uint64_t)mine >> 32);
+                const unsigned flo = __builtin_amdgcn_readfirstlane(mlo), fhi = __builtin_amdgcn_readfirstlane(mhi);
+                bool uniform = (mlo == flo) & (mhi == fhi);
+                int kt0 = kt * FWD_KT;  // position of the tile's first key
+                if (IDX) {
+                    const int rel0 = sKpos[cur][lane] - lane;
+                    kt0 = __builtin_amdgcn_readfirstlane(rel0);
+                    uniform &= rel0 == kt0;
+                }
+                if (__all(uniform)) {
+                    // last allowed key, relative to the first key this lane holds (4 hi): what it is compared with are
+                    // then compile-time constants, which occupy no registers
+                    const int rel = allow_bits(qb, flo, fhi) ? qb.lim - kt0 - 4 * hi : -1;
 #pragma unroll
                     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -494,6 +398,10 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             }
 
             // ---- online softmax (per-lane scalars) ----------------------------------------------
+            // (The maximum is looked at before any exponential.  Exponentials of one 32-key half beside the MFMAs of the other against the maximum of
+            // the tiles before, and the tile done again where one came out too large, gave 3 % with standard normal q and k where a launch's
+            // second round is half empty (3001 tokens, 32 / 8 heads, D 128), nothing elsewhere, and lost 4 to 19 % with scores of deviation 3
+            // to 8, as trained models have them; with the probabilities scaled afterwards instead it still lost 1 to 7 %.)
             // (four short chains instead of one long one: the wave issues in order and would sit out the latency of
             // every link)
             float mx[4];
@@ -517,56 +425,43 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
                     for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[0][i] = __builtin_amdgcn_exp2f(fmaf(s[0][i], c2, nb));
-#pragma unroll
-            for (int t = 0; t < 2; ++t) pb[0][t] = pack8<T>(s[0], 8 * t);
-            off = nb;
-            if (PIPED) settled = __all(!qvalid | (m_i != -INFINITY));
-        }
-
-        // ---- O^T += V^T P^T, and the row sums of the probabilities as that product sees them (rounded to T) ------------------------
-        // (the second half's exponentials are taken while the matrix cores work on the first)
-        if (cls != 0) {
-            if (!SUM_MFMA) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) s[1][i] = __builtin_amdgcn_exp2f(fmaf(s[1][i], c2, off));
-#pragma unroll
-                for (int t = 0; t < 2; ++t) pb[1][t] = pack8<T>(s[1], 8 * t);
-                float sums[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) sums[c] = T::add_pair(pb[c >> 1][c & 1][x], sums[c]);
-                l_i += (sums[0] + sums[1]) + (sums[2] + sums[3]);
+            for (int i = 0; i < 16; ++i) {
+                s[0][i] = __builtin_amdgcn_exp2f(fmaf(s[0][i], c2, nb));
+                s[1][i] = __builtin_amdgcn_exp2f(fmaf(s[1][i], c2, nb));
             }
+            u32x4 pb[2][2];
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) pb[kb][t] = pack8<T>(s[kb], 8 * t);
+            // row sum of the probabilities as the P V product sees them (rounded to T), two per instruction; a tile's are added up by
+            // themselves and meet the running sum once
+            {
+                float ps[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) ps[kb][t] = T::add_pair(pb[kb][t][x], ps[kb][t]);
+                l_i += (ps[0][0] + ps[0][1]) + (ps[1][0] + ps[1][1]);
+            }
+
+            // ---- O^T += V^T P^T -------------------------------------------------------------------
             __builtin_amdgcn_s_setprio(1);
             constexpr int PV = 2 * DB, VAHEAD = 3 < PV ? 3 : PV;
             const unsigned v_at = v_lane + cur * TILE_BYTES;
-            // A tile's probabilities are added up by themselves, 16 keys a chain, and meet the running sum once.  With every product of four added
-            // to it directly, small ones were lost one by one: 131072 keys with probabilities of 2^0 to 2^-12, lse off by 2.4e-5, here by
-            // less than 1.2e-6.  (Times alike.)
-            f32x4 sum[2];  // (all elements alike)
-            float half_sum[2];
             u32x4 va[2 * PV];
             auto read_v = [&](int j) { va[j] = v_operand(v_at, j / PV, j % PV / DB, j % DB); };
 #pragma unroll
             for (int j = 0; j < VAHEAD; ++j) read_v(j);
 #pragma unroll
             for (int j = 0; j < 2 * PV; ++j) {
-                const int kb = j / PV, t = j % PV / DB;
                 __builtin_amdgcn_sched_barrier(0);
                 if (j + VAHEAD < 2 * PV) read_v(j + VAHEAD);
-                o[j % DB] = T::mfma(va[j], pb[kb][t], o[j % DB]);
-#pragma unroll
-                for (int x = 0; x < 2; ++x)
-                    if (SUM_MFMA && j % DB == x * (DB / 2))
-                        sum[t] = add_four<T>(pb[kb][t][2 * x], pb[kb][t][2 * x + 1], x == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[t]);
-                if (SUM_MFMA && (j + 1) % PV == 0) half_sum[kb] = sum[0][0] + sum[1][0];
-                if (SUM_MFMA && kb == 0) exp_slot(s[1], pb[1], off, j, PV, 0);
-                if (SUM_MFMA && j == PV - 1) pb[1][1][3] = T::pack2(s[1][14], s[1][15]);
+                o[j % DB] = T::mfma(va[j], pb[j / PV][j % PV / DB], o[j % DB]);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (SUM_MFMA) l_i += half_sum[0] + half_sum[1];
             __builtin_amdgcn_s_setprio(0);
         }
     };
