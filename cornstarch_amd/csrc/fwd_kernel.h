@@ -311,15 +311,27 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             }
 
             // ---- bitfield rule in registers (partial tiles only) ------------------------------
+            // two_kinds: every row of the slice sees all keys of the tile or none.  The latter's scores stay as they are (they may be NaN), and their
+            // packed probabilities are cleared: 17 instructions for 64.  A slice with text and modality rows, or with padding, has such
+            // tiles all the way back, and its workgroup is often the longest of a launch: 3001 tokens with two segments, 32 / 8
+            // heads, D 128 80.6 -> 78.6 us, 4096 rows of a zigzag shard against 8192 keys 272 -> 263; text only and nothing hidden alike.
+            bool two_kinds = false, sees = true;
             if (DENSE) {
                 if (cls == 1 && row_bits_w != nullptr) {
-                    // (shifted by this lane's first key, 4 hi, once: the bit numbers tested are then constants)
-                    const unsigned w01[2] = {sRowBits[cur][wave][l32] >> (4 * hi), sRowBits[cur][wave][32 + l32] >> (4 * hi)};
+                    unsigned w01[2] = {sRowBits[cur][wave][l32], sRowBits[cur][wave][32 + l32]};
+                    sees = (w01[0] & w01[1]) == ~0u;
+                    two_kinds = __all(sees | ((w01[0] | w01[1]) == 0u));
+                    if (!two_kinds) {
+                        sees = true;
+                        // (shifted by this lane's first key, 4 hi, once: the bit numbers tested are then constants)
+                        w01[0] >>= 4 * hi;
+                        w01[1] >>= 4 * hi;
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
+                        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                        for (int i = 0; i < 16; ++i)
-                            s[kb][i] = ((w01[kb] >> (8 * (i >> 2) + (i & 3))) & 1u) ? s[kb][i] : -INFINITY;
+                            for (int i = 0; i < 16; ++i)
+                                s[kb][i] = ((w01[kb] >> (8 * (i >> 2) + (i & 3))) & 1u) ? s[kb][i] : -INFINITY;
+                    }
                 } else if (cls == 1) {
                     // mask bytes of this lane's query row: 4 consecutive keys per C-fragment group
                     const int kt0 = kt * FWD_KT;
@@ -367,11 +379,16 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
                     // last allowed key, relative to the first key this lane holds (4 hi): what it is compared with are
                     // then compile-time constants, which occupy no registers
                     const int rel = allow_bits(qb, flo, fhi) ? qb.lim - kt0 - 4 * hi : -1;
+                    sees = rel >= 59;  // (the last key of a lane: 32 + 24 + 3)
+                    two_kinds = __all(sees | (rel < 0));
+                    if (!two_kinds) {
+                        sees = true;
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
+                        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                        for (int i = 0; i < 16; ++i)
-                            s[kb][i] = (32 * kb + 8 * (i >> 2) + (i & 3) <= rel) ? s[kb][i] : -INFINITY;
+                            for (int i = 0; i < 16; ++i)
+                                s[kb][i] = (32 * kb + 8 * (i >> 2) + (i & 3) <= rel) ? s[kb][i] : -INFINITY;
+                    }
                 } else {
                     // natural positions: the row's limit relative to the first key this lane holds, so that the position
                     // test compares with compile-time constants
@@ -412,6 +429,7 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
                 for (int i = 1; i < 4; ++i) mx[c] = fmaxf(fmaxf(mx[c], s[0][4 * c + i]), s[1][4 * c + i]);
             }
             float mloc = half_swap_max(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
+            mloc = sees ? mloc : -INFINITY;
             if (__any(mloc > m_i + rescale_thr)) {  // wave-uniform; rare after the first tiles
                 const float mnew = fmaxf(m_i, mloc);
                 const float muse = (mnew == -INFINITY) ? 0.f : mnew;
@@ -434,6 +452,13 @@ __global__ __launch_bounds__(FWD_THREADS * STREAMS, D > 64 || STREAMS > 1 ? 2 : 
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                 for (int t = 0; t < 2; ++t) pb[kb][t] = pack8<T>(s[kb], 8 * t);
+            if (__builtin_expect(two_kinds, 0)) {
+                const unsigned keep = sees ? ~0u : 0u;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) pb[kb][t] &= u32x4{keep, keep, keep, keep};
+            }
             // row sum of the probabilities as the P V product sees them (rounded to T), two per instruction; a tile's are added up by
             // themselves and meet the running sum once
             {
